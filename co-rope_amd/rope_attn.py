@@ -235,6 +235,8 @@ class _FusedRopeAttn(torch.autograd.Function):
         # when a gradient will be asked for, the forward keeps its rotated q and k for the backward and the originals
         # are not saved (the reference saves q and k, fused_rope_attn.py:718, and re-rotates them in its backward)
         o, M, fc, fs, rotated = _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, keep_rotated=training)
+        if not training:   # nothing is kept: saving q, k, v here would also copy strided views of a fused projection
+            return o
         ctx.rotated = rotated is not None
         if ctx.rotated:
             ctx.save_for_backward(rotated[0], rotated[1], v, o, M, fc, fs)

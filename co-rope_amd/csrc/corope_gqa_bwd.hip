@@ -162,7 +162,7 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_rowdot_kernel(const uint
 template <int D, int G>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) void corope_bwd_scores_kernel(CoropeBwdParams p, CoropeBwdWs ws, CoropeBwdFreqs fr) {
   constexpr int HALF = D / 2;
-  constexpr int KS = D + 8, WS = kWave + 8, NVR = 2 * G, NDB = D / 32;
+  constexpr int KS = D + 8, WS = kWave + 8, NVR = 2 * G;
   constexpr int NI = 4 * ((2 * G - 1) / 8 + 1);                       // accumulator registers that hold rows < 2G
   __shared__ __attribute__((aligned(16))) uint16_t kt[kWave * KS];    // [key][d]: keys (bf16), rotated in place (fp16)
   __shared__ __attribute__((aligned(16))) uint16_t wts[NVR * WS];     // [virtual row][key] fp16 weights of the keys
@@ -608,99 +608,171 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dq_leader_kernel(CoropeB
   }
 }
 
+// ---------------------------------------------------------------------------------------------------- equal shares
+// The dv and dk kernels sum over query rows into blocks of 128 keys.  Key block kb sees the rows from its first key on, so
+// the blocks of a group differ in work by their number, and a group of 512 rows has four of them: a workgroup per block (or
+// per pair of a long and a short one) left most of the chip idle on short sequences.  Instead the row tiles of a group's
+// blocks, block after block, form one list that `shares` workgroups cut into equal pieces.  A piece that holds all of a block
+// writes the block's result; the others leave fp32 partial sums in a slot of their own, at most one at each end of a piece,
+// and corope_bwd_sum_kernel adds a block's slots in list order.  The cut depends on the sizes alone and not on how many
+// groups a pass handles, so a smaller workspace gives the same bits.
+// Measured: B2 Hq8 Hkv2 N512 D64 dk 414 -> 33 us and dv 55 -> 9 us, plus 7 us each for the sums; B2 Hq32 Hkv8 N4096 D128 dk
+// 4.69 -> 4.05 ms (two workgroups per compute unit, all of equal length, instead of one) and dv 0.67 -> 0.48 ms.
+constexpr int kDkKeys = 128;   // keys per block
+
+template <int ROWS>
+struct CoropeShares {
+  static_assert(kDkKeys % ROWS == 0, "a block starts on a tile");
+  int n_tiles, n_blocks, total;   // row tiles of block 0, key blocks, tiles of a whole group
+  __device__ __host__ explicit CoropeShares(int N) {
+    n_tiles = (N + ROWS - 1) / ROWS;
+    n_blocks = (N + kDkKeys - 1) / kDkKeys;
+    total = first(n_blocks);
+  }
+  __device__ __host__ int first(int kb) const { return kb * n_tiles - kDkKeys / ROWS * (kb * (kb - 1) / 2); }   // tiles before block kb
+  __device__ int begin(int share, int shares) const { return (int)((int64_t)share * total / shares); }
+  __device__ int owner(int tile, int shares) const { return (int)((((int64_t)tile + 1) * shares - 1) / total); }   // begin(owner) <= tile
+  // A piece's partial sums: slot 1 if they start at the block's first tile, slot 0 if an earlier piece started the block.
+  __device__ static int64_t slot(int share, bool starts_block) { return 2 * (int64_t)share + (starts_block ? 1 : 0); }
+};
+
+// Adds the partial sums of the blocks that were cut: out[key][d] = scale * sum over the block's pieces.
+template <int D, int ROWS>
+__global__ __launch_bounds__(256) void corope_bwd_sum_kernel(const float* parts, int64_t group_floats, uint16_t* out, int N, int shares,
+                                                             float scale) {
+  const CoropeShares<ROWS> sh(N);
+  const int kb = blockIdx.x, g = blockIdx.y;
+  const int w0 = sh.owner(sh.first(kb), shares), w1 = sh.owner(sh.first(kb + 1) - 1, shares);
+  if (w0 == w1) return;   // one piece holds all of the block and has written it
+  const float* src = parts + (int64_t)g * group_floats;
+  for (int e = blockIdx.z * 256 + threadIdx.x; e < kDkKeys * D / 4; e += 256 * gridDim.z) {
+    const int j = kb * kDkKeys + e / (D / 4);
+    if (j >= N) break;
+    f32x4 sum = *reinterpret_cast<const f32x4*>(src + sh.slot(w0, true) * (kDkKeys * D) + 4 * e);
+    for (int w = w0 + 1; w <= w1; w += 4) {   // four loads in flight
+      f32x4 x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const f32x4*>(src + sh.slot(min(w + u, w1), false) * (kDkKeys * D) + 4 * e);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (w + u <= w1) sum += x[u];
+    }
+    *reinterpret_cast<u32x2*>(out + ((int64_t)g * N + kb * kDkKeys) * D + 4 * e) =
+        u32x2{pack_elts(sum[0] * scale, sum[1] * scale), pack_elts(sum[2] * scale, sum[3] * scale)};
+  }
+}
+
 // ---------------------------------------------------------------------------------------------------- dv
 // dv_j = sum_{h, i} P^h_ij dO^h_i on the matrix cores: dv^T (d x keys) += dO^T (d x rows) P (rows x keys), 16 rows per
-// step.  One workgroup of 4 waves owns 128 keys (32 per wave) of one group; the 16 dO rows of every head are staged in
-// LDS and read transposed; P comes straight from the workspace (lane = key: 128-byte lines) and is rounded to bf16.
+// step.  A workgroup of 4 waves takes 128 keys at a time (32 per wave) of one group, equal shares of the rows as above; the 16 dO
+// rows of every head are staged in LDS and read transposed; P comes straight from the workspace (lane = key: 128-byte lines) and
+// is rounded to bf16.
+constexpr int kDvRows = 16;
+
 template <int D, int G>
-__global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParams p, CoropeBwdWs ws) {
-  constexpr int TS = D + 16, NDB = D / 32, NT = 4 * kWave, ROWS = 16;
+__global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParams p, CoropeBwdWs ws, float* parts, int64_t group_floats) {
+  constexpr int TS = D + 16, NDB = D / 32, NT = 4 * kWave, ROWS = kDvRows;
   constexpr int UNITS = G * ROWS * (D / 8), PER = (UNITS + NT - 1) / NT;   // 16-byte pieces of a dO tile, per thread
   __shared__ __attribute__((aligned(16))) uint16_t tile[G * ROWS * TS];
-  const int jb = blockIdx.x * 128, g = blockIdx.y;
+  const int g = blockIdx.y;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int r = lane % 32, hf = lane / 32;
   const int N = p.N, b = g / p.Hkv, kvh = g % p.Hkv;
   const int head0 = b * p.Hq + kvh * G;
-  const int jw = jb + 32 * wave, j = jw + r;
-  f32x16 acc[NDB];
-#pragma unroll
-  for (int db = 0; db < NDB; ++db) acc[db] = f32x16{0};
-
-  // Both streams run one step ahead in registers: the workgroup of the first key block walks N / 16 steps one after the
-  // other, and with a step's loads issued only when the step begins its time is N / 16 memory latencies.
-  u32x4 dreg[PER];
-  float pnext[G][8];
-  auto fetch = [&](int i0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = min((int)threadIdx.x + u * NT, UNITS - 1);
-      const int h = e / (ROWS * (D / 8)), rr = (e / (D / 8)) % ROWS, v8 = e % (D / 8);
-      dreg[u] = *reinterpret_cast<const u32x4*>(p.d_o + ((int64_t)(head0 + h) * N + min(i0 + rr, N - 1)) * D + 8 * v8);
-    }
-    const bool wave_on = i0 + ROWS - 1 >= jw && jw < N;   // wave-uniform: some row of the step sees a key of this wave
-    const int64_t row_len = 64 * (i0 / 64 + 1);           // the 16 rows of a step share a row length
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const float* prow = ws.p(head0 + h) + tri_row_start(min(i0, N - 1)) + j;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int i = i0 + 8 * hf + t;
-        pnext[h][t] = (wave_on && i < N && j <= i) ? prow[row_len * (8 * hf + t)] : 0.f;   // nothing outside the triangle is defined
-      }
-    }
-  };
-  if (jb < N) fetch(jb);
+  const CoropeShares<ROWS> sh(N);
+  const int shares = gridDim.x, share = blockIdx.x;
+  int kb = 0;
 #pragma unroll 1
-  for (int i0 = jb; i0 < N; i0 += ROWS) {
-    __syncthreads();   // the previous step's reads of the tile are done
+  for (int t = sh.begin(share, shares), t_end = sh.begin(share + 1, shares); t < t_end;) {
+    while (sh.first(kb + 1) <= t) ++kb;
+    const int b0 = sh.first(kb), b1 = sh.first(kb + 1), seg_end = min(t_end, b1);
+    const int jb = kb * kDkKeys, row_end = min(N, jb + ROWS * (seg_end - b0));
+    const int jw = jb + 32 * wave, j = jw + r;
+    f32x16 acc[NDB];
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = threadIdx.x + u * NT;
-      if (UNITS % NT == 0 || e < UNITS)
-        *reinterpret_cast<u32x4*>(tile + (e / (D / 8)) * TS + 8 * (e % (D / 8))) = dreg[u];   // rows are (head, row) pairs
-    }
-    u32x4 bop[G];
+    for (int db = 0; db < NDB; ++db) acc[db] = f32x16{0};
+
+    // Both streams run one step ahead in registers: the steps of a piece follow one after the other, and with a step's loads
+    // issued only when the step begins its time is that many memory latencies.
+    u32x4 dreg[PER];
+    float pnext[G][8];
+    auto fetch = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int h = 0; h < G; ++h)
-      bop[h] = u32x4{pack_elts(pnext[h][0], pnext[h][1]), pack_elts(pnext[h][2], pnext[h][3]),
-                     pack_elts(pnext[h][4], pnext[h][5]), pack_elts(pnext[h][6], pnext[h][7])};
-    const bool wave_on = i0 + ROWS - 1 >= jw && jw < N;
-    if (i0 + ROWS < N) fetch(i0 + ROWS);
-    __syncthreads();
-    if (wave_on) {
+      for (int u = 0; u < PER; ++u) {
+        const int e = min((int)threadIdx.x + u * NT, UNITS - 1);
+        const int h = e / (ROWS * (D / 8)), rr = (e / (D / 8)) % ROWS, v8 = e % (D / 8);
+        dreg[u] = *reinterpret_cast<const u32x4*>(p.d_o + ((int64_t)(head0 + h) * N + min(i0 + rr, N - 1)) * D + 8 * v8);
+      }
+      const bool wave_on = i0 + ROWS - 1 >= jw && jw < N;   // wave-uniform: some row of the step sees a key of this wave
+      const int64_t row_len = 64 * (i0 / 64 + 1);           // the 16 rows of a step share a row length
+#pragma unroll
+      for (int h = 0; h < G; ++h) {
+        const float* prow = ws.p(head0 + h) + tri_row_start(min(i0, N - 1)) + j;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          const int i = i0 + 8 * hf + x;
+          pnext[h][x] = (wave_on && i < N && j <= i) ? prow[row_len * (8 * hf + x)] : 0.f;   // nothing outside the triangle is defined
+        }
+      }
+    };
+    const int row_begin = jb + ROWS * (t - b0);
+    fetch(row_begin);
+#pragma unroll 1
+    for (int i0 = row_begin; i0 < row_end; i0 += ROWS) {
+      __syncthreads();   // the previous step's reads of the tile are done
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const int e = threadIdx.x + u * NT;
+        if (UNITS % NT == 0 || e < UNITS)
+          *reinterpret_cast<u32x4*>(tile + (e / (D / 8)) * TS + 8 * (e % (D / 8))) = dreg[u];   // rows are (head, row) pairs
+      }
+      u32x4 bop[G];
 #pragma unroll
       for (int h = 0; h < G; ++h)
+        bop[h] = u32x4{pack_elts(pnext[h][0], pnext[h][1]), pack_elts(pnext[h][2], pnext[h][3]),
+                       pack_elts(pnext[h][4], pnext[h][5]), pack_elts(pnext[h][6], pnext[h][7])};
+      const bool wave_on = i0 + ROWS - 1 >= jw && jw < N;
+      if (i0 + ROWS < row_end) fetch(i0 + ROWS);
+      __syncthreads();
+      if (wave_on) {
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
-          acc[db] = mfma32(load_a_trans_natural(tile + h * ROWS * TS, TS, 0, 32 * db), bop[h], acc[db]);
-    }
-  }
-  if (j < N) {
-    uint16_t* op = p.dv + ((int64_t)g * N + j) * D;
+        for (int h = 0; h < G; ++h)
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const u32x2 w = {pack_elts(acc[db][4 * g4], acc[db][4 * g4 + 1]), pack_elts(acc[db][4 * g4 + 2], acc[db][4 * g4 + 3])};
-        *reinterpret_cast<u32x2*>(op + db * 32 + 8 * g4 + 4 * hf) = w;
+          for (int db = 0; db < NDB; ++db)
+            acc[db] = mfma32(load_a_trans_natural(tile + h * ROWS * TS, TS, 0, 32 * db), bop[h], acc[db]);
       }
+    }
+    const bool whole = t == b0 && seg_end == b1;
+    if (j < N) {
+      uint16_t* op = p.dv + ((int64_t)g * N + j) * D;
+      float* pp = parts + (int64_t)g * group_floats + sh.slot(share, t == b0) * (kDkKeys * D) + (j - jb) * D;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const f32x4 x = {acc[db][4 * g4], acc[db][4 * g4 + 1], acc[db][4 * g4 + 2], acc[db][4 * g4 + 3]};
+          if (whole)
+            *reinterpret_cast<u32x2*>(op + db * 32 + 8 * g4 + 4 * hf) = u32x2{pack_elts(x[0], x[1]), pack_elts(x[2], x[3])};
+          else
+            *reinterpret_cast<f32x4*>(pp + db * 32 + 8 * g4 + 4 * hf) = x;
+        }
+    }
+    t = seg_end;
   }
 }
 
 // ---------------------------------------------------------------------------------------------------- dk
-// dk_j = c sum_i [ R(+delta_ij)(sum_h dS^h_ij q^h_i) + W_ij qL_i ].  One workgroup of 4 waves owns 128 keys of one group
-// (32 per wave) and walks the query rows from the block's first key to the end, 8 rows per staged tile.  Per row:
+// dk_j = c sum_i [ R(+delta_ij)(sum_h dS^h_ij q^h_i) + W_ij qL_i ].  A workgroup of 4 waves takes 128 keys of one group at a time
+// (32 per wave) and walks query rows, 8 per staged tile.  Per row:
 //   u = sum_h dS^h q^h for the wave's 32 keys and all D columns: a (32 keys x heads) x (heads x D) product on the
 //       matrix cores - the contraction is only G long, but it takes 2G multiply-adds per (key, pair) off the vector
 //       units; the result lands as lane = column (mod 32), registers = 16 of the wave's keys;
 //   rotation and accumulation on the vector units: lane (c, half) owns pairs c and c + 32 (D = 128) for the 16 keys of
 //       its half: one (sin, cos) and six multiply-adds per (row, key, pair).
-// Work per key block falls linearly with the block index, so a workgroup takes blocks b and (last - b) in turn: every
-// workgroup sees the same number of rows.  Tiles of DELTA, W, DS^h ([row][matrix][key], fp32) and the rows' queries
+// A workgroup takes its share of the group's (block, row tile) list as above.  Tiles of DELTA, W, DS^h ([row][matrix][key], fp32) and the rows' queries
 // ([row][column][head], bf16, heads padded to 8 with zeros: the B operand is then one 16-byte read) go through LDS,
 // fetched into registers one tile ahead.
-constexpr int kDkKeys = 128, kDkRows = 8, kDkWaves = 4;
+constexpr int kDkRows = 8, kDkWaves = 4;
 
 template <int D, int G>
 struct CoropeDkCfg {
@@ -712,7 +784,7 @@ struct CoropeDkCfg {
 
 template <int D, int G>
 __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu(2))) void corope_bwd_dk_kernel(CoropeBwdParams p, CoropeBwdWs ws,
-                                                                       CoropeBwdFreqs fr) {
+                                                                       CoropeBwdFreqs fr, float* parts, int64_t group_floats) {
   using Cfg = CoropeDkCfg<D, G>;
   constexpr int HALF = D / 2, NT = kDkWaves * kWave, MATS = Cfg::kMats, NP = D / 64;
   static_assert(D == 64 || D == 128, "pairs per lane are laid out for these head dims");
@@ -725,7 +797,8 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
   const int col = lane % 32, hf = lane / 32;
   const int N = p.N, b = g / p.Hkv, kvh = g % p.Hkv;
   const int head0 = b * p.Hq + kvh * G;
-  const int n_blocks = (N + kDkKeys - 1) / kDkKeys;
+  const CoropeShares<kDkRows> sh(N);
+  const int shares = gridDim.x, share = blockIdx.x;
   float w_turn[NP > 0 ? NP : 1];
 #pragma unroll
   for (int np = 0; np < (NP > 0 ? NP : 1); ++np) w_turn[np] = fr.turns[min(32 * np + col, HALF - 1)];
@@ -737,11 +810,13 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
   constexpr int kRowItems = kDkRows * G * (D / 8), RI = (kRowItems + NT - 1) / NT;  // 16-byte pieces of q rows
   static_assert(kTileElems % (4 * NT) == 0, "tile elements divide evenly over the threads, four keys at a time");
 
+  int kb = 0;
 #pragma unroll 1
-  for (int phase = 0; phase < 2; ++phase) {
-    const int kb = phase == 0 ? (int)blockIdx.x : n_blocks - 1 - (int)blockIdx.x;
-    if (phase == 1 && kb <= (int)blockIdx.x) break;   // odd number of blocks: the middle one has been done in phase 0
+  for (int t = sh.begin(share, shares), t_end = sh.begin(share + 1, shares); t < t_end;) {
+    while (sh.first(kb + 1) <= t) ++kb;
+    const int b0 = sh.first(kb), b1 = sh.first(kb + 1), seg_end = min(t_end, b1);
     const int jb = kb * kDkKeys, jw = jb + 32 * wave;
+    const int row_begin = jb + kDkRows * (t - b0), row_end = min(N, jb + kDkRows * (seg_end - b0));
 
     f32x4 mv[TI / 4];
     u32x4 qv[RI];
@@ -776,9 +851,9 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
       for (int e = 0; e < 16; ++e) dk1[np][e] = dk2[np][e] = 0.f;
 
-    fetch(jb);
+    fetch(row_begin);
 #pragma unroll 1
-    for (int i0 = jb; i0 < N; i0 += kDkRows) {
+    for (int i0 = row_begin; i0 < row_end; i0 += kDkRows) {
       __syncthreads();   // the previous tile has been consumed
       static_for<TI / 4>([&](auto k_c) __attribute__((always_inline)) {
         constexpr int k = decltype(k_c)::value;
@@ -795,7 +870,7 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
         }
       });
       __syncthreads();
-      if (i0 + kDkRows < N) fetch(i0 + kDkRows);
+      if (i0 + kDkRows < row_end) fetch(i0 + kDkRows);
       const int n_rows = min(kDkRows, N - i0);
 #pragma unroll 1
       for (int r = 0; r < n_rows; ++r) {
@@ -840,18 +915,26 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
         }
       }
     }
+    const bool whole = t == b0 && seg_end == b1;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int j = jw + acc_row(e, hf);
       if (j < N) {
         uint16_t* op = p.dk + ((int64_t)g * N + j) * D;
+        float* pp = parts + (int64_t)g * group_floats + sh.slot(share, t == b0) * (kDkKeys * D) + (j - jb) * D;
 #pragma unroll
         for (int np = 0; np < NP; ++np) {
-          op[32 * np + col] = f_to_elt(dk1[np][e] * p.sm_scale);
-          op[32 * np + col + HALF] = f_to_elt(dk2[np][e] * p.sm_scale);
+          if (whole) {
+            op[32 * np + col] = f_to_elt(dk1[np][e] * p.sm_scale);
+            op[32 * np + col + HALF] = f_to_elt(dk2[np][e] * p.sm_scale);
+          } else {
+            pp[32 * np + col] = dk1[np][e];
+            pp[32 * np + col + HALF] = dk2[np][e];
+          }
         }
       }
     }
+    t = seg_end;
   }
 }
 
@@ -860,8 +943,18 @@ int64_t corope_gqa_bwd_workspace_floats(int B, int Hq, int Hkv, int N, int D) {
   return tri_row_start(N) * (2 * (int64_t)B * Hkv + 3 * (int64_t)B * Hq) + (int64_t)B * Hkv * N * D;
 }
 
+// Workgroups per group of the kernels that cut a group's list into equal shares: as many as give every compute unit its two
+// workgroups once (a second, partly filled round would leave units idle), from 128 groups on, where that is too coarse, four
+// rounds' worth; no more than the tiles, nor than two slots each in the space for the partial sums.
+template <int ROWS>
+static int corope_bwd_shares(int N, int n_groups_total, int64_t slots) {
+  const int places = 2 * device_cu_count();
+  const int64_t want = places / n_groups_total >= 4 ? places / n_groups_total : (4 * places + n_groups_total - 1) / n_groups_total;
+  return (int)std::max<int64_t>(1, std::min({want, slots / 2, (int64_t)CoropeShares<ROWS>(N).total}));
+}
+
 template <int D, int G>
-static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr,
+static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, int n_groups_total,
                                         hipStream_t stream) {
   const dim3 rows(p.N, p.B * p.Hkv);
   const int nt = (p.N + 127) / 128;
@@ -872,28 +965,37 @@ static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBw
   hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G>), rows, dim3(kWave), 0, stream, p, ws, fr);
   hipLaunchKernelGGL(corope_bwd_dq_leader_kernel<D>, dim3((p.N + 127) / 128, p.B * p.Hkv), dim3(4 * kWave), 0, stream, p, ws);
   using Cfg = CoropeDkCfg<D, G>;
-  hipLaunchKernelGGL((corope_bwd_dv_kernel<D, G>), dim3((p.N + 127) / 128, p.B * p.Hkv), dim3(4 * kWave), 0, stream, p, ws);
+  // The dP matrices are not needed any more behind the scores kernel: they hold the partial sums, first of dv, then of dk.
+  const int64_t group_floats = G * ws.NN, slots = group_floats / (kDkKeys * D);
+  const int dv_shares = corope_bwd_shares<kDvRows>(p.N, n_groups_total, slots), dk_shares = corope_bwd_shares<kDkRows>(p.N, n_groups_total, slots);
+  float* parts = ws.dp(0);
+  const int n_groups = p.B * p.Hkv, n_blocks = (p.N + kDkKeys - 1) / kDkKeys;
+  hipLaunchKernelGGL((corope_bwd_dv_kernel<D, G>), dim3(dv_shares, n_groups), dim3(4 * kWave), 0, stream, p, ws, parts, group_floats);
+  if (dv_shares > 1)
+    hipLaunchKernelGGL((corope_bwd_sum_kernel<D, kDvRows>), dim3(n_blocks, n_groups, 8), dim3(256), 0, stream, parts, group_floats, p.dv,
+                       p.N, dv_shares, 1.f);
   auto kern = corope_bwd_dk_kernel<D, G>;
   static std::atomic<uint64_t> lds_ok{0};
   if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
-  const int n_key_blocks = (p.N + kDkKeys - 1) / kDkKeys;
-  hipLaunchKernelGGL(kern, dim3((n_key_blocks + 1) / 2, p.B * p.Hkv), dim3(kDkWaves * kWave), Cfg::kLdsBytes, stream, p, ws,
-                     fr);
+  hipLaunchKernelGGL(kern, dim3(dk_shares, n_groups), dim3(kDkWaves * kWave), Cfg::kLdsBytes, stream, p, ws, fr, parts, group_floats);
+  if (dk_shares > 1)
+    hipLaunchKernelGGL((corope_bwd_sum_kernel<D, kDkRows>), dim3(n_blocks, n_groups, 8), dim3(256), 0, stream, parts, group_floats, p.dk,
+                       p.N, dk_shares, p.sm_scale);
   return hipGetLastError();
 }
 
 template <int D>
-static hipError_t launch_corope_bwd_d(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr,
+static hipError_t launch_corope_bwd_d(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, int n_groups_total,
                                       hipStream_t stream) {
   switch (p.Hq / p.Hkv) {
-    case 1: return launch_corope_bwd_cfg<D, 1>(p, ws, fr, stream);
-    case 2: return launch_corope_bwd_cfg<D, 2>(p, ws, fr, stream);
-    case 3: return launch_corope_bwd_cfg<D, 3>(p, ws, fr, stream);
-    case 4: return launch_corope_bwd_cfg<D, 4>(p, ws, fr, stream);
-    case 5: return launch_corope_bwd_cfg<D, 5>(p, ws, fr, stream);
-    case 6: return launch_corope_bwd_cfg<D, 6>(p, ws, fr, stream);
-    case 7: return launch_corope_bwd_cfg<D, 7>(p, ws, fr, stream);
-    case 8: return launch_corope_bwd_cfg<D, 8>(p, ws, fr, stream);
+    case 1: return launch_corope_bwd_cfg<D, 1>(p, ws, fr, n_groups_total, stream);
+    case 2: return launch_corope_bwd_cfg<D, 2>(p, ws, fr, n_groups_total, stream);
+    case 3: return launch_corope_bwd_cfg<D, 3>(p, ws, fr, n_groups_total, stream);
+    case 4: return launch_corope_bwd_cfg<D, 4>(p, ws, fr, n_groups_total, stream);
+    case 5: return launch_corope_bwd_cfg<D, 5>(p, ws, fr, n_groups_total, stream);
+    case 6: return launch_corope_bwd_cfg<D, 6>(p, ws, fr, n_groups_total, stream);
+    case 7: return launch_corope_bwd_cfg<D, 7>(p, ws, fr, n_groups_total, stream);
+    case 8: return launch_corope_bwd_cfg<D, 8>(p, ws, fr, n_groups_total, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -932,7 +1034,7 @@ hipError_t launch_corope_gqa_bwd(const CoropeBwdParams& p, int D, float* workspa
     c.Hkv = gc;
     c.Hq = gc * G;
     CoropeBwdWs ws{workspace, tri_row_start(p.N), gc, gc * G};
-    const hipError_t e = D == 128 ? launch_corope_bwd_d<128>(c, ws, fr, stream) : launch_corope_bwd_d<64>(c, ws, fr, stream);
+    const hipError_t e = D == 128 ? launch_corope_bwd_d<128>(c, ws, fr, n_groups, stream) : launch_corope_bwd_d<64>(c, ws, fr, n_groups, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

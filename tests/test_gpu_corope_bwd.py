@@ -304,3 +304,12 @@ def test_corope_more_heads_than_a_grid_axis(pkg):
         for a, r in zip(grads, g1):
             assert torch.equal(a[sl], r), b
     mod.release_backward_workspace()
+
+
+# One key block cut among many workgroups, a cut inside and across blocks, a ragged last block, more groups than one round of
+# workgroups, and lengths whose scratch leaves room for few or no partial sums.
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 4, 1, 128, 64), (1, 2, 1, 129, 128), (1, 2, 2, 257, 64), (1, 1, 1, 256, 128), (1, 2, 1, 655, 64)])
+def test_corope_backward_cut_key_blocks(pkg, B, Hq, Hkv, N, D):
+    q, k, v, d_o = _inputs(B, Hq, Hkv, N, D, seed=11)
+    scale = 1 / math.sqrt(D)
+    _compare(_gpu_grads(pkg, q, k, v, d_o, scale, 1e4), _oracle_grads(q, k, v, d_o, scale, 1e4), Hq // Hkv)

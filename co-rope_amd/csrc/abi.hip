@@ -69,6 +69,17 @@ int check_ptrs(const char* what, std::initializer_list<const void*> ptrs) {
   return COROPE_OK;
 }
 
+// (batch, head, row) strides of a view: rows start on 16-byte boundaries and one (batch, head) slice stays below 4 GiB (32-bit
+// offsets inside it)
+int check_strides(const char* what, const int64_t* st, int N, int D) {
+  if (st[2] < D || st[0] < 0 || st[1] < 0 || st[0] % 8 != 0 || st[1] % 8 != 0 || st[2] % 8 != 0)
+    return fail(COROPE_E_BADARG, "%s: strides (%lld, %lld, %lld) must be non-negative multiples of 8 elements, rows at least D apart",
+                what, (long long)st[0], (long long)st[1], (long long)st[2]);
+  if ((int64_t)N * st[2] * 2 >= ((int64_t)1 << 32) || st[2] >= ((int64_t)1 << 30))
+    return fail(COROPE_E_UNSUPPORTED, "%s: one (batch, head) slice spans 4 GiB or more at row stride %lld", what, (long long)st[2]);
+  return COROPE_OK;
+}
+
 int launch_status(const char* what, hipError_t e) {
   if (e == hipSuccess) return COROPE_OK;
   return fail(COROPE_E_LAUNCH, "%s: HIP error %d (%s)", what, (int)e, hipGetErrorString(e));
@@ -76,7 +87,7 @@ int launch_status(const char* what, hipError_t e) {
 
 corope::BwdParams make_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                            const float* lse, float* delta, const float* c, const float* s, int64_t fstride, void* dq,
-                           void* dk, void* dv, int B, int H, int N, float sm_scale) {
+                           void* dk, void* dv, int B, int H, int N, int D, float sm_scale, int Hkv = 0) {
   corope::BwdParams p{};
   p.q = static_cast<const uint16_t*>(q);
   p.k = static_cast<const uint16_t*>(k);
@@ -95,7 +106,9 @@ corope::BwdParams make_bwd(const void* q, const void* k, const void* v, const vo
   p.qk_scale = sm_scale * kLog2e;
   p.N = N;
   p.BH = B * H;
-  p.H = p.Hkv = H;
+  p.H = H;
+  p.Hkv = Hkv > 0 ? Hkv : H;
+  p.contiguous(D);
   return p;
 }
 
@@ -335,7 +348,7 @@ int corope_rope_attn_bwd_preprocess(const void* o, const void* d_o, float* delta
   rc = check_ptrs("rope_attn_bwd_preprocess", {o, d_o, delta});
   if (rc) return rc;
   corope::BwdParams p = make_bwd(nullptr, nullptr, nullptr, o, d_o, nullptr, delta, nullptr, nullptr, D, nullptr,
-                                 nullptr, nullptr, B, H, N, 1.f);
+                                 nullptr, nullptr, B, H, N, D, 1.f);
   return launch_status("rope_attn_bwd_preprocess", corope::launch_bwd_preprocess(p, D, static_cast<hipStream_t>(stream)));
 }
 
@@ -370,7 +383,7 @@ int bwd_dv_impl(const char* what, bool prerot, const void* q, const void* k, con
   rc = check_ptrs(what, {q, k, d_o, lse, freqs_cos, freqs_sin, dv});
   if (rc) return rc;
   corope::BwdParams p = make_bwd(q, k, nullptr, nullptr, d_o, lse, nullptr, freqs_cos, freqs_sin, freq_row_stride,
-                                 nullptr, nullptr, dv, B, H, N, sm_scale);
+                                 nullptr, nullptr, dv, B, H, N, D, sm_scale);
   mark_prerotated(p, prerot);
   return launch_status(what, corope::launch_bwd_dv(p, D, causal != 0, static_cast<hipStream_t>(stream)));
 }
@@ -383,7 +396,7 @@ int bwd_dk_impl(const char* what, bool prerot, const void* q, const void* k, con
   rc = check_ptrs(what, {q, k, v, d_o, lse, delta, freqs_cos, freqs_sin, dk});
   if (rc) return rc;
   corope::BwdParams p = make_bwd(q, k, v, nullptr, d_o, lse, const_cast<float*>(delta), freqs_cos, freqs_sin,
-                                 freq_row_stride, nullptr, dk, nullptr, B, H, N, sm_scale);
+                                 freq_row_stride, nullptr, dk, nullptr, B, H, N, D, sm_scale);
   mark_prerotated(p, prerot);
   return launch_status(what, corope::launch_bwd_dk(p, D, causal != 0, static_cast<hipStream_t>(stream)));
 }
@@ -399,7 +412,7 @@ int bwd_dq_impl(const char* what, bool prerot, const void* q, const void* k, con
   if (rc) return rc;
   if (o != nullptr && !aligned16(o)) return fail(COROPE_E_ALIGN, "%s: pointer %p is not 16-byte aligned", what, o);
   corope::BwdParams p = make_bwd(q, k, v, o, d_o, lse, const_cast<float*>(delta), freqs_cos, freqs_sin,
-                                 freq_row_stride, dq, nullptr, nullptr, B, H, N, sm_scale);
+                                 freq_row_stride, dq, nullptr, nullptr, B, H, N, D, sm_scale);
   mark_prerotated(p, prerot);
   return launch_status(what, corope::launch_bwd_dq(p, D, causal != 0, static_cast<hipStream_t>(stream)));
 }
@@ -432,7 +445,7 @@ int corope_rope_attn_bwd_dkdv(const void* q, const void* k, const void* v, const
   if (rc) return rc;
   if (D == 64) {   // both sets of accumulators and the rotation's table values fit a wave's registers: one launch
     corope::BwdParams p = make_bwd(q, k, v, nullptr, d_o, lse, const_cast<float*>(delta), freqs_cos, freqs_sin,
-                                   freq_row_stride, nullptr, dk, dv, B, H, N, sm_scale);
+                                   freq_row_stride, nullptr, dk, dv, B, H, N, D, sm_scale);
     return launch_status("rope_attn_bwd_dkdv", corope::launch_bwd_dkdv_fused(p, D, causal != 0, static_cast<hipStream_t>(stream)));
   }
   rc = corope_rope_attn_bwd_dv(q, k, d_o, lse, freqs_cos, freqs_sin, freq_row_stride, dv, B, H, N, D, sm_scale, causal,
@@ -475,7 +488,7 @@ int corope_rope_attn_bwd_dkdv_prerotated(const void* q_rot, const void* k_rot, c
   rc = check_ptrs(what, {q_rot, k_rot, v, d_o, lse, delta, freqs_cos, freqs_sin, dk, dv});
   if (rc) return rc;
   corope::BwdParams p = make_bwd(q_rot, k_rot, v, nullptr, d_o, lse, const_cast<float*>(delta), freqs_cos, freqs_sin,
-                                 freq_row_stride, nullptr, dk, dv, B, H, N, sm_scale);
+                                 freq_row_stride, nullptr, dk, dv, B, H, N, D, sm_scale);
   mark_prerotated(p, true);
   return launch_status(what, corope::launch_bwd_dkdv_fused(p, D, causal != 0, static_cast<hipStream_t>(stream)));
 }
@@ -545,6 +558,47 @@ int corope_rope_attn_bwd_ws(const void* q, const void* k, const void* v, const v
                                          dv, B, H, N, D, sm_scale, causal, stream);
 }
 
+int64_t corope_rope_attn_bwd_rotated_parts_bytes(int B, int H, int Hkv, int N, int D, int causal) {
+  if (Hkv <= 0 || H % Hkv != 0 || corope_rope_attn_check(B, H, N, D, D, 1.f, 1)) return -1;
+  return corope::bwd_dkdv_parts_bytes(B, H, Hkv, N, D, causal != 0);
+}
+
+int corope_rope_attn_bwd_rotated(const void* q_rot, const void* k_rot, const void* v, const int64_t* v_strides, const void* o,
+                                 const void* d_o, const int64_t* do_strides, const float* lse, float* delta, const float* freqs_cos,
+                                 const float* freqs_sin, int64_t freq_row_stride, void* dq, void* dk, void* dv, int B, int H, int Hkv,
+                                 int N, int D, float sm_scale, int causal, int fp16, void* parts, int64_t parts_bytes, void* stream) {
+  const char* what = "rope_attn_bwd_rotated";
+  if (Hkv <= 0 || H % Hkv != 0) return fail(COROPE_E_BADARG, "%s: H=%d is not a multiple of Hkv=%d", what, H, Hkv);
+  int rc = validate_bwd(what, B, H, N, D, freq_row_stride, sm_scale,
+                        {q_rot, k_rot, v, o, d_o, lse, delta, freqs_cos, freqs_sin, dq, dk, dv});
+  if (rc) return rc;
+  corope::BwdParams p = make_bwd(q_rot, k_rot, v, o, d_o, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dq, dk, dv, B, H, N, D,
+                                 sm_scale, Hkv);
+  mark_prerotated(p, true);
+  if (D == 256 && (v_strides != nullptr || do_strides != nullptr)) return fail(COROPE_E_UNSUPPORTED, "%s: strided v or d_o at head dim 256", what);
+  if (v_strides != nullptr) {
+    if ((rc = check_strides(what, v_strides, N, D))) return rc;
+    p.v_sb = v_strides[0], p.v_sh = v_strides[1], p.v_sn = (int)v_strides[2];
+  }
+  if (do_strides != nullptr) {
+    if ((rc = check_strides(what, do_strides, N, D))) return rc;
+    p.do_sb = do_strides[0], p.do_sh = do_strides[1], p.do_sn = (int)do_strides[2];
+  }
+  if (parts != nullptr) {
+    if ((rc = check_ptrs(what, {parts}))) return rc;
+    const int64_t need = corope::bwd_dkdv_parts_bytes(B, H, Hkv, N, D, causal != 0);
+    if (parts_bytes < need)
+      return fail(COROPE_E_BADARG, "%s: parts of %lld bytes, %lld needed", what, (long long)parts_bytes, (long long)need);
+    p.parts = static_cast<float*>(parts);
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  // the dQ kernel computes delta for the rows it owns, the dK+dV kernel reads it
+  rc = launch_status(what, fp16 ? corope_f16::launch_bwd_dq(p, D, causal != 0, st) : corope::launch_bwd_dq(p, D, causal != 0, st));
+  if (rc) return rc;
+  return launch_status(what, fp16 ? corope_f16::launch_bwd_dkdv_fused(p, D, causal != 0, st)
+                                  : corope::launch_bwd_dkdv_fused(p, D, causal != 0, st));
+}
+
 int corope_rope_attn_fwd_gqa(const void* q, const void* k, const void* v, const float* freqs_cos, const float* freqs_sin,
                              int64_t freq_row_stride, void* o, float* lse, void* q_rot, void* k_rot, float* tile_kmax, int B,
                              int Hq, int Hkv, int N, int D, float sm_scale, int causal, void* stream) {
@@ -582,8 +636,7 @@ int corope_rope_attn_bwd_gqa(const void* q, const void* k, int prerotated, const
   rc = corope_rope_attn_bwd_preprocess(o, d_o, delta, B, Hq, N, D, stream);
   if (rc) return rc;
   corope::BwdParams p = make_bwd(q, k, v, nullptr, d_o, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dq, dk, dv, B, Hq,
-                                 N, sm_scale);
-  p.Hkv = Hkv;
+                                 N, D, sm_scale, Hkv);
   mark_prerotated(p, prerotated != 0);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (prerotated) {
@@ -650,8 +703,7 @@ int corope_rope_attn_bwd_f16(const void* q, const void* k, int prerotated, const
                         {q, k, v, o, d_o, lse, delta, freqs_cos, freqs_sin, dq, dk, dv});
   if (rc) return rc;
   corope::BwdParams p = make_bwd(q, k, v, o, d_o, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dq, dk, dv, B, H, N,
-                                 sm_scale);
-  p.Hkv = Hkv;
+                                 D, sm_scale, Hkv);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (prerotated) {
     // q, k are the rotated copies a two-launch forward kept: the dQ kernel computes delta on its way, dK and dV come
@@ -702,14 +754,8 @@ int corope_rope_attn_fwd_strided(const void* q, const int64_t* q_strides, const 
   rc = check_ptrs(what, {q, k, v, freqs_cos, freqs_sin, o, lse});
   if (rc) return rc;
   if (q_strides == nullptr || k_strides == nullptr || v_strides == nullptr) return fail(COROPE_E_BADARG, "%s: null strides", what);
-  for (const int64_t* st : {q_strides, k_strides, v_strides}) {
-    // rows start on 16-byte boundaries and one (batch, head) slice stays below 4 GiB (32-bit offsets inside it)
-    if (st[2] < D || st[0] < 0 || st[1] < 0 || st[0] % 8 != 0 || st[1] % 8 != 0 || st[2] % 8 != 0)
-      return fail(COROPE_E_BADARG, "%s: strides (%lld, %lld, %lld) must be non-negative multiples of 8 elements, rows at least D apart",
-                  what, (long long)st[0], (long long)st[1], (long long)st[2]);
-    if ((int64_t)N * st[2] * 2 >= ((int64_t)1 << 32) || st[2] >= ((int64_t)1 << 30))
-      return fail(COROPE_E_UNSUPPORTED, "%s: one (batch, head) slice spans 4 GiB or more at row stride %lld", what, (long long)st[2]);
-  }
+  for (const int64_t* st : {q_strides, k_strides, v_strides})
+    if ((rc = check_strides(what, st, N, D))) return rc;
   if (k_rot == nullptr && q_rot != nullptr) return fail(COROPE_E_BADARG, "%s: q_rot without k_rot", what);
   corope::FwdParams p{};
   p.q = static_cast<const uint16_t*>(q);

@@ -159,6 +159,21 @@ struct BwdParams {
   int BH;          // batch * query heads
   int H, Hkv;      // as in FwdParams; dk, dv have B * Hkv slabs and sum over the query heads of their group
   int num_blocks;  // filled in by the launcher
+  // Layout of v and d_o for the kernels on rotated operands (everything else is contiguous; last dimension contiguous):
+  // elements between batches, heads and rows.  contiguous(D) fills in (B, H, N, D) row-major.
+  int64_t v_sb, v_sh, do_sb, do_sh;
+  int v_sn, do_sn;
+  float* parts;    // partial sums of the dK+dV kernel's cut key blocks (bwd_dkdv_parts_bytes), or null: no block is cut
+  void contiguous(int D) {
+    v_sn = do_sn = D;
+    v_sh = do_sh = (int64_t)N * D;
+    v_sb = (int64_t)Hkv * N * D;
+    do_sb = (int64_t)H * N * D;
+  }
+#if defined(__HIPCC__)
+  __device__ __forceinline__ const uint16_t* v_slab(int kvs) const { return v + (kvs / Hkv) * v_sb + (kvs % Hkv) * v_sh; }
+  __device__ __forceinline__ const uint16_t* do_slab(int bh) const { return d_o + (bh / H) * do_sb + (bh % H) * do_sh; }
+#endif
 };
 
 struct CoropeParams {
@@ -216,6 +231,8 @@ hipError_t launch_bwd_preprocess(const BwdParams& p, int D, hipStream_t stream);
 hipError_t launch_bwd_dv(const BwdParams& p, int D, bool causal, hipStream_t stream);
 hipError_t launch_bwd_dk(const BwdParams& p, int D, bool causal, hipStream_t stream);
 hipError_t launch_bwd_dkdv_fused(const BwdParams& p, int D, bool causal, hipStream_t stream);  // dK and dV in one launch
+// bytes of BwdParams::parts with which launch_bwd_dkdv_fused on rotated operands cuts key blocks; 0: it is faster without
+int64_t bwd_dkdv_parts_bytes(int B, int H, int Hkv, int N, int D, bool causal);
 hipError_t launch_bwd_dq(const BwdParams& p, int D, bool causal, hipStream_t stream);
 hipError_t launch_corope_gqa_fwd(const CoropeParams& p, int D, hipStream_t stream);
 int64_t corope_gqa_bwd_workspace_floats(int B, int Hq, int Hkv, int N, int D);

@@ -13,6 +13,8 @@
 //
 // Operands that must be read "transposed" (contraction along the sequence axis of a row-major tile) use the
 // gfx950 transposing LDS read, so every tile is staged row-major exactly once.
+#include <algorithm>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -59,8 +61,83 @@ struct DkdvCfg {
   static_assert(kLdsBytes <= 160 * 1024, "LDS of a compute unit");
 };
 
+// v and d_o may be strided views (BwdParams) up to D = 128; at D = 256, where the registers for run-time strides cost the dK+dV
+// kernel 10 % (222 -> 245 us at B2 H16 N2048), they are contiguous.
+template <int D>
+__device__ __forceinline__ uint32_t do_row_bytes(const BwdParams& p) { return D > 128 ? D * 2 : (uint32_t)p.do_sn * 2; }
+template <int D>
+__device__ __forceinline__ uint32_t v_row_bytes(const BwdParams& p) { return D > 128 ? D * 2 : (uint32_t)p.v_sn * 2; }
+template <int D>
+__device__ __forceinline__ const uint16_t* v_slab_of(const BwdParams& p, int kvs) {
+  return D > 128 ? p.v + (int64_t)kvs * p.N * D : p.v_slab(kvs);
+}
+
+// What a workgroup of the dK+dV kernel works on.  CUT = false: whole items dealt in rounds (ItemList).  CUT = true: the query
+// tiles of all items, slab after slab, form one list that the workgroups cut into equal pieces, so that few or unequal items
+// (short sequences, few heads, grouped-query attention, where one key block sweeps the query tiles of several heads) still
+// keep every compute unit busy equally long.  A piece that holds all of an item writes its result; others leave fp32
+// accumulators in a slot of their own -- at most one at each end of a piece -- and rope_attn_bwd_dkdv_sum_kernel adds an
+// item's slots in list order.  Both number the items heaviest first: item i is key block i / slabs of slab i % slabs.
+template <bool CUT>
+struct DkdvWork;
+
+template <>
+struct DkdvWork<false> {
+  ItemList items;
+  int total;
+  __device__ __forceinline__ DkdvWork(int num_blocks, int slabs, int, int, int) : total(num_blocks * slabs) {}
+  __device__ __forceinline__ int at(int round) const { return items.at(round); }   // >= total: no such item
+  __device__ __forceinline__ int begin(int) const { return 0; }
+  __device__ __forceinline__ int end(int, int iters) const { return iters; }
+  __device__ __forceinline__ int share() const { return 0; }
+};
+
+struct DkdvTiles {
+  int nb, slabs, group, m_tiles, step, per_slab, total_tiles;
+  // step: query tiles by which a key block sees fewer than the one before it (0 when every key sees every query)
+  __host__ __device__ DkdvTiles(int nb_, int slabs_, int group_, int m_tiles_, int step_)
+      : nb(nb_), slabs(slabs_), group(group_), m_tiles(m_tiles_), step(step_) {
+    per_slab = first(nb);
+    total_tiles = per_slab * slabs;
+  }
+  __host__ __device__ int first(int kb) const { return group * (kb * m_tiles - step * (kb * (kb - 1) / 2)); }   // tiles of a slab before block kb
+  __device__ int start(int item) const { return (item % slabs) * per_slab + first(item / slabs); }
+  __device__ int begin_of_share(int w, int shares) const { return (int)((int64_t)w * total_tiles / shares); }
+  __device__ int share_of(int tile, int shares) const { return (int)((((int64_t)tile + 1) * shares - 1) / total_tiles); }
+};
+
+template <>
+struct DkdvWork<true> {
+  DkdvTiles t;
+  int total, t0, t1, li0, piece;
+  __device__ __forceinline__ DkdvWork(int num_blocks, int slabs, int group, int m_tiles, int step)
+      : t(num_blocks, slabs, group, m_tiles, step), total(num_blocks * slabs) {
+    // workgroup ids go round-robin to the 8 XCDs: neighbouring pieces, which share slabs, stay on one
+    const int n = gridDim.x, id = blockIdx.x;
+    piece = n % 8 == 0 ? (id % 8) * (n / 8) + id / 8 : id;
+    t0 = t.begin_of_share(piece, n);
+    t1 = t.begin_of_share(piece + 1, n);
+    const int slab = t0 / t.per_slab, rem = t0 % t.per_slab;
+    int kb = 0;
+    while (kb + 1 < t.nb && t.first(kb + 1) <= rem) ++kb;
+    li0 = slab * t.nb + kb;
+  }
+  __device__ __forceinline__ int at(int round) const {
+    const int li = li0 + round, slab = li / t.nb, kb = li % t.nb;
+    return li < total && slab * t.per_slab + t.first(kb) < t1 ? kb * t.slabs + slab : total;
+  }
+  __device__ __forceinline__ int begin(int item) const { return max(0, t0 - t.start(item)); }
+  __device__ __forceinline__ int end(int item, int iters) const { return min(iters, t1 - t.start(item)); }
+  __device__ __forceinline__ int share() const { return piece; }
+};
+
+// A slot of partial sums: NWAVES x 32 keys x D of dV, then of dK_r, as the accumulators lie ([32-key block][register quad][lane]).
+template <int D, int NWAVES>
+constexpr int64_t kDkdvSlotFloats = 2ll * NWAVES * 32 * D;
+__device__ __forceinline__ int64_t dkdv_slot(int share, bool starts_item) { return 2 * (int64_t)share + (starts_item ? 1 : 0); }
+
 // PREROT: Q and K come from copies that rope_rotate_kernel rotated beforehand (no table reads in the loop).
-template <int D, int NWAVES, int BLOCK_M, bool CAUSAL, bool DO_DV, bool DO_DK, bool PREROT>
+template <int D, int NWAVES, int BLOCK_M, bool CAUSAL, bool DO_DV, bool DO_DK, bool PREROT, bool CUT = false>
 __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<D>, kWavesPerSimd<D>))) void rope_attn_bwd_dkdv_kernel(BwdParams p) {
   constexpr int DO_PAD = DO_DK ? (DO_DV ? kDkdvBothWaysPad : 8) : 32;
   constexpr int Q_PAD = DO_DK ? kDkdvBothWaysPad : 8;
@@ -83,10 +160,10 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   // An item: a key block of one key/value slab; its workgroup sweeps the query tiles of every query head of the group
   // (one head without grouped-query attention), accumulating dK and dV over all of them.  Heaviest first: causal key
   // blocks see fewer query tiles the later they lie.
-  const ItemList items;
   const int BHkv = p.BH / p.H * p.Hkv, GQ = p.H / p.Hkv;
-  const int total = p.num_blocks * BHkv;   // item i: key block i / BHkv of slab i % BHkv
   const int m_tiles = (N + BLOCK_M - 1) / BLOCK_M;
+  const DkdvWork<CUT> items(p.num_blocks, BHkv, GQ, m_tiles, CAUSAL ? Cfg::kBlockN / BLOCK_M : 0);
+  const int total = items.total;           // item i: key block i / BHkv of slab i % BHkv
   const uint16_t* q_all = PREROT ? p.q_rot : p.q;
 
   // ---- the stream of query tiles: a cursor one tile ahead of the tile being consumed -----------------------------------
@@ -94,15 +171,18 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   qst.out_scale = p.qk_scale;
   CopyStage<D, BLOCK_M, NT, DO_PAD> dst;
   float st_lse = 0.f, st_delta = 0.f;
-  int l_round = 0, l_it = 0, l_iters, l_slab0, l_mt0, l_tph;
+  int l_round = 0, l_it, l_iters, l_slab0, l_mt0, l_tph;
+  const uint16_t* l_do;
   auto load_item = [&](int r) {    // false: no such item
     const int i = items.at(r);
     if (i >= total) return false;
     const int bkv = i % BHkv, n0 = (i / BHkv) * Cfg::kBlockN;
     l_slab0 = (bkv / p.Hkv) * p.H + (bkv % p.Hkv) * GQ;   // first query head of the group
+    if constexpr (D <= 128) l_do = p.do_slab(l_slab0);
     l_mt0 = CAUSAL ? n0 / BLOCK_M : 0;
     l_tph = max(m_tiles - l_mt0, 0);
-    l_iters = GQ * l_tph;
+    l_it = items.begin(i);
+    l_iters = items.end(i, GQ * l_tph);
     return true;
   };
   // iteration it of an item -> query head slab0 + it / tph, query tile mt0 + it % tph
@@ -112,12 +192,11 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
         ++l_it;
       } else if (load_item(l_round + 1)) {
         ++l_round;
-        l_it = 0;
       }   // else: past the last tile of the last item; the same tile is requested again and never used
     }
     const int qs = l_slab0 + l_it / l_tph, m0 = (l_mt0 + l_it % l_tph) * BLOCK_M;
     qst.load(q_all + (int64_t)qs * N * D, p.cos, p.sin, p.fstride, m0, N);
-    dst.load(p.d_o + (int64_t)qs * N * D, m0, N);
+    dst.load(D > 128 ? p.d_o + (int64_t)qs * N * D : l_do + (qs - l_slab0) * p.do_sh, m0, N, do_row_bytes<D>(p));
     if (threadIdx.x < BLOCK_M) {
       int qi = m0 + threadIdx.x;
       // -M and -delta: what the S and dP products start from.  Rows past the end: M = +inf makes P = 0, so they
@@ -159,7 +238,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     const int64_t base = (int64_t)(i % BHkv) * N * D;
     const int row0 = (i / BHkv) * Cfg::kBlockN + rb * 32, l = opaque_lane();
     krows.load((PREROT ? p.k_rot : p.k) + base, p.cos, p.sin, p.fstride, row0, N, l);
-    if constexpr (DO_DK) vrows_regs.load(p.v + base, nullptr, nullptr, 0, row0, N, l);
+    if constexpr (DO_DK) vrows_regs.load(v_slab_of<D>(p, i % BHkv), nullptr, nullptr, 0, row0, N, l, v_row_bytes<D>(p));
   };
   auto take_rows = [&]() __attribute__((always_inline)) {
     const int l = opaque_lane();
@@ -190,6 +269,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     const int64_t base = (int64_t)bkv * N * D;                           // k, v, dk, dv
     const int mt0 = CAUSAL ? n0 / BLOCK_M : 0;
     const int tiles_per_head = max(m_tiles - mt0, 0), n_iter = GQ * tiles_per_head;
+    const int it_begin = items.begin(item), it_end = items.end(item, n_iter);
     const int wk_lo = n0 + rb * 32, wk_hi = wk_lo + 31;
     const int key = wk_lo + lq;
     COROPE_ISTAMP(1);
@@ -213,7 +293,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       if constexpr (DO_DK && !V_LDS) asm volatile("" ::"v"(vb[kc]));
     }
 
-    for (int it = 0; it < n_iter; ++it) {
+    for (int it = it_begin; it < it_end; ++it) {
       const int m0 = (mt0 + it % tiles_per_head) * BLOCK_M;
 #ifdef COROPE_TRACE
       if (it == 1) COROPE_ISTAMP(3);
@@ -326,22 +406,72 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     // first and land while dV leaves (which waits for nothing); behind them (loads return in the order they were issued)
     // the next item's rows, which land while dK leaves.  After the last item its own rows are requested once more and
     // never used: the request is then unconditional, and the registers it fills are free during the tile loop on every path.
-    UnrotateTables<D> tb;
-    if constexpr (DO_DK && PREROT) tb.load(p.cos, p.sin, p.fstride, wk_lo, N, opaque_lane());
-    if constexpr (DO_DV) store_rows_via_wave_tile<D>(dvacc, p.dv + base, wk_lo, N, 1.f, wave_slot, opaque_lane());
     const int next_item = items.at(round + 1);
     const bool has_next = next_item < total;
-    request_rows(has_next ? next_item : item);
-    if constexpr (DO_DK) {
-      if constexpr (!PREROT) tb.load(p.cos, p.sin, p.fstride, wk_lo, N, opaque_lane());
-      // the Q_r operand carried sm_scale * log2(e): ln 2 is what is left of sm_scale
-      store_unrotated_rows_via_wave_tile<D>(dkacc, tb, p.dk + base, wk_lo, N, 0.6931471805599453f, wave_slot, opaque_lane());
+    if (!CUT || (it_begin == 0 && it_end == n_iter)) {   // workgroup-uniform
+      UnrotateTables<D> tb;
+      if constexpr (DO_DK && PREROT) tb.load(p.cos, p.sin, p.fstride, wk_lo, N, opaque_lane());
+      if constexpr (DO_DV) store_rows_via_wave_tile<D>(dvacc, p.dv + base, wk_lo, N, 1.f, wave_slot, opaque_lane());
+      request_rows(has_next ? next_item : item);
+      if constexpr (DO_DK) {
+        if constexpr (!PREROT) tb.load(p.cos, p.sin, p.fstride, wk_lo, N, opaque_lane());
+        // the Q_r operand carried sm_scale * log2(e): ln 2 is what is left of sm_scale
+        store_unrotated_rows_via_wave_tile<D>(dkacc, tb, p.dk + base, wk_lo, N, 0.6931471805599453f, wave_slot, opaque_lane());
+      }
+    } else if constexpr (CUT) {   // a piece of the item: its partial sums
+      float* slot = p.parts + dkdv_slot(items.share(), it_begin == 0) * kDkdvSlotFloats<D, NWAVES> + (int64_t)rb * 32 * D + 4 * opaque_lane();
+#pragma unroll
+      for (int i = 0; i < NDB * 4; ++i) {
+        const int db = i / 4, g = i % 4;
+        *reinterpret_cast<f32x4*>(slot + i * 4 * kWave) = f32x4{dvacc[db][4 * g], dvacc[db][4 * g + 1], dvacc[db][4 * g + 2], dvacc[db][4 * g + 3]};
+        *reinterpret_cast<f32x4*>(slot + NWAVES * 32 * D + i * 4 * kWave) = f32x4{dkacc[db][4 * g], dkacc[db][4 * g + 1], dkacc[db][4 * g + 2], dkacc[db][4 * g + 3]};
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      request_rows(has_next ? next_item : item);
     }
     COROPE_ISTAMP(6);
     if (!has_next) break;
     item = next_item;
     COROPE_ISTAMP(0);
     take_rows();
+  }
+}
+
+// dV and dK of the items that were cut: one wave per 32 keys of an item (blockIdx.x) and output (blockIdx.y: dV, dK) adds the
+// partial accumulators and stores them as the dK+dV kernel would have.
+template <int D, int NWAVES, int BLOCK_M, bool CAUSAL>
+__global__ __launch_bounds__(kWave) void rope_attn_bwd_dkdv_sum_kernel(BwdParams p, int shares) {
+  constexpr int NDB = D / 32, BLOCK_N = NWAVES * 32;
+  __shared__ __attribute__((aligned(16))) uint8_t tile[WaveTile<D>::kBytes];
+  const int N = p.N, slabs = p.BH / p.H * p.Hkv, GQ = p.H / p.Hkv, m_tiles = (N + BLOCK_M - 1) / BLOCK_M;
+  const DkdvTiles t(p.num_blocks, slabs, GQ, m_tiles, CAUSAL ? BLOCK_N / BLOCK_M : 0);
+  const int item = blockIdx.x / NWAVES, rb = blockIdx.x % NWAVES, kb = item / slabs, slab = item % slabs;
+  const int start = t.start(item), w0 = t.share_of(start, shares), w1 = t.share_of(start + t.first(kb + 1) - t.first(kb) - 1, shares);
+  const int row0 = kb * BLOCK_N + rb * 32;
+  if (w0 == w1 || row0 >= N) return;   // one piece holds all of the item and has written it
+  const float* src = p.parts + blockIdx.y * (NWAVES * 32 * D) + (int64_t)rb * 32 * D + 4 * threadIdx.x;
+  f32x16 acc[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) acc[db] = f32x16{0};
+#pragma unroll 1
+  for (int w = w0; w <= w1; ++w) {
+    const float* slot = src + dkdv_slot(w, w == w0) * kDkdvSlotFloats<D, NWAVES>;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(slot + (4 * db + g) * 4 * kWave);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[db][4 * g + e] += x[e];
+      }
+  }
+  const int64_t base = (int64_t)slab * N * D;
+  if (blockIdx.y == 0) {
+    store_rows_via_wave_tile<D>(acc, p.dv + base, row0, N, 1.f, tile);
+  } else {
+    UnrotateTables<D> tb;
+    tb.load(p.cos, p.sin, p.fstride, row0, N);
+    store_unrotated_rows_via_wave_tile<D>(acc, tb, p.dk + base, row0, N, 0.6931471805599453f, tile);
   }
 }
 
@@ -404,7 +534,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     if (i >= total) return false;
     const int64_t kv_base = (int64_t)kv_slab(i % p.BH, p.H, p.Hkv) * N * D;
     l_kg = (PREROT ? p.k_rot : p.k) + kv_base;
-    l_vg = p.v + kv_base;
+    l_vg = v_slab_of<D>(p, kv_slab(i % p.BH, p.H, p.Hkv));
     l_tiles = tiles_of(p.num_blocks - 1 - i / p.BH);
     return true;
   };
@@ -416,7 +546,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       l_tile = 0;
     }   // else: past the last tile of the last item; the same tile is requested again and never used
     kst.load(l_kg, p.cos, p.sin, p.fstride, l_tile * BLOCK_N, N);
-    vst.load(l_vg, l_tile * BLOCK_N, N);
+    vst.load(l_vg, l_tile * BLOCK_N, N, v_row_bytes<D>(p));
   };
   auto k_tile = [&](int buf) { return reinterpret_cast<uint16_t*>(smem + buf * Cfg::kStageBytes); };
   auto v_tile = [&](int buf) { return reinterpret_cast<uint16_t*>(smem + buf * Cfg::kStageBytes + Cfg::kKTileBytes); };
@@ -440,10 +570,11 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     const int64_t base = (int64_t)bh * N * D;
     const int l = opaque_lane();
     qrows.load((PREROT ? p.q_rot : p.q) + base, p.cos, p.sin, p.fstride, row0, N, l);
-    dorows.load(p.d_o + base, nullptr, nullptr, 0, row0, N, l);
+    const uint16_t* dog = D > 128 ? p.d_o + base : p.do_slab(bh);
+    dorows.load(dog, nullptr, nullptr, 0, row0, N, l, do_row_bytes<D>(p));
     // (without O the dO rows are requested twice: the request is then unconditional and the registers it fills are free
     // during the tile loop on every path)
-    orows.load((p.o != nullptr ? p.o : p.d_o) + base, nullptr, nullptr, 0, row0, N, l);
+    orows.load(p.o != nullptr ? p.o + base : dog, nullptr, nullptr, 0, row0, N, l, p.o != nullptr ? (uint32_t)D * 2 : do_row_bytes<D>(p));
     const int q_c = min(row0 + l % 32, N - 1);
     lse_q = p.lse[(int64_t)bh * N + q_c];
     // delta_i = sum_d o_id * do_id (reference _attn_bwd_preprocess, :324-337): read from the preprocess pass, or -- when the
@@ -488,7 +619,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   COROPE_ISTAMP(0);
   load_item(0);
   kst.load(l_kg, p.cos, p.sin, p.fstride, 0, N);
-  vst.load(l_vg, 0, N);
+  vst.load(l_vg, 0, N, v_row_bytes<D>(p));
   request_rows(item);
   take_rows(item);
   kst.store_rows(k_tile(0));
@@ -622,11 +753,17 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
 }
 
 // ===================================================================================== launchers
+template <int D>
+constexpr int kDkdvBlockM = D > 128 ? 32 : 64;   // what fits the LDS beside the waves' own slots
+template <int D>
+constexpr int kDkdvCutWaves = D > 128 ? 4 : 8;
+template <int D, bool DO_DV, bool DO_DK, int NWAVES>
+using DkdvCfgOf = DkdvCfg<D, NWAVES, kDkdvBlockM<D>, DO_DK ? (DO_DV ? kDkdvBothWaysPad : 8) : 32, DO_DK ? kDkdvBothWaysPad : 8>;
+
 template <int D, bool CAUSAL, bool DO_DV, bool DO_DK, bool PREROT, int NWAVES>
 static hipError_t launch_dkdv_waves(BwdParams p, hipStream_t stream) {
-  constexpr int BLOCK_M = D > 128 ? 32 : 64;   // what fits the LDS beside the waves' own slots
-  using Cfg = DkdvCfg<D, NWAVES, BLOCK_M, DO_DK ? (DO_DV ? kDkdvBothWaysPad : 8) : 32, DO_DK ? kDkdvBothWaysPad : 8>;
-  auto kern = rope_attn_bwd_dkdv_kernel<D, NWAVES, BLOCK_M, CAUSAL, DO_DV, DO_DK, PREROT>;
+  using Cfg = DkdvCfgOf<D, DO_DV, DO_DK, NWAVES>;
+  auto kern = rope_attn_bwd_dkdv_kernel<D, NWAVES, kDkdvBlockM<D>, CAUSAL, DO_DV, DO_DK, PREROT>;
   static std::atomic<uint64_t> lds_ok{0};
   if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
   p.num_blocks = (p.N + Cfg::kBlockN - 1) / Cfg::kBlockN;
@@ -638,14 +775,85 @@ static hipError_t launch_dkdv_waves(BwdParams p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <int D, bool DO_DV, bool DO_DK>
+static bool dkdv_small_tiles(int N, int slabs) {
+  return use_small_tiles(N, slabs, DkdvCfgOf<D, DO_DV, DO_DK, 4>::kLdsBytes);
+}
+
+// How many pieces the tiles of the fused dK+dV launch on rotated operands are cut into; 0: whole items.  Whole items take as
+// long as the workgroup that is dealt the most.  Cut, every workgroup has the same number of tiles, and what is added is the
+// partial sums' way through memory (each of the about `shares` + `items` pieces written and read once) and one more launch.
+// The constants are measured ones: microseconds per tile of a full chip (a tile of a 128-key item with four waves on its
+// compute unit takes 0.85 of a 256-key item's; with part of the chip idle the clock is higher and tiles are up to a quarter
+// shorter), 6 TB/s for the partial sums, 10 us for the launch and the longer change of items.  Backward, whole / cut, B Hq Hkv N at
+// D = 128: 1 32 8 3001 676 / 285 us, 4 8 1 1500 633 / 129, 1 8 8 4096 337 / 244, 1 16 16 2048 181 / 150, and on the other side
+// 2 16 16 2048 182 / 188, 2 40 40 1500 196 / 254.
+template <int D>
+static int dkdv_shares(int N, int slabs, int group, bool causal) {
+  constexpr int BM = kDkdvBlockM<D>, CW = kDkdvCutWaves<D>, kMost = 16;
+  if (g_tile_rows.load(std::memory_order_relaxed) != 0) return 0;   // a form was asked for
+  const int m_tiles = (N + BM - 1) / BM, cus = device_cu_count();
+  const bool small = D <= 128 && dkdv_small_tiles<D, true, true>(N, slabs);
+  const int block = small || D > 128 ? 128 : 256, nb = (N + block - 1) / block;
+  const int slots = cus * (small && fits_twice(DkdvCfgOf<D, true, true, 4>::kLdsBytes) ? 2 : 1);
+  const int64_t n_items = (int64_t)nb * slabs;
+  if (n_items > (int64_t)kMost * slots || (int64_t)n_items * group * m_tiles >= (1ll << 30)) return 0;   // many rounds even out
+  // the heaviest item of every round goes to the workgroup that was dealt the lightest of the round before (ItemList)
+  int64_t longest = 0;
+  const int grid = (int)std::min<int64_t>(n_items, slots);
+  for (int w = 0; w < grid; w += 8) {
+    int64_t sum = 0;
+    for (int r = 0; (int64_t)r * grid < n_items; ++r) {
+      const int64_t i = (int64_t)r * grid + ((r & 1) ? grid - 1 - w : w);
+      if (i < n_items) sum += group * (m_tiles - (causal ? (int)(i / slabs) * (block / BM) : 0));
+    }
+    longest = std::max(longest, sum);
+  }
+  const DkdvTiles t((N + CW * 32 - 1) / (CW * 32), slabs, group, m_tiles, causal ? CW * 32 / BM : 0);
+  const int shares = std::max(1, std::min(cus, t.total_tiles / 4));
+  const float tile_us = D == 64 ? 1.7f : 3.3f;
+  const float busy = std::min(1.f, (float)t.total_tiles * (block == CW * 32 ? 1.f : 2.f) / ((float)longest * cus));
+  const float whole = (small ? 0.85f : 1.f) * longest * tile_us * (0.75f + 0.25f * busy);
+  const float moved = (float)(shares + std::min<int64_t>(t.nb * (int64_t)slabs, shares)) * kDkdvSlotFloats<D, CW> * 8;
+  const float cut = t.total_tiles * tile_us / shares + 10.f + moved / 6e6f;
+  return cut < 0.95f * whole ? shares : 0;
+}
+
+int64_t bwd_dkdv_parts_bytes(int B, int H, int Hkv, int N, int D, bool causal) {
+  const int slabs = B * Hkv, group = H / Hkv;
+  if (D == 64) return 8 * dkdv_shares<64>(N, slabs, group, causal) * kDkdvSlotFloats<64, kDkdvCutWaves<64>>;
+  if (D == 128) return 8 * dkdv_shares<128>(N, slabs, group, causal) * kDkdvSlotFloats<128, kDkdvCutWaves<128>>;
+  return 8 * dkdv_shares<256>(N, slabs, group, causal) * kDkdvSlotFloats<256, kDkdvCutWaves<256>>;
+}
+
+template <int D, bool CAUSAL>
+static hipError_t launch_dkdv_cut(BwdParams p, int shares, hipStream_t stream) {
+  constexpr int NWAVES = kDkdvCutWaves<D>, BM = kDkdvBlockM<D>;
+  using Cfg = DkdvCfgOf<D, true, true, NWAVES>;
+  auto kern = rope_attn_bwd_dkdv_kernel<D, NWAVES, BM, CAUSAL, true, true, true, true>;
+  static std::atomic<uint64_t> lds_ok{0};
+  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
+  p.num_blocks = (p.N + Cfg::kBlockN - 1) / Cfg::kBlockN;
+#ifdef COROPE_TRACE
+  p.trace = nullptr;
+#endif
+  hipLaunchKernelGGL(kern, dim3(shares), dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, p);
+  const unsigned blocks = (unsigned)p.num_blocks * (p.BH / p.H * p.Hkv) * NWAVES;
+  hipLaunchKernelGGL((rope_attn_bwd_dkdv_sum_kernel<D, NWAVES, BM, CAUSAL>), dim3(blocks, 2), dim3(kWave), 0, stream, p, shares);
+  return hipGetLastError();
+}
+
 template <int D, bool CAUSAL, bool DO_DV, bool DO_DK, bool PREROT>
 static hipError_t launch_dkdv_cfg(const BwdParams& p, hipStream_t stream) {
+  if constexpr (DO_DV && DO_DK && PREROT)
+    if (p.parts != nullptr)
+      if (const int shares = dkdv_shares<D>(p.N, p.BH / p.H * p.Hkv, p.H / p.Hkv, CAUSAL); shares > 0)
+        return launch_dkdv_cut<D, CAUSAL>(p, shares, stream);
   if constexpr (D > 128) {
     return launch_dkdv_waves<D, CAUSAL, DO_DV, DO_DK, PREROT, 4>(p, stream);   // 4 waves x 512 registers
   } else {
-    using Small = DkdvCfg<D, 4, 64, DO_DK ? (DO_DV ? kDkdvBothWaysPad : 8) : 32, DO_DK ? kDkdvBothWaysPad : 8>;
-    return use_small_tiles(p.N, p.BH / p.H * p.Hkv, Small::kLdsBytes) ? launch_dkdv_waves<D, CAUSAL, DO_DV, DO_DK, PREROT, 4>(p, stream)
-                                                     : launch_dkdv_waves<D, CAUSAL, DO_DV, DO_DK, PREROT, 8>(p, stream);
+    return dkdv_small_tiles<D, DO_DV, DO_DK>(p.N, p.BH / p.H * p.Hkv) ? launch_dkdv_waves<D, CAUSAL, DO_DV, DO_DK, PREROT, 4>(p, stream)
+                                                                      : launch_dkdv_waves<D, CAUSAL, DO_DV, DO_DK, PREROT, 8>(p, stream);
   }
 }
 

@@ -223,6 +223,32 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
     return o, M, fc, fs, rotated
 
 
+def _backward_rotated(lib, q_rot, k_rot, v, o, do, M, fc, fs, sm_scale, causal):
+    """(dq, dk, dv, ...) of the operator from the rotated q and k its forward kept."""
+    B, H, N, D = q_rot.shape
+    Hkv = k_rot.shape[1]
+    v_st = do_st = None
+    if not v.is_contiguous():
+        v_st = _view_strides(v) if D <= 128 else None
+        v = v if v_st is not None else v.contiguous()
+    if not do.is_contiguous():
+        do_st = _view_strides(do) if D <= 128 else None
+        do = do if do_st is not None else do.contiguous()
+    dq, dk, dv = torch.empty_like(q_rot), torch.empty_like(k_rot), torch.empty_like(k_rot)
+    delta = torch.empty_like(M)
+    # scratch in which the dK+dV launch leaves the partial sums of key blocks it cuts among workgroups (0: none are cut)
+    nbytes = lib.corope_rope_attn_bwd_rotated_parts_bytes(B, H, Hkv, N, D, int(causal))
+    parts = torch.empty(nbytes, device=q_rot.device, dtype=torch.uint8) if nbytes > 0 else None
+    with _on_device(q_rot):
+        rc = lib.corope_rope_attn_bwd_rotated(q_rot.data_ptr(), k_rot.data_ptr(), v.data_ptr(), v_st, o.data_ptr(), do.data_ptr(), do_st,
+                                              M.data_ptr(), delta.data_ptr(), fc.data_ptr(), fs.data_ptr(), fc.stride(0), dq.data_ptr(),
+                                              dk.data_ptr(), dv.data_ptr(), B, H, Hkv, N, D, sm_scale, int(causal),
+                                              int(q_rot.dtype == torch.float16), parts.data_ptr() if parts is not None else None, nbytes,
+                                              _stream_ptr(q_rot))
+    _lib.check(rc, "corope_rope_attn_bwd_rotated")
+    return dq, dk, dv, None, None, None, None, None
+
+
 class _FusedRopeAttn(torch.autograd.Function):
 
     @staticmethod
@@ -230,8 +256,6 @@ class _FusedRopeAttn(torch.autograd.Function):
         _check_inputs(q, k, v, freqs_cos, freqs_sin)
         B, H, N, D = q.shape
         training = any(ctx.needs_input_grad[:3])
-        if training:
-            v = v.contiguous()         # the backward kernels read v row-major; q and k they read as the forward left them
         # when a gradient will be asked for, the forward keeps its rotated q and k for the backward and the originals
         # are not saved (the reference saves q and k, fused_rope_attn.py:718, and re-rotates them in its backward)
         o, M, fc, fs, rotated = _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, keep_rotated=training)
@@ -251,34 +275,30 @@ class _FusedRopeAttn(torch.autograd.Function):
     def backward(ctx, do):
         q, k, v, o, M, fc, fs = ctx.saved_tensors
         lib = _lib.load()
-        do = do.contiguous()
         if do.dtype != q.dtype:
             do = do.to(q.dtype)
         B, H, N, D = q.shape
+        if ctx.rotated:   # q, k are the rotated copies the forward kept; v and dO are read where they lie if their layout allows it
+            return _backward_rotated(lib, q, k, v, o, do, M, fc, fs, ctx.sm_scale, ctx.causal)
+        do = do.contiguous()
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         delta = torch.empty_like(M)
         with _on_device(q):
             if q.dtype == torch.float16:
                 ws, nbytes = None, 0
-                if not ctx.rotated and use_rotated_path(N, D, training=True):   # rotate q and k once, then the kernels on the copies
+                if use_rotated_path(N, D, training=True):   # rotate q and k once, then the kernels on the copies
                     nbytes = lib.corope_rope_attn_bwd_workspace_bytes(B, H, N, D)
                     ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-                rc = lib.corope_rope_attn_bwd_f16(q.data_ptr(), k.data_ptr(), int(ctx.rotated), v.data_ptr(), o.data_ptr(), do.data_ptr(),
+                rc = lib.corope_rope_attn_bwd_f16(q.data_ptr(), k.data_ptr(), 0, v.data_ptr(), o.data_ptr(), do.data_ptr(),
                                                   M.data_ptr(), delta.data_ptr(), fc.data_ptr(), fs.data_ptr(), fc.stride(0),
                                                   dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, H, k.shape[1], N, D,
                                                   ctx.sm_scale, int(ctx.causal), ws.data_ptr() if ws is not None else None,
                                                   nbytes, _stream_ptr(q))
             elif k.shape[1] != H:         # grouped-query attention
-                rc = lib.corope_rope_attn_bwd_gqa(q.data_ptr(), k.data_ptr(), int(ctx.rotated), v.data_ptr(), o.data_ptr(),
+                rc = lib.corope_rope_attn_bwd_gqa(q.data_ptr(), k.data_ptr(), 0, v.data_ptr(), o.data_ptr(),
                                                   do.data_ptr(), M.data_ptr(), delta.data_ptr(), fc.data_ptr(), fs.data_ptr(),
                                                   fc.stride(0), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, H,
                                                   k.shape[1], N, D, ctx.sm_scale, int(ctx.causal), _stream_ptr(q))
-            elif ctx.rotated:           # q, k are the rotated copies the forward kept
-                rc = lib.corope_rope_attn_bwd_prerotated(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                                         do.data_ptr(), M.data_ptr(), delta.data_ptr(), fc.data_ptr(),
-                                                         fs.data_ptr(), fc.stride(0), dq.data_ptr(), dk.data_ptr(),
-                                                         dv.data_ptr(), B, H, N, D, ctx.sm_scale, int(ctx.causal),
-                                                         _stream_ptr(q))
             elif use_rotated_path(N, D, training=True):   # rotate q and k once, then run the kernels on the rotated copies
                 nbytes = lib.corope_rope_attn_bwd_workspace_bytes(B, H, N, D)
                 ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)

@@ -283,6 +283,20 @@ int corope_rope_attn_bwd_gqa(const void *q, const void *k, int prerotated, const
                              void *dq, void *dk, void *dv,
                              int B, int Hq, int Hkv, int N, int D, float sm_scale, int causal, void *stream);
 
+/* The whole backward on the rotated copies a two-launch forward kept (q_rot carries sm_scale * log2 e), bf16 or fp16 (fp16 != 0),
+ * with or without grouped-query attention: the dQ kernel, which computes delta = rowsum(O o dO) on its way, then dK and dV in one
+ * launch.  Up to D = 128 v and d_o may be strided views (batch, head and row strides in elements, as
+ * corope_rope_attn_fwd_strided; NULL: contiguous); everything else is contiguous.  parts: scratch for partial sums, with which the dK+dV launch cuts its work into equal
+ * pieces; corope_rope_attn_bwd_rotated_parts_bytes says how much, 0 where whole key blocks fill the chip as well (then, and if
+ * NULL is passed, nothing is cut).  delta: (B,H,N) fp32 scratch.  Replaces _attention.backward
+ * (fused-rope/fused_rope_attn.py:725-777; group sum: assets/flashattn-gqa/triton_gqa.py:605-666). */
+int64_t corope_rope_attn_bwd_rotated_parts_bytes(int B, int H, int Hkv, int N, int D, int causal);
+int corope_rope_attn_bwd_rotated(const void *q_rot, const void *k_rot, const void *v, const int64_t *v_strides, const void *o,
+                                 const void *d_o, const int64_t *do_strides, const float *lse, float *delta,
+                                 const float *freqs_cos, const float *freqs_sin, int64_t freq_row_stride,
+                                 void *dq, void *dk, void *dv, int B, int H, int Hkv, int N, int D, float sm_scale, int causal,
+                                 int fp16, void *parts, int64_t parts_bytes, void *stream);
+
 /* Co-RoPE grouped-query attention forward (causal only).
  * q: (B,Hq,N,D), k/v: (B,Hkv,N,D), o: (B,Hq,N,D), group size Hq/Hkv in [1, 8].
  * Replaces the launch of _corope_fwd_backbone in _attention.forward

@@ -415,3 +415,33 @@ def test_seeded_sweep_over_shapes_and_paths(pkg, monkeypatch):
             print(f"  {name}: max-abs {err.max():.3e} mean-abs {err.mean():.3e} (|ref| max {b.abs().max():.2f})")
             assert a.shape == b.shape and torch.isfinite(a).all(), (it, name)
             assert within_bar(a, b, 1.5 * TOL * (math.sqrt(G) if name in ("dK", "dV") else 1.0))[0], (it, name)
+
+
+# Shapes whose dK+dV launch cuts key blocks into pieces (and, last, one that does not): cuts inside and across blocks and heads of
+# a group, a ragged last block, a last piece of one tile, every head dim, v and dO as strided views.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,cut", [(1, 8, 1, 700, 128, True), (1, 8, 2, 1100, 64, True), (1, 4, 1, 300, 256, True),
+                                              (2, 2, 2, 2049, 128, True), (1, 8, 8, 600, 128, False)])
+def test_backward_cut_key_blocks(pkg, B, Hq, Hkv, N, D, cut, causal, dtype):
+    dev = torch.device("cuda:0")
+    assert (pkg._lib.load().corope_rope_attn_bwd_rotated_parts_bytes(B, Hq, Hkv, N, D, int(causal)) > 0) == cut
+    G, scale = Hq // Hkv, 1 / math.sqrt(D)
+    q, g = (bf16_round(seeded((B, N, Hq, D), 30 + i)).transpose(1, 2) for i in range(2))
+    k, v = (bf16_round(seeded((B, N, Hkv, D), 40 + i)).transpose(1, 2) for i in range(2))
+    c, s = O.precompute_freqs_cis(D, N)
+    qd, kd, vd = (t.to(dev, dtype).requires_grad_(True) for t in (q, k, v))
+    assert Hkv == 1 or not vd.is_contiguous()
+    o = pkg.attention(qd, kd, vd, causal, scale, c.to(dev), s.to(dev))
+    grads = torch.autograd.grad(o, (qd, kd, vd), g.to(dev, dtype))
+    torch.cuda.synchronize()
+    kx, vx = k.repeat_interleave(G, dim=1), v.repeat_interleave(G, dim=1)
+    ref = O.rope_attn_fwd_bwd_blocked(q.contiguous(), kx, vx, g.contiguous(), causal, scale, c, s)
+    rdq, rdk, rdv = ref[2], *(t.reshape(B, Hkv, G, N, D).sum(2) for t in ref[3:5])
+    for name, a, b in (("dQ", grads[0], rdq), ("dK", grads[1], rdk), ("dV", grads[2], rdv)):
+        # dK and dV sum G heads' contributions before the one rounding.  On gradients of magnitude 2 to 4 that rounding alone is up
+        # to 7.8e-3 (half a bf16 step), on top of the errors of P and dS rounded to 8 bits that the bar of 2e-2 is met with at
+        # magnitude 1 to 2, where it is half as large: 2.4e-2.
+        ok, err = within_bar(a.float().cpu(), b, 2.4e-2 * (math.sqrt(G) if name != "dQ" else 1.0))[:2]
+        print(f"  {name}: max-abs {err:.3e} (|ref| max {b.abs().max():.2f})", flush=True)
+        assert ok, name

@@ -772,6 +772,19 @@ __device__ __forceinline__ u32x4 load_a_trans16(const uint16_t* tile, int stride
   return u32x4{a[0], a[1], b[0], b[1]};
 }
 
+// The same for contraction slots in the order in which two 16x16 accumulator blocks hand out their rows: slots j of lane group
+// l / 16 <-> k = kbase + 16*(j / 4) + 4*(l / 16) + j % 4.
+__device__ __forceinline__ u32x4 load_a_trans16_acc(const uint16_t* tile, int stride, int kbase, int m0) {
+  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+  const int l = threadIdx.x % kWave;
+  const int g = l / 16, s = l % 16;
+  const uint16_t* p = tile + (kbase + 4 * g + s / 4) * stride + m0 + 4 * (s % 4);
+  s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p));
+  s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + 16 * stride));
+  u32x2 a = __builtin_bit_cast(u32x2, lo), b = __builtin_bit_cast(u32x2, hi);
+  return u32x4{a[0], a[1], b[0], b[1]};
+}
+
 // Natural-order variant of load_a_trans: slot j of lane-half h <-> k = kbase + 8*h + j.
 __device__ __forceinline__ u32x4 load_a_trans_natural(const uint16_t* tile, int stride, int kbase, int m0) {
   typedef __attribute__((address_space(3))) s16x4* lds_ptr;
@@ -815,6 +828,15 @@ __device__ __forceinline__ float row16_sum(float x) {
   x += dpp_move<0x121, 0xf>(0.f, x);   // row_ror:1
   return x;
 }
+// The same within each row of 16 lanes, and the row's last lane's value in every lane of the row.
+__device__ __forceinline__ float row16_prefix_sum(float x) {
+  x += dpp_move<0x111, 0xf>(0.f, x);
+  x += dpp_move<0x112, 0xf>(0.f, x);
+  x += dpp_move<0x114, 0xf>(0.f, x);
+  x += dpp_move<0x118, 0xf>(0.f, x);
+  return x;
+}
+__device__ __forceinline__ float row16_last(float x) { return dpp_move<0x15f, 0xf>(0.f, x); }   // row_newbcast:15
 __device__ __forceinline__ float wave_last(float x) {          // lane 63's value, wave-uniform
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), kWave - 1));
 }
@@ -826,6 +848,14 @@ __device__ __forceinline__ float wave_max(float x) {
   x = fmaxf(x, dpp_move<0x142, 0xa>(-INFINITY, x));
   x = fmaxf(x, dpp_move<0x143, 0xc>(-INFINITY, x));
   return wave_last(x);
+}
+
+// 1 / (1 + e^-x): hardware exponential and reciprocal (one unit in the last place), the latter refined by one Newton step.
+__device__ __forceinline__ float sigmoid(float x) {
+  const float d = 1.f + __expf(-x);
+  if (d == INFINITY) return 0.f;
+  const float y = __builtin_amdgcn_rcpf(d);
+  return __builtin_fmaf(__builtin_fmaf(-d, y, 1.f), y, y);
 }
 
 __device__ __forceinline__ float bf16_to_f(uint16_t x) { return __builtin_bit_cast(float, (uint32_t)x << 16); }

@@ -13,20 +13,28 @@
 // swept right to left and delta accumulates directly: the reference's extra pass over all keys (:103-135) and the
 // cancellation in a[i,i] - a[i,j] disappear (online softmax does not care about chunk order).  (2) The angle is
 // shared by the whole group, so the key is rotated once per (i, j, d) - the only place sines and cosines are evaluated.
-// (3) With the rotated keys parked in LDS, everything that is a dot product with a key row runs on the matrix cores:
-// the leader logits q_leader K^T (bf16 x bf16: exact products), the scores q^h Kt^T (one (G x D) x (D x 64 keys)
-// product per chunk, rows beyond G idle), and O^T += V^T P^T.  The rotated keys are rounded to fp16, not bf16, and the
-// score product runs in fp16 (the bf16 queries convert exactly): 11 significant bits keep the scores as accurate as the
-// bf16 rounding of P afterwards, also at sm_scale = 1 where a bf16 key would cost several percent of a weight.
+// (3) Everything that is a dot product with a key or value row runs on the matrix cores: the leader logits q_leader K^T (bf16 x
+// bf16: exact products), the scores q^h Kt^T and O^T += V^T P^T.  The rotated keys are rounded to fp16, not bf16, and the score
+// product runs in fp16 (the bf16 queries convert exactly): 11 significant bits keep the scores as accurate as the bf16 rounding of P
+// afterwards, also at sm_scale = 1 where a bf16 key would cost several percent of a weight.
 //
-// Mapping: one wave (= one workgroup) per (batch, kv head, query row), longest rows first; lane = key inside a 64-key
-// chunk.  Per chunk: the contiguous 64 x D block of K is fetched with whole cache lines per instruction and parked in
-// the LDS tile -> logits (16x16x32 MFMA, every lane finds its key's logit in its own registers) -> gate, scan over the lanes,
-// delta -> each lane rotates its own key row in place -> scores (32x32x16 MFMA, rows moved back to lane = key with
-// v_permlane32_swap) -> online softmax against a wave-uniform
-// reference value per head (moved to the running maximum only when a score rises well above it) -> the block of V
-// replaces the rotated keys in the tile -> O accumulation (MFMA).  A wave's LDS instructions
-// execute in order, so the kernel needs no barriers; global loads for the next step are issued one step ahead.
+// Mapping: a wave owns R query rows of one (batch, kv head) group; four waves share a workgroup and the K and V tiles of 64 keys
+// it stages in LDS, sweeping from the diagonal to key 0.  Everything is laid out for 16x16x32 MFMAs with the R x G (row, head)
+// pairs as the 16 columns:
+//   logits   A = leaders (row m of A is the leader of query row m R / 16), B = keys: lane (key % 16, row group) finds the logits
+//            of its own rows in its own registers; gates and their suffix sums run along the 16 lanes of a DPP row and then over the
+//            four 16-key blocks in registers; delta crosses the lanes once, through LDS.
+//   rotation lane (key % 16, g) holds columns 8 g .. 8 g + 7 of every 32 of its key, both halves of each rotation pair, exactly as the
+//            A operand of the score product wants them: the rotated keys never leave the registers.  Keys are unpacked once for all R rows.
+//   scores   S^T = Kt Q^T per row: all 16 columns are multiplied, the row's own G are taken over.  The accumulators of the R rows
+//            together are one full tile: lane = (row, head), registers = 16 keys of the chunk, so the softmax has no idle lane and its
+//            row statistics are one register per lane.
+//   O^T += V^T P^T  for all R rows at once; P is the B operand as the scores left it (the keys of a contraction step in accumulator
+//            order, V read transposed in the same order).
+// What bounds it: the vector units, 10 issue slots per (row, key, pair) -- one multiply, one range reduction, sine and cosine at two
+// slots each, two multiplies, two multiply-adds that round to fp16 -- of about 12 in all.  Measured at B2 Hq32 Hkv8 N4096 D128:
+// 5.37 -> 3.33 ms (one wave per row, the rotated keys through LDS: 14 slots per pair, the keys four times through
+// LDS and a softmax per head over the lanes), B1 Hq32 Hkv8 N1111 D128 fp16 230 -> 152 us, B2 Hq8 Hkv2 N512 D64 20.9 -> 18.4 us.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -36,250 +44,283 @@ struct CoropeFreqs {
   float w[64];  // inverse frequencies divided by 2*pi (revolutions per unit of delta), D/2 entries used
 };
 
-template <int D, int G>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void corope_gqa_fwd_kernel(CoropeParams p,
+constexpr int kCoropeWaves = 4, kCoropeKeys = 64;
+
+template <int D, int R>
+struct CoropeFwdCfg {
+  static constexpr int kKStride = D + 8;    // K tile rows: 16 keys read at one column hit 16 different bank groups
+  static constexpr int kVStride = D + 16;   // V tile rows: the 4 rows x 32 bytes of a transposing read cover 32 banks once
+  static constexpr int kTileElems = kCoropeKeys * (kKStride + kVStride);
+  static constexpr int kDeltaFloats = 4 * R * 16;                            // per wave: [16-key block][row][key % 16]
+  static constexpr int kLdsBytes = 2 * kTileElems * 2 + kCoropeWaves * kDeltaFloats * 4;
+  static_assert(2 * kLdsBytes <= 160 * 1024, "two workgroups per compute unit");
+};
+
+// (At D = 64 the registers allow more than two waves per SIMD: with several rows per wave that is 4 % faster, B2 Hq16 Hkv16 N2688
+// 1458 -> 1397 us; with one, where the longest rows set the time, 7 % slower, B1 Hq2 Hkv1 N4096 173 -> 185 us.)
+template <int D, int G, int R>
+__global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_per_eu(2, R == 1 ? 2 : 8))) void corope_gqa_fwd_kernel(CoropeParams p,
                                                                                                        CoropeFreqs fr) {
-  constexpr int HALF = D / 2, KS = D + 8, WS = kWave + 8, PIECES = D / 8;
-  constexpr int NI = 4 * ((G - 1) / 8 + 1);                            // accumulator registers that hold rows < G
-  __shared__ __attribute__((aligned(16))) uint16_t tile[kWave * KS];   // [key][d]: K (bf16), then rotated K (fp16), then V (bf16)
-  __shared__ __attribute__((aligned(16))) uint16_t ql[D];              // the leader's query row (bf16)
-  __shared__ __attribute__((aligned(16))) uint16_t wts[G * WS];        // [head][key] bf16 softmax weights of the chunk
+  using Cfg = CoropeFwdCfg<D, R>;
+  constexpr int KS = Cfg::kKStride, VS = Cfg::kVStride, NT = kCoropeWaves * kWave, PIECES = D / 8;
+  constexpr int NKS = D / 32, HK = D / 64, NOB = D / 16, PER = kCoropeKeys * PIECES / NT;
+  constexpr int ZR = R > 4 ? R / 4 : 1;     // query rows whose gates a lane holds
+  static_assert(R * G <= 16 && 64 % (kCoropeWaves * R) == 0, "columns of a product; a workgroup's rows lie in one chunk");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int n = lane % 16, g = lane / 16;   // matrix-core identity: A row / B column, contraction group
+  uint16_t* const tiles = reinterpret_cast<uint16_t*>(smem);
+  float* const dbuf = reinterpret_cast<float*>(smem + 2 * Cfg::kTileElems * 2) + wave * Cfg::kDeltaFloats;
+
   const int n_groups = p.B * p.Hkv;
   const int grp = blockIdx.x % n_groups;
-  const int i = p.N - 1 - blockIdx.x / n_groups;                       // longest rows first
-  const int lane = threadIdx.x;
-  const int vr = lane % 32, hf = lane / 32;                            // matrix-core identity of this lane
-  const int b = grp / p.Hkv, kvh = grp % p.Hkv;
-  const int N = p.N;
-  const int head0 = b * p.Hq + kvh * G;
+  const int i0 = (p.num_m_blocks - 1 - (int)(blockIdx.x / n_groups)) * (kCoropeWaves * R);   // longest rows first
+  const int N = p.N, iw = i0 + wave * R;
+  const int head0 = (grp / p.Hkv) * p.Hq + (grp % p.Hkv) * G;
   const uint16_t* kbase = p.k + (int64_t)grp * N * D;
   const uint16_t* vbase = p.v + (int64_t)grp * N * D;
-  const int n_chunks = i / kWave + 1;
+  const int n_chunks = i0 / kCoropeKeys + 1;
   const float scale2 = p.sm_scale * 1.4426950408889634f;               // scores in the base-2 domain
 
-  // A operand of the score product, constant over the row: lane (vr, hf) holds columns 16 ks + 8 hf .. + 7 of q^vr as fp16
-  // for vr < G, zeros otherwise.  The logit product takes the leader's row in the element type from LDS.
-  // (This product stays on 32x32x16: with rows m of a 16x16x32 A operand holding head m % 4, which also needs no exchange
-  // between lanes, the kernel was 3.7 % slower at G = 4, D = 128 -- unlike the logit product below.)
-  u32x4 aop[D / 16];
+  // column n of the score product: (query row, head) = (iw + n / G, n % G); columns from R G on are idle
+  const int crow = n < R * G ? n / G : 0, chead = n < R * G ? n % G : 0;
+  u32x4 qop[NKS], lop[NKS];   // B operand of the score product (fp16), A operand of the logit product (element type)
   {
-    const uint16_t* qrow = p.q + ((int64_t)(head0 + (vr < G ? vr : 0)) * N + i) * D + 8 * hf;
+    const uint16_t* qrow = p.q + ((int64_t)(head0 + chead) * N + min(iw + crow, N - 1)) * D + 8 * g;
+    const uint16_t* lrow = p.q + ((int64_t)head0 * N + min(iw + n * R / 16, N - 1)) * D + 8 * g;
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      const u32x4 raw = *reinterpret_cast<const u32x4*>(qrow + 16 * ks);
-      u32x4 h16;
+    for (int ks = 0; ks < NKS; ++ks) {
+      const u32x4 raw = *reinterpret_cast<const u32x4*>(qrow + 32 * ks);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) h16[e] = pack_f16(elt_lo(raw[e]), elt_hi(raw[e]));
-      aop[ks] = vr < G ? h16 : u32x4{0, 0, 0, 0};
+      for (int e = 0; e < 4; ++e) qop[ks][e] = n < R * G ? pack_f16(elt_lo(raw[e]), elt_hi(raw[e])) : 0u;
+      lop[ks] = *reinterpret_cast<const u32x4*>(lrow + 32 * ks);
     }
-    const uint16_t* lrow = p.q + ((int64_t)head0 * N + i) * D;
-    for (int d = lane; d < D; d += kWave) ql[d] = lrow[d];
   }
+  float turns[HK][8];         // w_d / 2 pi of this lane's columns d = 32 hk + 8 g + e
+#pragma unroll
+  for (int hk = 0; hk < HK; ++hk)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int d = 32 * hk + e;
+      turns[hk][e] = g == 0 ? fr.w[d] : g == 1 ? fr.w[d + 8] : g == 2 ? fr.w[d + 16] : fr.w[d + 24];
+    }
 
-  // one 64 x D block of K or V: consecutive 16-byte pieces per lane, parked as rows of the tile
-  u32x4 blk[PIECES];
-  // may_run_past_end: only the chunk on the diagonal can; the form without the clamped variant keeps one address per
-  // lane (with both forms present the compiler merges them into loads behind sixteen selected 64-bit addresses)
-  auto fetch_block = [&](const uint16_t* base, int c, auto may_run_past_end) __attribute__((always_inline)) {
-    const uint16_t* block = base + (int64_t)c * kWave * D;   // wave-uniform
-    if (!decltype(may_run_past_end)::value || c * kWave + kWave <= N) {
 #pragma unroll
-      for (int it = 0; it < PIECES; ++it)
-        blk[it] = *reinterpret_cast<const u32x4*>(byte_offset(block, 16u * lane + 1024u * it));
-    } else {   // the block runs past the last key: clamp the rows (only the chunk on the diagonal can get here)
+  for (int hk = 0; hk < HK; ++hk)
 #pragma unroll
-      for (int it = 0; it < PIECES; ++it) {
-        const int row = (it * kWave + lane) / PIECES, piece = lane % PIECES;
-        blk[it] = *reinterpret_cast<const u32x4*>(base + (int64_t)min(c * kWave + row, N - 1) * D + 8 * piece);
-      }
+    for (int e = 0; e < 8; ++e) asm volatile("" ::"v"(turns[hk][e]));   // landed before the loop: left to their first use, the wait sits in it
+
+  // K and V of a chunk: global memory -> registers one chunk ahead -> the other LDS stage
+  u32x4 kst[PER], vst[PER];
+  auto fetch = [&](int c, auto may_run_past_end) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = threadIdx.x + u * NT;
+      int row = c * kCoropeKeys + e / PIECES;
+      if (decltype(may_run_past_end)::value) row = min(row, N - 1);   // only the chunk on the diagonal can
+      const uint32_t off = (uint32_t)row * (D * 2) + (e % PIECES) * 16;
+      kst[u] = *reinterpret_cast<const u32x4*>(byte_offset(kbase, off));
+      vst[u] = *reinterpret_cast<const u32x4*>(byte_offset(vbase, off));
     }
   };
-  auto park_block = [&]() __attribute__((always_inline)) {
+  auto park = [&](int buf) __attribute__((always_inline)) {
+    uint16_t* kt = tiles + buf * Cfg::kTileElems;
+    uint16_t* vt = kt + kCoropeKeys * KS;
 #pragma unroll
-    for (int it = 0; it < PIECES; ++it) {
-      const int row = (it * kWave + lane) / PIECES, piece = lane % PIECES;
-      *reinterpret_cast<u32x4*>(tile + row * KS + 8 * piece) = blk[it];
+    for (int u = 0; u < PER; ++u) {
+      const int e = threadIdx.x + u * NT;
+      *reinterpret_cast<u32x4*>(kt + (e / PIECES) * KS + 8 * (e % PIECES)) = kst[u];
+      *reinterpret_cast<u32x4*>(vt + (e / PIECES) * VS + 8 * (e % PIECES)) = vst[u];
     }
-  };
-  // (rows < G of a 64-key product) -> this lane's key: swapping the upper half of the keys-below-32 result with the lower
-  // half of the keys-from-32 result puts every key's rows into its own lane
-  auto rows_of_key = [&](const f32x16& c0, const f32x16& c1, float (&out)[G]) __attribute__((always_inline)) {
-    float lo_rows[NI], hi_rows[NI];   // rows 8 (n / 4) + n % 4 and the same + 4
-#pragma unroll
-    for (int n = 0; n < NI; ++n) {
-      const float x0 = c0[n], x1 = c1[n];   // (a bit_cast applied directly to a vector element reads element 0)
-      const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x0), __builtin_bit_cast(uint32_t, x1),
-                                                      false, false);
-      lo_rows[n] = __builtin_bit_cast(float, (uint32_t)r[0]);
-      hi_rows[n] = __builtin_bit_cast(float, (uint32_t)r[1]);
-    }
-#pragma unroll
-    for (int h = 0; h < G; ++h) out[h] = (h / 4) % 2 ? hi_rows[4 * (h / 8) + h % 4] : lo_rows[4 * (h / 8) + h % 4];
-  };
-  // Leader logits of the 64 keys (K as parked): a 1 x D by D x 64 product, run as 16x16x32 products with the leader's row in
-  // every row of A.  All rows of a result block are then equal, block kb holds keys 16 kb .. 16 kb + 15 in the lanes with
-  // that l % 16, so every lane finds its own key's logit in block (lane / 16) of its own registers.
-  auto leader_logit = [&]() __attribute__((always_inline)) {
-    const int r = lane / 16, c = lane % 16;
-    f32x4 acc[4];
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) acc[kb] = f32x4{0, 0, 0, 0};
-#pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) {
-      const u32x4 a = *reinterpret_cast<const u32x4*>(ql + 32 * ks + 8 * r);   // a broadcast read per 16 lanes
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-        acc[kb] = mfma16(a, *reinterpret_cast<const u32x4*>(tile + (16 * kb + c) * KS + 32 * ks + 8 * r), acc[kb]);
-    }
-    return r == 0 ? acc[0][0] : r == 1 ? acc[1][0] : r == 2 ? acc[2][0] : acc[3][0];
-  };
-  // scores of the G heads against the rotated keys (fp16) -> this lane's key: sc[h]
-  auto scores_of_key = [&](float (&sc)[G]) __attribute__((always_inline)) {
-    f32x16 c0 = f32x16{0}, c1 = f32x16{0};
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      c0 = mfma32_f16(aop[ks], *reinterpret_cast<const u32x4*>(tile + vr * KS + 16 * ks + 8 * hf), c0);
-      c1 = mfma32_f16(aop[ks], *reinterpret_cast<const u32x4*>(tile + (32 + vr) * KS + 16 * ks + 8 * hf), c1);
-    }
-    rows_of_key(c0, c1, sc);
   };
 
-  // O^T += V^T P^T as 16x16x32 products (16 output columns x 16 heads per block, of which G are used: half the matrix-pipe
-  // time and half the accumulator registers of the 32x32x16 form).  oacc[db][e]: column 16 db + 4 (lane / 16) + e of head
-  // lane % 16's output row (lanes with lane % 16 >= G idle).
-  constexpr int NOB = D / 16;
-  const int oh = lane % 16, og = lane / 16;
-  f32x4 oacc[NOB];
+  f32x4 oacc[NOB];            // O^T: column n, d = 16 db + 4 g + e
 #pragma unroll
   for (int db = 0; db < NOB; ++db) oacc[db] = f32x4{0, 0, 0, 0};
-  float m_run[G], l_run[G];   // running maximum (wave-uniform, base-2 domain) and this lane's sum of 2^(s - m)
+  // reference value of the exponentials of this lane's column (base-2 units; far below every score until the first chunk) and
+  // this lane's share of its denominator
+  float m_run = -1e30f, l_run = 0.f;
+  float carry[ZR];            // sum of the gates to the right of the chunk
 #pragma unroll
-  for (int h = 0; h < G; ++h) {
-    m_run[h] = -INFINITY;
-    l_run[h] = 0.f;
-  }
-  float carry = 0.f;          // sum of the gates of the chunks to the right (up to the diagonal)
+  for (int z = 0; z < ZR; ++z) carry[z] = 0.f;
 
-  // the chunk on the diagonal, the only one that can run past the last key, is fetched here; the loop's own fetches
-  // are for chunks inside the sequence
-  fetch_block(kbase, n_chunks - 1, std::true_type{});
-  park_block();
-  fetch_block(vbase, n_chunks - 1, std::true_type{});
+  fetch(n_chunks - 1, std::true_type{});
+  park(0);
+  __syncthreads();
+  int buf = 0;
 #pragma unroll 1
   for (int c = n_chunks - 1; c >= 0; --c) {
-    const int j = c * kWave + lane;
-    const bool valid = j <= i;
-    if (c != n_chunks - 1) {
-      park_block();                                  // K of this chunk
-      fetch_block(vbase, c, std::false_type{});      // V of this chunk: needed after the scores
-    }
-    lds_order();                  // (also orders the one-time write of the leader's row before its first read)
+    if (c > 0) fetch(c - 1, std::false_type{});
+    const uint16_t* kt = tiles + buf * Cfg::kTileElems;
+    const uint16_t* vt = kt + kCoropeKeys * KS;
+    const bool diagonal = c == n_chunks - 1;   // wave-uniform
 
-    // leader logits (row 0 of the product), gates, delta
-    const float lg0 = leader_logit();
-    const float z = valid ? 1.f / (1.f + __expf(-lg0 * p.sm_scale)) : 0.f;   // gates beyond the diagonal do not count
-    const float zpre = wave_prefix_sum(z), ztot = wave_last(zpre);
-    const float delta = carry + (ztot - zpre);   // gates strictly to the right of this key, up to the diagonal
-    carry += ztot;
-
-    // each lane rotates its own key row in place: one step of look-ahead in two alternating register sets; the scheduling
-    // barriers keep the LDS reads from all moving to the top
-    u32x2 wa[2][2];
-    wa[0][0] = *reinterpret_cast<const u32x2*>(tile + lane * KS);
-    wa[0][1] = *reinterpret_cast<const u32x2*>(tile + lane * KS + HALF);
-    static_for<HALF / 4>([&](auto step_c) __attribute__((always_inline)) {
-      constexpr int step = decltype(step_c)::value, d0 = step * 4;
-      if (d0 + 4 < HALF) {
-        wa[(step + 1) % 2][0] = *reinterpret_cast<const u32x2*>(tile + lane * KS + d0 + 4);
-        wa[(step + 1) % 2][1] = *reinterpret_cast<const u32x2*>(tile + lane * KS + HALF + d0 + 4);
-      }
-      const u32x2 w1 = wa[step % 2][0], w2 = wa[step % 2][1];
-      float r1v[4], r2v[4];
+    // ---- leader logits, gates, delta: lane (key 16 b + n, query rows (4 g + e) R / 16) -------------------------------------
+    {
+      f32x4 lg[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float x = __builtin_amdgcn_fractf(delta * fr.w[d0 + e]);
-        const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
-        const float k1 = e % 2 ? elt_hi(w1[e / 2]) : elt_lo(w1[e / 2]);
-        const float k2 = e % 2 ? elt_hi(w2[e / 2]) : elt_lo(w2[e / 2]);
-        r1v[e] = __builtin_fmaf(cs, k1, sn * k2);
-        r2v[e] = __builtin_fmaf(cs, k2, -(sn * k1));
+      for (int b = 0; b < 4; ++b) {
+        lg[b] = f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+          lg[b] = mfma16(lop[ks], *reinterpret_cast<const u32x4*>(kt + (16 * b + n) * KS + 32 * ks + 8 * g), lg[b]);
       }
-      *reinterpret_cast<u32x2*>(tile + lane * KS + d0) = u32x2{pack_f16(r1v[0], r1v[1]), pack_f16(r1v[2], r1v[3])};
-      *reinterpret_cast<u32x2*>(tile + lane * KS + HALF + d0) = u32x2{pack_f16(r2v[0], r2v[1]), pack_f16(r2v[2], r2v[3])};
-      __builtin_amdgcn_sched_barrier(0);
-    });
+#pragma unroll
+      for (int z = 0; z < ZR; ++z) {
+        const int r = R > 4 ? g * ZR + z : 4 * g * R / 16;
+        float pre[4], tot[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          float x = sigmoid(lg[b][z * (4 / ZR)] * p.sm_scale);
+          if (diagonal && c * kCoropeKeys + 16 * b + n > iw + r) x = 0.f;   // gates beyond the diagonal do not count
+          pre[b] = row16_prefix_sum(x);
+          tot[b] = row16_last(pre[b]);
+        }
+        float right = carry[z];
+#pragma unroll
+        for (int b = 3; b >= 0; --b) {
+          dbuf[(b * R + r) * 16 + n] = right + (tot[b] - pre[b]);   // gates strictly to the right of the key, up to the diagonal
+          right += tot[b];
+        }
+        carry[z] = right;
+      }
+    }
     lds_order();
 
-    // scores of every head, online softmax
-    float sc[G];
-    scores_of_key(sc);
-    // The reference value m_run[h] of the exponentials only has to keep them in range, it need not be the running
-    // maximum: it moves (to the exact maximum so far, with the usual rescaling) only when some score of the chunk lies
-    // more than kLazyMargin above it, which after the first chunks of a row is rare.  The common case then costs one
-    // comparison per head instead of a cross-lane maximum.
-    constexpr float kLazyMargin = 8.f;   // base-2 units: weights stay below 2^8
-    float (&s2)[G] = sc;   // scaled in place
-    bool exceeds = false;
+    // ---- rotated keys and scores: 16 keys at a time ---------------------------------------------------------------------
+    f32x4 sacc[4];
+    static_for<4>([&](auto b_c) __attribute__((always_inline)) {
+      constexpr int b = decltype(b_c)::value;
+      float k1[HK][8], k2[HK][8];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      s2[h] = valid ? sc[h] * scale2 : -INFINITY;
-      exceeds |= s2[h] > m_run[h] + kLazyMargin;   // m_run starts at -inf: the first chunk always moves it
-    }
-    if (__builtin_amdgcn_ballot_w64(exceeds) != 0) {   // wave-uniform
-      float al = 1.f;          // this lane's head's rescale factor
+      for (int hk = 0; hk < HK; ++hk) {
+        const u32x4 x1 = *reinterpret_cast<const u32x4*>(kt + (16 * b + n) * KS + 32 * hk + 8 * g);
+        const u32x4 x2 = *reinterpret_cast<const u32x4*>(kt + (16 * b + n) * KS + D / 2 + 32 * hk + 8 * g);
 #pragma unroll
-      for (int h = 0; h < G; ++h) {
-        const float m_new = fmaxf(m_run[h], wave_max(s2[h]));   // finite: the chunk holds a key <= i
-        const float a = fast_exp2(m_run[h] - m_new);
-        m_run[h] = m_new;
-        l_run[h] *= a;
-        al = oh == h ? a : al;
+        for (int e = 0; e < 4; ++e) {
+          k1[hk][2 * e] = elt_lo(x1[e]);
+          k1[hk][2 * e + 1] = elt_hi(x1[e]);
+          k2[hk][2 * e] = elt_lo(x2[e]);
+          k2[hk][2 * e + 1] = elt_hi(x2[e]);
+        }
       }
+      float delta = dbuf[b * R * 16 + n];
+#pragma unroll 1
+      for (int r = 0; r < R; ++r) {
+        const float delta_r = delta;
+        delta = dbuf[(b * R + min(r + 1, R - 1)) * 16 + n];
+        f32x4 acc = f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int hk = 0; hk < HK; ++hk) {
+          f16x8 y1, y2;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float x = __builtin_amdgcn_fractf(delta_r * turns[hk][e]);
+            const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
+            y1[e] = (_Float16)__builtin_fmaf(cs, k1[hk][e], sn * k2[hk][e]);
+            y2[e] = (_Float16)__builtin_fmaf(cs, k2[hk][e], -(sn * k1[hk][e]));
+          }
+          acc = mfma16_f16(__builtin_bit_cast(u32x4, y1), qop[hk], acc);
+          acc = mfma16_f16(__builtin_bit_cast(u32x4, y2), qop[HK + hk], acc);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sacc[b][e] = crow == r ? acc[e] : sacc[b][e];
+      }
+    });
+
+    // ---- softmax: lane = (row, head), 16 keys 16 b + 4 g + e of the chunk ------------------------------------------------
+    if (diagonal) {
+      int rel = iw + crow - c * kCoropeKeys - 4 * g;   // last key the row sees, relative to this lane's first
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (16 * b + e > rel) sacc[b][e] = scale2 < 0.f ? INFINITY : -INFINITY;
+    }
+    // The reference value only has to keep the exponentials in range, it need not be the running maximum: it moves (to the exact
+    // maximum so far, with the usual rescaling) only when some score of the chunk lies more than kLazyMargin above it, which after
+    // the first chunks of a row is rare.
+    constexpr float kLazyMargin = 8.f;   // base-2 units: weights stay below 2^8
+    float x[4][4], top = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[b][e] = __builtin_fmaf(sacc[b][e], scale2, -m_run);
+        top = fmaxf(top, x[b][e]);
+      }
+    if (__builtin_amdgcn_ballot_w64(top > kLazyMargin) != 0) {   // wave-uniform
+      top = -INFINITY;
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) top = fmaxf(top, sacc[b][e] * scale2);
+      top = fmaxf(top, __shfl_xor(top, 16));
+      top = fmaxf(top, __shfl_xor(top, 32));
+      const float m_new = fmaxf(m_run, top);   // finite: the chunk holds a key <= row
+      const float al = fast_exp2(m_run - m_new);
+      m_run = m_new;
+      l_run *= al;
 #pragma unroll
       for (int db = 0; db < NOB; ++db)
 #pragma unroll
         for (int e = 0; e < 4; ++e) oacc[db][e] *= al;
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[b][e] = __builtin_fmaf(sacc[b][e], scale2, -m_run);
     }
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const float e = fast_exp2(s2[h] - m_run[h]);   // 0 for the keys beyond the diagonal
-      l_run[h] += e;
-      wts[h * WS + lane] = f_to_elt(e);
-    }
-    park_block();                          // V replaces the rotated keys
-    if (c > 0) fetch_block(kbase, c - 1, std::false_type{});  // K of the next chunk
-    lds_order();
+    for (int t = 0; t < 2; ++t) {   // 32 keys per product
+      float w[8];
 #pragma unroll
-    for (int ks = 0; ks < kWave / 32; ++ks) {   // 32 keys per product
-      u32x4 bop = u32x4{0, 0, 0, 0};
-      if (oh < G) bop = *reinterpret_cast<const u32x4*>(wts + oh * WS + 32 * ks + 8 * og);
+      for (int j = 0; j < 8; ++j) {
+        w[j] = fast_exp2(x[2 * t + j / 4][j % 4]);   // 0 for the keys beyond the diagonal
+        l_run += w[j];
+      }
+      const u32x4 bop = {pack_elts(w[0], w[1]), pack_elts(w[2], w[3]), pack_elts(w[4], w[5]), pack_elts(w[6], w[7])};
 #pragma unroll
-      for (int db = 0; db < NOB; ++db) oacc[db] = mfma16(load_a_trans16(tile, KS, 32 * ks, 16 * db), bop, oacc[db]);
+      for (int db = 0; db < NOB; ++db) oacc[db] = mfma16(load_a_trans16_acc(vt, VS, 32 * t, 16 * db), bop, oacc[db]);
     }
-    lds_order();
+    if (c > 0) park(buf ^ 1);
+    buf ^= 1;
+    __syncthreads();
   }
 
-  float inv_l = 0.f;
-#pragma unroll
-  for (int h = 0; h < G; ++h) {
-    const float l = wave_sum(l_run[h]);
-    inv_l = oh == h ? (l > 0.f ? 1.f / l : 0.f) : inv_l;   // same guard as the reference's epilogue (:343-345)
-  }
-  if (oh < G) {
-    uint16_t* op = p.o + ((int64_t)(head0 + oh) * N + i) * D;
+  float l = l_run + __shfl_xor(l_run, 16);
+  l += __shfl_xor(l, 32);
+  const float inv_l = l > 0.f ? 1.f / l : 0.f;   // same guard as the reference's epilogue (:343-345)
+  if (n < R * G && iw + crow < N) {
+    uint16_t* op = p.o + ((int64_t)(head0 + chead) * N + iw + crow) * D;
 #pragma unroll
     for (int db = 0; db < NOB; ++db) {
       const u32x2 w = {pack_elts(oacc[db][0] * inv_l, oacc[db][1] * inv_l), pack_elts(oacc[db][2] * inv_l, oacc[db][3] * inv_l)};
-      *reinterpret_cast<u32x2*>(op + db * 16 + 4 * og) = w;
+      *reinterpret_cast<u32x2*>(op + db * 16 + 4 * g) = w;
     }
   }
 }
 
-template <int D, int G>
-static hipError_t launch_corope_cfg(CoropeParams p, const CoropeFreqs& fr, hipStream_t stream) {
-  p.num_m_blocks = p.N;   // one query row per workgroup
-  hipLaunchKernelGGL((corope_gqa_fwd_kernel<D, G>), dim3(p.N * p.B * p.Hkv), dim3(kWave), 0, stream, p, fr);
+template <int D, int G, int R>
+static hipError_t launch_corope_rows(CoropeParams p, const CoropeFreqs& fr, hipStream_t stream) {
+  using Cfg = CoropeFwdCfg<D, R>;
+  auto kern = corope_gqa_fwd_kernel<D, G, R>;
+  static std::atomic<uint64_t> lds_ok{0};
+  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
+  p.num_m_blocks = (p.N + kCoropeWaves * R - 1) / (kCoropeWaves * R);
+  hipLaunchKernelGGL(kern, dim3((unsigned)p.num_m_blocks * p.B * p.Hkv), dim3(kCoropeWaves * kWave), Cfg::kLdsBytes, stream, p, fr);
   return hipGetLastError();
+}
+
+template <int D, int G>
+static hipError_t launch_corope_cfg(const CoropeParams& p, const CoropeFreqs& fr, hipStream_t stream) {
+  // Rows per wave: as many as fill the 16 columns where that leaves four waves per SIMD, of which two run at a time; below that
+  // the longest rows, whose chunks follow one after the other, set the time, and fewer rows per wave shorten it (B1 Hq32 Hkv8
+  // N1111 D128: 190 us with four rows, 165 with two).
+  constexpr int kMost = G <= 2 ? 8 : G <= 4 ? 4 : 2;
+  const int64_t rows = (int64_t)p.N * p.B * p.Hkv, simds = 4 * device_cu_count();
+  if (rows >= 4 * simds * kMost) return launch_corope_rows<D, G, kMost>(p, fr, stream);
+  if (kMost > 2 && rows >= 8 * simds) return launch_corope_rows<D, G, 2>(p, fr, stream);
+  return launch_corope_rows<D, G, 1>(p, fr, stream);
 }
 
 template <int D>

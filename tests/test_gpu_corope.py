@@ -118,3 +118,20 @@ def test_corope_forward_fp16(pkg, B, Hq, Hkv, N, D, scale):
         assert err.max() <= TOL
     else:
         assert err.max() <= 0.15 and err.mean() <= 5e-3
+
+
+# Many short groups: every number of query rows a wave takes (by group size and by how many rows there are), with lengths that end
+# inside a wave's rows, a workgroup's rows and a chunk.  Three of the groups against the oracle.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("groups,G,N,D", [(470, 1, 70, 64), (480, 2, 69, 128), (240, 3, 73, 128), (240, 4, 70, 64), (120, 4, 75, 128),
+                                          (120, 5, 71, 64), (120, 8, 70, 128), (60, 1, 139, 128)])
+def test_forward_many_groups(pkg, groups, G, N, D, dtype):
+    dev = torch.device("cuda:0")
+    q, k, v = (bf16_round(seeded((groups, h, N, D), 20 + i)) for i, h in enumerate((G, 1, 1)))
+    scale = 1 / math.sqrt(D)
+    o = pkg.corope_attention(*(t.to(dev, dtype) for t in (q, k, v)), True, scale, 10000.0)
+    torch.cuda.synchronize()
+    for g in (0, groups // 2, groups - 1):
+        ref = C.corope_gqa_forward(q[g:g + 1].double(), k[g:g + 1].double(), v[g:g + 1].double(), True, scale, 10000.0, torch.float64)
+        err = (o[g:g + 1].double().cpu() - ref).abs().max().item()
+        assert err <= 2e-2, (g, err)

@@ -77,6 +77,11 @@ __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) { return mf
 __device__ __forceinline__ f32x4 mfma16_f16(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
+// D(16x16) += A(16x16) * B(16x16): lane l holds row / column (l % 16), contraction slots 4*(l / 16) .. +3; D as above.
+typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
+__device__ __forceinline__ f32x4 mfma16x16_f16(u32x2 a, u32x2 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
+}
 #ifdef COROPE_F16
 __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) { return mfma16_f16(a, b, c); }
 #else
@@ -785,6 +790,15 @@ __device__ __forceinline__ u32x4 load_a_trans16_acc(const uint16_t* tile, int st
   return u32x4{a[0], a[1], b[0], b[1]};
 }
 
+// A operand of mfma16x16 (16 rows m x 16 contraction slots) read transposed from a row-major tile of 16 rows: lane l gets
+// T[4*(l / 16) + j][m0 + l % 16] for slots j = 0..3.
+__device__ __forceinline__ u32x2 load_a_trans16_block(const uint16_t* tile, int stride, int m0) {
+  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+  const int l = threadIdx.x % kWave;
+  const int g = l / 16, s = l % 16;
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(tile + (4 * g + s / 4) * stride + m0 + 4 * (s % 4))));
+}
+
 // Natural-order variant of load_a_trans: slot j of lane-half h <-> k = kbase + 8*h + j.
 __device__ __forceinline__ u32x4 load_a_trans_natural(const uint16_t* tile, int stride, int kbase, int m0) {
   typedef __attribute__((address_space(3))) s16x4* lds_ptr;
@@ -837,8 +851,26 @@ __device__ __forceinline__ float row16_prefix_sum(float x) {
   return x;
 }
 __device__ __forceinline__ float row16_last(float x) { return dpp_move<0x15f, 0xf>(0.f, x); }   // row_newbcast:15
+__device__ __forceinline__ uint32_t row16_ror8(uint32_t x) {   // lane l gets lane l ^ 8's value
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, false);
+}
 __device__ __forceinline__ float wave_last(float x) {          // lane 63's value, wave-uniform
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), kWave - 1));
+}
+// The prefix sum within each segment of 16, 32 or 64 lanes, and the segment's last lane's value in every lane of it.
+template <int SEG>
+__device__ __forceinline__ float segment_prefix_sum(float x) {
+  static_assert(SEG == 16 || SEG == 32 || SEG == 64, "whole rows of 16 lanes");
+  if constexpr (SEG == 64) return wave_prefix_sum(x);
+  x = row16_prefix_sum(x);
+  if constexpr (SEG == 32) x += dpp_move<0x142, 0xa>(0.f, x);
+  return x;
+}
+template <int SEG>
+__device__ __forceinline__ float segment_last(float x) {
+  if constexpr (SEG == 64) return wave_last(x);
+  if constexpr (SEG == 32) return __shfl(x, (int)(threadIdx.x % kWave) | 31);
+  return row16_last(x);
 }
 __device__ __forceinline__ float wave_max(float x) {
   x = fmaxf(x, dpp_move<0x111, 0xf>(-INFINITY, x));

@@ -21,17 +21,15 @@
 // and where the dS-weighted sum of the group's queries is rotated (dk kernel) - the angle is shared by the group and
 // rotation is linear, so one vector is rotated per (i, j), not one per head.  Everything that is a dot product with an
 // already rotated or an unrotated row runs on the matrix cores.  Launches, in order:
-//   rowdot (x2)  leader logits qL K^T per group and dP = dO V^T per head, fp32 into the workspace (32x32x16 bf16 MFMA,
-//                128 rows x 128 keys per workgroup, operands fetched with whole cache lines and parked in LDS)
-//   scores       one wave per (group, query row), lane = key:
-//                  right to left over 64-key chunks: z, delta by a scan, the rotated keys Kt -> LDS (fp16); on the matrix
-//                  cores S = q Kt^T and dS/ddelta = [-w q2, w q1] Kt^T for all heads at once, then - with running softmax
+//   scores       a wave per R query rows of a group, 16 keys at a time:
+//                  right to left: leader logits, z, delta by a scan, the rotated keys Kt in registers (fp16); on the matrix cores
+//                  dP = V dO^T, S = Kt q^T and dS/ddelta = Kt [-w q2, w q1]^T for all heads, then - with running softmax
 //                  statistics, flash-attention style - the two sums that make dq: sum_j e_j dP_j kt_j and sum_j e_j kt_j;
-//                  left to right: P, dS, G and its running sum, W;
-//                  writes dq of the heads 1..G-1, the leader's dq without its gate path (fp32, workspace) and the workspace
-//                  matrices DELTA, W [group] and P, DS [head] (packed lower triangles)
+//                  left to right: dP again, dS, G and its running sum, W;
+//                  writes dq of the heads 1..G-1, the leader's dq without its gate path (fp32, workspace), the workspace
+//                  matrices DELTA, W [group] and S, DS [head] (packed lower triangles) and the row statistics that make P of S
 //   dq_leader    dq_leader = c (partial + W K): a plain product on the matrix cores, 128 rows per workgroup
-//   dv           dv^T += dO^T P on the matrix cores, 128 keys per workgroup
+//   dv           dv^T += dO^T P on the matrix cores, P from S and the row statistics, 128 keys per workgroup
 //   dk           one workgroup per (group, 128 keys): sum_h dS^h q^h on the matrix cores, then lane = rotation pair x 16
 //                keys rotates it per (i, j) and adds the gate path W qL; tiles of DELTA, W, DS staged through LDS
 // Rounding: the rotated keys and what multiplies them (queries, the softmax weights e and e dP) are fp16 - the bf16
@@ -46,8 +44,8 @@
 namespace COROPE_NS {
 
 struct CoropeBwdFreqs {
-  float turns[64];   // w_d / (2 pi): phase in revolutions per unit of delta (what v_sin_f32 / v_cos_f32 take)
-  float rad[64];     // w_d
+  alignas(16) float turns[64];   // w_d / (2 pi): phase in revolutions per unit of delta (what v_sin_f32 / v_cos_f32 take)
+  alignas(16) float rad[64];     // w_d
 };
 
 // Row i of a workspace matrix holds the keys j <= i only: rows are packed, each padded to the 64-key chunk it ends in
@@ -64,462 +62,536 @@ struct CoropeBwdWs {
   int n_groups, n_heads;
   __device__ __host__ float* delta(int g) const { return base + (int64_t)g * NN; }
   __device__ __host__ float* w(int g) const { return base + (int64_t)(n_groups + g) * NN; }
-  __device__ __host__ float* p(int h) const { return base + (int64_t)(2 * n_groups + h) * NN; }               // S, then P
+  __device__ __host__ float* s(int h) const { return base + (int64_t)(2 * n_groups + h) * NN; }               // scores, base-2 units
   __device__ __host__ float* ds(int h) const { return base + (int64_t)(2 * n_groups + n_heads + h) * NN; }    // dS/ddelta, then dS
-  __device__ __host__ float* dp(int h) const { return base + (int64_t)(2 * n_groups + 2 * n_heads + h) * NN; }
+  // What the last n_heads matrices' worth of space holds, per group: the partial sums of dv, then of dk, from the front, and per
+  // head and query row, at the end, the reference value of the exponentials and 1 / their sum.
+  __device__ __host__ static int padded_rows(int N) { return (N + 15) / 16 * 16; }
+  __device__ __host__ int64_t part_floats(int G, int N) const { return G * (NN - 2 * padded_rows(N)); }
+  __device__ __host__ float* parts(int g, int G) const { return base + (int64_t)(2 * n_groups + 2 * n_heads + g * G) * NN; }
+  __device__ __host__ float* row_max(int g, int G, int N, int h) const { return parts(g, G) + part_floats(G, N) + h * padded_rows(N); }
+  __device__ __host__ float* row_inv(int g, int G, int N, int h) const { return row_max(g, G, N, G + h); }
   // (N, D) per group: the leader head's dq without the gate path and without the factor sm_scale
   __device__ __host__ float* dql(int g, int N, int D) const {
     return base + (int64_t)(2 * n_groups + 3 * n_heads) * NN + (int64_t)g * N * D;
   }
 };
 
-// ---------------------------------------------------------------------------------------------------- row dots
-// out[idx][i][j] = a[idx * a_mul][i] . b[idx / b_div][j] for the tiles that touch the causal triangle: the two plain
-// matrix products of the backward (leader logits qL K^T per group: a_mul = G, b_div = 1; dP = dO V^T per head: a_mul
-// = 1, b_div = G) on the matrix cores.  A workgroup of 4 waves owns 128 rows x 128 keys; the rows of both operands are
-// fetched with whole cache lines and parked in LDS (an operand piece read straight from global memory is 16 bytes of a
-// row per lane: every instruction would touch 64 different lines); one wave owns 32 rows and sweeps the keys in two
-// halves of 64, the second half fetched while the first is multiplied.
-constexpr int kRowdotRows = 128, kRowdotKeys = 64;
-
-template <int D>
-__global__ __launch_bounds__(4 * kWave) void corope_bwd_rowdot_kernel(const uint16_t* a, const uint16_t* b, float* out,
-                                                                      int64_t NN, int N, int a_mul, int b_div) {
-  constexpr int TS = D + 8, NT = 4 * kWave, PIECES = D / 8;
-  constexpr int A_PER = kRowdotRows * PIECES / NT, B_PER = kRowdotKeys * PIECES / NT;
-  __shared__ __attribute__((aligned(16))) uint16_t atile[kRowdotRows * TS];
-  __shared__ __attribute__((aligned(16))) uint16_t btile[kRowdotKeys * TS];
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int r = lane % 32, hf = lane / 32;
-  const int idx = blockIdx.z;
-  const int ib = blockIdx.y * kRowdotRows, j0 = blockIdx.x * 128;
-  if (j0 > ib + kRowdotRows - 1 || ib >= N) return;   // every key of the block lies beyond its rows (workgroup-uniform)
-  const int i0 = ib + wave * 32;
-  const uint16_t* arows = a + (int64_t)idx * a_mul * N * D;
-  const uint16_t* brows = b + (int64_t)(idx / b_div) * N * D;
-  u32x4 breg[B_PER];
-  auto fetch_b = [&](int jh) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < B_PER; ++u) {
-      const int e = threadIdx.x + u * NT;
-      breg[u] = *reinterpret_cast<const u32x4*>(brows + (int64_t)min(jh + e / PIECES, N - 1) * D + 8 * (e % PIECES));
-    }
-  };
-  auto park_b = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < B_PER; ++u) {
-      const int e = threadIdx.x + u * NT;
-      *reinterpret_cast<u32x4*>(btile + (e / PIECES) * TS + 8 * (e % PIECES)) = breg[u];
-    }
-  };
-  fetch_b(j0);
-#pragma unroll
-  for (int u = 0; u < A_PER; ++u) {
-    const int e = threadIdx.x + u * NT;
-    *reinterpret_cast<u32x4*>(atile + (e / PIECES) * TS + 8 * (e % PIECES)) =
-        *reinterpret_cast<const u32x4*>(arows + (int64_t)min(ib + e / PIECES, N - 1) * D + 8 * (e % PIECES));
-  }
-  park_b();
-  __syncthreads();
-  u32x4 af[D / 16];
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) af[ks] = *reinterpret_cast<const u32x4*>(atile + (wave * 32 + r) * TS + 16 * ks + 8 * hf);
-  float* obase = out + (int64_t)idx * NN;
-  // the 32 rows of the wave lie in one 64-row band, so they share a row length; a column <= i0 + 31 is inside the padded row
-  const int64_t row0 = tri_row_start(min(i0, N - 1)), row_len = 64 * (i0 / 64 + 1);
-#pragma unroll 1
-  for (int half = 0; half < 2; ++half) {
-    const int jh = j0 + kRowdotKeys * half;
-    const bool more = half == 0 && jh + kRowdotKeys <= ib + kRowdotRows - 1 && jh + kRowdotKeys < N;   // workgroup-uniform
-    if (more) fetch_b(jh + kRowdotKeys);
-#pragma unroll
-    for (int jt = 0; jt < kRowdotKeys / 32; ++jt) {
-      const int jj0 = jh + 32 * jt;
-      if (jj0 > i0 + 31 || jj0 >= N || i0 >= N) continue;   // wave-uniform
-      f32x16 c = f32x16{0};
-#pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks)
-        c = mfma32(af[ks], *reinterpret_cast<const u32x4*>(btile + (32 * jt + r) * TS + 16 * ks + 8 * hf), c);
-      const int col = jj0 + r;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int dr = acc_row(e, hf);
-        if (i0 + dr < N && col < N) obase[row0 + row_len * dr + col] = c[e];
-      }
-    }
-    if (!more) break;
-    __syncthreads();   // every wave is done with the first half of the keys
-    park_b();
-    __syncthreads();
-  }
-}
-
 // ---------------------------------------------------------------------------------------------------- scores
-// One wave per (group, query row i), all G heads at once, lane = key.  Per 64-key chunk the lanes rotate their keys
-// (the only place sines and cosines are evaluated) and park them in LDS as fp16; everything that is a dot product with
-// the rotated key then runs on the matrix cores: the raw scores q^h . kt and their derivatives with respect to delta
-// (rows [-w q2, w q1] . kt) as one (2G x D) x (D x 64 keys) product, and the dq sums as (weights x keys) x (keys x D).
-template <int D, int G>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) void corope_bwd_scores_kernel(CoropeBwdParams p, CoropeBwdWs ws, CoropeBwdFreqs fr) {
-  constexpr int HALF = D / 2;
-  constexpr int KS = D + 8, WS = kWave + 8, NVR = 2 * G;
-  constexpr int NI = 4 * ((2 * G - 1) / 8 + 1);                       // accumulator registers that hold rows < 2G
-  __shared__ __attribute__((aligned(16))) uint16_t kt[kWave * KS];    // [key][d]: keys (bf16), rotated in place (fp16)
-  __shared__ __attribute__((aligned(16))) uint16_t wts[NVR * WS];     // [virtual row][key] fp16 weights of the keys
-  const int i = p.N - 1 - blockIdx.x, g = blockIdx.y, lane = threadIdx.x;   // longest rows first
-  const int vr = lane % 32, hf = lane / 32;                                  // matrix-core identity of this lane
-  const int N = p.N, b = g / p.Hkv, kvh = g % p.Hkv;
-  const int head0 = b * p.Hq + kvh * G;   // first head of the group, as a (batch, head) slab index
-  // A operand of the score products, constant over the row: lane (vr, hf) holds columns 16 ks + 8 hf .. + 7 of matrix row vr;
-  // rows h < G are q^h, rows G + h are [-w q2^h, w q1^h] (the derivative with respect to delta), the rest zero
-  u32x4 aop[D / 16];
-  {
-    const int h = vr < G ? vr : vr - G;
-    const uint16_t* qrow = p.q + ((int64_t)(head0 + (vr < 2 * G ? h : 0)) * N + i) * D;
+// A wave owns R query rows of one (batch, kv head) group, all G heads at once, and sweeps 16 keys at a time.  The R x G (row, head)
+// pairs are columns of 16x16 products: rows 0 .. R/2 - 1 are columns 0 .. 7, the others columns 8 .. 15 (R = 1: columns 0 .. 7).
+//   keys     lane (key % 16, g) holds columns 8 g .. 8 g + 7 of every 32 of its key, fetched straight from global memory (a key
+//            block is 4 KB, read once for all R rows) and unpacked once; the rotation happens in that layout, row by row.
+//   scores   the rotated keys are the A operand as they are.  A row needs its own columns of S = Kt q^T only, and of
+//            dS/ddelta = Kt [-w q2, w q1]^T; one product gives both: the B operand of a row of the lower half carries q in columns
+//            0 .. 7 and the derivative's rows in columns 8 .. 15, of the upper half the other way round.
+//   softmax  lane = (row, head), registers = 4 of the 16 keys: no idle lane, row statistics are one register per lane.
+//   dq       needs the rotated keys transposed: they go through LDS (16 keys x D x R rows per wave) and come back through the
+//            transposing read.  The weights of the two sums, e (dP - ref) and e, share the 16 columns in the same way (a rotation by 8
+//            lanes), and two rows share the 32 contraction slots of a product (the other row's columns of B are zero).
+// No barriers: a wave is a workgroup.  What bounds it: in the first sweep the vector units (busy 82 % of it; 10 issue slots per (row, key,
+// pair) as in the forward, of about 12.3 in all), in the second the memory (9 floats in, 5 out per (row, key) at G = 4); two waves a
+// SIMD hide one under the other only in part.  dP is computed in both sweeps, and P is left to the dv kernel: kept in the workspace they cost
+// 12 floats more per (row, key) and a launch.
+// Measured at B2 Hq32 Hkv8 N4096 D128: 8.2 -> 5.9 ms, first sweep 4.6 (one wave per row with the rotated keys in LDS, behind launches for the
+// logits and dP); B2 Hq8 Hkv2 N512 D64 52 -> 40 us.
+template <int D, int G, int R>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void corope_bwd_scores_kernel(CoropeBwdParams p, CoropeBwdWs ws,
+                                                                                                          CoropeBwdFreqs fr) {
+  constexpr int TS = D + 16, HALF = D / 2;   // LDS row stride: the row-wise writes and the transposing reads both spread over the banks
+  constexpr int NKS = D / 32, HK = D / 64, NDB = D / 16;
+  constexpr int NS = R > 1 ? 2 : 1, RH = R / NS;             // halves of the columns, rows in each
+  static_assert(RH * G <= 8 && (R == 1 || R == 2 || R == 4), "eight columns for each half of the rows");
+  // [row][key][d]: rotated keys, fp16.  Before they come and after they have been used, a block of 16 rows of K or V on its way from whole
+  // cache lines to operand order; second sweep: such a block, and behind it dP [column][key], fp32
+  constexpr int BS = D + 8, PS = kWave + 4;   // row strides: block (elements), dP (floats)
+  constexpr int kKtElems = R * 16 * TS, kBlockElems = 2 * 16 * BS, kSecondElems = 16 * BS + NS * 8 * PS * 2;
+  __shared__ __attribute__((aligned(16))) uint16_t kt[std::max({kKtElems, kBlockElems, kSecondElems})];
+  __shared__ __attribute__((aligned(16))) uint16_t lead[R * (D + 8)];  // the leader's rows
+  const int lane = threadIdx.x, n = lane % 16, g = lane / 16;
+  // longest rows of all groups first: with one group after the other the last group's longest rows started when the chip was
+  // already running empty (23 % of the compute units' time idle)
+  const int n_groups = p.B * p.Hkv, grp = (int)(blockIdx.x % n_groups);
+  const int iw = R * ((int)(gridDim.x / n_groups) - 1 - (int)(blockIdx.x / n_groups));
+  const int N = p.N, b_ = grp / p.Hkv, kvh = grp % p.Hkv;
+  const int head0 = b_ * p.Hq + kvh * G;   // first head of the group, as a (batch, head) slab index
+  const int sub = n % 8;                   // place within a half
+  const bool low = n < 8;
+  // Idle columns repeat the first one of their half, rows past the end the last row, operands and all: they come to the same values
+  // and may store them to the same places.  With no lane switched off around the loops' stores their number is known to the compiler,
+  // and a wait for a prefetched load does not wait for the stores behind it.
+  const bool busy = sub / G < RH;
+  const int place = busy ? sub / G : 0, head = busy ? sub % G : 0;      // this lane's column: row of the half, head
+  const int half = NS > 1 ? n / 8 : 0;                                  // (R = 1: the lanes from 8 on hold dS/ddelta only)
+  const int own_row = min(iw + half * RH + place, N - 1);
+  const float scale2 = p.sm_scale * 1.4426950408889634f;                // scores in the base-2 domain
+
+  // w_d / 2 pi and w_d of this lane's columns d = 32 hk + 8 g + e
+  float turns[HK][8], rad[HK][8];
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      const int d0 = 16 * ks + 8 * hf;                      // first of this lane's 8 columns
-      u32x4 val = u32x4{0, 0, 0, 0};
-      if (vr < G) {
-        const u32x4 raw = *reinterpret_cast<const u32x4*>(qrow + d0);
+  for (int hk = 0; hk < HK; ++hk)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) val[e] = pack_f16(elt_lo(raw[e]), elt_hi(raw[e]));   // exact
-      } else if (vr < 2 * G) {
-        const bool upper = d0 >= HALF;                       // columns of the second half take w q1, the first half -w q2
-        const u32x4 src = *reinterpret_cast<const u32x4*>(qrow + (upper ? d0 - HALF : d0 + HALF));
-        const float* wr = fr.rad + (upper ? d0 - HALF : d0);
-        float x[8];
+    for (int e = 0; e < 8; e += 4) {
+      const f32x4 t = *reinterpret_cast<const f32x4*>(fr.turns + 32 * hk + 8 * g + e);
+      const f32x4 w = *reinterpret_cast<const f32x4*>(fr.rad + 32 * hk + 8 * g + e);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float qv = e % 2 ? elt_hi(src[e / 2]) : elt_lo(src[e / 2]);
-          x[e] = upper ? wr[e] * qv : -wr[e] * qv;
-        }
-        val = u32x4{pack_f16(x[0], x[1]), pack_f16(x[2], x[3]), pack_f16(x[4], x[5]), pack_f16(x[6], x[7])};
+      for (int x = 0; x < 4; ++x) {
+        turns[hk][e + x] = t[x];
+        rad[hk][e + x] = w[x];
       }
-      aop[ks] = val;
+    }
+
+  // B operands of the score products (fp16): columns of half s, the derivative's rows in the other half's places
+  u32x4 qop[NS][NKS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const bool deriv = n / 8 != s;
+    const uint16_t* qrow = p.q + ((int64_t)(head0 + head) * N + min(iw + s * RH + place, N - 1)) * D;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      const int d0 = 32 * ks + 8 * g;
+      const u32x4 raw = *reinterpret_cast<const u32x4*>(qrow + (deriv ? d0 ^ HALF : d0));
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float w = rad[ks % HK][e], qv = e % 2 ? elt_hi(raw[e / 2]) : elt_lo(raw[e / 2]);
+        x[e] = (deriv ? (2 * ks < NKS ? -w : w) : 1.f) * qv;   // first half of the columns: -w q2, second: w q1
+      }
+      qop[s][ks] = u32x4{pack_f16(x[0], x[1]), pack_f16(x[2], x[3]), pack_f16(x[4], x[5]), pack_f16(x[6], x[7])};
     }
   }
-  const uint16_t* kbase = p.k + (int64_t)g * N * D;
-  const int64_t rowoff = tri_row_start(i);
-  const int n_chunks = i / kWave + 1;
-  // this row of every workspace matrix: wave-uniform bases, addressed with 32-bit byte offsets of the key index
-  float* const d_row = ws.delta(g) + rowoff;
-  float* const w_row = ws.w(g) + rowoff;
-  float *p_row[G], *ds_row[G];
-  const float* dp_row[G];
-#pragma unroll
-  for (int h = 0; h < G; ++h) {
-    p_row[h] = ws.p(head0 + h) + rowoff;
-    ds_row[h] = ws.ds(head0 + h) + rowoff;
-    dp_row[h] = ws.dp(head0 + h) + rowoff;
-  }
-
-  // ---- right to left: gates, delta, raw scores, dS/ddelta, softmax statistics, dq sums --------------------------------
   // dq^h = c sum_j dS_j kt_j = c (sum_j e_j dP_j kt_j - Delta sum_j e_j kt_j) / L with e_j = exp(s_j - m): both sums are
-  // accumulated on the matrix cores as rows 2h and 2h + 1 of W (virtual rows x keys) times Kt (keys x d), rescaled
-  // flash-attention style when the row's running maximum m moves.  The 2G <= 16 virtual rows are the columns of 16x16x32
-  // products (half the matrix-pipe time and accumulator registers of the 32x32x16 form, whose other 16 columns would be
-  // idle): dqa[db][e] belongs to virtual row `qv` = lane % 16 and column 16 db + 4 (lane / 16) + e.
-  constexpr int NQB = D / 16;
-  const int qv = lane % 16, qg = lane / 16;
-  f32x4 dqa[NQB];
-#pragma unroll
-  for (int db = 0; db < NQB; ++db) dqa[db] = f32x4{0, 0, 0, 0};
-  float m_run[G], l_run[G], pd_run[G];   // running maximum (wave-uniform); per lane: sum of exp(s - m), of exp(s - m) dP
-#pragma unroll
-  for (int h = 0; h < G; ++h) {
-    m_run[h] = -INFINITY;
-    l_run[h] = pd_run[h] = 0.f;
-  }
-  float carry = 0.f;   // sum of z over the keys to the right of the current chunk (up to the diagonal)
+  // accumulated on the matrix cores, rescaled flash-attention style when the row's reference value m moves.
   // Reference value for Delta = rowsum(P o dP), which is only known at the end of the row: the dq sums take e (dP - ref)
   // as weights and are corrected by (Delta - ref) afterwards, which is exact for any ref; the closer ref is to Delta, the
   // less the two sums cancel (rows dominated by one key would otherwise lose the 11 bits of the weights).  With the forward
   // output at hand ref = rowsum(O o dO), equal to Delta up to O's rounding; without it ref = 0.
   // The weights e (dP - ref) go to the matrix cores as fp16, whose 5 exponent bits would tie the result to the scale of
   // dO (overflow from |dP - ref| ~ 1e3 on, nothing left of a mean-reduced loss's 1e-7): they are divided by a power of two
-  // w_scale >= 4 |dO_i| first (|dP_ij| <= |dO_i| |v_j|, so the scaled weights are at most e^4 |v_j| / 4 whatever dO is)
+  // w_scale >= 4 |dO_i| first (|dP_ij| <= |dO_i| |v_j|, so the scaled weights are at most 2^5 |v_j| / 4 whatever dO is)
   // and the sum is multiplied back afterwards -- exact both ways.
-  float dref[G];
-  int w_exp[G];   // w_scale = 2^w_exp, wave-uniform (scalar registers)
+  float dref = 0.f, w_mul, w_inv;
+  const uint16_t* const do_l = p.d_o + ((int64_t)(head0 + head) * N + own_row) * D + 8 * g;   // B operand of dP = V dO^T, column n
+  {
+    float sq = 0.f;
+    const int64_t off = ((int64_t)(head0 + head) * N + own_row) * D + 8 * g;
 #pragma unroll
-  for (int h = 0; h < G; ++h) {
-    float acc = 0.f, sq = 0.f;
-    const int64_t off = ((int64_t)(head0 + h) * N + i) * D;
-    for (int d = lane; d < D; d += kWave) {
-      const float g_d = elt_to_f(p.d_o[off + d]);
-      sq = __builtin_fmaf(g_d, g_d, sq);
-      if (p.o != nullptr) acc = __builtin_fmaf(elt_to_f(p.o[off + d]), g_d, acc);
+    for (int ks = 0; ks < NKS; ++ks) {
+      const u32x4 x = *reinterpret_cast<const u32x4*>(do_l + 32 * ks);
+      u32x4 y = u32x4{0, 0, 0, 0};
+      if (p.o != nullptr) y = *reinterpret_cast<const u32x4*>(p.o + off + 32 * ks);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sq = __builtin_fmaf(elt_lo(x[e]), elt_lo(x[e]), __builtin_fmaf(elt_hi(x[e]), elt_hi(x[e]), sq));
+        dref = __builtin_fmaf(elt_lo(x[e]), elt_lo(y[e]), __builtin_fmaf(elt_hi(x[e]), elt_hi(y[e]), dref));
+      }
     }
-    dref[h] = wave_sum(acc);
+    sq += __shfl_xor(sq, 16);
+    sq += __shfl_xor(sq, 32);
+    dref += __shfl_xor(dref, 16);
+    dref += __shfl_xor(dref, 32);
     int ex = 0;
-    (void)frexpf(__builtin_sqrtf(wave_sum(sq)), &ex);       // |dO_i| = m 2^ex with m in [0.5, 1); 0 gives ex = 0
-    w_exp[h] = __builtin_amdgcn_readfirstlane(max(-100, min(100, ex + 2)));
+    (void)frexpf(__builtin_sqrtf(sq), &ex);       // |dO_i| = m 2^ex with m in [0.5, 1); 0 gives ex = 0
+    const int w_exp = max(-100, min(100, ex + 2));
+    w_mul = ldexpf(1.f, w_exp);
+    w_inv = ldexpf(1.f, -w_exp);
   }
-  // A chunk's 64 key rows are one contiguous block of global memory: the wave fetches it with consecutive 16-byte pieces
-  // per lane (full cache lines per instruction) and parks it in the LDS tile, where each lane then finds its own key's
-  // row.  The block, the leader logits (from the row-dot pass; their slot then takes delta) and dP are each requested
-  // for the next chunk at the point where the current values have been used up.
-  constexpr int PIECES = D / 8;   // 16-byte pieces per row = fetch instructions per chunk
-  u32x4 kv[PIECES];
-  // may_run_past_end: only the chunk on the diagonal can; the form without the clamped variant keeps one address per
-  // lane (with both forms present the compiler merges them into loads behind sixteen selected 64-bit addresses)
-  auto fetch_keys = [&](int c, auto may_run_past_end) __attribute__((always_inline)) {
-    const uint16_t* block = kbase + (int64_t)c * kWave * D;   // wave-uniform
-    if (!decltype(may_run_past_end)::value || c * kWave + kWave <= N) {
-#pragma unroll
-      for (int it = 0; it < PIECES; ++it)
-        kv[it] = *reinterpret_cast<const u32x4*>(byte_offset(block, 16u * lane + 1024u * it));
-    } else {   // the block runs past the last key: clamp the rows (only the chunk on the diagonal can get here)
-#pragma unroll
-      for (int it = 0; it < PIECES; ++it) {
-        const int row = (it * kWave + lane) / PIECES, piece = lane % PIECES;
-        kv[it] = *reinterpret_cast<const u32x4*>(kbase + (int64_t)min(c * kWave + row, N - 1) * D + 8 * piece);
-      }
-    }
-  };
-  auto park_keys = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int it = 0; it < PIECES; ++it) {
-      const int row = (it * kWave + lane) / PIECES, piece = lane % PIECES;
-      *reinterpret_cast<u32x4*>(kt + row * KS + 8 * piece) = kv[it];
-    }
-  };
-  float logit, dpv[G];
-  {
-    const int jc = min((n_chunks - 1) * kWave + lane, i);
-    fetch_keys(n_chunks - 1, std::true_type{});
-    logit = *byte_offset(d_row, 4u * jc);
-#pragma unroll
-    for (int h = 0; h < G; ++h) dpv[h] = *byte_offset(dp_row[h], 4u * jc);
-  }
-#pragma unroll 1
-  for (int c = n_chunks - 1; c >= 0; --c) {
-    const int j = c * kWave + lane;
-    const bool valid = j <= i;
-    park_keys();
-    const float z = valid ? 1.f / (1.f + __expf(-logit * p.sm_scale)) : 0.f;
-    const int jn = j - kWave;   // this lane's key in the next chunk: at or below the diagonal whenever that chunk exists
-    if (c > 0) logit = *byte_offset(d_row, 4u * jn);
-    const float zpre = wave_prefix_sum(z), ztot = wave_last(zpre);
-    const float delta = carry + (ztot - zpre);   // gates strictly to the right, up to and including the diagonal
-    carry += ztot;
+  const float ref_scaled = dref * w_inv;
 
-    // the key rotated by -delta w_d replaces the key in LDS (bf16, row = this lane's key)
+  const uint16_t* kbase = p.k + (int64_t)grp * N * D;
+  const uint16_t* vbase = p.v + (int64_t)grp * N * D;
+  const int row_len = 64 * (iw / 64 + 1);                    // the rows of a wave lie in one 64-row band: one row length
+  const int64_t rows0 = tri_row_start(iw);
+  // this lane's places in the matrices: the score of a column; dS/ddelta of the column eight on; gates of key n
+  // of query row z_row
+  const int z_row = min(iw + g * R / 4, N - 1);
+  // (stored by lane (column, keys) = (lane / 4, 4 (lane % 4) ..): four lanes complete a 64-byte piece)
+  float *s_l, *g_l;
+  const int from = lane / 4 + 16 * (lane % 4);   // the lane that computes what this one stores
+  {
+    const int c = lane / 4, csub = c % 8, chalf = NS > 1 ? c / 8 : 0;
+    const int cplace = csub / G < RH ? csub / G : 0, chead = csub / G < RH ? csub % G : 0;
+    const int64_t c_own = rows0 + row_len * (min(iw + chalf * RH + cplace, N - 1) - iw) + 4 * (lane % 4);
+    const int64_t c_other = rows0 + row_len * (min(iw + (NS - 1 - chalf) * RH + cplace, N - 1) - iw) + 4 * (lane % 4);
+    s_l = (NS == 1 && c >= 8 ? ws.ds(head0 + chead) : ws.s(head0 + chead)) + c_own;
+    g_l = ws.ds(head0 + chead) + c_other;
+  }
+  float* const d_l = ws.delta(grp) + rows0 + row_len * (z_row - iw) + n;
+  float* const slope_l = ws.w(grp) + rows0 + row_len * (z_row - iw) + n;
+
+  f32x4 dqa[NS][NDB];    // half s: columns 0..7 sum e (dP - ref) kt, 8..15 sum e kt of the half's columns; d = 16 db + 4 g + e
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) dqa[s][db] = f32x4{0, 0, 0, 0};
+  float m_run = -1e30f, l_run = 0.f, pd_run = 0.f;   // reference value of the exponentials; this lane's sums of e and e dP
+  float carry = 0.f;                                  // gates to the right of the block, up to the diagonal
+
+  const int nb = iw / 16 + 1;
+  // A block of 16 rows of K or V: an operand piece read straight from memory is 16 bytes of a row per lane, neighbouring lanes in different
+  // rows, and the address unit then handles one lane per cycle (it was busy 81 % of this kernel's time).  So a block is requested with
+  // consecutive pieces in consecutive lanes and takes its operand order in LDS.
+  auto request = [&](u32x4 (&x)[NKS], const uint16_t* base, int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NKS; ++u) {
+      const int e = lane + u * kWave;
+      const uint32_t row = min(16 * b + e / (D / 8), N - 1);   // (only the block on the diagonal can reach past the end)
+      x[u] = *reinterpret_cast<const u32x4*>(byte_offset(base, row * (D * 2) + e % (D / 8) * 16));
+    }
+  };
+  auto park = [&](const u32x4 (&x)[NKS], uint16_t* tile) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < NKS; ++u) {
+      const int e = lane + u * kWave;
+      *reinterpret_cast<u32x4*>(tile + e / (D / 8) * BS + e % (D / 8) * 8) = x[u];
+    }
+  };
+  auto take = [&](u32x4 (&x)[NKS], const uint16_t* tile) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) x[ks] = *reinterpret_cast<const u32x4*>(tile + n * BS + 32 * ks + 8 * g);
+  };
+  u32x4 kraw[NKS];
+  u32x4 va[NKS], da[NKS];
+  f32x4 dp;   // dP of this lane's column for the block at hand
+  auto fetch_dp = [&](int b) __attribute__((always_inline)) {
+    request(va, vbase, b);
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) da[ks] = *reinterpret_cast<const u32x4*>(do_l + 32 * ks);
+  };
+  // What a block needs before its keys can be rotated, done for the next block at the end of this one: its keys and values in operand order,
+  // dP, the leader logits (row m of A is the leader of query row m R / 16, so lane (key n, g) finds the logit of its own query row z_row),
+  // gates and delta of (z_row, key n).  The steps are short and each waits for the one before: together their waits overlap.
+  float z, delta;
+  auto prepare = [&](int b, bool diagonal) __attribute__((always_inline)) {
     lds_order();
-    // one step of look-ahead in two alternating register sets; the scheduling barriers keep the reads from all moving up
-    u32x2 wa[2][2];
-    wa[0][0] = *reinterpret_cast<const u32x2*>(kt + lane * KS);
-    wa[0][1] = *reinterpret_cast<const u32x2*>(kt + lane * KS + HALF);
-    static_for<HALF / 4>([&](auto step_c) __attribute__((always_inline)) {
-      constexpr int step = decltype(step_c)::value, d0 = step * 4;
-      if (d0 + 4 < HALF) {
-        wa[(step + 1) % 2][0] = *reinterpret_cast<const u32x2*>(kt + lane * KS + d0 + 4);
-        wa[(step + 1) % 2][1] = *reinterpret_cast<const u32x2*>(kt + lane * KS + HALF + d0 + 4);
-      }
-      const u32x2 w1 = wa[step % 2][0], w2 = wa[step % 2][1];
-      float r1v[4], r2v[4];
+    park(va, kt);
+    park(kraw, kt + 16 * BS);
+    lds_order();
+    take(va, kt);
+    take(kraw, kt + 16 * BS);
+    lds_order();
+    f32x4 lg = f32x4{0, 0, 0, 0};
+    dp = f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      lg = mfma16(*reinterpret_cast<const u32x4*>(lead + n * R / 16 * (D + 8) + 32 * ks + 8 * g), kraw[ks], lg);
+      dp = mfma16(va[ks], da[ks], dp);
+    }
+    z = sigmoid(lg[0] * p.sm_scale);
+    if (diagonal && 16 * b + n > z_row) z = 0.f;
+    const float zpre = row16_prefix_sum(z), ztot = row16_last(zpre);
+    delta = carry + (ztot - zpre);   // gates strictly to the right, up to and including the diagonal
+    carry += ztot;
+  };
+  fetch_dp(nb - 1);
+  for (int e = lane; e < R * (D / 8); e += kWave)
+    *reinterpret_cast<u32x4*>(lead + e / (D / 8) * (D + 8) + e % (D / 8) * 8) =
+        *reinterpret_cast<const u32x4*>(p.q + ((int64_t)head0 * N + min(iw + e / (D / 8), N - 1)) * D + e % (D / 8) * 8);
+  lds_order();
+  request(kraw, kbase, nb - 1);
+  prepare(nb - 1, true);
+#pragma unroll
+  for (int hk = 0; hk < HK; ++hk)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) asm volatile("" ::"v"(turns[hk][e]));
+#pragma unroll 1
+  for (int b = nb - 1; b >= 0; --b) {
+    const bool diagonal = b == nb - 1;   // wave-uniform
+    float k1[HK][8], k2[HK][8];
+#pragma unroll
+    for (int hk = 0; hk < HK; ++hk)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float x = __builtin_amdgcn_fractf(delta * fr.turns[d0 + e]);
-        const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
-        const float k1 = e % 2 ? elt_hi(w1[e / 2]) : elt_lo(w1[e / 2]);
-        const float k2 = e % 2 ? elt_hi(w2[e / 2]) : elt_lo(w2[e / 2]);
-        r1v[e] = __builtin_fmaf(cs, k1, sn * k2);
-        r2v[e] = __builtin_fmaf(cs, k2, -(sn * k1));
+        k1[hk][2 * e] = elt_lo(kraw[hk][e]);
+        k1[hk][2 * e + 1] = elt_hi(kraw[hk][e]);
+        k2[hk][2 * e] = elt_lo(kraw[HK + hk][e]);
+        k2[hk][2 * e + 1] = elt_hi(kraw[HK + hk][e]);
       }
-      *reinterpret_cast<u32x2*>(kt + lane * KS + d0) = u32x2{pack_f16(r1v[0], r1v[1]), pack_f16(r1v[2], r1v[3])};
-      *reinterpret_cast<u32x2*>(kt + lane * KS + HALF + d0) = u32x2{pack_f16(r2v[0], r2v[1]), pack_f16(r2v[2], r2v[3])};
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    lds_order();   // rotated keys are in LDS
+    request(kraw, kbase, max(b - 1, 0));
+    *byte_offset(d_l, 64u * b) = delta;
+    *byte_offset(slope_l, 64u * b) = z * (1.f - z);   // the sigmoid's slope; replaced by W in the second sweep
 
-    // (2G rows x D) x (D x 64 keys): lane = (row vr, half hf) for the A operand, (key vr [+ 32], half hf) for B
-    f32x16 c0 = f32x16{0}, c1 = f32x16{0};
+    // rotated keys -> LDS, scores and dS/ddelta
+    f32x4 m[NS];
+    static_for<R>([&](auto r_c) __attribute__((always_inline)) {
+      constexpr int r = decltype(r_c)::value, s = r / RH;
+      const float delta_r = R == 1 ? delta : __shfl(delta, 64 / R * r + n);
+      f32x4 acc = f32x4{0, 0, 0, 0};
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      c0 = mfma32_f16(aop[ks], *reinterpret_cast<const u32x4*>(kt + vr * KS + 16 * ks + 8 * hf), c0);
-      c1 = mfma32_f16(aop[ks], *reinterpret_cast<const u32x4*>(kt + (32 + vr) * KS + 16 * ks + 8 * hf), c1);
-    }
-    // the results sit at lane = key % 32 with rows split over the lane halves; swapping the upper half of the keys-below-
-    // 32 result with the lower half of the keys-from-32 result puts every key's rows into its own lane
-    float lo_rows[NI], hi_rows[NI];   // rows 8 (n / 4) + n % 4 and the same + 4
+      for (int hk = 0; hk < HK; ++hk) {
+        f16x8 y1, y2;
 #pragma unroll
-    for (int n = 0; n < NI; ++n) {
-      const float x0 = c0[n], x1 = c1[n];   // (a bit_cast applied directly to a vector element reads element 0)
-      const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x0), __builtin_bit_cast(uint32_t, x1),
-                                                      false, false);
-      lo_rows[n] = __builtin_bit_cast(float, (uint32_t)r[0]);
-      hi_rows[n] = __builtin_bit_cast(float, (uint32_t)r[1]);
-    }
-    // the registers of the product are free again: request the next chunk's keys (a chunk left of the diagonal one lies
-    // inside the sequence)
-    if (c > 0) fetch_keys(c - 1, std::false_type{});
-    float acc[G], gacc[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const int ra = h, rb = G + h;
-      acc[h] = (ra / 4) % 2 ? hi_rows[4 * (ra / 8) + ra % 4] : lo_rows[4 * (ra / 8) + ra % 4];
-      gacc[h] = (rb / 4) % 2 ? hi_rows[4 * (rb / 8) + rb % 4] : lo_rows[4 * (rb / 8) + rb % 4];
-    }
-    if (valid) {
-      *byte_offset(d_row, 4u * j) = delta;
-      *byte_offset(w_row, 4u * j) = z * (1.f - z);   // the sigmoid's slope; replaced by W in the second sweep
-    }
-    // The reference value m_run[h] of the exponentials only has to keep them in range, it need not be the running
-    // maximum (any value gives the same P once the row is normalised): it moves, to the exact maximum so far and with the
-    // usual rescaling, only when some score of the chunk lies more than kLazyMargin above it -- rare after the first
-    // chunks of a row -- and the common case costs one comparison per head instead of a cross-lane maximum.  The margin
-    // bounds the weights e (dP - ref) that go to the matrix cores as fp16.
-    constexpr float kLazyMargin = 4.f;
-    bool exceeds = false;
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const float sc = acc[h] * p.sm_scale;
-      if (valid) {
-        *byte_offset(p_row[h], 4u * j) = sc;
-        *byte_offset(ds_row[h], 4u * j) = gacc[h] * p.sm_scale;
+        for (int e = 0; e < 8; ++e) {
+          const float x = __builtin_amdgcn_fractf(delta_r * turns[hk][e]);
+          const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
+          y1[e] = (_Float16)__builtin_fmaf(cs, k1[hk][e], sn * k2[hk][e]);
+          y2[e] = (_Float16)__builtin_fmaf(cs, k2[hk][e], -(sn * k1[hk][e]));
+        }
+        const u32x4 w1 = __builtin_bit_cast(u32x4, y1), w2 = __builtin_bit_cast(u32x4, y2);
+        uint16_t* dst = kt + (r * 16 + n) * TS + 32 * hk + 8 * g;
+        *reinterpret_cast<u32x4*>(dst) = w1;
+        *reinterpret_cast<u32x4*>(dst + HALF) = w2;
+        acc = mfma16_f16(w1, qop[s][hk], acc);
+        acc = mfma16_f16(w2, qop[s][HK + hk], acc);
       }
-      acc[h] = valid ? sc : -INFINITY;
-      exceeds |= acc[h] > m_run[h] + kLazyMargin;   // m_run starts at -inf: the first chunk always moves it
-    }
-    if (__builtin_amdgcn_ballot_w64(exceeds) != 0) {   // wave-uniform
-      float al = 1.f;          // this lane's virtual row's rescale factor
+      if (r % RH == 0) {
+        m[s] = acc;
+      } else {
 #pragma unroll
-      for (int h = 0; h < G; ++h) {
-        const float m_new = fmaxf(m_run[h], wave_max(acc[h]));   // finite: the chunk holds a key <= i
-        const float a = __expf(m_run[h] - m_new);
-        m_run[h] = m_new;
-        l_run[h] *= a;
-        pd_run[h] *= a;
-        al = qv / 2 == h ? a : al;
+        for (int e = 0; e < 4; ++e) m[s][e] = place == r % RH ? acc[e] : m[s][e];
+      }
+    });
+    // The operands of the next block's dP take the registers that this block's keys have left: requested here, used at the end
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_dp(max(b - 1, 0));
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 sc, gd;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x0 = m[0][e], x1 = m[NS - 1][e];
+      sc[e] = (low ? x0 : x1) * scale2;
+      gd[e] = (NS > 1 && low ? x1 : x0) * p.sm_scale;
+    }
+    {
+      f32x4 s_out, g_out;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s_out[e] = __shfl(NS == 1 && !low ? gd[e] : sc[e], from);
+        if constexpr (NS > 1) g_out[e] = __shfl(gd[e], from);
+      }
+      *reinterpret_cast<f32x4*>(byte_offset(s_l, 64u * b)) = s_out;
+      if constexpr (NS > 1) *reinterpret_cast<f32x4*>(byte_offset(g_l, 64u * b)) = g_out;
+    }
+    if (diagonal) {
+      const int rel = own_row - 16 * b - 4 * g;   // last key the row sees, relative to this lane's first
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sc[e] = e > rel ? -INFINITY : sc[e];
+        dp[e] = e > rel ? 0.f : dp[e];              // not defined there
+      }
+    }
+    // The reference value only has to keep the exponentials in range, it need not be the running maximum (any value gives the
+    // same P once the row is normalised): it moves, to the exact maximum so far and with the usual rescaling, only when some score
+    // of the block lies more than kLazyMargin above it.  The margin bounds the weights that go to the matrix cores as fp16.
+    constexpr float kLazyMargin = 5.f;   // base-2 units
+    float x[4], top = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[e] = sc[e] - m_run;
+      top = fmaxf(top, x[e]);
+    }
+    if (__builtin_amdgcn_ballot_w64(top > kLazyMargin) != 0) {   // wave-uniform
+      top = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
+      top = fmaxf(top, __shfl_xor(top, 16));
+      top = fmaxf(top, __shfl_xor(top, 32));
+      const float m_new = fmaxf(m_run, top);   // finite: the block holds a key <= row
+      const float al = fast_exp2(m_run - m_new);
+      m_run = m_new;
+      l_run *= al;
+      pd_run *= al;
+      const float al_x = __shfl_xor(al, 8);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const float f = (n / 8 == s) ? al : al_x;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dqa[s][db][e] *= f;
       }
 #pragma unroll
-      for (int db = 0; db < NQB; ++db)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) dqa[db][e] *= al;
+      for (int e = 0; e < 4; ++e) x[e] = sc[e] - m_run;
     }
+    float we[4], wd[4];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const float e = __expf(acc[h] - m_run[h]);   // 0 for the keys beyond the diagonal
-      l_run[h] += e;
-      pd_run[h] = __builtin_fmaf(e, dpv[h], pd_run[h]);
+    for (int e = 0; e < 4; ++e) {
+      we[e] = fast_exp2(x[e]);   // 0 for the keys beyond the diagonal
+      l_run += we[e];
+      pd_run = __builtin_fmaf(we[e], dp[e], pd_run);
       // (clamped to fp16's range: a value row |v_j| in the thousands saturates instead of turning into infinity)
-      wts[(2 * h) * WS + lane] = f_to_f16(fminf(fmaxf(e * ldexpf(dpv[h] - dref[h], -w_exp[h]), -65504.f), 65504.f));
-      wts[(2 * h + 1) * WS + lane] = f_to_f16(e);
+      wd[e] = fminf(fmaxf(we[e] * __builtin_fmaf(dp[e], w_inv, -ref_scaled), -65504.f), 65504.f);
     }
-    if (c > 0) {
+    const u32x2 pd = {pack_f16(wd[0], wd[1]), pack_f16(wd[2], wd[3])}, pe = {pack_f16(we[0], we[1]), pack_f16(we[2], we[3])};
+    u32x2 wts[NS];
 #pragma unroll
-      for (int h = 0; h < G; ++h) dpv[h] = *byte_offset(dp_row[h], 4u * jn);
+    for (int t = 0; t < 2; ++t) {
+      const uint32_t pe_x = row16_ror8(pe[t]), pd_x = row16_ror8(pd[t]);   // all lanes active
+      wts[0][t] = low ? pd[t] : pe_x;
+      if constexpr (NS > 1) wts[NS - 1][t] = low ? pd_x : pe[t];
     }
-    lds_order();   // rotated keys and weights are in LDS
+    lds_order();   // rotated keys are in LDS
+    static_for<NS>([&](auto s_c) __attribute__((always_inline)) {
+      constexpr int s = decltype(s_c)::value;
+      u32x4 bop;
 #pragma unroll
-    for (int ks = 0; ks < kWave / 32; ++ks) {   // 32 keys per product
-      u32x4 bop = u32x4{0, 0, 0, 0};
-      if (qv < 2 * G) bop = *reinterpret_cast<const u32x4*>(wts + qv * WS + 32 * ks + 8 * qg);
+      for (int t = 0; t < 2; ++t) {
+        bop[t] = busy && place == 0 ? wts[s][t] : 0u;
+        bop[2 + t] = place == 1 ? wts[s][t] : 0u;
+      }
 #pragma unroll
-      for (int db = 0; db < NQB; ++db) dqa[db] = mfma16_f16(load_a_trans16(kt, KS, 32 * ks, 16 * db), bop, dqa[db]);
-    }
-    lds_order();   // ... and consumed: the next chunk may overwrite them
+      for (int db = 0; db < NDB; ++db) {
+        const u32x2 a0 = load_a_trans16_block(kt + s * RH * 16 * TS, TS, 16 * db);
+        if constexpr (RH > 1) {
+          const u32x2 a1 = load_a_trans16_block(kt + (s * RH + 1) * 16 * TS, TS, 16 * db);
+          dqa[s][db] = mfma16_f16(u32x4{a0[0], a0[1], a1[0], a1[1]}, bop, dqa[s][db]);
+        } else {
+          dqa[s][db] = mfma16x16_f16(a0, u32x2{bop[0], bop[1]}, dqa[s][db]);
+        }
+      }
+    });
+    lds_order();   // ... and consumed: the next block may overwrite them
+    prepare(b - 1, false);   // (before block 0: again block 0, unused)
   }
-  // row statistics: largest score, 1 / sum of exponentials, rowsum(P o dP)
-  float m_row[G], inv_l[G], dsum[G];
+  // row statistics: 1 / sum of exponentials, rowsum(P o dP)
+  l_run += __shfl_xor(l_run, 16);
+  l_run += __shfl_xor(l_run, 32);
+  pd_run += __shfl_xor(pd_run, 16);
+  pd_run += __shfl_xor(pd_run, 32);
+  const float inv_l = 1.f / l_run, dsum = pd_run * inv_l;
+
+  if ((NS > 1 || low) && busy && g == 0 && iw + half * RH + place < N) {   // for the dv kernel
+    ws.row_max(grp, G, N, head)[own_row] = m_run;
+    ws.row_inv(grp, G, N, head)[own_row] = inv_l;
+  }
+
+  // (sum e (dP - ref) kt - (Delta - ref) sum e kt) / L, the second sum sitting eight lanes up.  dq of the heads 1..G-1 is final; the
+  // leader's still lacks the gate path W K, which a separate plain matrix product adds (corope_bwd_dq_leader_kernel): its row
+  // goes to the workspace in fp32, unscaled
+  {
+    const float corr = dsum - dref;
+    const float inv_x = __shfl_xor(inv_l, 8), corr_x = __shfl_xor(corr, 8), mul_x = __shfl_xor(w_mul, 8);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int row = iw + s * RH + place;
+      const float my_inv = s == 0 ? inv_l : inv_x, my_corr = s == 0 ? corr : corr_x, my_mul = s == 0 ? w_mul : mul_x;
+      const bool mine = low && busy && row < N;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) {
+        f32x4 val;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float a = dqa[s][db][e], plain = __shfl_xor(a, 8);
+          val[e] = (a * my_mul - my_corr * plain) * my_inv;
+        }
+        if (mine) {
+          if (head == 0)
+            *reinterpret_cast<f32x4*>(ws.dql(grp, N, D) + (int64_t)row * D + db * 16 + 4 * g) = val;
+          else
+            *reinterpret_cast<u32x2*>(p.dq + ((int64_t)(head0 + head) * N + row) * D + db * 16 + 4 * g) =
+                u32x2{pack_elts(val[0] * p.sm_scale, val[1] * p.sm_scale), pack_elts(val[2] * p.sm_scale, val[3] * p.sm_scale)};
+        }
+      }
+    }
+  }
+
+  // ---- left to right: dS, G_ij = sum_h dS dS/ddelta, its running sum over the keys, W: 64 keys at a time, lane = (row, R keys) ------
+  // dP once more from V and dO: lane = column there, through LDS to lane = (row, keys).  What the lanes read here other lanes of this
+  // wave wrote above.
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  constexpr int SEG = kWave / R;   // lanes of a row
+  typedef float keys_t __attribute__((ext_vector_type(R)));
+  float* const dpt = reinterpret_cast<float*>(kt + 16 * BS);
+  const int row2 = lane / SEG, key0 = (lane % SEG) * R, i2 = min(iw + row2, N - 1);
+  const int col2 = row2 / RH * 8 + row2 % RH * G;   // column of (row2, head 0)
+  float m_row[G], l_row[G], d_row[G];
 #pragma unroll
   for (int h = 0; h < G; ++h) {
-    m_row[h] = m_run[h];
-    const float l = wave_sum(l_run[h]), pd = wave_sum(pd_run[h]);
-    inv_l[h] = 1.f / l;
-    dsum[h] = pd * inv_l[h];
+    m_row[h] = __shfl(m_run, col2 + h);
+    l_row[h] = __shfl(inv_l, col2 + h);
+    d_row[h] = __shfl(dsum, col2 + h);
   }
-
-  // even virtual row 2h: (sum e (dP - ref) kt - (Delta - ref) sum e kt) / L, the second sum sitting in the neighbouring lane; the rows from
-  // 2G on are idle
-  {
-    float my_inv = 0.f, my_dsum = 0.f;
-    int my_exp = 0;
+  const uint32_t at = 4u * (row_len * (i2 - iw) + key0);
+  float* const w_base = ws.w(grp) + rows0;   // wave-uniform bases, addressed with 32-bit byte offsets
+  const float* const s_base = ws.s(head0) + rows0;
+  float* const ds_base = ws.ds(head0) + rows0;
+  u32x4 dop[NKS], vraw[4][NKS];
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) dop[ks] = *reinterpret_cast<const u32x4*>(do_l + 32 * ks);
+  // The matrices come from memory and are requested two chunks ahead, in two register sets; V comes from the cache, one chunk ahead.
+  keys_t sl_n[2], sv_n[2][G], gv_n[2][G];
+  const int n_chunks = iw / kWave + 1;
+  auto fetch_v = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) request(vraw[t], vbase, 4 * c + t);
+  };
+  auto fetch_rows = [&](int c, auto set_c) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value;
+    const uint32_t off = at + 256u * c;
+    sl_n[set] = *reinterpret_cast<const keys_t*>(byte_offset(w_base, off));
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-      my_inv = qv / 2 == h ? inv_l[h] : my_inv;
-      my_dsum = qv / 2 == h ? dsum[h] - dref[h] : my_dsum;
-      my_exp = qv / 2 == h ? w_exp[h] : my_exp;
-    }
-#pragma unroll
-    for (int db = 0; db < NQB; ++db)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float other = __shfl_xor(dqa[db][e], 1);
-        if (qv < 2 * G) dqa[db][e] = (ldexpf(dqa[db][e], my_exp) - my_dsum * other) * my_inv;
-      }
-  }
-  // dq of the heads 1..G-1 is final; the leader's still lacks the gate path W K, which a separate plain matrix product
-  // adds (corope_bwd_dq_leader_kernel): its row goes to the workspace in fp32, unscaled
-  if (qv < 2 * G && qv % 2 == 0) {
-    if (qv == 0) {
-      float* op = ws.dql(g, N, D) + (int64_t)i * D;
-#pragma unroll
-      for (int db = 0; db < NQB; ++db) *reinterpret_cast<f32x4*>(op + db * 16 + 4 * qg) = dqa[db];
-    } else {
-      uint16_t* op = p.dq + ((int64_t)(head0 + qv / 2) * N + i) * D;
-#pragma unroll
-      for (int db = 0; db < NQB; ++db) {
-        const u32x2 w = {pack_elts(dqa[db][0] * p.sm_scale, dqa[db][1] * p.sm_scale),
-                         pack_elts(dqa[db][2] * p.sm_scale, dqa[db][3] * p.sm_scale)};
-        *reinterpret_cast<u32x2*>(op + db * 16 + 4 * qg) = w;
-      }
-    }
-  }
-
-  // ---- left to right: P, dS, G_ij = sum_h dS dS/ddelta, its running sum over the keys, W ------------------------------
-  float gcarry = 0.f;
-  // one chunk of look-ahead here too
-  float sl_n, sv_n[G], gv_n[G], dp_n[G];
-  auto fetch = [&](int c) __attribute__((always_inline)) {
-    const int j = c * kWave + lane;
-    const int jc = min(j, i);
-    sl_n = *byte_offset(w_row, 4u * jc);
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      sv_n[h] = *byte_offset(p_row[h], 4u * jc);
-      gv_n[h] = *byte_offset(ds_row[h], 4u * jc);
-      dp_n[h] = *byte_offset(dp_row[h], 4u * jc);
+      sv_n[set][h] = *reinterpret_cast<const keys_t*>(byte_offset(s_base + h * ws.NN, off));
+      gv_n[set][h] = *reinterpret_cast<const keys_t*>(byte_offset(ds_base + h * ws.NN, off));
     }
   };
-  fetch(0);
-#pragma unroll 1
-  for (int c = 0; c < n_chunks; ++c) {
-    const int j = c * kWave + lane;
-    const bool valid = j <= i;
-    // take this chunk's values out of the look-ahead registers and request the next chunk's before anything is stored,
+  float gcarry = 0.f;
+  auto chunk = [&](int c, auto set_c) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      lds_order();
+      park(vraw[t], kt);
+      lds_order();
+      take(vraw[t], kt);
+      f32x4 dp = f32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) dp = mfma16(vraw[t][ks], dop[ks], dp);
+      *reinterpret_cast<f32x4*>(dpt + (half * 8 + sub) * PS + 16 * t + 4 * g) = dp;
+    }
+    // take this chunk's values out of the look-ahead registers and request the later chunks' before anything is stored,
     // so that waiting for them never waits for this chunk's stores
-    const float slope = sl_n;
-    float sv[G], gv[G], dpc[G];
+    const keys_t slope = sl_n[set];
+    keys_t sv[G], gv[G];
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-      sv[h] = sv_n[h];
-      gv[h] = gv_n[h];
-      dpc[h] = dp_n[h];
+      sv[h] = sv_n[set][h];
+      gv[h] = gv_n[set][h];
     }
-    if (c + 1 < n_chunks) fetch(c + 1);
-    float gij = 0.f;
-    float prv[G], dsv[G];
+    fetch_v(min(c + 1, n_chunks - 1));
+    fetch_rows(min(c + 2, n_chunks - 1), set_c);
+    lds_order();   // dP is in LDS
+    float gij[R];
+#pragma unroll
+    for (int x = 0; x < R; ++x) gij[x] = 0.f;
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-      prv[h] = __expf(sv[h] - m_row[h]) * inv_l[h];
-      dsv[h] = prv[h] * (dpc[h] - dsum[h]);
-      gij = __builtin_fmaf(dsv[h], gv[h], gij);
-    }
-    gij = valid ? gij : 0.f;
-    const float pre = wave_prefix_sum(gij);   // over the keys at and to the left of this one
-    const float wij = valid ? (gcarry + pre - gij) * slope : 0.f;   // (sum of G over the keys j < t) z'(t)
-    gcarry += wave_last(pre);
-    if (valid) {
+      const keys_t dp = *reinterpret_cast<const keys_t*>(dpt + (col2 + h) * PS + key0);
 #pragma unroll
-      for (int h = 0; h < G; ++h) {
-        *byte_offset(p_row[h], 4u * j) = prv[h];
-        *byte_offset(ds_row[h], 4u * j) = dsv[h];
+      for (int x = 0; x < R; ++x) {
+        const float pr = fast_exp2(sv[h][x] - m_row[h]) * l_row[h];
+        const float ds = pr * (dp[x] - d_row[h]);
+        gij[x] = __builtin_fmaf(ds, gv[h][x], gij[x]);
+        gv[h][x] = ds;
       }
-      *byte_offset(w_row, 4u * j) = wij;
     }
+    lds_order();   // ... and read: the next chunk's may overwrite it
+    float tot = 0.f;
+#pragma unroll
+    for (int x = 0; x < R; ++x) {
+      if (c * kWave + key0 + x > i2) gij[x] = 0.f;   // nothing beyond the diagonal is defined
+      tot += gij[x];
+    }
+    const float pre = segment_prefix_sum<SEG>(tot);
+    float left = gcarry + (pre - tot);               // G over the keys to the left of this lane's first
+    gcarry += segment_last<SEG>(pre);
+    keys_t wij;
+#pragma unroll
+    for (int x = 0; x < R; ++x) {
+      wij[x] = left * slope[x];                      // (sum of G over the keys j < t) z'(t)
+      left += gij[x];
+    }
+    const uint32_t off = at + 256u * c;
+#pragma unroll
+    for (int h = 0; h < G; ++h) *reinterpret_cast<keys_t*>(byte_offset(ds_base + h * ws.NN, off)) = gv[h];
+    *reinterpret_cast<keys_t*>(byte_offset(w_base, off)) = wij;
+  };
+  fetch_rows(0, std::integral_constant<int, 0>{});
+  fetch_v(0);
+  fetch_rows(min(1, n_chunks - 1), std::integral_constant<int, 1>{});
+#pragma unroll 1
+  for (int c = 0; c < n_chunks; c += 2) {
+    chunk(c, std::integral_constant<int, 0>{});
+    if (c + 1 == n_chunks) break;
+    chunk(c + 1, std::integral_constant<int, 1>{});
   }
 }
 
@@ -533,8 +605,8 @@ template <int D>
 __global__ __launch_bounds__(4 * kWave) void corope_bwd_dq_leader_kernel(CoropeBwdParams p, CoropeBwdWs ws) {
   constexpr int TS = D + 16, NDB = D / 32, NT = 4 * kWave, STEP = 16;
   __shared__ __attribute__((aligned(16))) uint16_t tile[STEP * TS];
-  const int g = blockIdx.y;
-  const int rb = (int)gridDim.x - 1 - (int)blockIdx.x;            // the last row blocks see the most keys: first
+  const int n_groups = p.B * p.Hkv, g = (int)(blockIdx.x % n_groups);
+  const int rb = (int)(gridDim.x / n_groups) - 1 - (int)(blockIdx.x / n_groups);   // the last row blocks of all groups see the most keys: first
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int r = lane % 32, hf = lane / 32;
   const int N = p.N, b = g / p.Hkv, kvh = g % p.Hkv, G = p.Hq / p.Hkv;
@@ -665,8 +737,8 @@ __global__ __launch_bounds__(256) void corope_bwd_sum_kernel(const float* parts,
 // ---------------------------------------------------------------------------------------------------- dv
 // dv_j = sum_{h, i} P^h_ij dO^h_i on the matrix cores: dv^T (d x keys) += dO^T (d x rows) P (rows x keys), 16 rows per
 // step.  A workgroup of 4 waves takes 128 keys at a time (32 per wave) of one group, equal shares of the rows as above; the 16 dO
-// rows of every head are staged in LDS and read transposed; P comes straight from the workspace (lane = key: 128-byte lines) and
-// is rounded to bf16.
+// rows of every head are staged in LDS and read transposed; S comes straight from the workspace (lane = key: 128-byte lines), becomes P
+// with the row's statistics and is rounded to the element type.
 constexpr int kDvRows = 16;
 
 template <int D, int G>
@@ -674,6 +746,8 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
   constexpr int TS = D + 16, NDB = D / 32, NT = 4 * kWave, ROWS = kDvRows;
   constexpr int UNITS = G * ROWS * (D / 8), PER = (UNITS + NT - 1) / NT;   // 16-byte pieces of a dO tile, per thread
   __shared__ __attribute__((aligned(16))) uint16_t tile[G * ROWS * TS];
+  __shared__ __attribute__((aligned(16))) float stat[2][2 * G * ROWS];   // two steps' [reference values, 1 / sums][head][row]
+  static_assert(2 * G * ROWS <= NT, "one statistic per thread");
   const int g = blockIdx.y;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int r = lane % 32, hf = lane / 32;
@@ -695,7 +769,14 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
     // Both streams run one step ahead in registers: the steps of a piece follow one after the other, and with a step's loads
     // issued only when the step begins its time is that many memory latencies.
     u32x4 dreg[PER];
-    float pnext[G][8];
+    float pnext[G][8], stat_next = 0.f;
+    auto fetch_stat = [&](int i0) __attribute__((always_inline)) {
+      const int i = i0 + threadIdx.x % ROWS;
+      if (threadIdx.x < 2 * G * ROWS) stat_next = i < N ? ws.row_max(g, G, N, threadIdx.x / ROWS)[i] : 0.f;
+    };
+    auto park_stat = [&](int step) __attribute__((always_inline)) {
+      if (threadIdx.x < 2 * G * ROWS) stat[step % 2][threadIdx.x] = stat_next;
+    };
     auto fetch = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < PER; ++u) {
@@ -707,30 +788,40 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
       const int64_t row_len = 64 * (i0 / 64 + 1);           // the 16 rows of a step share a row length
 #pragma unroll
       for (int h = 0; h < G; ++h) {
-        const float* prow = ws.p(head0 + h) + tri_row_start(min(i0, N - 1)) + j;
+        const float* srow = ws.s(head0 + h) + tri_row_start(min(i0, N - 1)) + j;
 #pragma unroll
         for (int x = 0; x < 8; ++x) {
           const int i = i0 + 8 * hf + x;
-          pnext[h][x] = (wave_on && i < N && j <= i) ? prow[row_len * (8 * hf + x)] : 0.f;   // nothing outside the triangle is defined
+          pnext[h][x] = (wave_on && i < N && j <= i) ? srow[row_len * (8 * hf + x)] : -INFINITY;   // nothing outside the triangle is defined
         }
       }
     };
     const int row_begin = jb + ROWS * (t - b0);
     fetch(row_begin);
+    fetch_stat(row_begin);
+    __syncthreads();   // the previous piece's reads are done
+    park_stat(0);
+    fetch_stat(row_begin + ROWS);
 #pragma unroll 1
-    for (int i0 = row_begin; i0 < row_end; i0 += ROWS) {
-      __syncthreads();   // the previous step's reads of the tile are done
+    for (int i0 = row_begin, step = 0; i0 < row_end; i0 += ROWS, ++step) {
+      __syncthreads();   // the previous step's reads of the tile are done, this step's statistics are there
 #pragma unroll
       for (int u = 0; u < PER; ++u) {
         const int e = threadIdx.x + u * NT;
         if (UNITS % NT == 0 || e < UNITS)
           *reinterpret_cast<u32x4*>(tile + (e / (D / 8)) * TS + 8 * (e % (D / 8))) = dreg[u];   // rows are (head, row) pairs
       }
+      park_stat(step + 1);   // (two steps ahead of their use, so that the weights are ready when the tile is)
+      fetch_stat(i0 + 2 * ROWS);
+      const float* st = stat[step % 2];
       u32x4 bop[G];
 #pragma unroll
-      for (int h = 0; h < G; ++h)
-        bop[h] = u32x4{pack_elts(pnext[h][0], pnext[h][1]), pack_elts(pnext[h][2], pnext[h][3]),
-                       pack_elts(pnext[h][4], pnext[h][5]), pack_elts(pnext[h][6], pnext[h][7])};
+      for (int h = 0; h < G; ++h) {
+        float w[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) w[x] = fast_exp2(pnext[h][x] - st[h * ROWS + 8 * hf + x]) * st[(G + h) * ROWS + 8 * hf + x];
+        bop[h] = u32x4{pack_elts(w[0], w[1]), pack_elts(w[2], w[3]), pack_elts(w[4], w[5]), pack_elts(w[6], w[7])};
+      }
       const bool wave_on = i0 + ROWS - 1 >= jw && jw < N;
       if (i0 + ROWS < row_end) fetch(i0 + ROWS);
       __syncthreads();
@@ -953,22 +1044,33 @@ static int corope_bwd_shares(int N, int n_groups_total, int64_t slots) {
   return (int)std::max<int64_t>(1, std::min({want, slots / 2, (int64_t)CoropeShares<ROWS>(N).total}));
 }
 
+// Rows per wave of the scores kernel: as many as fill the 16 columns where that leaves two waves per SIMD twice over; below that
+// fewer rows per wave give more waves.  Decided on the whole call's groups, so a smaller workspace gives the same bits.
+template <int D, int G>
+static void launch_corope_bwd_scores(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, int n_groups_total,
+                                     hipStream_t stream) {
+  constexpr int kMost = G <= 4 ? 4 : 2;
+  const int64_t rows = (int64_t)p.N * n_groups_total, simds = 4 * device_cu_count();
+  const int n_groups = p.B * p.Hkv;
+  auto blocks = [&](int R) { return dim3((unsigned)((p.N + R - 1) / R) * n_groups); };
+  if (kMost > 2 && rows >= 4 * simds * kMost)
+    hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, kMost>), blocks(kMost), dim3(kWave), 0, stream, p, ws, fr);
+  else if (rows >= 8 * simds)
+    hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, 2>), blocks(2), dim3(kWave), 0, stream, p, ws, fr);
+  else
+    hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, 1>), blocks(1), dim3(kWave), 0, stream, p, ws, fr);
+}
+
 template <int D, int G>
 static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, int n_groups_total,
                                         hipStream_t stream) {
-  const dim3 rows(p.N, p.B * p.Hkv);
   const int nt = (p.N + 127) / 128;
-  hipLaunchKernelGGL(corope_bwd_rowdot_kernel<D>, dim3(nt, nt, p.B * p.Hkv), dim3(4 * kWave), 0, stream, p.q, p.k,
-                     ws.delta(0), ws.NN, p.N, G, 1);
-  hipLaunchKernelGGL(corope_bwd_rowdot_kernel<D>, dim3(nt, nt, p.B * p.Hq), dim3(4 * kWave), 0, stream, p.d_o, p.v,
-                     ws.dp(0), ws.NN, p.N, 1, G);
-  hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G>), rows, dim3(kWave), 0, stream, p, ws, fr);
-  hipLaunchKernelGGL(corope_bwd_dq_leader_kernel<D>, dim3((p.N + 127) / 128, p.B * p.Hkv), dim3(4 * kWave), 0, stream, p, ws);
+  launch_corope_bwd_scores<D, G>(p, ws, fr, n_groups_total, stream);
+  hipLaunchKernelGGL(corope_bwd_dq_leader_kernel<D>, dim3((unsigned)nt * p.B * p.Hkv), dim3(4 * kWave), 0, stream, p, ws);
   using Cfg = CoropeDkCfg<D, G>;
-  // The dP matrices are not needed any more behind the scores kernel: they hold the partial sums, first of dv, then of dk.
-  const int64_t group_floats = G * ws.NN, slots = group_floats / (kDkKeys * D);
+  const int64_t group_floats = G * ws.NN, slots = ws.part_floats(G, p.N) / (kDkKeys * D);
   const int dv_shares = corope_bwd_shares<kDvRows>(p.N, n_groups_total, slots), dk_shares = corope_bwd_shares<kDkRows>(p.N, n_groups_total, slots);
-  float* parts = ws.dp(0);
+  float* parts = ws.parts(0, G);
   const int n_groups = p.B * p.Hkv, n_blocks = (p.N + kDkKeys - 1) / kDkKeys;
   hipLaunchKernelGGL((corope_bwd_dv_kernel<D, G>), dim3(dv_shares, n_groups), dim3(4 * kWave), 0, stream, p, ws, parts, group_floats);
   if (dv_shares > 1)

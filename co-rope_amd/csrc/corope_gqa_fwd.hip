@@ -41,7 +41,7 @@
 namespace COROPE_NS {
 
 struct CoropeFreqs {
-  float w[64];  // inverse frequencies divided by 2*pi (revolutions per unit of delta), D/2 entries used
+  alignas(16) float w[64];  // inverse frequencies divided by 2*pi (revolutions per unit of delta), D/2 entries used
 };
 
 constexpr int kCoropeWaves = 4, kCoropeKeys = 64;
@@ -100,9 +100,10 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
 #pragma unroll
   for (int hk = 0; hk < HK; ++hk)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int d = 32 * hk + e;
-      turns[hk][e] = g == 0 ? fr.w[d] : g == 1 ? fr.w[d + 8] : g == 2 ? fr.w[d + 16] : fr.w[d + 24];
+    for (int e = 0; e < 8; e += 4) {
+      const f32x4 t = *reinterpret_cast<const f32x4*>(fr.w + 32 * hk + 8 * g + e);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) turns[hk][e + x] = t[x];
     }
 
 #pragma unroll

@@ -313,3 +313,20 @@ def test_corope_backward_cut_key_blocks(pkg, B, Hq, Hkv, N, D):
     q, k, v, d_o = _inputs(B, Hq, Hkv, N, D, seed=11)
     scale = 1 / math.sqrt(D)
     _compare(_gpu_grads(pkg, q, k, v, d_o, scale, 1e4), _oracle_grads(q, k, v, d_o, scale, 1e4), Hq // Hkv)
+
+
+# Many short groups: every number of query rows a wave of the scores kernel takes (by group size and by how many rows there are), with
+# lengths that end inside a wave's rows, a block of 16 keys and a chunk.  Three of the groups against the oracle.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("groups,G,N,D", [(240, 1, 70, 64), (240, 2, 69, 128), (240, 3, 73, 128), (240, 4, 70, 64), (120, 4, 75, 128),
+                                          (120, 5, 71, 64), (120, 8, 70, 128), (120, 7, 97, 64), (120, 2, 81, 64)])
+def test_corope_backward_many_groups(pkg, groups, G, N, D, dtype):
+    dev = torch.device("cuda:0")
+    q, k, v, d_o = _inputs(groups, G, 1, N, D, seed=23)
+    scale = 1 / math.sqrt(D)
+    qd, kd, vd = (t.to(dev, dtype).requires_grad_(True) for t in (q, k, v))
+    pkg.corope_attention(qd, kd, vd, True, scale, 10000.0).backward(d_o.to(dev, dtype))
+    torch.cuda.synchronize()
+    for g in (0, groups // 2, groups - 1):
+        sl = slice(g, g + 1)
+        _compare([t.grad[sl].float().cpu() for t in (qd, kd, vd)], _oracle_grads(q[sl], k[sl], v[sl], d_o[sl], scale, 10000.0), G)

@@ -236,10 +236,11 @@ def _backward_rotated(lib, q_rot, k_rot, v, o, do, M, fc, fs, sm_scale, causal):
         do = do if do_st is not None else do.contiguous()
     dq, dk, dv = torch.empty_like(q_rot), torch.empty_like(k_rot), torch.empty_like(k_rot)
     delta = torch.empty_like(M)
-    # scratch in which the dK+dV launch leaves the partial sums of key blocks it cuts among workgroups (0: none are cut)
-    nbytes = lib.corope_rope_attn_bwd_rotated_parts_bytes(B, H, Hkv, N, D, int(causal))
-    parts = torch.empty(nbytes, device=q_rot.device, dtype=torch.uint8) if nbytes > 0 else None
     with _on_device(q_rot):
+        # scratch in which the dK+dV launch leaves the partial sums of key blocks it cuts among workgroups (0: none are cut); how
+        # many pieces there are depends on the device
+        nbytes = lib.corope_rope_attn_bwd_rotated_parts_bytes(B, H, Hkv, N, D, int(causal))
+        parts = torch.empty(nbytes, device=q_rot.device, dtype=torch.uint8) if nbytes > 0 else None
         rc = lib.corope_rope_attn_bwd_rotated(q_rot.data_ptr(), k_rot.data_ptr(), v.data_ptr(), v_st, o.data_ptr(), do.data_ptr(), do_st,
                                               M.data_ptr(), delta.data_ptr(), fc.data_ptr(), fs.data_ptr(), fc.stride(0), dq.data_ptr(),
                                               dk.data_ptr(), dv.data_ptr(), B, H, Hkv, N, D, sm_scale, int(causal),
@@ -259,7 +260,9 @@ class _FusedRopeAttn(torch.autograd.Function):
         # when a gradient will be asked for, the forward keeps its rotated q and k for the backward and the originals
         # are not saved (the reference saves q and k, fused_rope_attn.py:718, and re-rotates them in its backward)
         o, M, fc, fs, rotated = _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, keep_rotated=training)
-        if not training:   # nothing is kept: saving q, k, v here would also copy strided views of a fused projection
+        # nothing to differentiate, nothing kept: saving q, k, v would also copy strided views of a fused projection.  (Tables that
+        # ask for a gradient get None, but the backward that says so runs and wants its tensors.)
+        if not any(ctx.needs_input_grad):
             return o
         ctx.rotated = rotated is not None
         if ctx.rotated:

@@ -445,3 +445,15 @@ def test_backward_cut_key_blocks(pkg, B, Hq, Hkv, N, D, cut, causal, dtype):
         ok, err = within_bar(a.float().cpu(), b, 2.4e-2 * (math.sqrt(G) if name != "dQ" else 1.0))[:2]
         print(f"  {name}: max-abs {err:.3e} (|ref| max {b.abs().max():.2f})", flush=True)
         assert ok, name
+
+
+# Only the tables ask for a gradient: the operator has none for them, and its backward says so with the tensors its forward kept.
+@pytest.mark.parametrize("N", [130, 1024])
+def test_backward_when_only_the_tables_ask_for_a_gradient(pkg, N):
+    dev = torch.device("cuda:0")
+    q, k, v, _, c, s = _case(1, 2, N, 64)
+    c = c.to(dev).requires_grad_(True)
+    o = pkg.attention(*(t.to(dev, torch.bfloat16) for t in (q, k, v)), True, 0.125, c, s.to(dev))
+    assert o.requires_grad
+    o.sum().backward()
+    assert c.grad is None

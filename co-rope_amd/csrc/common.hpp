@@ -92,10 +92,12 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
 
 // ---- the element type of the attention kernels: two elements per 32-bit word, element 0 in the low half -------------
 #ifdef COROPE_F16
+constexpr bool kEltIsF16 = true;
 __device__ __forceinline__ float elt_lo(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[0]; }
 __device__ __forceinline__ float elt_hi(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[1]; }
 __device__ __forceinline__ uint32_t pack_elts(float lo, float hi) { return pack_f16(lo, hi); }
 #else
+constexpr bool kEltIsF16 = false;
 __device__ __forceinline__ float elt_lo(uint32_t w) { return bf16_lo(w); }
 __device__ __forceinline__ float elt_hi(uint32_t w) { return bf16_hi(w); }
 __device__ __forceinline__ uint32_t pack_elts(float lo, float hi) { return pack_bf16(lo, hi); }

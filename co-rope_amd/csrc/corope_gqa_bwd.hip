@@ -859,7 +859,11 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
 //       matrix cores - the contraction is only G long, but it takes 2G multiply-adds per (key, pair) off the vector
 //       units; the result lands as lane = column (mod 32), registers = 16 of the wave's keys;
 //   rotation and accumulation on the vector units: lane (c, half) owns pairs c and c + 32 (D = 128) for the 16 keys of
-//       its half: one (sin, cos) and six multiply-adds per (row, key, pair).
+//       its half: one (sin, cos) and four multiply-adds per (row, key, pair).
+// The gate path W qL contracts over rows, so a tile's 8 rows are one more product into the same accumulators (on the vector units it was 2 of
+// 12 issue slots per (row, key, pair)).  W is split into three bf16 parts, 24 bits whatever its scale, and an fp16 query into two.
+// What bounds it: the vector units, 10 issue slots per (row, key, pair).  Measured with the gate path moved: B2 Hq32 Hkv8 N4096 D128
+// forward + backward 15.0 -> 14.6 ms, B2 Hq8 Hkv2 N512 D64 133 -> 130.5 us.
 // A workgroup takes its share of the group's (block, row tile) list as above.  Tiles of DELTA, W, DS^h ([row][matrix][key], fp32) and the rows' queries
 // ([row][column][head], bf16, heads padded to 8 with zeros: the B operand is then one 16-byte read) go through LDS,
 // fetched into registers one tile ahead.
@@ -936,11 +940,9 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
         }
       });
     };
-    float dk1[NP][16], dk2[NP][16];
+    f32x16 dk1[NP], dk2[NP];
 #pragma unroll
-    for (int np = 0; np < NP; ++np)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) dk1[np][e] = dk2[np][e] = 0.f;
+    for (int np = 0; np < NP; ++np) dk1[np] = dk2[np] = f32x16{0};
 
     fetch(row_begin);
 #pragma unroll 1
@@ -962,10 +964,48 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
       });
       __syncthreads();
       if (i0 + kDkRows < row_end) fetch(i0 + kDkRows);
+      if (i0 < jw) continue;   // wave-uniform: all keys of this wave lie above the diagonal of the tile's rows
+      // gate path: dk += W^T qL over the tile's 8 rows.  W enters as three bf16 parts (24 bits, any range), an fp16 query as two.
+      {
+        float hi[8], mid[8], lo[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          const float wij = tile[(x * MATS + 1) * kDkKeys + 32 * wave + col];
+          hi[x] = bf16_to_f(f_to_bf16(wij));
+          const float rest = wij - hi[x];
+          mid[x] = bf16_to_f(f_to_bf16(rest));
+          lo[x] = rest - mid[x];
+        }
+        u32x4 a1, a2;   // contraction slots of half 0: hi, then lo; of half 1: mid, then nothing
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const uint32_t h2 = pack_bf16(hi[2 * x], hi[2 * x + 1]), m2 = pack_bf16(mid[2 * x], mid[2 * x + 1]);
+          const uint32_t l2 = pack_bf16(lo[2 * x], lo[2 * x + 1]);
+          a1[x] = hf == 0 ? h2 : m2;
+          a2[x] = hf == 0 ? l2 : 0u;
+        }
+#pragma unroll
+        for (int cb = 0; cb < 2 * NP; ++cb) {
+          const uint16_t* ql = qT + (32 * cb + col) * 8;
+          u32x4 b1, b2;
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const uint32_t q2 = ql[2 * x * D * 8] | (uint32_t)ql[(2 * x + 1) * D * 8] << 16;
+            b1[x] = kEltIsF16 ? pack_bf16(elt_lo(q2), elt_hi(q2)) : q2;
+            if constexpr (kEltIsF16) b2[x] = pack_bf16(elt_lo(q2) - bf16_lo(b1[x]), elt_hi(q2) - bf16_hi(b1[x]));
+          }
+          f32x16& acc = cb < NP ? dk1[cb % NP] : dk2[cb % NP];
+          if constexpr (kEltIsF16) {
+            acc = mfma32_bf16(a2, b2, acc);
+            acc = mfma32_bf16(a1, b2, acc);
+          }
+          acc = mfma32_bf16(a2, b1, acc);
+          acc = mfma32_bf16(a1, b1, acc);
+        }
+      }
       const int n_rows = min(kDkRows, N - i0);
 #pragma unroll 1
       for (int r = 0; r < n_rows; ++r) {
-        if (i0 + r < jw) continue;   // wave-uniform: all keys of this wave lie above the diagonal of this row
         const float* trow = tile + r * MATS * kDkKeys + 32 * wave;
         // A: (32 keys x 16 contraction slots): lane (key, half 0) holds dS^h for h = 0..7 rounded to bf16, half 1 what the
         // rounding left over (again as bf16); with the queries of heads 0..7 in both halves of B the product carries dS to
@@ -980,28 +1020,23 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
           }
           aop = u32x4{pack_elts(dsv[0], dsv[1]), pack_elts(dsv[2], dsv[3]), pack_elts(dsv[4], dsv[5]), pack_elts(dsv[6], dsv[7])};
         }
-        // delta and W of this lane's 16 keys: keys 8 n + 4 half + 0..3 for n = 0..3, as the accumulator rows are laid out
-        f32x4 dl[4], wg[4];
+        // delta of this lane's 16 keys: keys 8 n + 4 half + 0..3 for n = 0..3, as the accumulator rows are laid out
+        f32x4 dl[4];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) {
-          dl[n] = *reinterpret_cast<const f32x4*>(trow + 8 * n + 4 * hf);
-          wg[n] = *reinterpret_cast<const f32x4*>(trow + kDkKeys + 8 * n + 4 * hf);
-        }
-        // B: (heads x 32 columns) per column block; the same read also carries the leader's (head 0) value of the column.
-        // One rotation pair per pass (columns 32 np + col and the same + D/2), so that only two product blocks are live.
+        for (int n = 0; n < 4; ++n) dl[n] = *reinterpret_cast<const f32x4*>(trow + 8 * n + 4 * hf);
+        // B: (heads x 32 columns) per column block.  One rotation pair per pass (columns 32 np + col and the same + D/2), so that only two product blocks are live.
 #pragma unroll
         for (int np = 0; np < NP; ++np) {
           const u32x4 bq1 = *reinterpret_cast<const u32x4*>(qT + (r * D + 32 * np + col) * 8);
           const u32x4 bq2 = *reinterpret_cast<const u32x4*>(qT + (r * D + 32 * (NP + np) + col) * 8);
-          const float ql1 = elt_lo(bq1[0]), ql2 = elt_lo(bq2[0]);
           const f32x16 u1 = mfma32(aop, bq1, f32x16{0}), u2 = mfma32(aop, bq2, f32x16{0});
 #pragma unroll
           for (int e = 0; e < 16; ++e) {
-            const float delta = dl[e / 4][e % 4], wij = wg[e / 4][e % 4];
+            const float delta = dl[e / 4][e % 4];
             const float x = __builtin_amdgcn_fractf(delta * w_turn[np]);
             const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
-            dk1[np][e] = __builtin_fmaf(cs, u1[e], __builtin_fmaf(-sn, u2[e], __builtin_fmaf(wij, ql1, dk1[np][e])));
-            dk2[np][e] = __builtin_fmaf(cs, u2[e], __builtin_fmaf(sn, u1[e], __builtin_fmaf(wij, ql2, dk2[np][e])));
+            dk1[np][e] = __builtin_fmaf(cs, u1[e], __builtin_fmaf(-sn, u2[e], dk1[np][e]));
+            dk2[np][e] = __builtin_fmaf(cs, u2[e], __builtin_fmaf(sn, u1[e], dk2[np][e]));
           }
         }
       }

@@ -898,6 +898,21 @@ __device__ __forceinline__ uint16_t f_to_f16(float x) { return (uint16_t)(pack_f
 __device__ __forceinline__ uint16_t f_to_elt(float x) { return (uint16_t)(pack_elts(x, 0.f) & 0xffffu); }
 __device__ __forceinline__ float elt_to_f(uint16_t x) { return elt_lo((uint32_t)x); }
 
+// Co-RoPE's phase in revolutions, as v_sin_f32 / v_cos_f32 take it: their input domain is [-256, 256], so it is reduced only where it can
+// leave that.  Over [0, 256) the unreduced sine differs from the reduced one by at most 7e-10 (23 of 65536 values a unit) and the cosine not
+// at all; the error against 64 bits is the same 1.2e-7.
+template <bool REDUCE>
+__device__ __forceinline__ float corope_phase(float x) { return REDUCE ? __builtin_amdgcn_fractf(x) : x; }
+// How many leading blocks of 32 rotation pairs have to be reduced: delta is a sum of at most N gates of at most 1.  turns: revolutions per
+// unit of delta, D / 2 of them.  A template argument of the kernels, because the reduction is one of ten issue slots per (row, key,
+// pair): forward B1 Hq32 Hkv8 N1111 D128 152.8 -> 144.8 us (none reduced), forward + backward B2 Hq32 Hkv8 N4096 D128 15.00 -> 14.66 ms (half).
+inline int corope_reduced_blocks(const float* turns, int D, int N) {
+  int blocks = 0;
+  for (int d = 0; d < D / 2; ++d)
+    if (!(turns[d] * (float)N < 255.f)) blocks = d / 32 + 1;
+  return blocks;
+}
+
 // f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>): a loop whose index is a compile-time constant
 // in the body, so register arrays indexed with it never look dynamically indexed to the optimiser.
 template <int... I, class F>

@@ -95,7 +95,7 @@ struct CoropeBwdWs {
 // 12 floats more per (row, key) and a launch.
 // Measured at B2 Hq32 Hkv8 N4096 D128: 8.2 -> 5.9 ms, first sweep 4.6 (one wave per row with the rotated keys in LDS, behind launches for the
 // logits and dP); B2 Hq8 Hkv2 N512 D64 52 -> 40 us.
-template <int D, int G, int R>
+template <int D, int G, int R, int REDUCED>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void corope_bwd_scores_kernel(CoropeBwdParams p, CoropeBwdWs ws,
                                                                                                           CoropeBwdFreqs fr) {
   constexpr int TS = D + 16, HALF = D / 2;   // LDS row stride: the row-wise writes and the transposing reads both spread over the banks
@@ -317,12 +317,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
       constexpr int r = decltype(r_c)::value, s = r / RH;
       const float delta_r = R == 1 ? delta : __shfl(delta, 64 / R * r + n);
       f32x4 acc = f32x4{0, 0, 0, 0};
-#pragma unroll
-      for (int hk = 0; hk < HK; ++hk) {
+      static_for<HK>([&](auto hk_c) __attribute__((always_inline)) {
+        constexpr int hk = decltype(hk_c)::value;
         f16x8 y1, y2;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float x = __builtin_amdgcn_fractf(delta_r * turns[hk][e]);
+          const float x = corope_phase<(hk < REDUCED)>(delta_r * turns[hk][e]);
           const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
           y1[e] = (_Float16)__builtin_fmaf(cs, k1[hk][e], sn * k2[hk][e]);
           y2[e] = (_Float16)__builtin_fmaf(cs, k2[hk][e], -(sn * k1[hk][e]));
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
         *reinterpret_cast<u32x4*>(dst + HALF) = w2;
         acc = mfma16_f16(w1, qop[s][hk], acc);
         acc = mfma16_f16(w2, qop[s][HK + hk], acc);
-      }
+      });
       if (r % RH == 0) {
         m[s] = acc;
       } else {
@@ -877,7 +877,7 @@ struct CoropeDkCfg {
   static constexpr int kLdsBytes = kMatBytes + kQBytes;
 };
 
-template <int D, int G>
+template <int D, int G, int REDUCED>
 __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu(2))) void corope_bwd_dk_kernel(CoropeBwdParams p, CoropeBwdWs ws,
                                                                        CoropeBwdFreqs fr, float* parts, int64_t group_floats) {
   using Cfg = CoropeDkCfg<D, G>;
@@ -1025,20 +1025,20 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
         for (int n = 0; n < 4; ++n) dl[n] = *reinterpret_cast<const f32x4*>(trow + 8 * n + 4 * hf);
         // B: (heads x 32 columns) per column block.  One rotation pair per pass (columns 32 np + col and the same + D/2), so that only two product blocks are live.
-#pragma unroll
-        for (int np = 0; np < NP; ++np) {
+        static_for<NP>([&](auto np_c) __attribute__((always_inline)) {
+          constexpr int np = decltype(np_c)::value;
           const u32x4 bq1 = *reinterpret_cast<const u32x4*>(qT + (r * D + 32 * np + col) * 8);
           const u32x4 bq2 = *reinterpret_cast<const u32x4*>(qT + (r * D + 32 * (NP + np) + col) * 8);
           const f32x16 u1 = mfma32(aop, bq1, f32x16{0}), u2 = mfma32(aop, bq2, f32x16{0});
 #pragma unroll
           for (int e = 0; e < 16; ++e) {
             const float delta = dl[e / 4][e % 4];
-            const float x = __builtin_amdgcn_fractf(delta * w_turn[np]);
+            const float x = corope_phase<(np < REDUCED)>(delta * w_turn[np]);
             const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
             dk1[np][e] = __builtin_fmaf(cs, u1[e], __builtin_fmaf(-sn, u2[e], dk1[np][e]));
             dk2[np][e] = __builtin_fmaf(cs, u2[e], __builtin_fmaf(sn, u1[e], dk2[np][e]));
           }
-        }
+        });
       }
     }
     const bool whole = t == b0 && seg_end == b1;
@@ -1081,7 +1081,7 @@ static int corope_bwd_shares(int N, int n_groups_total, int64_t slots) {
 
 // Rows per wave of the scores kernel: as many as fill the 16 columns where that leaves two waves per SIMD twice over; below that
 // fewer rows per wave give more waves.  Decided on the whole call's groups, so a smaller workspace gives the same bits.
-template <int D, int G>
+template <int D, int G, int REDUCED>
 static void launch_corope_bwd_scores(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, int n_groups_total,
                                      hipStream_t stream) {
   constexpr int kMost = G <= 4 ? 4 : 2;
@@ -1089,18 +1089,18 @@ static void launch_corope_bwd_scores(const CoropeBwdParams& p, const CoropeBwdWs
   const int n_groups = p.B * p.Hkv;
   auto blocks = [&](int R) { return dim3((unsigned)((p.N + R - 1) / R) * n_groups); };
   if (kMost > 2 && rows >= 4 * simds * kMost)
-    hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, kMost>), blocks(kMost), dim3(kWave), 0, stream, p, ws, fr);
+    hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, kMost, REDUCED>), blocks(kMost), dim3(kWave), 0, stream, p, ws, fr);
   else if (rows >= 8 * simds)
-    hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, 2>), blocks(2), dim3(kWave), 0, stream, p, ws, fr);
+    hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, 2, REDUCED>), blocks(2), dim3(kWave), 0, stream, p, ws, fr);
   else
-    hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, 1>), blocks(1), dim3(kWave), 0, stream, p, ws, fr);
+    hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, 1, REDUCED>), blocks(1), dim3(kWave), 0, stream, p, ws, fr);
 }
 
-template <int D, int G>
+template <int D, int G, int REDUCED>
 static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, int n_groups_total,
                                         hipStream_t stream) {
   const int nt = (p.N + 127) / 128;
-  launch_corope_bwd_scores<D, G>(p, ws, fr, n_groups_total, stream);
+  launch_corope_bwd_scores<D, G, REDUCED>(p, ws, fr, n_groups_total, stream);
   hipLaunchKernelGGL(corope_bwd_dq_leader_kernel<D>, dim3((unsigned)nt * p.B * p.Hkv), dim3(4 * kWave), 0, stream, p, ws);
   using Cfg = CoropeDkCfg<D, G>;
   const int64_t group_floats = G * ws.NN, slots = ws.part_floats(G, p.N) / (kDkKeys * D);
@@ -1111,7 +1111,7 @@ static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBw
   if (dv_shares > 1)
     hipLaunchKernelGGL((corope_bwd_sum_kernel<D, kDvRows>), dim3(n_blocks, n_groups, 8), dim3(256), 0, stream, parts, group_floats, p.dv,
                        p.N, dv_shares, 1.f);
-  auto kern = corope_bwd_dk_kernel<D, G>;
+  auto kern = corope_bwd_dk_kernel<D, G, REDUCED>;
   static std::atomic<uint64_t> lds_ok{0};
   if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3(dk_shares, n_groups), dim3(kDkWaves * kWave), Cfg::kLdsBytes, stream, p, ws, fr, parts, group_floats);
@@ -1121,18 +1121,18 @@ static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBw
   return hipGetLastError();
 }
 
-template <int D>
+template <int D, int REDUCED>
 static hipError_t launch_corope_bwd_d(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, int n_groups_total,
                                       hipStream_t stream) {
   switch (p.Hq / p.Hkv) {
-    case 1: return launch_corope_bwd_cfg<D, 1>(p, ws, fr, n_groups_total, stream);
-    case 2: return launch_corope_bwd_cfg<D, 2>(p, ws, fr, n_groups_total, stream);
-    case 3: return launch_corope_bwd_cfg<D, 3>(p, ws, fr, n_groups_total, stream);
-    case 4: return launch_corope_bwd_cfg<D, 4>(p, ws, fr, n_groups_total, stream);
-    case 5: return launch_corope_bwd_cfg<D, 5>(p, ws, fr, n_groups_total, stream);
-    case 6: return launch_corope_bwd_cfg<D, 6>(p, ws, fr, n_groups_total, stream);
-    case 7: return launch_corope_bwd_cfg<D, 7>(p, ws, fr, n_groups_total, stream);
-    case 8: return launch_corope_bwd_cfg<D, 8>(p, ws, fr, n_groups_total, stream);
+    case 1: return launch_corope_bwd_cfg<D, 1, REDUCED>(p, ws, fr, n_groups_total, stream);
+    case 2: return launch_corope_bwd_cfg<D, 2, REDUCED>(p, ws, fr, n_groups_total, stream);
+    case 3: return launch_corope_bwd_cfg<D, 3, REDUCED>(p, ws, fr, n_groups_total, stream);
+    case 4: return launch_corope_bwd_cfg<D, 4, REDUCED>(p, ws, fr, n_groups_total, stream);
+    case 5: return launch_corope_bwd_cfg<D, 5, REDUCED>(p, ws, fr, n_groups_total, stream);
+    case 6: return launch_corope_bwd_cfg<D, 6, REDUCED>(p, ws, fr, n_groups_total, stream);
+    case 7: return launch_corope_bwd_cfg<D, 7, REDUCED>(p, ws, fr, n_groups_total, stream);
+    case 8: return launch_corope_bwd_cfg<D, 8, REDUCED>(p, ws, fr, n_groups_total, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1171,7 +1171,11 @@ hipError_t launch_corope_gqa_bwd(const CoropeBwdParams& p, int D, float* workspa
     c.Hkv = gc;
     c.Hq = gc * G;
     CoropeBwdWs ws{workspace, tri_row_start(p.N), gc, gc * G};
-    const hipError_t e = D == 128 ? launch_corope_bwd_d<128>(c, ws, fr, n_groups, stream) : launch_corope_bwd_d<64>(c, ws, fr, n_groups, stream);
+    const int reduced = corope_reduced_blocks(fr.turns, D, p.N);
+    const hipError_t e = D == 64 ? (reduced == 0 ? launch_corope_bwd_d<64, 0>(c, ws, fr, n_groups, stream) : launch_corope_bwd_d<64, 1>(c, ws, fr, n_groups, stream))
+                         : reduced == 0 ? launch_corope_bwd_d<128, 0>(c, ws, fr, n_groups, stream)
+                         : reduced == 1 ? launch_corope_bwd_d<128, 1>(c, ws, fr, n_groups, stream)
+                                        : launch_corope_bwd_d<128, 2>(c, ws, fr, n_groups, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

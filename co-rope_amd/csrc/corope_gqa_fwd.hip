@@ -31,10 +31,11 @@
 //            row statistics are one register per lane.
 //   O^T += V^T P^T  for all R rows at once; P is the B operand as the scores left it (the keys of a contraction step in accumulator
 //            order, V read transposed in the same order).
-// What bounds it: the vector units, 10 issue slots per (row, key, pair) -- one multiply, one range reduction, sine and cosine at two
-// slots each, two multiplies, two multiply-adds that round to fp16 -- of about 12 in all.  Measured at B2 Hq32 Hkv8 N4096 D128:
-// 5.37 -> 3.33 ms (one wave per row, the rotated keys through LDS: 14 slots per pair, the keys four times through
-// LDS and a softmax per head over the lanes), B1 Hq32 Hkv8 N1111 D128 fp16 230 -> 152 us, B2 Hq8 Hkv2 N512 D64 20.9 -> 18.4 us.
+// What bounds it: the vector units, 9 or 10 issue slots per (row, key, pair) -- one multiply, a range reduction where the phase can leave
+// the sine unit's domain (REDUCED: in that many blocks of 32 pairs), sine and cosine at two slots each, two multiplies, two multiply-adds
+// that round to fp16 -- of about 11.5 in all.  Measured at B2 Hq32 Hkv8 N4096 D128: 5.37 -> 3.20 ms (3.33 with every phase reduced; before, one wave per
+// row, the rotated keys through LDS: 14 slots per pair, the keys four times through LDS and a softmax per head over the lanes),
+// B1 Hq32 Hkv8 N1111 D128 fp16 224 -> 145 us (152 with every phase reduced), B2 Hq8 Hkv2 N512 D64 20.9 -> 18.4 us.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -58,7 +59,7 @@ struct CoropeFwdCfg {
 
 // (At D = 64 the registers allow more than two waves per SIMD: with several rows per wave that is 4 % faster, B2 Hq16 Hkv16 N2688
 // 1458 -> 1397 us; with one, where the longest rows set the time, 7 % slower, B1 Hq2 Hkv1 N4096 173 -> 185 us.)
-template <int D, int G, int R>
+template <int D, int G, int R, int REDUCED>
 __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_per_eu(2, R == 1 ? 2 : 8))) void corope_gqa_fwd_kernel(CoropeParams p,
                                                                                                        CoropeFreqs fr) {
   using Cfg = CoropeFwdCfg<D, R>;
@@ -211,19 +212,19 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
         const float delta_r = delta;
         delta = dbuf[(b * R + min(r + 1, R - 1)) * 16 + n];
         f32x4 acc = f32x4{0, 0, 0, 0};
-#pragma unroll
-        for (int hk = 0; hk < HK; ++hk) {
+        static_for<HK>([&](auto hk_c) __attribute__((always_inline)) {
+          constexpr int hk = decltype(hk_c)::value;
           f16x8 y1, y2;
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const float x = __builtin_amdgcn_fractf(delta_r * turns[hk][e]);
+            const float x = corope_phase<(hk < REDUCED)>(delta_r * turns[hk][e]);
             const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
             y1[e] = (_Float16)__builtin_fmaf(cs, k1[hk][e], sn * k2[hk][e]);
             y2[e] = (_Float16)__builtin_fmaf(cs, k2[hk][e], -(sn * k1[hk][e]));
           }
           acc = mfma16_f16(__builtin_bit_cast(u32x4, y1), qop[hk], acc);
           acc = mfma16_f16(__builtin_bit_cast(u32x4, y2), qop[HK + hk], acc);
-        }
+        });
 #pragma unroll
         for (int e = 0; e < 4; ++e) sacc[b][e] = crow == r ? acc[e] : sacc[b][e];
       }
@@ -301,10 +302,10 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
   }
 }
 
-template <int D, int G, int R>
+template <int D, int G, int R, int REDUCED>
 static hipError_t launch_corope_rows(CoropeParams p, const CoropeFreqs& fr, hipStream_t stream) {
   using Cfg = CoropeFwdCfg<D, R>;
-  auto kern = corope_gqa_fwd_kernel<D, G, R>;
+  auto kern = corope_gqa_fwd_kernel<D, G, R, REDUCED>;
   static std::atomic<uint64_t> lds_ok{0};
   if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
   p.num_m_blocks = (p.N + kCoropeWaves * R - 1) / (kCoropeWaves * R);
@@ -312,29 +313,29 @@ static hipError_t launch_corope_rows(CoropeParams p, const CoropeFreqs& fr, hipS
   return hipGetLastError();
 }
 
-template <int D, int G>
+template <int D, int G, int REDUCED>
 static hipError_t launch_corope_cfg(const CoropeParams& p, const CoropeFreqs& fr, hipStream_t stream) {
   // Rows per wave: as many as fill the 16 columns where that leaves four waves per SIMD, of which two run at a time; below that
   // the longest rows, whose chunks follow one after the other, set the time, and fewer rows per wave shorten it (B1 Hq32 Hkv8
   // N1111 D128: 190 us with four rows, 165 with two).
   constexpr int kMost = G <= 2 ? 8 : G <= 4 ? 4 : 2;
   const int64_t rows = (int64_t)p.N * p.B * p.Hkv, simds = 4 * device_cu_count();
-  if (rows >= 4 * simds * kMost) return launch_corope_rows<D, G, kMost>(p, fr, stream);
-  if (kMost > 2 && rows >= 8 * simds) return launch_corope_rows<D, G, 2>(p, fr, stream);
-  return launch_corope_rows<D, G, 1>(p, fr, stream);
+  if (rows >= 4 * simds * kMost) return launch_corope_rows<D, G, kMost, REDUCED>(p, fr, stream);
+  if (kMost > 2 && rows >= 8 * simds) return launch_corope_rows<D, G, 2, REDUCED>(p, fr, stream);
+  return launch_corope_rows<D, G, 1, REDUCED>(p, fr, stream);
 }
 
-template <int D>
+template <int D, int REDUCED>
 static hipError_t launch_corope_d(const CoropeParams& p, const CoropeFreqs& fr, hipStream_t stream) {
   switch (p.Hq / p.Hkv) {
-    case 1: return launch_corope_cfg<D, 1>(p, fr, stream);
-    case 2: return launch_corope_cfg<D, 2>(p, fr, stream);
-    case 3: return launch_corope_cfg<D, 3>(p, fr, stream);
-    case 4: return launch_corope_cfg<D, 4>(p, fr, stream);
-    case 5: return launch_corope_cfg<D, 5>(p, fr, stream);
-    case 6: return launch_corope_cfg<D, 6>(p, fr, stream);
-    case 7: return launch_corope_cfg<D, 7>(p, fr, stream);
-    case 8: return launch_corope_cfg<D, 8>(p, fr, stream);
+    case 1: return launch_corope_cfg<D, 1, REDUCED>(p, fr, stream);
+    case 2: return launch_corope_cfg<D, 2, REDUCED>(p, fr, stream);
+    case 3: return launch_corope_cfg<D, 3, REDUCED>(p, fr, stream);
+    case 4: return launch_corope_cfg<D, 4, REDUCED>(p, fr, stream);
+    case 5: return launch_corope_cfg<D, 5, REDUCED>(p, fr, stream);
+    case 6: return launch_corope_cfg<D, 6, REDUCED>(p, fr, stream);
+    case 7: return launch_corope_cfg<D, 7, REDUCED>(p, fr, stream);
+    case 8: return launch_corope_cfg<D, 8, REDUCED>(p, fr, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -347,7 +348,11 @@ hipError_t launch_corope_gqa_fwd(const CoropeParams& p, int D, hipStream_t strea
     float inv = 1.0f / powf(p.theta, e);
     fr.w[d] = (float)((double)inv / 6.283185307179586);
   }
-  return D == 128 ? launch_corope_d<128>(p, fr, stream) : launch_corope_d<64>(p, fr, stream);
+  const int reduced = corope_reduced_blocks(fr.w, D, p.N);
+  if (D == 64) return reduced == 0 ? launch_corope_d<64, 0>(p, fr, stream) : launch_corope_d<64, 1>(p, fr, stream);
+  return reduced == 0   ? launch_corope_d<128, 0>(p, fr, stream)
+         : reduced == 1 ? launch_corope_d<128, 1>(p, fr, stream)
+                        : launch_corope_d<128, 2>(p, fr, stream);
 }
 
 }  // namespace COROPE_NS

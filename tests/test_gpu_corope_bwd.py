@@ -330,3 +330,28 @@ def test_corope_backward_many_groups(pkg, groups, G, N, D, dtype):
     for g in (0, groups // 2, groups - 1):
         sl = slice(g, g + 1)
         _compare([t.grad[sl].float().cpu() for t in (qd, kd, vd)], _oracle_grads(q[sl], k[sl], v[sl], d_o[sl], scale, 10000.0), G)
+
+
+# The phase delta w_d is reduced only where it can leave the sine unit's domain: N w_d / 2 pi <= 255 keeps it inside, so with w_0 = 1
+# the kernels change form between N = 1602 and 1603; theta = 1 makes every pair that fast.  dO is zero but for the rows that the oracle
+# follows, the last ones -- the largest phases -- among them, so their gradients are all there is.
+@pytest.mark.parametrize("theta", [10000.0, 1.0])
+@pytest.mark.parametrize("Hq,Hkv,N,D", [(2, 1, 1602, 64), (2, 1, 1603, 64), (4, 1, 1602, 128), (4, 1, 1603, 128), (1, 1, 2100, 128)])
+def test_corope_phase_beyond_the_sine_units_domain(pkg, Hq, Hkv, N, D, theta):
+    dev = torch.device("cuda:0")
+    rows = list(range(0, 6)) + [N // 2] + list(range(N - 6, N))
+    q, k, v, d_o = _inputs(1, Hq, Hkv, N, D, seed=29)
+    keep = torch.zeros(N, 1)
+    keep[rows] = 1.0
+    d_o, scale = d_o * keep, 1 / math.sqrt(D)
+    qg, kg, vg = (t.to(dev, torch.bfloat16).requires_grad_(True) for t in (q, k, v))
+    o = pkg.corope_attention(qg, kg, vg, True, scale, theta)
+    got = (o[:, :, rows],) + torch.autograd.grad(o, (qg, kg, vg), d_o.to(dev, torch.bfloat16))
+    qr, kr, vr = (t.double().requires_grad_(True) for t in (q, k, v))
+    ref = C.corope_gqa_forward_rows(qr, kr, vr, True, scale, theta, torch.tensor(rows), torch.float64)
+    ref = (ref,) + torch.autograd.grad(ref, (qr, kr, vr), d_o[:, :, rows].double())
+    for name, a, b in zip(("O", "dQ", "dK", "dV"), got, ref):
+        # bf16 operands of the products and bf16 results: 1.7e-3 to 2.4e-3 where nothing cancels, and the bar at about four times that
+        err = ((a.double().cpu() - b).norm() / b.norm()).item()
+        print(f"  {name} rel {err:.3e}", flush=True)
+        assert err <= 8e-3, name

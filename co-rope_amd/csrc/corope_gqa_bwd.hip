@@ -28,8 +28,8 @@
 //                  left to right: dP again, dS, G and its running sum, W;
 //                  writes dq of the heads 1..G-1, the leader's dq without its gate path (fp32, workspace), the workspace
 //                  matrices DELTA, W [group] and S, DS [head] (packed lower triangles) and the row statistics that make P of S
-//   dq_leader    dq_leader = c (partial + W K): a plain product on the matrix cores, 128 rows per workgroup
-//   dv           dv^T += dO^T P on the matrix cores, P from S and the row statistics, 128 keys per workgroup
+//   dv           dq_leader = c (partial + W K), 128 rows per workgroup, and beside it dv^T += dO^T P, P from S and the row statistics, 128
+//                keys per workgroup: plain products on the matrix cores
 //   dk           one workgroup per (group, 128 keys): sum_h dS^h q^h on the matrix cores, then lane = rotation pair x 16
 //                keys rotates it per (i, j) and adds the gate path W qL; tiles of DELTA, W, DS staged through LDS
 // Rounding: the rotated keys and what multiplies them (queries, the softmax weights e and e dP) are fp16 - the bf16
@@ -89,8 +89,8 @@ struct CoropeBwdWs {
 //   dq       needs the rotated keys transposed: they go through LDS (16 keys x D x R rows per wave) and come back through the
 //            transposing read.  The weights of the two sums, e (dP - ref) and e, share the 16 columns in the same way (a rotation by 8
 //            lanes), and two rows share the 32 contraction slots of a product (the other row's columns of B are zero).
-// No barriers: a wave is a workgroup.  What bounds it: in the first sweep the vector units (busy 82 % of it; 10 issue slots per (row, key,
-// pair) as in the forward, of about 12.3 in all), in the second the memory (9 floats in, 5 out per (row, key) at G = 4); two waves a
+// No barriers: a wave is a workgroup.  What bounds it: in the first sweep the vector units (busy 82 % of it; 9 or 10 issue slots per (row, key,
+// pair) as in the forward, of about 12 in all), in the second the memory (9 floats in, 5 out per (row, key) at G = 4); two waves a
 // SIMD hide one under the other only in part.  dP is computed in both sweeps, and P is left to the dv kernel: kept in the workspace they cost
 // 12 floats more per (row, key) and a launch.
 // Measured at B2 Hq32 Hkv8 N4096 D128: 8.2 -> 5.9 ms, first sweep 4.6 (one wave per row with the rotated keys in LDS, behind launches for the
@@ -454,7 +454,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
   }
 
   // (sum e (dP - ref) kt - (Delta - ref) sum e kt) / L, the second sum sitting eight lanes up.  dq of the heads 1..G-1 is final; the
-  // leader's still lacks the gate path W K, which a separate plain matrix product adds (corope_bwd_dq_leader_kernel): its row
+  // leader's still lacks the gate path W K, which a separate plain matrix product adds (corope_bwd_dq_leader): its row
   // goes to the workspace in fp32, unscaled
   {
     const float corr = dsum - dref;
@@ -600,23 +600,22 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
 // computed transposed (dq^T += K^T W^T) so that W is read along its packed rows: lane = query row, 8 consecutive keys per
 // step, each value split into two bf16 parts (the keys are exact, so the product carries W to about 16 bits).  One
 // workgroup of 4 waves owns 128 rows (32 per wave) of one group; the 16 key rows of a step are staged in LDS and read
-// transposed.
+// transposed.  Its workgroups come first in the dv launch.
+constexpr int kLeaderRows = 128;
+
 template <int D>
-__global__ __launch_bounds__(4 * kWave) void corope_bwd_dq_leader_kernel(CoropeBwdParams p, CoropeBwdWs ws) {
+__device__ __forceinline__ void corope_bwd_dq_leader(const CoropeBwdParams& p, const CoropeBwdWs& ws, uint16_t* tile, int g, int rb) {
   constexpr int TS = D + 16, NDB = D / 32, NT = 4 * kWave, STEP = 16;
-  __shared__ __attribute__((aligned(16))) uint16_t tile[STEP * TS];
-  const int n_groups = p.B * p.Hkv, g = (int)(blockIdx.x % n_groups);
-  const int rb = (int)(gridDim.x / n_groups) - 1 - (int)(blockIdx.x / n_groups);   // the last row blocks of all groups see the most keys: first
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int r = lane % 32, hf = lane / 32;
   const int N = p.N, b = g / p.Hkv, kvh = g % p.Hkv, G = p.Hq / p.Hkv;
-  const int iw = rb * 128 + 32 * wave, i = iw + r;                // this wave's first row, this lane's row
+  const int iw = rb * kLeaderRows + 32 * wave, i = iw + r;              // this wave's first row, this lane's row
   const uint16_t* kbase = p.k + (int64_t)g * N * D;
   const float* wrow = ws.w(g) + tri_row_start(min(i, N - 1));
   f32x16 acc[NDB];
 #pragma unroll
   for (int db = 0; db < NDB; ++db) acc[db] = f32x16{0};
-  const int t_end = min(N, rb * 128 + 128);                       // keys up to the block's last row
+  const int t_end = min(N, (rb + 1) * kLeaderRows);                      // keys up to the block's last row
   // the key rows and this lane's W values of a step are fetched into registers one step ahead (the workgroup of the last
   // row block walks N / 16 steps one after the other)
   constexpr int UNITS = STEP * (D / 8), PER = (UNITS + NT - 1) / NT;
@@ -739,22 +738,29 @@ __global__ __launch_bounds__(256) void corope_bwd_sum_kernel(const float* parts,
 // step.  A workgroup of 4 waves takes 128 keys at a time (32 per wave) of one group, equal shares of the rows as above; the 16 dO
 // rows of every head are staged in LDS and read transposed; S comes straight from the workspace (lane = key: 128-byte lines), becomes P
 // with the row's statistics and is rounded to the element type.
+// The leader's dq needs nothing of dv's and both wait for memory, so their workgroups share a launch: forward + backward
+// B2 Hq8 Hkv2 N512 D64 129.7 -> 127.3 us, and 5 % where the groups are fewer; at N = 4096, where each fills the chip by itself, no difference.
 constexpr int kDvRows = 16;
 
 template <int D, int G>
-__global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParams p, CoropeBwdWs ws, float* parts, int64_t group_floats) {
+__global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParams p, CoropeBwdWs ws, float* parts, int64_t group_floats,
+                                                                     int shares) {
   constexpr int TS = D + 16, NDB = D / 32, NT = 4 * kWave, ROWS = kDvRows;
   constexpr int UNITS = G * ROWS * (D / 8), PER = (UNITS + NT - 1) / NT;   // 16-byte pieces of a dO tile, per thread
   __shared__ __attribute__((aligned(16))) uint16_t tile[G * ROWS * TS];
   __shared__ __attribute__((aligned(16))) float stat[2][2 * G * ROWS];   // two steps' [reference values, 1 / sums][head][row]
   static_assert(2 * G * ROWS <= NT, "one statistic per thread");
-  const int g = blockIdx.y;
+  const int n_groups = p.B * p.Hkv, leader_blocks = (p.N + kLeaderRows - 1) / kLeaderRows * n_groups;
+  if ((int)blockIdx.x < leader_blocks) {   // the last row blocks of all groups see the most keys: first
+    corope_bwd_dq_leader<D>(p, ws, tile, blockIdx.x % n_groups, (leader_blocks - 1 - (int)blockIdx.x) / n_groups);
+    return;
+  }
+  const int g = ((int)blockIdx.x - leader_blocks) / shares, share = ((int)blockIdx.x - leader_blocks) % shares;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int r = lane % 32, hf = lane / 32;
   const int N = p.N, b = g / p.Hkv, kvh = g % p.Hkv;
   const int head0 = b * p.Hq + kvh * G;
   const CoropeShares<ROWS> sh(N);
-  const int shares = gridDim.x, share = blockIdx.x;
   int kb = 0;
 #pragma unroll 1
   for (int t = sh.begin(share, shares), t_end = sh.begin(share + 1, shares); t < t_end;) {
@@ -862,7 +868,7 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
 //       its half: one (sin, cos) and four multiply-adds per (row, key, pair).
 // The gate path W qL contracts over rows, so a tile's 8 rows are one more product into the same accumulators (on the vector units it was 2 of
 // 12 issue slots per (row, key, pair)).  W is split into three bf16 parts, 24 bits whatever its scale, and an fp16 query into two.
-// What bounds it: the vector units, 10 issue slots per (row, key, pair).  Measured with the gate path moved: B2 Hq32 Hkv8 N4096 D128
+// What bounds it: the vector units, 9 or 10 issue slots per (row, key, pair).  Measured with the gate path moved: B2 Hq32 Hkv8 N4096 D128
 // forward + backward 15.0 -> 14.6 ms, B2 Hq8 Hkv2 N512 D64 133 -> 130.5 us.
 // A workgroup takes its share of the group's (block, row tile) list as above.  Tiles of DELTA, W, DS^h ([row][matrix][key], fp32) and the rows' queries
 // ([row][column][head], bf16, heads padded to 8 with zeros: the B operand is then one 16-byte read) go through LDS,
@@ -1099,15 +1105,15 @@ static void launch_corope_bwd_scores(const CoropeBwdParams& p, const CoropeBwdWs
 template <int D, int G, int REDUCED>
 static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, int n_groups_total,
                                         hipStream_t stream) {
-  const int nt = (p.N + 127) / 128;
   launch_corope_bwd_scores<D, G, REDUCED>(p, ws, fr, n_groups_total, stream);
-  hipLaunchKernelGGL(corope_bwd_dq_leader_kernel<D>, dim3((unsigned)nt * p.B * p.Hkv), dim3(4 * kWave), 0, stream, p, ws);
   using Cfg = CoropeDkCfg<D, G>;
   const int64_t group_floats = G * ws.NN, slots = ws.part_floats(G, p.N) / (kDkKeys * D);
   const int dv_shares = corope_bwd_shares<kDvRows>(p.N, n_groups_total, slots), dk_shares = corope_bwd_shares<kDkRows>(p.N, n_groups_total, slots);
   float* parts = ws.parts(0, G);
   const int n_groups = p.B * p.Hkv, n_blocks = (p.N + kDkKeys - 1) / kDkKeys;
-  hipLaunchKernelGGL((corope_bwd_dv_kernel<D, G>), dim3(dv_shares, n_groups), dim3(4 * kWave), 0, stream, p, ws, parts, group_floats);
+  const unsigned leader_blocks = (unsigned)((p.N + kLeaderRows - 1) / kLeaderRows) * n_groups;
+  hipLaunchKernelGGL((corope_bwd_dv_kernel<D, G>), dim3(leader_blocks + (unsigned)dv_shares * n_groups), dim3(4 * kWave), 0, stream, p, ws,
+                     parts, group_floats, dv_shares);
   if (dv_shares > 1)
     hipLaunchKernelGGL((corope_bwd_sum_kernel<D, kDvRows>), dim3(n_blocks, n_groups, 8), dim3(256), 0, stream, parts, group_floats, p.dv,
                        p.N, dv_shares, 1.f);

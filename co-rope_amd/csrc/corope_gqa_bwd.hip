@@ -922,20 +922,18 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
     f32x4 mv[TI / 4];
     u32x4 qv[RI];
     auto fetch = [&](int i0) __attribute__((always_inline)) {
-      // the 8 rows of a tile share a row length; rows past the end repeat the last one (and are zeroed below)
+      // the 8 rows of a tile share a row length; rows past the end repeat the last one
       const int64_t tile0 = tri_row_start(i0);
       const int row_len = 64 * (i0 / 64 + 1);
       static_for<TI / 4>([&](auto k_c) __attribute__((always_inline)) {
         constexpr int k = decltype(k_c)::value;
         const int e = 4 * (threadIdx.x + k * NT);
         const int key = e % kDkKeys, m = (e / kDkKeys) % MATS, r = e / (kDkKeys * MATS);
-        const int i = i0 + r, j = jb + key;
-        const float* src = m == 0 ? ws.delta(g) : m == 1 ? ws.w(g) : ws.ds(head0 + m - 2);
-        // four keys with one load, always inside the padded row (no branch); what lies outside the causal triangle or
-        // past N is not defined there and becomes zero
-        const f32x4 v = *reinterpret_cast<const f32x4*>(src + tile0 + (int64_t)row_len * min(r, N - 1 - i0) + min(j, row_len - 4));
-#pragma unroll
-        for (int x = 0; x < 4; ++x) mv[k][x] = (i < N && j + x <= i) ? v[x] : 0.f;
+        const int mat = m == 0 ? g : m == 1 ? ws.n_groups + g : 2 * ws.n_groups + ws.n_heads + head0 + m - 2;   // (as CoropeBwdWs counts them)
+        const float* src = ws.base + mat * ws.NN;
+        // four keys with one load, always inside the padded row (no branch); what is not defined there becomes zero on its way into
+        // LDS (here the select would wait for the load)
+        mv[k] = *reinterpret_cast<const f32x4*>(src + tile0 + (int64_t)row_len * min(r, N - 1 - i0) + min(jb + key, row_len - 4));
       });
       static_for<RI>([&](auto k_c) __attribute__((always_inline)) {
         constexpr int k = decltype(k_c)::value;
@@ -956,7 +954,11 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
       __syncthreads();   // the previous tile has been consumed
       static_for<TI / 4>([&](auto k_c) __attribute__((always_inline)) {
         constexpr int k = decltype(k_c)::value;
-        *reinterpret_cast<f32x4*>(tile + 4 * (threadIdx.x + k * NT)) = mv[k];
+        const int e = 4 * (threadIdx.x + k * NT), i = i0 + e / (kDkKeys * MATS), j = jb + e % kDkKeys;
+        f32x4 v;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[x] = (i < N && j + x <= i) ? mv[k][x] : 0.f;   // outside the causal triangle or past N
+        *reinterpret_cast<f32x4*>(tile + e) = v;
       });
       static_for<RI>([&](auto k_c) __attribute__((always_inline)) {
         constexpr int k = decltype(k_c)::value;
@@ -1010,6 +1012,13 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
         }
       }
       const int n_rows = min(kDkRows, N - i0);
+      // dS of a row is read from LDS under the row before: what begins a row is a chain from there through the conversion and the product
+      float ds_next[G];
+      auto read_ds = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < G; ++h) ds_next[h] = tile[(r * MATS + 2 + h) * kDkKeys + 32 * wave + col];
+      };
+      read_ds(0);
 #pragma unroll 1
       for (int r = 0; r < n_rows; ++r) {
         const float* trow = tile + r * MATS * kDkKeys + 32 * wave;
@@ -1021,11 +1030,12 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
           float dsv[8];
 #pragma unroll
           for (int h = 0; h < 8; ++h) {
-            const float x = h < G ? trow[(2 + h) * kDkKeys + col] : 0.f;
+            const float x = h < G ? ds_next[h < G ? h : 0] : 0.f;
             dsv[h] = hf == 0 ? x : x - elt_to_f(f_to_elt(x));
           }
           aop = u32x4{pack_elts(dsv[0], dsv[1]), pack_elts(dsv[2], dsv[3]), pack_elts(dsv[4], dsv[5]), pack_elts(dsv[6], dsv[7])};
         }
+        read_ds(min(r + 1, kDkRows - 1));
         // delta of this lane's 16 keys: keys 8 n + 4 half + 0..3 for n = 0..3, as the accumulator rows are laid out
         f32x4 dl[4];
 #pragma unroll
@@ -1045,6 +1055,8 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
             dk2[np][e] = __builtin_fmaf(cs, u2[e], __builtin_fmaf(sn, u1[e], dk2[np][e]));
           }
         });
+#pragma unroll
+        for (int h = 0; h < G; ++h) asm volatile("" : "+v"(ds_next[h]));   // (or the read sinks to its use)
       }
     }
     const bool whole = t == b0 && seg_end == b1;

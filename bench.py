@@ -41,10 +41,11 @@ HBM_TRAFFIC_BYTES = {
     ("c3", "rope_attn_bwd_dq"): int((404872 * 2.0 + 91136) * 1024),
     ("c3", "rope_attn_bwd_dkdv"): int((312964 * 2.0 + 131072) * 1024),
     ("c4", "rope_attn_fwd"): int((1073484 * 2.0 + 243220) * 1024),
-    # Co-RoPE at C5 (profiles/corope_gqa_c5_hbm_traffic.md): the forward kernel; the backward's six launches together
-    ("c5", "corope_gqa_fwd"): int((70416 * 2.0 + 65536) * 1024),
-    ("c5", "corope_gqa_bwd"): int(((2 * 22429 + 701939 + 48483 + 226967 + 298542) * 2.0
-                                   + (2 * 188709 + 1422980 + 2364 + 2341 + 2341)) * 1024),
+    # Co-RoPE at C5 (profiles/corope_gqa_c5_hbm_traffic.md): the forward kernel; the backward's launches together, with
+    # the workspace for one pass
+    ("c5", "corope_gqa_fwd"): int((73773 * 2.0 + 65536) * 1024),
+    ("c5", "corope_gqa_bwd"): int(((3564006 + 1865385 + 2086161 + 26643 + 26649) * 2.0
+                                   + (9566621 + 74243 + 57856 + 11776 + 11776)) * 1024),
 }
 
 CONFIGS = {
@@ -422,15 +423,11 @@ def bench_corope(args):
         ws_bytes = groups * one
         by_workspace[f"{groups} of {B * Hkv} groups per pass, {ws_bytes / 2**30:.2f} GiB"] = round(time_bwd(), 4)
     ws_bytes = full_bytes
-    # issue slots per (sin, cos) pair, counted as for the forward (a transcendental = 2 slots): scores kernel 11 + 4 (phase
-    # 2, unpack 2, rotate 4, pack 1, LDS 2; sin, cos); dk kernel 8 + 4 (phase 2, rotate-accumulate 4, gate path 2; sin, cos);
-    # the per-head sums run on the matrix cores
-    bwd_instr = pairs * (15 + 12)
-    # VALU roofline: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz issue slots/s.  Per (sin, cos) pair the forward needs 14 slots:
-    # 10 full-rate instructions (phase 2, unpack 2, rotate 4, pack 1, LDS 1) and two transcendentals, which issue at half
-    # the rate (measured on this chip: v_sin_f32 16.0 T lanes/s against 33.3 for v_fma_f32), so 2 slots each; the per-head
-    # dot products run on the matrix cores
-    fwd_instr = pairs * 14
+    # VALU roofline: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz issue slots/s.  Issue slots per (sin, cos) pair, the same in the forward, the
+    # backward's scores kernel and its dk kernel: phase 1, reduced for half of the pairs at this N and theta (0.5), two
+    # transcendentals at half rate (measured on this chip: v_sin_f32 16.0 T lanes/s against 33.3 for v_fma_f32), so 2 slots
+    # each, and 4 to rotate; the dot products run on the matrix cores
+    fwd_instr, bwd_instr = pairs * 9.5, 2 * pairs * 9.5
     out = {"metric": "Co-RoPE GQA fwd, B2 Hq32 Hkv8 N4096 D128 causal", "value": round(flops / (ms * 1e-3) * 1e-12, 2),
            "unit": "TFLOP/s (attention-equivalent)", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
            "ms_per_step": round(ms, 4), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
@@ -445,7 +442,7 @@ def bench_corope(args):
            "backward": {"ms": round(bms, 4), "steps": bsteps, "workspace_gib": round(ws_bytes / 2**30, 2), "ms_by_workspace": by_workspace,
                         "sincos_pairs_per_s": round(2 * pairs / (bms * 1e-3), 1),
                         "tflops_attention_equivalent": round(2.5 * flops / (bms * 1e-3) * 1e-12, 2),
-                        "roofline": {"bound": "valu", "kernel": "corope_gqa_bwd (6 launches)",
+                        "roofline": {"bound": "valu", "kernel": "corope_gqa_bwd (5 launches)",
                                      "achieved": round(bwd_instr / (bms * 1e-3) * 1e-12, 3),
                                      "peak": round(256 * 4 * 16 * 2.4e9 * 1e-12, 3), "unit": "T issue slots/s",
                                      "frac": round(bwd_instr / (bms * 1e-3) / (256 * 4 * 16 * 2.4e9), 4),

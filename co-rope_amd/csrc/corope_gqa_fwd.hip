@@ -231,14 +231,16 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
     });
 
     // ---- softmax: lane = (row, head), 16 keys 16 b + 4 g + e of the chunk ------------------------------------------------
-    if (diagonal) {
-      int rel = iw + crow - c * kCoropeKeys - 4 * g;   // last key the row sees, relative to this lane's first
+    // Keys beyond the diagonal are masked behind the scaling: sm_scale may be zero or negative.
+    auto mask = [&](float (&y)[4][4]) __attribute__((always_inline)) {
+      if (!diagonal) return;
+      const int rel = iw + crow - c * kCoropeKeys - 4 * g;   // last key the row sees, relative to this lane's first
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (16 * b + e > rel) sacc[b][e] = scale2 < 0.f ? INFINITY : -INFINITY;
-    }
+          if (16 * b + e > rel) y[b][e] = -INFINITY;
+    };
     // The reference value only has to keep the exponentials in range, it need not be the running maximum: it moves (to the exact
     // maximum so far, with the usual rescaling) only when some score of the chunk lies more than kLazyMargin above it, which after
     // the first chunks of a row is rare.
@@ -247,16 +249,23 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        x[b][e] = __builtin_fmaf(sacc[b][e], scale2, -m_run);
-        top = fmaxf(top, x[b][e]);
-      }
+      for (int e = 0; e < 4; ++e) x[b][e] = __builtin_fmaf(sacc[b][e], scale2, -m_run);
+    mask(x);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) top = fmaxf(top, x[b][e]);
     if (__builtin_amdgcn_ballot_w64(top > kLazyMargin) != 0) {   // wave-uniform
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[b][e] = sacc[b][e] * scale2;
+      mask(x);
       top = -INFINITY;
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) top = fmaxf(top, sacc[b][e] * scale2);
+        for (int e = 0; e < 4; ++e) top = fmaxf(top, x[b][e]);
       top = fmaxf(top, __shfl_xor(top, 16));
       top = fmaxf(top, __shfl_xor(top, 32));
       const float m_new = fmaxf(m_run, top);   // finite: the chunk holds a key <= row
@@ -271,6 +280,7 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
       for (int b = 0; b < 4; ++b)
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[b][e] = __builtin_fmaf(sacc[b][e], scale2, -m_run);
+      mask(x);
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {   // 32 keys per product

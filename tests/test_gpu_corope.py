@@ -135,3 +135,18 @@ def test_forward_many_groups(pkg, groups, G, N, D, dtype):
         ref = C.corope_gqa_forward(q[g:g + 1].double(), k[g:g + 1].double(), v[g:g + 1].double(), True, scale, 10000.0, torch.float64)
         err = (o[g:g + 1].double().cpu() - ref).abs().max().item()
         assert err <= 2e-2, (g, err)
+
+
+# A zero temperature (every weight the same) and a negative one: what lies beyond the diagonal has to vanish whatever the scale does to
+# it.  One, two and four query rows per wave, lengths that end inside a chunk.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("scale", [0.0, -0.0, -0.125])
+@pytest.mark.parametrize("groups,G,N,D", [(1, 2, 100, 64), (2, 8, 77, 128), (130, 4, 70, 64), (240, 4, 70, 64), (240, 3, 73, 128)])
+def test_forward_scale_zero_or_negative(pkg, groups, G, N, D, scale, dtype):
+    dev = torch.device("cuda:0")
+    q, k, v = (bf16_round(seeded((groups, h, N, D), 50 + i)) for i, h in enumerate((G, 1, 1)))
+    o = pkg.corope_attention(*(t.to(dev, dtype) for t in (q, k, v)), True, scale, 10000.0)
+    torch.cuda.synchronize()
+    for g in {0, groups // 2, groups - 1}:
+        ref = C.corope_gqa_forward(q[g:g + 1].double(), k[g:g + 1].double(), v[g:g + 1].double(), True, scale, 10000.0, torch.float64)
+        assert (o[g:g + 1].double().cpu() - ref).abs().max() <= TOL, g

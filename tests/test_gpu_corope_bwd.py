@@ -355,3 +355,11 @@ def test_corope_phase_beyond_the_sine_units_domain(pkg, Hq, Hkv, N, D, theta):
         err = ((a.double().cpu() - b).norm() / b.norm()).item()
         print(f"  {name} rel {err:.3e}", flush=True)
         assert err <= 8e-3, name
+
+
+# A zero and a negative temperature: O, the reference value of the row sums, and through it every gradient.
+@pytest.mark.parametrize("scale", [0.0, -0.125])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 4, 2, 100, 64), (1, 8, 1, 77, 128), (1, 1, 1, 130, 128)])
+def test_corope_backward_scale_zero_or_negative(pkg, B, Hq, Hkv, N, D, scale):
+    q, k, v, d_o = _inputs(B, Hq, Hkv, N, D, seed=51)
+    _compare(_gpu_grads(pkg, q, k, v, d_o, scale, 10000.0), _oracle_grads(q, k, v, d_o, scale, 10000.0), Hq // Hkv)

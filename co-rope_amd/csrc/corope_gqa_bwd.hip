@@ -798,7 +798,7 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
 #pragma unroll
         for (int x = 0; x < 8; ++x) {
           const int i = i0 + 8 * hf + x;
-          pnext[h][x] = (wave_on && i < N && j <= i) ? srow[row_len * (8 * hf + x)] : -INFINITY;   // nothing outside the triangle is defined
+          pnext[h][x] = (wave_on && i < N && j <= i) ? srow[row_len * (8 * hf + x)] : 0.f;   // nothing outside the triangle is defined
         }
       }
     };
@@ -825,7 +825,10 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
       for (int h = 0; h < G; ++h) {
         float w[8];
 #pragma unroll
-        for (int x = 0; x < 8; ++x) w[x] = fast_exp2(pnext[h][x] - st[h * ROWS + 8 * hf + x]) * st[(G + h) * ROWS + 8 * hf + x];
+        for (int x = 0; x < 8; ++x) {   // (a key the row does not see has weight zero also where the row's statistics are NaN)
+          const float e = fast_exp2(pnext[h][x] - st[h * ROWS + 8 * hf + x]) * st[(G + h) * ROWS + 8 * hf + x];
+          w[x] = j <= i0 + 8 * hf + x ? e : 0.f;
+        }
         bop[h] = u32x4{pack_elts(w[0], w[1]), pack_elts(w[2], w[3]), pack_elts(w[4], w[5]), pack_elts(w[6], w[7])};
       }
       const bool wave_on = i0 + ROWS - 1 >= jw && jw < N;

@@ -363,3 +363,37 @@ def test_corope_phase_beyond_the_sine_units_domain(pkg, Hq, Hkv, N, D, theta):
 def test_corope_backward_scale_zero_or_negative(pkg, B, Hq, Hkv, N, D, scale):
     q, k, v, d_o = _inputs(B, Hq, Hkv, N, D, seed=51)
     _compare(_gpu_grads(pkg, q, k, v, d_o, scale, 10000.0), _oracle_grads(q, k, v, d_o, scale, 10000.0), Hq // Hkv)
+
+
+def _bad_row_grads(pkg, groups, G, N, D, row, head, what, dtype):
+    """Gradients of many short groups, and the same with one query row of group 3 spoilt; everything the spoilt row cannot reach (other
+    groups are compared bit for bit) has to stay as it was."""
+    dev = torch.device("cuda:0")
+    q, k, v, d_o = (t.to(dev, dtype) for t in _inputs(groups, G, 1, N, D, seed=61))
+    bad = q.clone()
+    bad[3, head, row, 1] = what
+    out = []
+    for x in (q, bad):
+        x, kd, vd = (t.clone().requires_grad_(True) for t in (x, k, v))
+        out.append(torch.autograd.grad(pkg.corope_attention(x, kd, vd, True, 1 / math.sqrt(D), 10000.0), (x, kd, vd), d_o))
+    torch.cuda.synchronize()
+    for clean, spoilt in zip(*out):
+        assert torch.equal(clean[:3], spoilt[:3]) and torch.equal(clean[4:], spoilt[4:])
+    return [[t[3].float().cpu() for t in side] for side in out]
+
+
+BAD_ROWS = [(240, 4, 70, 64, 37), (240, 2, 70, 128, 50), (240, 4, 70, 128, 0), (60, 8, 139, 64, 66), (4, 4, 200, 128, 101), (240, 1, 70, 64, 69)]
+
+
+# A row whose leader's or own query is not finite has NaN statistics.  Keys behind it do not see it.  (Where a rescaling falls moves by
+# what the spoilt row does, so its neighbours agree to the suite's bar, not bit for bit.)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("what", [float("nan"), float("inf")])
+@pytest.mark.parametrize("groups,G,N,D,row", BAD_ROWS)
+def test_corope_dv_of_keys_behind_a_row_that_is_not_finite(pkg, groups, G, N, D, row, what, dtype):
+    for head in {0, G - 1}:
+        clean, spoilt = _bad_row_grads(pkg, groups, G, N, D, row, head, what, dtype)
+        assert torch.isfinite(spoilt[2][:, row + 1:]).all()
+        if row + 1 < N:
+            assert (clean[2][:, row + 1:] - spoilt[2][:, row + 1:]).abs().max() <= TOL
+        assert not torch.isfinite(spoilt[2][:, :row + 1]).any()

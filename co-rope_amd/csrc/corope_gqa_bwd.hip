@@ -362,6 +362,27 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
       *reinterpret_cast<f32x4*>(byte_offset(s_l, 64u * b)) = s_out;
       if constexpr (NS > 1) *reinterpret_cast<f32x4*>(byte_offset(g_l, 64u * b)) = g_out;
     }
+    // Two rows share the contraction slots of the dq products, the other row's columns of B being zero: a rotated key that is not
+    // finite (a leader's row that is not, a key beyond fp16 once rotated) would reach the other row's dq.  It shows in its own row's scores,
+    // and through them in that row's statistics and dq; in LDS it is then replaced by zero.  Rare: the common case costs five instructions a
+    // block.
+    if constexpr (RH > 1) {
+      float poison = 0.f;   // NaN if a score is not finite
+#pragma unroll
+      for (int e = 0; e < 4; ++e) poison = __builtin_fmaf(sc[e], 0.f, poison);
+      if (__builtin_amdgcn_ballot_w64(poison != poison) != 0) {   // wave-uniform
+        lds_order();
+#pragma unroll 1
+        for (int e = lane; e < R * 16 * (D / 2); e += kWave) {
+          uint32_t* at = reinterpret_cast<uint32_t*>(kt + e / (D / 2) * TS) + e % (D / 2);
+          uint32_t w = *at;
+          if ((w & 0x7c00u) == 0x7c00u) w &= 0xffff0000u;
+          if ((w & 0x7c000000u) == 0x7c000000u) w &= 0xffffu;
+          *at = w;
+        }
+        lds_order();
+      }
+    }
     if (diagonal) {
       const int rel = own_row - 16 * b - 4 * g;   // last key the row sees, relative to this lane's first
 #pragma unroll

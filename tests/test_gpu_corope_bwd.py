@@ -397,3 +397,40 @@ def test_corope_dv_of_keys_behind_a_row_that_is_not_finite(pkg, groups, G, N, D,
         if row + 1 < N:
             assert (clean[2][:, row + 1:] - spoilt[2][:, row + 1:]).abs().max() <= TOL
         assert not torch.isfinite(spoilt[2][:, :row + 1]).any()
+
+
+# Rows of one wave share matrix products: a row whose rotated keys are not finite must not reach the dq of the rows beside it.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("what", [float("nan"), float("inf")])
+@pytest.mark.parametrize("groups,G,N,D,row", BAD_ROWS)
+def test_corope_dq_beside_a_row_that_is_not_finite(pkg, groups, G, N, D, row, what, dtype):
+    clean, spoilt = _bad_row_grads(pkg, groups, G, N, D, row, 0, what, dtype)
+    others = [i for i in range(N) if i != row]
+    assert torch.isfinite(spoilt[0][:, others]).all()
+    assert (clean[0][:, others] - spoilt[0][:, others]).abs().max() <= TOL
+    assert not torch.isfinite(spoilt[0][0, row]).any()
+
+
+# A key that is NaN spoils the rows that see it and no row before its block of 32 (the leader's gate path multiplies 32 rows at once).  One that leaves fp16's range only where its rotation
+# takes it there (here |cos| + |sin| > 65504 / 49920 of the first pair, about half of the rows) spoils none of the others.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("groups,G,N,D,key", [(240, 4, 70, 64, 33), (240, 2, 70, 128, 20), (240, 3, 73, 128, 34)])
+def test_corope_dq_of_rows_beside_those_a_key_spoils(pkg, groups, G, N, D, key, dtype):
+    dev = torch.device("cuda:0")
+    q, k, v, d_o = _inputs(groups, G, 1, N, D, seed=71)
+    for what in (float("nan"), 49920.0):
+        bad = k.clone()
+        bad[3, 0, key, ::D // 2] = what
+        x, kd, vd = (t.to(dev, dtype).requires_grad_(True) for t in (q, bad, v))
+        dq = torch.autograd.grad(pkg.corope_attention(x, kd, vd, True, 1 / math.sqrt(D), 10000.0), x, d_o.to(dev, dtype))[0][3].float().cpu()
+        assert torch.isfinite(dq[:, :key // 32 * 32]).all()
+        if what != what:
+            assert not torch.isfinite(dq[:, key:]).any()
+            continue
+        sl = slice(3, 4)
+        aux = C.corope_gqa_forward(q[sl].double(), bad[sl].double(), v[sl].double(), True, 1 / math.sqrt(D), 10000.0, torch.float64, return_aux=True)[1]
+        phi = aux["delta"][0, 0, :, key]   # the first pair turns by delta itself
+        kept = (phi.cos().abs() + phi.sin().abs()) * what < 65000
+        kept[:key] = False
+        assert 5 < kept.sum() < N - key - 5
+        assert torch.isfinite(dq[:, kept]).all()

@@ -243,19 +243,17 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
     };
     // The reference value only has to keep the exponentials in range, it need not be the running maximum: it moves (to the exact
     // maximum so far, with the usual rescaling) only when some score of the chunk lies more than kLazyMargin above it, which after
-    // the first chunks of a row is rare.
+    // the first chunks of a row is rare.  On the diagonal, a row's first chunk, it always does, so only that branch masks.
     constexpr float kLazyMargin = 8.f;   // base-2 units: weights stay below 2^8
     float x[4][4], top = -INFINITY;
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[b][e] = __builtin_fmaf(sacc[b][e], scale2, -m_run);
-    mask(x);
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) top = fmaxf(top, x[b][e]);
-    if (__builtin_amdgcn_ballot_w64(top > kLazyMargin) != 0) {   // wave-uniform
+      for (int e = 0; e < 4; ++e) {
+        x[b][e] = __builtin_fmaf(sacc[b][e], scale2, -m_run);
+        top = fmaxf(top, x[b][e]);
+      }
+    if (diagonal || __builtin_amdgcn_ballot_w64(top > kLazyMargin) != 0) {   // wave-uniform
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll

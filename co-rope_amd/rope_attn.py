@@ -227,10 +227,7 @@ def _backward_rotated(lib, q_rot, k_rot, v, o, do, M, fc, fs, sm_scale, causal):
     """(dq, dk, dv, ...) of the operator from the rotated q and k its forward kept."""
     B, H, N, D = q_rot.shape
     Hkv = k_rot.shape[1]
-    v_st = do_st = None
-    if not v.is_contiguous():
-        v_st = _view_strides(v) if D <= 128 else None
-        v = v if v_st is not None else v.contiguous()
+    do_st = None
     if not do.is_contiguous():
         do_st = _view_strides(do) if D <= 128 else None
         do = do if do_st is not None else do.contiguous()
@@ -241,7 +238,7 @@ def _backward_rotated(lib, q_rot, k_rot, v, o, do, M, fc, fs, sm_scale, causal):
         # many pieces there are depends on the device
         nbytes = lib.corope_rope_attn_bwd_rotated_parts_bytes(B, H, Hkv, N, D, int(causal))
         parts = torch.empty(nbytes, device=q_rot.device, dtype=torch.uint8) if nbytes > 0 else None
-        rc = lib.corope_rope_attn_bwd_rotated(q_rot.data_ptr(), k_rot.data_ptr(), v.data_ptr(), v_st, o.data_ptr(), do.data_ptr(), do_st,
+        rc = lib.corope_rope_attn_bwd_rotated(q_rot.data_ptr(), k_rot.data_ptr(), v.data_ptr(), None, o.data_ptr(), do.data_ptr(), do_st,
                                               M.data_ptr(), delta.data_ptr(), fc.data_ptr(), fs.data_ptr(), fc.stride(0), dq.data_ptr(),
                                               dk.data_ptr(), dv.data_ptr(), B, H, Hkv, N, D, sm_scale, int(causal),
                                               int(q_rot.dtype == torch.float16), parts.data_ptr() if parts is not None else None, nbytes,
@@ -257,10 +254,15 @@ class _FusedRopeAttn(torch.autograd.Function):
         _check_inputs(q, k, v, freqs_cos, freqs_sin)
         B, H, N, D = q.shape
         training = any(ctx.needs_input_grad[:3])
+        if training:
+            # v is kept for the backward, and a view kept as it is would hold the fused projection it is cut from, and would be lost
+            # if the caller overwrites that before the backward: a view is copied (377 -> 386 us forward and backward at B1 Hq32 Hkv8 N3001 D128), q and k are kept
+            # rotated, in tensors of their own
+            v = v.contiguous()
         # when a gradient will be asked for, the forward keeps its rotated q and k for the backward and the originals
         # are not saved (the reference saves q and k, fused_rope_attn.py:718, and re-rotates them in its backward)
         o, M, fc, fs, rotated = _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, keep_rotated=training)
-        # nothing to differentiate, nothing kept: saving q, k, v would also copy strided views of a fused projection.  (Tables that
+        # nothing to differentiate, nothing kept: saving q and k would copy strided views of a fused projection.  (Tables that
         # ask for a gradient get None, but the backward that says so runs and wants its tensors.)
         if not any(ctx.needs_input_grad):
             return o
@@ -281,7 +283,7 @@ class _FusedRopeAttn(torch.autograd.Function):
         if do.dtype != q.dtype:
             do = do.to(q.dtype)
         B, H, N, D = q.shape
-        if ctx.rotated:   # q, k are the rotated copies the forward kept; v and dO are read where they lie if their layout allows it
+        if ctx.rotated:   # q, k are the rotated copies the forward kept; dO is read where it lies if its layout allows it
             return _backward_rotated(lib, q, k, v, o, do, M, fc, fs, ctx.sm_scale, ctx.causal)
         do = do.contiguous()
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)

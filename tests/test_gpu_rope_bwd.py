@@ -457,3 +457,26 @@ def test_backward_when_only_the_tables_ask_for_a_gradient(pkg, N):
     assert o.requires_grad
     o.sum().backward()
     assert c.grad is None
+
+
+# What the backward needs of a view is its own by the time the forward returns: the fused projection may be overwritten, and is not kept.
+@pytest.mark.parametrize("N,D", [(200, 64), (1100, 64), (640, 128), (300, 256)])
+def test_fused_projection_overwritten_before_the_backward(pkg, N, D):
+    dev = torch.device("cuda:0")
+    fused, g = (seeded(s, 80 + i).to(dev, torch.bfloat16) for i, s in enumerate(((1, N, 3, 2, D), (1, N, 2, D))))
+    c, s = (t.to(dev) for t in O.precompute_freqs_cis(D, N))
+    grads = []
+    for overwrite in (False, True):
+        x = fused.clone().requires_grad_(True)
+        buf = x * 1                    # (an intermediate, as a projection's output is)
+        o = pkg.attention(*(buf[:, :, i].transpose(1, 2) for i in range(3)), True, 0.1, c, s)
+        if overwrite:
+            with torch.no_grad():
+                buf.zero_()
+        del buf
+        grads.append(torch.autograd.grad(o, x, g.transpose(1, 2))[0])
+    assert torch.equal(*grads)
+    v = torch.zeros(1, N, 64, 2, D, device=dev, dtype=torch.bfloat16)[:, :, 0].transpose(1, 2).requires_grad_(True)
+    q, k = (torch.zeros(1, 2, N, D, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    o = pkg.attention(q, k, v, True, 0.1, c, s)
+    assert max(t.untyped_storage().nbytes() for t in o.grad_fn.saved_tensors if t.dtype == torch.bfloat16) <= 2 * 2 * N * D

@@ -235,9 +235,12 @@ def _backward_rotated(lib, q_rot, k_rot, v, o, do, M, fc, fs, sm_scale, causal):
     delta = torch.empty_like(M)
     with _on_device(q_rot):
         # scratch in which the dK+dV launch leaves the partial sums of key blocks it cuts among workgroups (0: none are cut); how
-        # many pieces there are depends on the device
+        # many pieces there are depends on the device (at most 128 MiB with 256 compute units).  Only speed needs it
         nbytes = lib.corope_rope_attn_bwd_rotated_parts_bytes(B, H, Hkv, N, D, int(causal))
-        parts = torch.empty(nbytes, device=q_rot.device, dtype=torch.uint8) if nbytes > 0 else None
+        try:
+            parts = torch.empty(nbytes, device=q_rot.device, dtype=torch.uint8) if nbytes > 0 else None
+        except torch.cuda.OutOfMemoryError:
+            parts = None
         rc = lib.corope_rope_attn_bwd_rotated(q_rot.data_ptr(), k_rot.data_ptr(), v.data_ptr(), None, o.data_ptr(), do.data_ptr(), do_st,
                                               M.data_ptr(), delta.data_ptr(), fc.data_ptr(), fs.data_ptr(), fc.stride(0), dq.data_ptr(),
                                               dk.data_ptr(), dv.data_ptr(), B, H, Hkv, N, D, sm_scale, int(causal),

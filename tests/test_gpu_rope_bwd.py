@@ -480,3 +480,34 @@ def test_fused_projection_overwritten_before_the_backward(pkg, N, D):
     q, k = (torch.zeros(1, 2, N, D, device=dev, dtype=torch.bfloat16) for _ in range(2))
     o = pkg.attention(q, k, v, True, 0.1, c, s)
     assert max(t.untyped_storage().nbytes() for t in o.grad_fn.saved_tensors if t.dtype == torch.bfloat16) <= 2 * 2 * N * D
+
+
+# The scratch for cut key blocks only buys time: where there is no memory for it the backward runs without.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_backward_without_memory_for_cut_key_blocks(pkg, monkeypatch, dtype):
+    dev = torch.device("cuda:0")
+    B, Hq, Hkv, N, D = 1, 8, 1, 700, 128
+    q, g = (seeded((B, Hq, N, D), 90 + i).to(dev, dtype) for i in range(2))
+    k, v = (seeded((B, Hkv, N, D), 92 + i).to(dev, dtype) for i in range(2))
+    c, s = (t.to(dev) for t in O.precompute_freqs_cis(D, N))
+    nbytes = pkg._lib.load().corope_rope_attn_bwd_rotated_parts_bytes(B, Hq, Hkv, N, D, 1)
+    assert nbytes > 0
+    x = [t.requires_grad_(True) for t in (q, k, v)]
+    o = pkg.attention(*x, True, 1 / math.sqrt(D), c, s)
+    cut = torch.autograd.grad(o, x, g, retain_graph=True)
+    empty, refused = torch.empty, []
+
+    def short_of_memory(*args, **kwargs):
+        if args[0] == nbytes:
+            refused.append(nbytes)
+            raise torch.cuda.OutOfMemoryError("no memory")
+        return empty(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", short_of_memory)
+    whole = torch.autograd.grad(o, x, g)
+    monkeypatch.undo()
+    assert refused and torch.equal(cut[0], whole[0])
+    # the same products summed in another order in fp32, then one rounding: half a step of the element type, twice
+    step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for a, b in zip(cut[1:], whole[1:]):
+        assert (a.float() - b.float()).abs().max() <= 2 * step * b.float().abs().max() + 1e-5

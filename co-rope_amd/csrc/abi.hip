@@ -521,16 +521,11 @@ int corope_rope_attn_bwd_prerotated(const void* q_rot, const void* k_rot, const 
                                     const float* lse, float* delta, const float* freqs_cos, const float* freqs_sin,
                                     int64_t freq_row_stride, void* dq, void* dk, void* dv, int B, int H, int N, int D,
                                     float sm_scale, int causal, void* stream) {
-  // two launches: the dQ kernel computes delta for the rows it owns on its way (no separate pass over o and dO), the
-  // fused dK+dV kernel reads it afterwards
-  int rc = validate_bwd("rope_attn_bwd_prerotated", B, H, N, D, freq_row_stride, sm_scale,
-                        {q_rot, k_rot, v, o, d_o, lse, delta, freqs_cos, freqs_sin, dq, dk, dv});
+  const int rc = validate_bwd("rope_attn_bwd_prerotated", B, H, N, D, freq_row_stride, sm_scale,
+                              {q_rot, k_rot, v, o, d_o, lse, delta, freqs_cos, freqs_sin, dq, dk, dv});
   if (rc) return rc;
-  rc = corope_rope_attn_bwd_dq_prerotated(q_rot, k_rot, v, o, d_o, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dq, B,
-                                          H, N, D, sm_scale, causal, stream);
-  if (rc) return rc;
-  return corope_rope_attn_bwd_dkdv_prerotated(q_rot, k_rot, v, d_o, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dk,
-                                              dv, B, H, N, D, sm_scale, causal, stream);
+  return corope_rope_attn_bwd_rotated(q_rot, k_rot, v, nullptr, o, d_o, nullptr, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dq, dk,
+                                      dv, B, H, H, N, D, sm_scale, causal, 0, nullptr, 0, stream);
 }
 
 int64_t corope_rope_attn_bwd_workspace_bytes(int B, int H, int N, int D) {
@@ -633,18 +628,16 @@ int corope_rope_attn_bwd_gqa(const void* q, const void* k, int prerotated, const
   if (rc) return rc;
   rc = check_ptrs(what, {q, k, v, o, d_o, lse, delta, freqs_cos, freqs_sin, dq, dk, dv});
   if (rc) return rc;
+  if (prerotated)
+    return corope_rope_attn_bwd_rotated(q, k, v, nullptr, o, d_o, nullptr, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dq, dk, dv, B,
+                                        Hq, Hkv, N, D, sm_scale, causal, 0, nullptr, 0, stream);
   rc = corope_rope_attn_bwd_preprocess(o, d_o, delta, B, Hq, N, D, stream);
   if (rc) return rc;
   corope::BwdParams p = make_bwd(q, k, v, nullptr, d_o, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dq, dk, dv, B, Hq,
                                  N, D, sm_scale, Hkv);
-  mark_prerotated(p, prerotated != 0);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (prerotated) {
-    rc = launch_status(what, corope::launch_bwd_dkdv_fused(p, D, causal != 0, st));
-  } else {
-    rc = launch_status(what, corope::launch_bwd_dv(p, D, causal != 0, st));
-    if (rc == 0) rc = launch_status(what, corope::launch_bwd_dk(p, D, causal != 0, st));
-  }
+  rc = launch_status(what, corope::launch_bwd_dv(p, D, causal != 0, st));
+  if (rc == 0) rc = launch_status(what, corope::launch_bwd_dk(p, D, causal != 0, st));
   if (rc) return rc;
   return launch_status(what, corope::launch_bwd_dq(p, D, causal != 0, st));
 }
@@ -702,17 +695,12 @@ int corope_rope_attn_bwd_f16(const void* q, const void* k, int prerotated, const
   int rc = validate_bwd(what, B, H, N, D, freq_row_stride, sm_scale,
                         {q, k, v, o, d_o, lse, delta, freqs_cos, freqs_sin, dq, dk, dv});
   if (rc) return rc;
+  if (prerotated)
+    return corope_rope_attn_bwd_rotated(q, k, v, nullptr, o, d_o, nullptr, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dq, dk, dv, B,
+                                        H, Hkv, N, D, sm_scale, causal, 1, nullptr, 0, stream);
   corope::BwdParams p = make_bwd(q, k, v, o, d_o, lse, delta, freqs_cos, freqs_sin, freq_row_stride, dq, dk, dv, B, H, N,
                                  D, sm_scale, Hkv);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (prerotated) {
-    // q, k are the rotated copies a two-launch forward kept: the dQ kernel computes delta on its way, dK and dV come
-    // from one kernel
-    mark_prerotated(p, true);
-    rc = launch_status(what, corope_f16::launch_bwd_dq(p, D, causal != 0, st));
-    if (rc) return rc;
-    return launch_status(what, corope_f16::launch_bwd_dkdv_fused(p, D, causal != 0, st));
-  }
   if (workspace != nullptr) {
     // as corope_rope_attn_bwd_ws: q (scaled) and k are rotated once, then as above
     if (!aligned16(workspace)) return fail(COROPE_E_ALIGN, "%s: pointer %p is not 16-byte aligned", what, workspace);

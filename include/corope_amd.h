@@ -203,8 +203,8 @@ int corope_rope_attn_bwd_dq_prerotated(const void *q_rot, const void *k_rot, con
                                        void *dq,
                                        int B, int H, int N, int D, float sm_scale, int causal, void *stream);
 
-/* Whole backward on rotated operands kept from corope_rope_attn_fwd_train (or made by corope_rope_rotate): preprocess,
- * dV, dK, dQ.  Replaces _attention.backward like corope_rope_attn_bwd (reference fused-rope/fused_rope_attn.py:720-777). */
+/* Whole backward on rotated operands kept from corope_rope_attn_fwd_train (or made by corope_rope_rotate):
+ * corope_rope_attn_bwd_rotated on contiguous bf16 tensors without grouped queries and without parts.  Replaces _attention.backward like corope_rope_attn_bwd (reference fused-rope/fused_rope_attn.py:720-777). */
 int corope_rope_attn_bwd_prerotated(const void *q_rot, const void *k_rot, const void *v, const void *o, const void *d_o,
                                     const float *lse, float *delta,
                                     const float *freqs_cos, const float *freqs_sin, int64_t freq_row_stride,
@@ -235,8 +235,7 @@ int corope_rope_attn_bwd_ws(const void *q, const void *k, const void *v, const v
  * rotated Q times sm_scale*log2(e), and (q_rot, k_rot) are then the operands of a backward with prerotated = 1.
  * k_rot != NULL with tile_kmax == NULL: K is rotated once into k_rot and the single-launch kernel runs on the copy, without
  * the rotation in its loop and with its own bookkeeping -- P and V stay fp16, as in the reference -- and q_rot as above.
- * Backward: prerotated = 1: q, k are those rotated copies (dQ kernel, which computes delta on its way, then the fused dK+dV
- * kernel); else preprocess + dV + dK + dQ as in corope_rope_attn_bwd, or -- given a workspace of
+ * Backward: prerotated = 1: q, k are those rotated copies (corope_rope_attn_bwd_rotated without parts); else preprocess + dV + dK + dQ as in corope_rope_attn_bwd, or -- given a workspace of
  * corope_rope_attn_bwd_workspace_bytes (may be NULL) -- the rotation of q and k into it followed by the dQ and the fused
  * dK+dV kernel as in corope_rope_attn_bwd_ws, the faster form from N * D = 65536 on.  `delta` is (B,H,N) fp32 scratch.
  * k, v, dk, dv have Hkv heads (H a multiple of Hkv; Hkv = H: the reference's form), as in the grouped-query entry points below.
@@ -272,7 +271,8 @@ int corope_rope_attn_fwd_strided(const void *q, const int64_t *q_strides, const 
  * reduction its archived GQA experiment (assets/flashattn-gqa/triton_gqa.py:605-666).
  * forward: k_rot NULL = single launch (q_rot and tile_kmax must be NULL too); otherwise K is rotated into k_rot
  * (B,Hkv,N,D) with tile_kmax (B*Hkv*ceil(N/64) floats, scratch) and q_rot (may be NULL) receives the rotated q.
- * backward: prerotated != 0 means q and k are those rotated copies (fused dK+dV kernel); delta (B,Hq,N) is scratch. */
+ * backward: prerotated != 0 means q and k are those rotated copies (corope_rope_attn_bwd_rotated without parts); delta (B,Hq,N) is
+ * scratch. */
 int corope_rope_attn_fwd_gqa(const void *q, const void *k, const void *v,
                              const float *freqs_cos, const float *freqs_sin, int64_t freq_row_stride,
                              void *o, float *lse, void *q_rot, void *k_rot, float *tile_kmax,

@@ -2,6 +2,7 @@
 
 Everything goes through the torch.autograd.Function, i.e. through the C ABI.  Bar: max-abs <= 2e-2 per tensor
 against the fp32 oracle evaluated on the same bf16-rounded q, k, v, dO."""
+import ctypes
 import math
 
 import numpy as np
@@ -511,3 +512,48 @@ def test_backward_without_memory_for_cut_key_blocks(pkg, monkeypatch, dtype):
     step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     for a, b in zip(cut[1:], whole[1:]):
         assert (a.float() - b.float()).abs().max() <= 2 * step * b.float().abs().max() + 1e-5
+
+
+# The C entry points that take rotated copies are one backward: with fewer arguments (bf16 without and with grouped queries, fp16), and
+# with v and dO as strided views.  Without scratch no key block is cut, and all agree bit for bit (with the operator too, where it cuts none).
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 8, 8, 600, 128), (2, 6, 6, 1030, 64), (4, 24, 12, 1100, 128), (1, 2, 2, 300, 256), (1, 1, 1, 513, 128)])
+def test_entry_points_on_rotated_copies_agree(pkg, B, Hq, Hkv, N, D, causal):
+    lib, dev = pkg._lib.load(), torch.device("cuda:0")
+    cut = lib.corope_rope_attn_bwd_rotated_parts_bytes(B, Hq, Hkv, N, D, int(causal)) > 0
+    scale, st = 1 / math.sqrt(D), torch.cuda.current_stream().cuda_stream
+    c, s = (t.to(dev) for t in O.precompute_freqs_cis(D, N))
+    for dtype in (torch.bfloat16, torch.float16):
+        q, k, v = (seeded((B, h, N, D), 100 + i).to(dev, dtype).requires_grad_(True) for i, h in enumerate((Hq, Hkv, Hkv)))
+        g = seeded((B, Hq, N, D), 103).to(dev, dtype)
+        out = pkg.attention(q, k, v, causal, scale, c, s)
+        qr, kr, vs, o, M, fc, fs = (t.detach() for t in out.grad_fn.saved_tensors)
+        want = operator = torch.autograd.grad(out, (q, k, v), g)
+        delta, got = torch.empty_like(M), [torch.empty_like(t) for t in want]
+        tables, grads, scalars = (M, delta, fc, fs), [t.data_ptr() for t in got], (N, D, scale, int(causal))
+
+        def check(name, *args):
+            for t in got:
+                t.fill_(float("nan"))
+            delta.fill_(float("nan"))
+            rc = getattr(lib, name)(*(a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args))
+            assert rc == 0, (name, pkg._lib.last_error())
+            torch.cuda.synchronize()
+            assert cut and want is operator or all(torch.equal(a, b) for a, b in zip(got, want)), (name, dtype)
+
+        check("corope_rope_attn_bwd_rotated", qr, kr, vs, None, o, g, None, *tables, fc.stride(0), *grads, B, Hq, Hkv, *scalars,
+              int(dtype == torch.float16), None, 0, st)
+        want = [t.clone() for t in got]
+        assert all(within_bar(a.float().cpu(), b.float().cpu(), TOL * math.sqrt(Hq // Hkv))[0] for a, b in zip(want, operator))
+        if dtype == torch.float16:
+            check("corope_rope_attn_bwd_f16", qr, kr, 1, vs, o, g, *tables, fc.stride(0), *grads, B, Hq, Hkv, *scalars, None, 0, st)
+        else:
+            check("corope_rope_attn_bwd_gqa", qr, kr, 1, vs, o, g, *tables, fc.stride(0), *grads, B, Hq, Hkv, *scalars, st)
+            if Hq == Hkv:
+                check("corope_rope_attn_bwd_prerotated", qr, kr, vs, o, g, *tables, fc.stride(0), *grads, B, Hq, *scalars, st)
+        if D <= 128:   # rows of the heads interleaved, and a fused projection's row stride
+            gv = g.transpose(1, 2).contiguous().transpose(1, 2)
+            vv = torch.stack((vs, vs, vs), 2).permute(0, 3, 2, 1, 4).contiguous()[:, :, 2].transpose(1, 2)
+            sv, sg = ((ctypes.c_int64 * 3)(*t.stride()[:3]) for t in (vv, gv))
+            check("corope_rope_attn_bwd_rotated", qr, kr, vv, sv, o, gv, sg, *tables, fc.stride(0), *grads, B, Hq, Hkv, *scalars,
+                  int(dtype == torch.float16), None, 0, st)

@@ -440,10 +440,13 @@ def test_backward_cut_key_blocks(pkg, B, Hq, Hkv, N, D, cut, causal, dtype):
     ref = O.rope_attn_fwd_bwd_blocked(q.contiguous(), kx, vx, g.contiguous(), causal, scale, c, s)
     rdq, rdk, rdv = ref[2], *(t.reshape(B, Hkv, G, N, D).sum(2) for t in ref[3:5])
     for name, a, b in (("dQ", grads[0], rdq), ("dK", grads[1], rdk), ("dV", grads[2], rdv)):
-        # dK and dV sum G heads' contributions before the one rounding.  On gradients of magnitude 2 to 4 that rounding alone is up
-        # to 7.8e-3 (half a bf16 step), on top of the errors of P and dS rounded to 8 bits that the bar of 2e-2 is met with at
-        # magnitude 1 to 2, where it is half as large: 2.4e-2.
-        ok, err = within_bar(a.float().cpu(), b, 2.4e-2 * (math.sqrt(G) if name != "dQ" else 1.0))[:2]
+        a = a.float().cpu()
+        err, heads = (a - b).abs().max(), math.sqrt(G) if name != "dQ" else 1.0   # dK and dV sum G heads' contributions
+        # From magnitude 2 on bf16's rounding alone is up to 2^-7 (half a step), 3.9e-3 more than at magnitude 1 to 2, where the bar of
+        # 2e-2 holds with it: 2.4e-2 there.
+        large = b.abs() >= 2
+        ok = within_bar(a[~large], b[~large], TOL * heads)[0] and (
+            not large.any() or within_bar(a[large], b[large], (TOL if name == "dQ" else 2.4e-2) * heads)[0])
         print(f"  {name}: max-abs {err:.3e} (|ref| max {b.abs().max():.2f})", flush=True)
         assert ok, name
 

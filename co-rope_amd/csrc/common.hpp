@@ -766,21 +766,9 @@ __device__ __forceinline__ void store_rows_via_lds(const f32x16 (&acc)[D / 32], 
   lds_order();
 }
 
-// A operand of mfma16 (16 rows m x 32 contraction slots) read transposed from a row-major tile T[k][m]: lane l gets
-// T[kbase + 8*(l / 16) + j][m0 + l % 16] for slots j = 0..7 (two transposing reads of 4 contraction rows each).
-__device__ __forceinline__ u32x4 load_a_trans16(const uint16_t* tile, int stride, int kbase, int m0) {
-  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
-  const int l = threadIdx.x % kWave;
-  const int g = l / 16, s = l % 16;
-  const uint16_t* p = tile + (kbase + 8 * g + s / 4) * stride + m0 + 4 * (s % 4);
-  s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p));
-  s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + 4 * stride));
-  u32x2 a = __builtin_bit_cast(u32x2, lo), b = __builtin_bit_cast(u32x2, hi);
-  return u32x4{a[0], a[1], b[0], b[1]};
-}
-
-// The same for contraction slots in the order in which two 16x16 accumulator blocks hand out their rows: slots j of lane group
-// l / 16 <-> k = kbase + 16*(j / 4) + 4*(l / 16) + j % 4.
+// A operand of mfma16 (16 rows m x 32 contraction slots) read transposed from a row-major tile T[k][m], contraction slots in the order in
+// which two 16x16 accumulator blocks hand out their rows: lane l gets T[k][m0 + l % 16], k = kbase + 16*(j / 4) + 4*(l / 16) + j % 4, for
+// slots j = 0..7 (two transposing reads of 4 contraction rows each).
 __device__ __forceinline__ u32x4 load_a_trans16_acc(const uint16_t* tile, int stride, int kbase, int m0) {
   typedef __attribute__((address_space(3))) s16x4* lds_ptr;
   const int l = threadIdx.x % kWave;
@@ -814,11 +802,6 @@ __device__ __forceinline__ u32x4 load_a_trans_natural(const uint16_t* tile, int 
 }
 
 // ---- wave-wide reductions and scans ---------------------------------------------------------------------------------
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m);
-  return x;
-}
 // Wave-wide scan and maximum with data-parallel-primitive moves (no LDS round trips): shifts by 1, 2, 4, 8 inside each
 // row of 16 lanes, then lane 15 of rows 0 and 2 is broadcast into rows 1 and 3, then lane 31 into rows 2 and 3.  Lanes
 // without a source take `identity`.  All 64 lanes must be active.
@@ -894,7 +877,6 @@ __device__ __forceinline__ float sigmoid(float x) {
 
 __device__ __forceinline__ float bf16_to_f(uint16_t x) { return __builtin_bit_cast(float, (uint32_t)x << 16); }
 __device__ __forceinline__ uint16_t f_to_bf16(float x) { return (uint16_t)(pack_bf16(x, 0.f) & 0xffffu); }
-__device__ __forceinline__ uint16_t f_to_f16(float x) { return (uint16_t)(pack_f16(x, 0.f) & 0xffffu); }
 __device__ __forceinline__ uint16_t f_to_elt(float x) { return (uint16_t)(pack_elts(x, 0.f) & 0xffffu); }
 __device__ __forceinline__ float elt_to_f(uint16_t x) { return elt_lo((uint32_t)x); }
 

@@ -147,7 +147,7 @@ int corope_gqa_check(int B, int Hq, int Hkv, int N, int D, float sm_scale, float
   if (D != 64 && D != 128) return fail(COROPE_E_UNSUPPORTED, "corope_gqa: head dim %d not built (64 and 128 are)", D);
   if (!std::isfinite(sm_scale)) return fail(COROPE_E_BADARG, "corope_gqa: sm_scale must be finite");
   if (!(theta > 0.f) || !std::isfinite(theta)) return fail(COROPE_E_BADARG, "corope_gqa: theta must be positive and finite");
-  // one workgroup per (batch, kv head, query row) on a single grid axis; slabs addressed with 32-bit byte offsets
+  // at most one wave per (batch, kv head, query row), on a single grid axis; slabs addressed with 32-bit byte offsets
   if ((int64_t)B * Hkv * N >= ((int64_t)1 << 31) || (int64_t)N * D * 2 >= ((int64_t)1 << 32))
     return fail(COROPE_E_UNSUPPORTED, "corope_gqa: B * Hkv * N = %lld rows exceed the grid, or one slab exceeds 4 GiB",
                 (long long)B * Hkv * N);

@@ -324,8 +324,9 @@ static hipError_t launch_corope_rows(CoropeParams p, const CoropeFreqs& fr, hipS
 template <int D, int G, int REDUCED>
 static hipError_t launch_corope_cfg(const CoropeParams& p, const CoropeFreqs& fr, hipStream_t stream) {
   // Rows per wave: as many as fill the 16 columns where that leaves four waves per SIMD, of which two run at a time; below that
-  // the longest rows, whose chunks follow one after the other, set the time, and fewer rows per wave shorten it (B1 Hq32 Hkv8
-  // N1111 D128: 190 us with four rows, 165 with two).
+  // the longest rows, whose chunks follow one after the other, set the time, and fewer rows per wave shorten it.  us with four / two /
+  // one row per wave at D = 128, fp16 B1 Hq32 Hkv8 N1111 171 / 143 / 179, bf16 B2 Hq16 Hkv4 N1024 152 / 122 / 153 and N2048 418 / 466 / 582;
+  // at D = 64, B2 Hq8 Hkv2 N512 39 / 24 / 18.
   constexpr int kMost = G <= 2 ? 8 : G <= 4 ? 4 : 2;
   const int64_t rows = (int64_t)p.N * p.B * p.Hkv, simds = 4 * device_cu_count();
   if (rows >= 4 * simds * kMost) return launch_corope_rows<D, G, kMost, REDUCED>(p, fr, stream);

@@ -888,7 +888,7 @@ template <bool DO_DV, bool DO_DK>
 static hipError_t launch_dkdv(const BwdParams& p, int D, bool causal, hipStream_t stream) {
   const bool pre = p.q_rot != nullptr && p.k_rot != nullptr;
 #define COROPE_DKDV(DD, CC, PP) launch_dkdv_cfg<DD, CC, DO_DV, DO_DK, PP>(p, stream)
-  if (D == 256) {   // separate dV and dK only: the accumulators of both do not fit one wave
+  if (D == 256) {   // separate dV and dK only: both in one launch is built for rotated copies alone (launch_bwd_dkdv_fused)
     if (DO_DV && DO_DK) return hipErrorInvalidValue;
     if constexpr (!(DO_DV && DO_DK)) {
       if (pre) return causal ? COROPE_DKDV(256, true, true) : COROPE_DKDV(256, false, true);

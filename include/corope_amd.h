@@ -289,7 +289,8 @@ int corope_rope_attn_bwd_gqa(const void *q, const void *k, int prerotated, const
  * corope_rope_attn_fwd_strided; NULL: contiguous); everything else is contiguous.  parts: scratch for partial sums, with which the dK+dV launch cuts its work into equal
  * pieces; corope_rope_attn_bwd_rotated_parts_bytes says how much, 0 where whole key blocks fill the chip as well (then, and if
  * NULL is passed, nothing is cut).  delta: (B,H,N) fp32 scratch.  Replaces _attention.backward
- * (fused-rope/fused_rope_attn.py:725-777; group sum: assets/flashattn-gqa/triton_gqa.py:605-666). */
+ * (fused-rope/fused_rope_attn.py:725-777; group sum: assets/flashattn-gqa/triton_gqa.py:605-666).  parts takes at most two slots per
+ * compute unit: with 256 of them 64 MiB at D = 64, 128 MiB at D = 128 and 256, whatever the tensors' sizes. */
 int64_t corope_rope_attn_bwd_rotated_parts_bytes(int B, int H, int Hkv, int N, int D, int causal);
 int corope_rope_attn_bwd_rotated(const void *q_rot, const void *k_rot, const void *v, const int64_t *v_strides, const void *o,
                                  const void *d_o, const int64_t *do_strides, const float *lse, float *delta,
@@ -314,15 +315,16 @@ int corope_gqa_fwd_f16(const void *q, const void *k, const void *v, void *o,
 
 /* Bytes of device workspace corope_gqa_bwd needs for these sizes (-1 for sizes corope_gqa_check rejects):
  * packed lower-triangular N x N fp32 matrices (about N*N/2 + 32*N floats each): two per key/value head (accumulated
- * gates; gate gradients) and three per query head (attention weights; score gradients; dO V^T), plus N*D floats per
- * key/value head (the leader head's dq before its gate-path term is added). */
+ * gates; gate gradients) and two per query head (scores; score gradients), one matrix's space more per query head for the row
+ * statistics and the partial sums of dv and dk, plus N*D floats per key/value head (the leader head's dq before its gate-path
+ * term is added). */
 int64_t corope_gqa_bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D);
 
 /* The smallest workspace corope_gqa_bwd accepts: the matrices of ONE (batch, key/value head) group, i.e. the figure above
  * divided by B*Hkv.  Groups are independent, so with a workspace between the two sizes the launch sequence runs once per
- * batch of as many groups as fit.  Fewer, larger passes are much faster, because two of the kernels spread over key blocks
- * x groups only: at B2 Hq32 Hkv8 N4096 D128 on MI355X 14.3 ms with all 16 groups in one pass (7.1 GiB), 31 ms with 4 per
- * pass (1.8 GiB), 94 ms with 1 (0.45 GiB) -- give it what memory allows.  -1 for sizes corope_gqa_check rejects. */
+ * batch of as many groups as fit.  Fewer, larger passes are faster, because a pass of few groups has too few rows to fill the
+ * chip and waits for its longest ones: at B2 Hq32 Hkv8 N4096 D128 on MI355X 10.9 ms with all 16 groups in one pass (7.1 GiB), 16.3 ms
+ * with 4 per pass (1.8 GiB), 51.9 ms with 1 (0.45 GiB) -- give it what memory allows.  -1 for sizes corope_gqa_check rejects. */
 int64_t corope_gqa_bwd_min_workspace_bytes(int B, int Hq, int Hkv, int N, int D);
 
 /* Co-RoPE grouped-query attention backward (causal only): dq (B,Hq,N,D), dk/dv (B,Hkv,N,D) from q, k, v and dO.

@@ -61,15 +61,17 @@ struct DkdvCfg {
   static_assert(kLdsBytes <= 160 * 1024, "LDS of a compute unit");
 };
 
-// v and d_o may be strided views (BwdParams) up to D = 128; at D = 256, where the registers for run-time strides cost the dK+dV
-// kernel 10 % (222 -> 245 us at B2 H16 N2048), they are contiguous.
-template <int D>
-__device__ __forceinline__ uint32_t do_row_bytes(const BwdParams& p) { return D > 128 ? D * 2 : (uint32_t)p.do_sn * 2; }
-template <int D>
-__device__ __forceinline__ uint32_t v_row_bytes(const BwdParams& p) { return D > 128 ? D * 2 : (uint32_t)p.v_sn * 2; }
-template <int D>
+// v and d_o may be strided views (BwdParams) on rotated copies up to D = 128; the kernels' STRIDED says whether they read them through
+// run-time strides.  At D = 256 the registers for these cost the dK+dV kernel 10 % (222 -> 245 us at B2 H16 N2048).  On unrotated
+// operands, which have none, they cost dK and dV up to 3 % (dK B6 H4 N274 D128 not causal 24.7 -> 25.5 us, dV B4 H32 N900 D64 33.7 -> 34.3),
+// and dQ nothing (B4 H32 N448 D128 44.1 us with, 44.5 without).
+template <int D, bool STRIDED>
+__device__ __forceinline__ uint32_t do_row_bytes(const BwdParams& p) { return STRIDED ? (uint32_t)p.do_sn * 2 : D * 2; }
+template <int D, bool STRIDED>
+__device__ __forceinline__ uint32_t v_row_bytes(const BwdParams& p) { return STRIDED ? (uint32_t)p.v_sn * 2 : D * 2; }
+template <int D, bool STRIDED>
 __device__ __forceinline__ const uint16_t* v_slab_of(const BwdParams& p, int kvs) {
-  return D > 128 ? p.v + (int64_t)kvs * p.N * D : p.v_slab(kvs);
+  return STRIDED ? p.v_slab(kvs) : p.v + (int64_t)kvs * p.N * D;
 }
 
 // What a workgroup of the dK+dV kernel works on.  CUT = false: whole items dealt in rounds (ItemList).  CUT = true: the query
@@ -141,7 +143,7 @@ template <int D, int NWAVES, int BLOCK_M, bool CAUSAL, bool DO_DV, bool DO_DK, b
 __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<D>, kWavesPerSimd<D>))) void rope_attn_bwd_dkdv_kernel(BwdParams p) {
   constexpr int DO_PAD = DO_DK ? (DO_DV ? kDkdvBothWaysPad : 8) : 32;
   constexpr int Q_PAD = DO_DK ? kDkdvBothWaysPad : 8;
-  constexpr bool V_LDS = DO_DV && DO_DK;
+  constexpr bool V_LDS = DO_DV && DO_DK, STRIDED = PREROT && D <= 128;
   using Cfg = DkdvCfg<D, NWAVES, BLOCK_M, DO_PAD, Q_PAD>;
   constexpr int NT = Cfg::kThreads;
   constexpr int KC = D / 16, NDB = D / 32, NQB = BLOCK_M / 32;
@@ -178,7 +180,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     if (i >= total) return false;
     const int bkv = i % BHkv, n0 = (i / BHkv) * Cfg::kBlockN;
     l_slab0 = (bkv / p.Hkv) * p.H + (bkv % p.Hkv) * GQ;   // first query head of the group
-    if constexpr (D <= 128) l_do = p.do_slab(l_slab0);
+    if constexpr (STRIDED) l_do = p.do_slab(l_slab0);
     l_mt0 = CAUSAL ? n0 / BLOCK_M : 0;
     l_tph = max(m_tiles - l_mt0, 0);
     l_it = items.begin(i);
@@ -196,7 +198,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     }
     const int qs = l_slab0 + l_it / l_tph, m0 = (l_mt0 + l_it % l_tph) * BLOCK_M;
     qst.load(q_all + (int64_t)qs * N * D, p.cos, p.sin, p.fstride, m0, N);
-    dst.load(D > 128 ? p.d_o + (int64_t)qs * N * D : l_do + (qs - l_slab0) * p.do_sh, m0, N, do_row_bytes<D>(p));
+    dst.load(STRIDED ? l_do + (qs - l_slab0) * p.do_sh : p.d_o + (int64_t)qs * N * D, m0, N, do_row_bytes<D, STRIDED>(p));
     if (threadIdx.x < BLOCK_M) {
       int qi = m0 + threadIdx.x;
       // -M and -delta: what the S and dP products start from.  Rows past the end: M = +inf makes P = 0, so they
@@ -238,7 +240,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     const int64_t base = (int64_t)(i % BHkv) * N * D;
     const int row0 = (i / BHkv) * Cfg::kBlockN + rb * 32, l = opaque_lane();
     krows.load((PREROT ? p.k_rot : p.k) + base, p.cos, p.sin, p.fstride, row0, N, l);
-    if constexpr (DO_DK) vrows_regs.load(v_slab_of<D>(p, i % BHkv), nullptr, nullptr, 0, row0, N, l, v_row_bytes<D>(p));
+    if constexpr (DO_DK) vrows_regs.load(v_slab_of<D, STRIDED>(p, i % BHkv), nullptr, nullptr, 0, row0, N, l, v_row_bytes<D, STRIDED>(p));
   };
   auto take_rows = [&]() __attribute__((always_inline)) {
     const int l = opaque_lane();
@@ -504,6 +506,7 @@ template <int D, int NWAVES, int BLOCK_N, bool CAUSAL, bool PREROT>
 __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<D>, kWavesPerSimd<D>))) void rope_attn_bwd_dq_kernel(BwdParams p) {
   using Cfg = DqCfg<D, NWAVES, BLOCK_N>;
   constexpr int NT = Cfg::kThreads;
+  constexpr bool STRIDED = D <= 128;
   constexpr int KC = D / 16, NDB = D / 32, NKB = BLOCK_N / 32;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
@@ -534,7 +537,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     if (i >= total) return false;
     const int64_t kv_base = (int64_t)kv_slab(i % p.BH, p.H, p.Hkv) * N * D;
     l_kg = (PREROT ? p.k_rot : p.k) + kv_base;
-    l_vg = v_slab_of<D>(p, kv_slab(i % p.BH, p.H, p.Hkv));
+    l_vg = v_slab_of<D, STRIDED>(p, kv_slab(i % p.BH, p.H, p.Hkv));
     l_tiles = tiles_of(p.num_blocks - 1 - i / p.BH);
     return true;
   };
@@ -546,7 +549,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       l_tile = 0;
     }   // else: past the last tile of the last item; the same tile is requested again and never used
     kst.load(l_kg, p.cos, p.sin, p.fstride, l_tile * BLOCK_N, N);
-    vst.load(l_vg, l_tile * BLOCK_N, N, v_row_bytes<D>(p));
+    vst.load(l_vg, l_tile * BLOCK_N, N, v_row_bytes<D, STRIDED>(p));
   };
   auto k_tile = [&](int buf) { return reinterpret_cast<uint16_t*>(smem + buf * Cfg::kStageBytes); };
   auto v_tile = [&](int buf) { return reinterpret_cast<uint16_t*>(smem + buf * Cfg::kStageBytes + Cfg::kKTileBytes); };
@@ -570,11 +573,11 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     const int64_t base = (int64_t)bh * N * D;
     const int l = opaque_lane();
     qrows.load((PREROT ? p.q_rot : p.q) + base, p.cos, p.sin, p.fstride, row0, N, l);
-    const uint16_t* dog = D > 128 ? p.d_o + base : p.do_slab(bh);
-    dorows.load(dog, nullptr, nullptr, 0, row0, N, l, do_row_bytes<D>(p));
+    const uint16_t* dog = STRIDED ? p.do_slab(bh) : p.d_o + base;
+    dorows.load(dog, nullptr, nullptr, 0, row0, N, l, do_row_bytes<D, STRIDED>(p));
     // (without O the dO rows are requested twice: the request is then unconditional and the registers it fills are free
     // during the tile loop on every path)
-    orows.load(p.o != nullptr ? p.o + base : dog, nullptr, nullptr, 0, row0, N, l, p.o != nullptr ? (uint32_t)D * 2 : do_row_bytes<D>(p));
+    orows.load(p.o != nullptr ? p.o + base : dog, nullptr, nullptr, 0, row0, N, l, p.o != nullptr ? (uint32_t)D * 2 : do_row_bytes<D, STRIDED>(p));
     const int q_c = min(row0 + l % 32, N - 1);
     lse_q = p.lse[(int64_t)bh * N + q_c];
     // delta_i = sum_d o_id * do_id (reference _attn_bwd_preprocess, :324-337): read from the preprocess pass, or -- when the
@@ -619,7 +622,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   COROPE_ISTAMP(0);
   load_item(0);
   kst.load(l_kg, p.cos, p.sin, p.fstride, 0, N);
-  vst.load(l_vg, 0, N, v_row_bytes<D>(p));
+  vst.load(l_vg, 0, N, v_row_bytes<D, STRIDED>(p));
   request_rows(item);
   take_rows(item);
   kst.store_rows(k_tile(0));

@@ -89,11 +89,11 @@ struct CoropeBwdWs {
 //   dq       needs the rotated keys transposed: they go through LDS (16 keys x D x R rows per wave) and come back through the
 //            transposing read.  The weights of the two sums, e (dP - ref) and e, share the 16 columns in the same way (a rotation by 8
 //            lanes), and two rows share the 32 contraction slots of a product (the other row's columns of B are zero).
-// No barriers: a wave is a workgroup.  What bounds it: in the first sweep the vector units (busy 82 % of it; 9 or 10 issue slots per (row, key,
+// No barriers: a wave is a workgroup.  What bounds it: in the first sweep the vector units (busy 71 % of both sweeps together; 9 or 10 issue slots per (row, key,
 // pair) as in the forward, of about 12 in all), in the second the memory (9 floats in, 5 out per (row, key) at G = 4); two waves a
 // SIMD hide one under the other only in part.  dP is computed in both sweeps, and P is left to the dv kernel: kept in the workspace they cost
 // 12 floats more per (row, key) and a launch.
-// Measured at B2 Hq32 Hkv8 N4096 D128: 8.2 -> 5.9 ms, first sweep 4.6 (one wave per row with the rotated keys in LDS, behind launches for the
+// Measured at B2 Hq32 Hkv8 N4096 D128: 8.2 -> 6.1 ms, three quarters of it the first sweep (one wave per row with the rotated keys in LDS, behind launches for the
 // logits and dP); B2 Hq8 Hkv2 N512 D64 52 -> 40 us.
 template <int D, int G, int R, int REDUCED>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void corope_bwd_scores_kernel(CoropeBwdParams p, CoropeBwdWs ws,
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
 
   const int nb = iw / 16 + 1;
   // A block of 16 rows of K or V: an operand piece read straight from memory is 16 bytes of a row per lane, neighbouring lanes in different
-  // rows, and the address unit then handles one lane per cycle (it was busy 81 % of this kernel's time).  So a block is requested with
+  // rows, and the address unit then handles one lane per cycle (which bound this kernel).  So a block is requested with
   // consecutive pieces in consecutive lanes and takes its operand order in LDS.
   auto request = [&](u32x4 (&x)[NKS], const uint16_t* base, int b) __attribute__((always_inline)) {
 #pragma unroll

@@ -323,8 +323,8 @@ int64_t corope_gqa_bwd_workspace_bytes(int B, int Hq, int Hkv, int N, int D);
 /* The smallest workspace corope_gqa_bwd accepts: the matrices of ONE (batch, key/value head) group, i.e. the figure above
  * divided by B*Hkv.  Groups are independent, so with a workspace between the two sizes the launch sequence runs once per
  * batch of as many groups as fit.  Fewer, larger passes are faster, because a pass of few groups has too few rows to fill the
- * chip and waits for its longest ones: at B2 Hq32 Hkv8 N4096 D128 on MI355X 10.9 ms with all 16 groups in one pass (7.1 GiB), 16.3 ms
- * with 4 per pass (1.8 GiB), 51.9 ms with 1 (0.45 GiB) -- give it what memory allows.  -1 for sizes corope_gqa_check rejects. */
+ * chip and waits for its longest ones: at B2 Hq32 Hkv8 N4096 D128 on MI355X 11.1 ms with all 16 groups in one pass (7.1 GiB), 16.8 ms
+ * with 4 per pass (1.8 GiB), 52.3 ms with 1 (0.45 GiB) -- give it what memory allows.  -1 for sizes corope_gqa_check rejects. */
 int64_t corope_gqa_bwd_min_workspace_bytes(int B, int Hq, int Hkv, int N, int D);
 
 /* Co-RoPE grouped-query attention backward (causal only): dq (B,Hq,N,D), dk/dv (B,Hkv,N,D) from q, k, v and dO.

@@ -895,6 +895,14 @@ inline int corope_reduced_blocks(const float* turns, int D, int N) {
   return blocks;
 }
 
+// The same in groups of 16 pairs.
+inline int corope_reduced_groups(const float* turns, int D, int N) {
+  int groups = 0;
+  for (int d = 0; d < D / 2; ++d)
+    if (!(turns[d] * (float)N < 255.f)) groups = d / 16 + 1;
+  return groups;
+}
+
 // f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>): a loop whose index is a compile-time constant
 // in the body, so register arrays indexed with it never look dynamically indexed to the optimiser.
 template <int... I, class F>
@@ -905,5 +913,130 @@ template <int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
 }
+
+// ---- Co-RoPE's slow pairs ------------------------------------------------------------------------------------------------------
+// Within a chunk of 64 keys a row's delta moves by at most 64: delta = mid + x, |x| <= kCoropeReach.  For a pair that turns slowly the
+// rotation by x is a short polynomial, and with complex numbers for the pairs and a = q e^(i mid w)
+//   conj(q) k e^(-i delta w) = conj(a) k e^(-i x w) = sum_n x^n conj(a (i w)^n / n!) k :
+// a row's scores of the chunk are a few products with the keys AS THEY ARE, one per power of x, which the matrix cores do for all rows at
+// once, instead of one rotation per (row, key, pair) on the vector units; what is rotated per (row, head, pair) and chunk is the query.
+//   class 0  |x w| <= 0.34:   powers 0 .. 4, remainder below 1e-5 (z^5 / 120 of the sine is folded into its cubic term)
+//   class 1  |x w| <= 0.04:   powers 0 .. 2, remainder below 1.1e-5
+// against half a unit of fp16, 2.4e-4, that rounding a rotated key costs.  Precision of the operands: the keys are exact; power 0 is carried
+// as two parts of the element type, and so is power 1 of class 0 with bf16.
+constexpr float kCoropeReach = 32.f, kCoropeLow0 = 0.34f, kCoropeLow1 = 0.04f;
+
+// How many trailing groups of 16 pairs may take the polynomial: the first of them class 0, a second one class 1.
+inline int corope_low_groups(const float* turns, int D) {
+  const int ng = D / 32;
+  auto slow = [&](int group, float limit) { return turns[16 * group] * 6.2831853f * kCoropeReach <= limit; };
+  if (ng > 2 && slow(ng - 2, kCoropeLow0) && slow(ng - 1, kCoropeLow1)) return 2;
+  return slow(ng - 1, kCoropeLow0) ? 1 : 0;
+}
+
+// x as one or two operands of the element type, second = what the first leaves over.
+__device__ __forceinline__ u32x4 pack_elts8(const float (&x)[8]) {
+  return u32x4{pack_elts(x[0], x[1]), pack_elts(x[2], x[3]), pack_elts(x[4], x[5]), pack_elts(x[6], x[7])};
+}
+__device__ __forceinline__ u32x4 pack_rest8(const float (&x)[8], u32x4 first) {
+  float r[8];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    r[2 * e] = x[2 * e] - elt_lo(first[e]);
+    r[2 * e + 1] = x[2 * e + 1] - elt_hi(first[e]);
+  }
+  return pack_elts8(r);
+}
+
+// B operands of the products above for one column (row, head) per lane, for LOW trailing groups of 16 pairs.
+template <int LOW>
+struct CoropeLowOps {
+  static_assert(LOW == 1 || LOW == 2, "a class 0 group and perhaps a class 1 group behind it");
+  // (an fp16 query of 60000 would leave fp16's range on its way round: halved, and the scores doubled again)
+  static constexpr float kScale = kEltIsF16 ? 0.5f : 1.f;
+  u32x4 c[5], c0r, c1r;   // class 0: powers 0..4, remainders of powers 0 and 1
+  u32x4 d[3], d0r;        // class 1
+
+  // raw: the column's query, groups in operand order; turns: w / 2 pi of this lane's pairs; mid: the chunk's middle
+  __device__ __forceinline__ void build(const u32x4* raw, const float (*turns)[4], float mid) {
+    static_for<LOW>([&](auto u_c) __attribute__((always_inline)) {
+      constexpr int u = decltype(u_c)::value;
+      float v[8], w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t w1 = raw[u][e / 2], w2 = raw[u][2 + e / 2];
+        const float q1 = (e % 2 ? elt_hi(w1) : elt_lo(w1)) * kScale, q2 = (e % 2 ? elt_hi(w2) : elt_lo(w2)) * kScale;
+        const float x = __builtin_amdgcn_fractf(mid * turns[u][e]);
+        const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
+        v[e] = __builtin_fmaf(cs, q1, -(sn * q2));
+        v[4 + e] = __builtin_fmaf(cs, q2, sn * q1);
+        float t = turns[u][e];
+        asm volatile("" : "+v"(t));   // (or its multiples below are kept in registers across the caller's loop)
+        w[e] = t * (6.2831853f * kCoropeReach);
+      }
+      auto times_iw = [&](float f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float a = v[e], b = v[4 + e], we = w[e] * f;
+          v[e] = -b * we;
+          v[4 + e] = a * we;
+        }
+      };
+      if constexpr (u == 0) {
+        // sine: z - z^3 (1 / 6 - 0.8 Z^2 / 120), cosine: 1 - z^2 / 2 + z^4 / 24
+        constexpr float c3 = 1.f / 6.f - 0.8f * kCoropeLow0 * kCoropeLow0 / 120.f;
+        c[0] = pack_elts8(v);
+        c0r = pack_rest8(v, c[0]);
+        times_iw(1.f);
+        c[1] = pack_elts8(v);
+        if constexpr (!kEltIsF16) c1r = pack_rest8(v, c[1]);
+        times_iw(0.5f);
+        c[2] = pack_elts8(v);
+        times_iw(2.f * c3);
+        c[3] = pack_elts8(v);
+        times_iw(1.f / (24.f * c3));
+        c[4] = pack_elts8(v);
+      } else {
+        d[0] = pack_elts8(v);
+        d0r = pack_rest8(v, d[0]);
+        times_iw(1.f);
+        d[1] = pack_elts8(v);
+        times_iw(0.5f);
+        d[2] = pack_elts8(v);
+      }
+    });
+  }
+
+  // s = the slow pairs' share of q . kt for B blocks of 16 keys: column = this lane's, rows (keys) 4 (lane / 16) ..; kf: the keys as A
+  // operands, y = x / kCoropeReach of those keys
+  template <int B>
+  __device__ __forceinline__ void scores(const u32x4 (&kf)[B][LOW], const f32x4 (&y)[B], f32x4 (&s)[B]) const {
+#pragma unroll
+    for (int b = 0; b < B; ++b) s[b] = mfma16(kf[b][0], c[4], f32x4{0, 0, 0, 0});
+#pragma unroll
+    for (int b = 0; b < B; ++b) s[b] = mfma16(kf[b][0], c[3], s[b] * y[b]);
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      s[b] = mfma16(kf[b][0], c[2], s[b] * y[b]);
+      if constexpr (LOW > 1) s[b] = mfma16(kf[b][1], d[2], s[b]);
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      s[b] *= y[b];
+      if constexpr (!kEltIsF16) s[b] = mfma16(kf[b][0], c1r, s[b]);
+      s[b] = mfma16(kf[b][0], c[1], s[b]);
+      if constexpr (LOW > 1) s[b] = mfma16(kf[b][1], d[1], s[b]);
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      s[b] *= y[b];
+      s[b] = mfma16(kf[b][0], c0r, s[b]);
+      if constexpr (LOW > 1) s[b] = mfma16(kf[b][1], d0r, s[b]);
+      s[b] = mfma16(kf[b][0], c[0], s[b]);
+      if constexpr (LOW > 1) s[b] = mfma16(kf[b][1], d[0], s[b]);
+      if constexpr (kEltIsF16) s[b] *= 1.f / kScale;
+    }
+  }
+};
 
 }  // namespace COROPE_NS

@@ -185,6 +185,7 @@ struct CoropeParams {
   float theta;  // RoPE base; inverse frequencies are theta^(-2d/D)
   int B, Hq, Hkv, N;
   int num_m_blocks;
+  int turn_from, turn_to;   // workgroups that take their items in reverse order (multiples of 8; none: 0, 0)
 };
 
 struct CoropeBwdParams {

@@ -150,3 +150,40 @@ def test_forward_scale_zero_or_negative(pkg, groups, G, N, D, scale, dtype):
     for g in {0, groups // 2, groups - 1}:
         ref = C.corope_gqa_forward(q[g:g + 1].double(), k[g:g + 1].double(), v[g:g + 1].double(), True, scale, 10000.0, torch.float64)
         assert (o[g:g + 1].double().cpu() - ref).abs().max() <= TOL, g
+
+
+# Sizes at which the forward takes the slow pairs through the polynomial: two, four and eight rows per wave (the group sizes' most), both
+# head dims, ragged lengths, fewer columns than 16.  "open": leaders that see every gate open, so that delta moves by 64 over a chunk of 64 keys
+# and the polynomials are used out to their ends; "shut": by next to nothing.
+LOW_CASES = [(1, 64, 16, 257, 64, 1e4), (1, 64, 8, 385, 128, 1e4), (1, 64, 16, 449, 128, 1e4), (2, 48, 16, 259, 64, 1e4), (2, 64, 32, 129, 128, 1e4),
+             (4, 32, 32, 130, 64, 1e4), (4, 64, 32, 131, 128, 1e4), (1, 256, 32, 130, 64, 9300.0), (1, 64, 16, 449, 128, 5e5), (1, 64, 16, 449, 128, 3000.0)]
+
+
+@pytest.mark.parametrize("gates", ["random", "open", "shut"])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,theta", LOW_CASES)
+def test_corope_forward_slow_pairs(pkg, B, Hq, Hkv, N, D, theta, gates):
+    """fp16, because its rounding hides the least: |O - O64| <= 4e-3 follows from P's rounding (2^-11 of sum P |v|, |v| < 4.7) and the
+    output's own (2^-12 of |O|), a fourth of which is left for the scores; where theta is too small for the polynomial a rotated key
+    is rounded, 12 nats of a leader's score by 2^-12, and |O| moves by up to 2e-2.  A leader row that is not finite stays its own."""
+    print(f"case B={B} Hq={Hq} Hkv={Hkv} N={N} D={D} theta={theta} {gates}", flush=True)
+    G, scale = Hq // Hkv, 1 / math.sqrt(D)
+    q, k, v = (torch.randn(B, h, N, D, generator=torch.Generator().manual_seed(9 + i)).half() for i, h in enumerate((Hq, Hkv, Hkv)))
+    if gates != "random":   # logits of +-12 from the slowest pair (no rounded rotation in them): sigmoid within 1e-4 of 1 or 0
+        k[..., D // 2 - 1] = 4.0
+        q[:, ::G, :, D // 2 - 1] = (1 if gates == "open" else -1) * 3.0 * math.sqrt(D)
+    dev = torch.device("cuda:0")
+    o = pkg.corope_attention(q.to(dev), k.to(dev), v.to(dev), True, scale, theta)
+    q_bad = q.clone()
+    q_bad[0, 0, N - 3] = float("nan")
+    o_bad = pkg.corope_attention(q_bad.to(dev), k.to(dev), v.to(dev), True, scale, theta)
+    torch.cuda.synchronize()
+    rows = torch.ones(N, dtype=torch.bool)
+    rows[N - 3] = False
+    assert torch.isfinite(o).all() and torch.isnan(o_bad[0, 0, N - 3]).all()
+    assert torch.equal(o_bad[0, :, rows], o[0, :, rows]) and torch.equal(o_bad[1:], o[1:])
+    for b, kv in ((0, 0), (B - 1, Hkv - 1)):
+        hs, sl = (slice(b, b + 1), slice(kv * G, (kv + 1) * G)), (slice(b, b + 1), slice(kv, kv + 1))
+        ref = C.corope_gqa_forward_rows(q[hs].double(), k[sl].double(), v[sl].double(), True, scale, theta, torch.arange(N), torch.float64)
+        err = (o[hs].double().cpu() - ref).abs()
+        print(f"  O max-abs {err.max():.3e} mean-abs {err.mean():.3e}")
+        assert err.max() <= (4e-3 if theta > 9222 else TOL)

@@ -892,30 +892,45 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
 //       its half: one (sin, cos) and four multiply-adds per (row, key, pair).
 // The gate path W qL contracts over rows, so a tile's 8 rows are one more product into the same accumulators (on the vector units it was 2 of
 // 12 issue slots per (row, key, pair)).  W is split into three bf16 parts, 24 bits whatever its scale, and an fp16 query into two.
-// What bounds it: the vector units, 9 or 10 issue slots per (row, key, pair).  Measured with the gate path moved: B2 Hq32 Hkv8 N4096 D128
-// forward + backward 15.0 -> 14.6 ms, B2 Hq8 Hkv2 N512 D64 133 -> 130.5 us.
+// The slow pairs (common.hpp; D = 128: half of all with theta = 10000) are not rotated per (row, key): with delta = mid_i + x, |x| <= kDkReach over
+// the block's 128 keys, and complex numbers for the pairs,
+//   dk_j = sum_i e^(i delta w) sum_h dS^h_ij q^h_i = sum_n sum_{i, h} (x_ij^n dS^h_ij) [ (i w)^n / n! e^(i mid_i w) q^h_i ] :
+// products that contract over rows and heads, one per power.  The bracket is shared by the block's keys: the four waves prepare it once per tile,
+// a wave per head.  Class 0 (|x w| <= 0.68) takes the powers 0 .. 5, class 1 (<= 0.08) 0 .. 2, the last coefficients lowered to spread the
+// remainder: below 1e-5 and 2.2e-5.  Operands are bf16 parts: two of dS and two of the bracket (16 bits) up to the power whose share is so small that
+// one keeps the sum as accurate.  Built for up to five heads a group, whose LDS leaves two workgroups to a compute unit.
+// What bounds it: the vector units, 9 or 10 issue slots per (row, key, pair) that is rotated.  Measured with the gate path moved: B2 Hq32 Hkv8 N4096 D128
+// forward + backward 15.0 -> 14.6 ms, B2 Hq8 Hkv2 N512 D64 133 -> 130.5 us; with the slow pairs as products the former 13.43 -> 12.70 ms, error of
+// dk against 64 bits 1.68e-3 (bf16) and 3.18e-4 (fp16) as before.
 // A workgroup takes its share of the group's (block, row tile) list as above.  Tiles of DELTA, W, DS^h ([row][matrix][key], fp32) and the rows' queries
 // ([row][column][head], bf16, heads padded to 8 with zeros: the B operand is then one 16-byte read) go through LDS,
 // fetched into registers one tile ahead.
 constexpr int kDkRows = 8, kDkWaves = 4;
+constexpr float kDkReach = kDkKeys / 2, kDkLow0 = kCoropeLow0 * kDkReach / kCoropeReach, kDkLow1 = kCoropeLow1 * kDkReach / kCoropeReach;
 
-template <int D, int G>
+template <int D, int G, int LOW>
 struct CoropeDkCfg {
   static constexpr int kMats = 2 + G;                                       // DELTA, W, DS^h
   static constexpr int kMatBytes = kDkRows * kMats * kDkKeys * 4;
   static constexpr int kQBytes = kDkRows * D * 8 * 2;                       // [row][column][8 heads] bf16
-  static constexpr int kLdsBytes = kMatBytes + kQBytes;
+  // slow pairs: [part][head][column][row] bf16, the parts of class 0, then of class 1; the rows' reference values of delta behind them
+  static constexpr int kParts0 = kEltIsF16 ? 9 : 8, kParts1 = kEltIsF16 ? 5 : 4;
+  static constexpr int kSlowElems = (LOW > 0 ? kParts0 : 0) * G * 32 * kDkRows + (LOW > 1 ? kParts1 : 0) * G * 32 * kDkRows;
+  static constexpr int kLdsBytes = kMatBytes + kQBytes + kSlowElems * 2 + (LOW > 0 ? kDkRows * 4 : 0);
 };
 
-template <int D, int G, int REDUCED>
+template <int D, int G, int REDUCED, int LOW>
 __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu(2))) void corope_bwd_dk_kernel(CoropeBwdParams p, CoropeBwdWs ws,
                                                                        CoropeBwdFreqs fr, float* parts, int64_t group_floats) {
-  using Cfg = CoropeDkCfg<D, G>;
-  constexpr int HALF = D / 2, NT = kDkWaves * kWave, MATS = Cfg::kMats, NP = D / 64;
-  static_assert(D == 64 || D == 128, "pairs per lane are laid out for these head dims");
+  using Cfg = CoropeDkCfg<D, G, LOW>;
+  constexpr int HALF = D / 2, NT = kDkWaves * kWave, MATS = Cfg::kMats;
+  constexpr int FAST = HALF - 16 * LOW, NP = FAST / 32;   // pairs rotated per (row, key), in blocks of 32
+  static_assert((D == 64 || D == 128) && FAST % 32 == 0, "pairs per lane are laid out for these head dims");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   float* tile = reinterpret_cast<float*>(smem);                                   // [row][matrix][key]
   uint16_t* qT = reinterpret_cast<uint16_t*>(smem + Cfg::kMatBytes);             // [row][column][8 heads]
+  uint16_t* slow_q = qT + Cfg::kQBytes / 2;                                       // [part][head][column][row]
+  float* mids = reinterpret_cast<float*>(slow_q + Cfg::kSlowElems);
 
   const int g = blockIdx.y;
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -924,9 +939,12 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
   const int head0 = b * p.Hq + kvh * G;
   const CoropeShares<kDkRows> sh(N);
   const int shares = gridDim.x, share = blockIdx.x;
-  float w_turn[NP > 0 ? NP : 1];
+  float w_turn[NP];
 #pragma unroll
-  for (int np = 0; np < (NP > 0 ? NP : 1); ++np) w_turn[np] = fr.turns[min(32 * np + col, HALF - 1)];
+  for (int np = 0; np < NP; ++np) w_turn[np] = fr.turns[32 * np + col];
+  float slow_turn[LOW > 0 ? LOW : 1] = {};   // of the pair whose queries this lane prepares
+#pragma unroll
+  for (int u = 0; u < LOW; ++u) slow_turn[u] = fr.turns[FAST + 16 * u + lane % 16];
 
   // heads G..7 of the query tile stay zero for the whole kernel
   for (int e = threadIdx.x; e < Cfg::kQBytes / 16; e += NT) reinterpret_cast<u32x4*>(qT)[e] = u32x4{0, 0, 0, 0};
@@ -971,6 +989,11 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
     f32x16 dk1[NP], dk2[NP];
 #pragma unroll
     for (int np = 0; np < NP; ++np) dk1[np] = dk2[np] = f32x16{0};
+    // slow group u: lane = column, 16 of the first half and their 16 partners
+    f32x16 slow[LOW > 0 ? LOW : 1];
+#pragma unroll
+    for (int u = 0; u < (LOW > 0 ? LOW : 1); ++u) slow[u] = f32x16{0};
+    auto slow_column = [&](int u) __attribute__((always_inline)) { return FAST + 16 * u + col % 16 + (col < 16 ? 0 : HALF); };
 
     fetch(row_begin);
 #pragma unroll 1
@@ -996,6 +1019,76 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
       });
       __syncthreads();
       if (i0 + kDkRows < row_end) fetch(i0 + kDkRows);
+      if constexpr (LOW > 0) {
+        // the slow pairs' B operands: lane = (pair, two rows), a wave = one head
+#pragma unroll 1
+        for (int h = wave; h < G; h += kDkWaves) {
+          const int pair = lane % 16, r0 = lane / 16 * 2;
+          float mid[2];
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const float* trow = tile + (r0 + x) * MATS * kDkKeys;   // (keys beyond the diagonal hold zero, what delta comes to there)
+            const float m = 0.5f * (trow[0] + trow[kDkKeys - 1]);
+            mid[x] = __builtin_fabsf(m) < 1e30f ? m : 0.f;          // (NaN: or keys the row does not see would meet it)
+            if (h == 0 && pair == 0) mids[r0 + x] = mid[x];
+          }
+          static_for<LOW>([&](auto u_c) __attribute__((always_inline)) {
+            constexpr int u = decltype(u_c)::value;
+            float v1[2], v2[2];
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+              const uint16_t* src = qT + ((r0 + x) * D + FAST + 16 * u + pair) * 8 + h;
+              const float q1 = elt_to_f(src[0]), q2 = elt_to_f(src[HALF * 8]);
+              const float ph = __builtin_amdgcn_fractf(mid[x] * slow_turn[u]);
+              const float sn = __builtin_amdgcn_sinf(ph), cs = __builtin_amdgcn_cosf(ph);
+              v1[x] = __builtin_fmaf(cs, q1, -(sn * q2));
+              v2[x] = __builtin_fmaf(cs, q2, sn * q1);
+            }
+            uint32_t* dst = reinterpret_cast<uint32_t*>(slow_q + (((u * Cfg::kParts0) * G + h) * 32 + pair) * kDkRows + r0);
+            auto put = [&](bool rest) __attribute__((always_inline)) {   // (the next part, and what its rounding leaves over as another)
+              const uint32_t p1 = pack_bf16(v1[0], v1[1]), p2 = pack_bf16(v2[0], v2[1]);
+              dst[0] = p1;
+              dst[16 * kDkRows / 2] = p2;
+              dst += G * 32 * kDkRows / 2;
+              if (!rest) return;
+              dst[0] = pack_bf16(v1[0] - bf16_lo(p1), v1[1] - bf16_hi(p1));
+              dst[16 * kDkRows / 2] = pack_bf16(v2[0] - bf16_lo(p2), v2[1] - bf16_hi(p2));
+              dst += G * 32 * kDkRows / 2;
+            };
+            const float w = slow_turn[u] * (6.2831853f * kDkReach);
+            auto times_iw = [&](float f) __attribute__((always_inline)) {
+#pragma unroll
+              for (int x = 0; x < 2; ++x) {
+                const float a = v1[x];
+                v1[x] = -(v2[x] * (w * f));
+                v2[x] = a * (w * f);
+              }
+            };
+            put(true);
+            if constexpr (u == 0) {   // cos z ~ 1 - a2 z^2 + a4 z^4, sin z ~ z - z^3 / 6 + a5 z^5
+              constexpr float Z2 = kDkLow0 * kDkLow0, a4 = 1.f / 24.f - 1.5f * Z2 / 720.f, a2 = 0.5f - 0.5625f * Z2 * Z2 / 720.f;
+              constexpr float a5 = 1.f / 120.f - 0.8f * Z2 / 5040.f;
+              times_iw(1.f);
+              put(true);
+              times_iw(a2);
+              put(kEltIsF16);
+              times_iw(1.f / (6.f * a2));
+              put(false);
+              times_iw(6.f * a4);
+              put(false);
+              times_iw(a5 / a4);
+              put(false);
+            } else {                  // cos z ~ 1 - z^2 / 2, sin z ~ a1 z
+              constexpr float a1 = 1.f - kDkLow1 * kDkLow1 / 8.f;
+              times_iw(a1);
+              put(kEltIsF16);
+              times_iw(0.5f / a1);
+              put(false);
+            }
+          });
+        }
+        __syncthreads();
+      }
       if (i0 < jw) continue;   // wave-uniform: all keys of this wave lie above the diagonal of the tile's rows
       // gate path: dk += W^T qL over the tile's 8 rows.  W enters as three bf16 parts (24 bits, any range), an fp16 query as two.
       {
@@ -1017,8 +1110,8 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
           a2[x] = hf == 0 ? l2 : 0u;
         }
 #pragma unroll
-        for (int cb = 0; cb < 2 * NP; ++cb) {
-          const uint16_t* ql = qT + (32 * cb + col) * 8;
+        for (int cb = 0; cb < 2 * NP + LOW; ++cb) {
+          const uint16_t* ql = qT + (cb < NP ? 32 * cb + col : cb < 2 * NP ? HALF + 32 * (cb - NP) + col : slow_column(cb - 2 * NP)) * 8;
           u32x4 b1, b2;
 #pragma unroll
           for (int x = 0; x < 4; ++x) {
@@ -1026,13 +1119,66 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
             b1[x] = kEltIsF16 ? pack_bf16(elt_lo(q2), elt_hi(q2)) : q2;
             if constexpr (kEltIsF16) b2[x] = pack_bf16(elt_lo(q2) - bf16_lo(b1[x]), elt_hi(q2) - bf16_hi(b1[x]));
           }
-          f32x16& acc = cb < NP ? dk1[cb % NP] : dk2[cb % NP];
+          f32x16& acc = cb < NP ? dk1[cb % NP] : cb < 2 * NP ? dk2[cb % NP] : slow[cb - 2 * NP];
           if constexpr (kEltIsF16) {
             acc = mfma32_bf16(a2, b2, acc);
             acc = mfma32_bf16(a1, b2, acc);
           }
           acc = mfma32_bf16(a2, b1, acc);
           acc = mfma32_bf16(a1, b1, acc);
+        }
+      }
+      if constexpr (LOW > 0) {
+        // the slow pairs: A = dS y^n, lane = (key, two heads), registers = the tile's rows
+        float y[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) y[x] = (tile[x * MATS * kDkKeys + 32 * wave + col] - mids[x]) * (1.f / kDkReach);
+#pragma unroll
+        for (int h0 = 0; h0 < G; h0 += 2) {
+          const int h = min(h0 + hf, G - 1);
+          float a[8];
+#pragma unroll
+          for (int x = 0; x < 8; ++x) a[x] = h0 + hf < G ? tile[(x * MATS + 2 + h) * kDkKeys + 32 * wave + col] : 0.f;
+          const uint16_t* bp = slow_q + (h * 32 + col) * kDkRows;
+          auto part = [&](int n) __attribute__((always_inline)) { return *reinterpret_cast<const u32x4*>(bp + n * G * 32 * kDkRows); };
+          u32x4 hi, lo;
+          auto split = [&]() __attribute__((always_inline)) {
+            hi = u32x4{pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3]), pack_bf16(a[4], a[5]), pack_bf16(a[6], a[7])};
+#pragma unroll
+            for (int x = 0; x < 4; ++x) lo[x] = pack_bf16(a[2 * x] - bf16_lo(hi[x]), a[2 * x + 1] - bf16_hi(hi[x]));
+          };
+          auto times_y = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int x = 0; x < 8; ++x) a[x] *= y[x];
+          };
+          auto full = [&](int u, int n) __attribute__((always_inline)) {   // with parts n and n + 1 of the group
+            const u32x4 b = part(n), rest = part(n + 1);
+            slow[u] = mfma32_bf16(hi, rest, slow[u]);
+            slow[u] = mfma32_bf16(lo, b, slow[u]);
+            slow[u] = mfma32_bf16(hi, b, slow[u]);
+          };
+          constexpr int F = kEltIsF16 ? 1 : 0, C1 = Cfg::kParts0;
+          split();
+          full(0, 0);
+          if constexpr (LOW > 1) full(1, C1);
+          times_y();
+          split();
+          full(0, 2);
+          if constexpr (LOW > 1) {
+            if constexpr (kEltIsF16) full(1, C1 + 2);
+            else slow[1] = mfma32_bf16(hi, part(C1 + 2), slow[1]);
+          }
+          times_y();
+          split();
+          if constexpr (kEltIsF16) full(0, 4);
+          else slow[0] = mfma32_bf16(hi, part(4), slow[0]);
+          if constexpr (LOW > 1) slow[1] = mfma32_bf16(hi, part(C1 + 3 + F), slow[1]);
+#pragma unroll
+          for (int n = 3; n < 6; ++n) {
+            times_y();
+            split();
+            slow[0] = mfma32_bf16(hi, part(n + 2 + F), slow[0]);
+          }
         }
       }
       const int n_rows = min(kDkRows, N - i0);
@@ -1068,7 +1214,7 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
         static_for<NP>([&](auto np_c) __attribute__((always_inline)) {
           constexpr int np = decltype(np_c)::value;
           const u32x4 bq1 = *reinterpret_cast<const u32x4*>(qT + (r * D + 32 * np + col) * 8);
-          const u32x4 bq2 = *reinterpret_cast<const u32x4*>(qT + (r * D + 32 * (NP + np) + col) * 8);
+          const u32x4 bq2 = *reinterpret_cast<const u32x4*>(qT + (r * D + HALF + 32 * np + col) * 8);
           const f32x16 u1 = mfma32(aop, bq1, f32x16{0}), u2 = mfma32(aop, bq2, f32x16{0});
 #pragma unroll
           for (int e = 0; e < 16; ++e) {
@@ -1099,6 +1245,13 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
             pp[32 * np + col] = dk1[np][e];
             pp[32 * np + col + HALF] = dk2[np][e];
           }
+        }
+#pragma unroll
+        for (int u = 0; u < LOW; ++u) {
+          if (whole)
+            op[slow_column(u)] = f_to_elt(slow[u][e] * p.sm_scale);
+          else
+            pp[slow_column(u)] = slow[u][e];
         }
       }
     }
@@ -1138,11 +1291,21 @@ static void launch_corope_bwd_scores(const CoropeBwdParams& p, const CoropeBwdWs
     hipLaunchKernelGGL((corope_bwd_scores_kernel<D, G, 1, REDUCED>), blocks(1), dim3(kWave), 0, stream, p, ws, fr);
 }
 
+template <int D, int G, int REDUCED, int LOW>
+static hipError_t launch_corope_bwd_dk(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, float* parts, int shares,
+                                       hipStream_t stream) {
+  constexpr int kLdsBytes = CoropeDkCfg<D, G, LOW>::kLdsBytes;
+  auto kern = corope_bwd_dk_kernel<D, G, REDUCED, LOW>;
+  static std::atomic<uint64_t> lds_ok{0};
+  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), kLdsBytes, lds_ok); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(shares, p.B * p.Hkv), dim3(kDkWaves * kWave), kLdsBytes, stream, p, ws, fr, parts, G * ws.NN);
+  return hipSuccess;
+}
+
 template <int D, int G, int REDUCED>
 static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBwdWs& ws, const CoropeBwdFreqs& fr, int n_groups_total,
                                         hipStream_t stream) {
   launch_corope_bwd_scores<D, G, REDUCED>(p, ws, fr, n_groups_total, stream);
-  using Cfg = CoropeDkCfg<D, G>;
   const int64_t group_floats = G * ws.NN, slots = ws.part_floats(G, p.N) / (kDkKeys * D);
   const int dv_shares = corope_bwd_shares<kDvRows>(p.N, n_groups_total, slots), dk_shares = corope_bwd_shares<kDkRows>(p.N, n_groups_total, slots);
   float* parts = ws.parts(0, G);
@@ -1153,10 +1316,10 @@ static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBw
   if (dv_shares > 1)
     hipLaunchKernelGGL((corope_bwd_sum_kernel<D, kDvRows>), dim3(n_blocks, n_groups, 8), dim3(256), 0, stream, parts, group_floats, p.dv,
                        p.N, dv_shares, 1.f);
-  auto kern = corope_bwd_dk_kernel<D, G, REDUCED>;
-  static std::atomic<uint64_t> lds_ok{0};
-  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3(dk_shares, n_groups), dim3(kDkWaves * kWave), Cfg::kLdsBytes, stream, p, ws, fr, parts, group_floats);
+  constexpr int kLow = D == 128 && CoropeDkCfg<D, G, 2>::kLdsBytes <= 80 * 1024 ? 2 : 0;   // (two workgroups a compute unit: up to five heads)
+  const hipError_t e = corope_low_groups(fr.turns, D) >= 2 ? launch_corope_bwd_dk<D, G, std::min(REDUCED, D / 64 - kLow / 2), kLow>(p, ws, fr, parts, dk_shares, stream)
+                                                           : launch_corope_bwd_dk<D, G, REDUCED, 0>(p, ws, fr, parts, dk_shares, stream);
+  if (e != hipSuccess) return e;
   if (dk_shares > 1)
     hipLaunchKernelGGL((corope_bwd_sum_kernel<D, kDkRows>), dim3(n_blocks, n_groups, 8), dim3(256), 0, stream, parts, group_floats, p.dk,
                        p.N, dk_shares, p.sm_scale);

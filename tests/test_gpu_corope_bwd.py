@@ -435,3 +435,38 @@ def test_corope_dq_of_rows_beside_those_a_key_spoils(pkg, groups, G, N, D, key, 
         kept[:key] = False
         assert 5 < kept.sum() < N - key - 5
         assert torch.isfinite(dq[:, kept]).all()
+
+
+# The slow pairs' products of the dk kernel (D = 128): every group size they are built for and one beyond, key blocks of 128 cut short, one row past a
+# tile; theta = 3000 turns too fast for them.  "open": leaders that see every gate open, so that delta moves by 128 over a block and the
+# polynomials are used out to their ends; "shut": by next to nothing.
+@pytest.mark.parametrize("gates", ["random", "open", "shut"])
+@pytest.mark.parametrize("Hq,Hkv,N,theta,dtype", [(1, 1, 257, 1e4, torch.float16), (4, 2, 129, 1e4, torch.bfloat16), (3, 1, 300, 5e5, torch.float16),
+                                                  (8, 2, 265, 1e4, torch.float16), (5, 1, 200, 1e4, torch.bfloat16), (5, 1, 136, 1e4, torch.float16),
+                                                  (6, 1, 150, 1e4, torch.float16), (4, 1, 140, 3000.0, torch.float16)])
+def test_corope_backward_slow_pairs(pkg, Hq, Hkv, N, theta, dtype, gates):
+    """Relative 2-norm of the gradients' error: rounding the result alone costs up to 2^-12 (fp16) or 2^-9 (bf16), the scores' fp16 rounded keys about as
+    much as the former; the bar is twice their sum.  A leader's score of +-12 nats moves by 12 times that rounding, and its weights with it."""
+    print(f"case Hq={Hq} Hkv={Hkv} N={N} theta={theta} {dtype} {gates}", flush=True)
+    G, D = Hq // Hkv, 128
+    scale = 1 / math.sqrt(D)
+    q, k, v, d_o = (torch.randn(1, h, N, D, generator=torch.Generator().manual_seed(19 + i)).to(dtype) for i, h in enumerate((Hq, Hkv, Hkv, Hq)))
+    if gates != "random":   # logits of +-12 from the slowest pair: sigmoid within 1e-4 of 1 or 0
+        k[..., D // 2 - 1] = 4.0
+        q[:, ::G, :, D // 2 - 1] = (1 if gates == "open" else -1) * 3.0 * math.sqrt(D)
+    dev = torch.device("cuda:0")
+    qg, kg, vg = (t.to(dev).requires_grad_(True) for t in (q, k, v))
+    o = pkg.corope_attention(qg, kg, vg, True, scale, theta)
+    got = torch.autograd.grad(o, (qg, kg, vg), d_o.to(dev), retain_graph=True)
+    bad = d_o.clone()
+    bad[0, 0, N - 60] = float("nan")
+    dk_bad = torch.autograd.grad(o, kg, bad.to(dev))[0]
+    torch.cuda.synchronize()
+    qd, kd, vd = (t.double().requires_grad_(True) for t in (q, k, v))
+    ref = torch.autograd.grad(C.corope_gqa_forward(qd, kd, vd, True, scale, theta, torch.float64), (qd, kd, vd), d_o.double())
+    bar = 2 * (2.0 ** -12 + (2.0 ** -12 if dtype == torch.float16 else 2.0 ** -9)) + (0 if gates == "random" else 12 * 2.0 ** -12)
+    for name, a, b in zip(("dQ", "dK", "dV"), got, ref):
+        err = ((a.double().cpu() - b).norm() / b.norm()).item()
+        print(f"  {name} relative error {err:.3e}")
+        assert err <= bar, name
+    assert torch.isnan(dk_bad[0, 0, : N - 59]).any() and torch.equal(dk_bad[0, 0, N - 59:], got[1][0, 0, N - 59:])

@@ -28,7 +28,7 @@
 //                  left to right: dP again, dS, G and its running sum, W;
 //                  writes dq of the heads 1..G-1, the leader's dq without its gate path (fp32, workspace), the workspace
 //                  matrices DELTA, W [group] and S, DS [head] (packed lower triangles) and the row statistics that make P of S
-//   dv           dq_leader = c (partial + W K), 128 rows per workgroup, and beside it dv^T += dO^T P, P from S and the row statistics, 128
+//   dv           dq_leader = c (partial + W K), 32 rows per workgroup, and beside it dv^T += dO^T P, P from S and the row statistics, 128
 //                keys per workgroup: plain products on the matrix cores
 //   dk           one workgroup per (group, 128 keys): sum_h dS^h q^h on the matrix cores, then lane = rotation pair x 16
 //                keys rotates it per (i, j) and adds the gate path W qL; tiles of DELTA, W, DS staged through LDS
@@ -620,83 +620,105 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
 // dq_leader_i = c (partial_i + sum_{t <= i} W_it k_t): a plain (rows x keys) x (keys x D) product on the matrix cores,
 // computed transposed (dq^T += K^T W^T) so that W is read along its packed rows: lane = query row, 8 consecutive keys per
 // step, each value split into two bf16 parts (the keys are exact, so the product carries W to about 16 bits).  One
-// workgroup of 4 waves owns 128 rows (32 per wave) of one group; the 16 key rows of a step are staged in LDS and read
-// transposed.  Its workgroups come first in the dv launch.
-constexpr int kLeaderRows = 128;
+// workgroup of 4 waves owns 32 rows of one group; every wave takes each fourth step of 16 keys, staged in LDS of its own and read
+// transposed, and the four sums are added at the end.  Its workgroups come first in the dv launch.
+// What bounds it: the chain of steps of the last rows (short sequences), the reads of W (long ones).  128 rows per workgroup, 32 a wave, every wave all
+// steps behind two barriers each -> this: the dv launch B2 Hq8 Hkv2 N512 D64 25.3 -> 11.0 us, B2 Hq32 Hkv8 N4096 D128 990 -> 921 us; forward +
+// backward B1 Hq8 Hkv2 N1024 D64 190 -> 157 us, B2 Hq16 Hkv16 N700 D64 fp16 435 -> 386 us.
+constexpr int kLeaderRows = 32;
 
 template <int D>
-__device__ __forceinline__ void corope_bwd_dq_leader(const CoropeBwdParams& p, const CoropeBwdWs& ws, uint16_t* tile, int g, int rb) {
-  constexpr int TS = D + 16, NDB = D / 32, NT = 4 * kWave, STEP = 16;
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+struct CoropeLeaderCfg {
+  static constexpr int TS = D + 16, STEP = 16, kSumStride = 36;   // key rows; a wave's sums, [row][32 columns], fp32
+  static constexpr int kElems = std::max(4 * STEP * TS, 4 * kLeaderRows * kSumStride * 2);
+};
+
+template <int D>
+__device__ __forceinline__ void corope_bwd_dq_leader(const CoropeBwdParams& p, const CoropeBwdWs& ws, uint16_t* lds, int g, int rb) {
+  using Cfg = CoropeLeaderCfg<D>;
+  constexpr int TS = Cfg::TS, NDB = D / 32, STEP = Cfg::STEP, PER = STEP * (D / 8) / kWave, SS = Cfg::kSumStride;
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int r = lane % 32, hf = lane / 32;
   const int N = p.N, b = g / p.Hkv, kvh = g % p.Hkv, G = p.Hq / p.Hkv;
-  const int iw = rb * kLeaderRows + 32 * wave, i = iw + r;              // this wave's first row, this lane's row
+  const int i0 = rb * kLeaderRows, i = i0 + r;                           // the workgroup's first row, this lane's row
   const uint16_t* kbase = p.k + (int64_t)g * N * D;
   const float* wrow = ws.w(g) + tri_row_start(min(i, N - 1));
+  uint16_t* const tile = lds + wave * STEP * TS;
   f32x16 acc[NDB];
 #pragma unroll
   for (int db = 0; db < NDB; ++db) acc[db] = f32x16{0};
-  const int t_end = min(N, (rb + 1) * kLeaderRows);                      // keys up to the block's last row
-  // the key rows and this lane's W values of a step are fetched into registers one step ahead (the workgroup of the last
-  // row block walks N / 16 steps one after the other)
-  constexpr int UNITS = STEP * (D / 8), PER = (UNITS + NT - 1) / NT;
-  u32x4 kreg[PER];
-  f32x4 w0 = f32x4{0.f, 0.f, 0.f, 0.f}, w1 = w0;
-  auto fetch = [&](int t0) __attribute__((always_inline)) {
+  const int steps = (min(N, i0 + kLeaderRows) + STEP - 1) / STEP;        // up to the last row's diagonal
+  // the key rows and this lane's W values are fetched into registers two of the wave's steps ahead
+  u32x4 kreg[2][PER];
+  f32x4 w0[2], w1[2];
+  auto fetch = [&](int step, auto set_c) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value;
+    const int t0 = min(step, steps - 1) * STEP;
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const int e = min((int)threadIdx.x + u * NT, UNITS - 1);
-      kreg[u] = *reinterpret_cast<const u32x4*>(kbase + (int64_t)min(t0 + e / (D / 8), N - 1) * D + 8 * (e % (D / 8)));
+      const int e = lane + u * kWave;
+      kreg[set][u] = *reinterpret_cast<const u32x4*>(kbase + (int64_t)min(t0 + e / (D / 8), N - 1) * D + 8 * (e % (D / 8)));
     }
     const int t = t0 + 8 * hf;     // first of this lane's 8 keys; t <= i keeps the 32-byte read inside the padded row
-    w0 = w1 = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (t0 <= iw + 31 && iw < N && i < N && t <= i) {
-      w0 = *reinterpret_cast<const f32x4*>(wrow + t);
-      w1 = *reinterpret_cast<const f32x4*>(wrow + t + 4);
+    w0[set] = w1[set] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (i < N && t <= i) {
+      w0[set] = *reinterpret_cast<const f32x4*>(wrow + t);
+      w1[set] = *reinterpret_cast<const f32x4*>(wrow + t + 4);
     }
   };
-  if (t_end > 0) fetch(0);
-#pragma unroll 1
-  for (int t0 = 0; t0 < t_end; t0 += STEP) {
-    __syncthreads();   // the previous step's reads of the tile are done
+  auto multiply = [&](int step, auto set_c) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value;
+    lds_order();   // the previous step's reads of the tile are done
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const int e = threadIdx.x + u * NT;
-      if (UNITS % NT == 0 || e < UNITS) *reinterpret_cast<u32x4*>(tile + (e / (D / 8)) * TS + 8 * (e % (D / 8))) = kreg[u];
+      const int e = lane + u * kWave;
+      *reinterpret_cast<u32x4*>(tile + (e / (D / 8)) * TS + 8 * (e % (D / 8))) = kreg[set][u];
     }
-    const int t = t0 + 8 * hf;
+    const int t = step * STEP + 8 * hf;
     float hi[8], lo[8];
 #pragma unroll
     for (int x = 0; x < 8; ++x) {
-      const float wv = (i < N && t + x <= i) ? (x < 4 ? w0[x] : w1[x - 4]) : 0.f;   // nothing beyond the diagonal is defined
+      const float wv = (i < N && t + x <= i) ? (x < 4 ? w0[set][x] : w1[set][x - 4]) : 0.f;   // nothing beyond the diagonal is defined
       hi[x] = elt_to_f(f_to_elt(wv));
       lo[x] = wv - hi[x];
     }
     const u32x4 bhi = {pack_elts(hi[0], hi[1]), pack_elts(hi[2], hi[3]), pack_elts(hi[4], hi[5]), pack_elts(hi[6], hi[7])};
     const u32x4 blo = {pack_elts(lo[0], lo[1]), pack_elts(lo[2], lo[3]), pack_elts(lo[4], lo[5]), pack_elts(lo[6], lo[7])};
-    if (t0 + STEP < t_end) fetch(t0 + STEP);
-    __syncthreads();
-    if (t0 <= iw + 31 && iw < N) {   // wave-uniform: some row of this wave sees a key of the step
+    fetch(step + 8, set_c);
+    lds_order();
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) {
-        const u32x4 a = load_a_trans_natural(tile, TS, 0, 32 * db);
-        acc[db] = mfma32(a, bhi, acc[db]);
-        acc[db] = mfma32(a, blo, acc[db]);
-      }
+    for (int db = 0; db < NDB; ++db) {
+      const u32x4 a = load_a_trans_natural(tile, TS, 0, 32 * db);
+      acc[db] = mfma32(a, bhi, acc[db]);
+      acc[db] = mfma32(a, blo, acc[db]);
     }
+  };
+  fetch(wave, std::integral_constant<int, 0>{});
+  fetch(wave + 4, std::integral_constant<int, 1>{});
+#pragma unroll 1
+  for (int step = wave; step < steps; step += 8) {
+    multiply(step, std::integral_constant<int, 0>{});
+    if (step + 4 >= steps) break;
+    multiply(step + 4, std::integral_constant<int, 1>{});
   }
-  if (i < N) {
-    const float* part = ws.dql(g, N, D) + (int64_t)i * D;
-    uint16_t* op = p.dq + ((int64_t)(b * p.Hq + kvh * G) * N + i) * D;
+  // the four waves' sums, 32 columns at a time: thread = (row, 4 columns)
+  float* const sums = reinterpret_cast<float*>(lds);
+  const int row = threadIdx.x / 8, d4 = threadIdx.x % 8 * 4;
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
+  for (int db = 0; db < NDB; ++db) {
+    __syncthreads();
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const f32x4 pv = *reinterpret_cast<const f32x4*>(part + db * 32 + 8 * g4 + 4 * hf);
-        const u32x2 w = {pack_elts((acc[db][4 * g4] + pv[0]) * p.sm_scale, (acc[db][4 * g4 + 1] + pv[1]) * p.sm_scale),
-                         pack_elts((acc[db][4 * g4 + 2] + pv[2]) * p.sm_scale, (acc[db][4 * g4 + 3] + pv[3]) * p.sm_scale)};
-        *reinterpret_cast<u32x2*>(op + db * 32 + 8 * g4 + 4 * hf) = w;
-      }
+    for (int g4 = 0; g4 < 4; ++g4)
+      *reinterpret_cast<f32x4*>(sums + (wave * kLeaderRows + r) * SS + 8 * g4 + 4 * hf) =
+          f32x4{acc[db][4 * g4], acc[db][4 * g4 + 1], acc[db][4 * g4 + 2], acc[db][4 * g4 + 3]};
+    __syncthreads();
+    if (i0 + row < N) {
+      f32x4 sum = *reinterpret_cast<const f32x4*>(ws.dql(g, N, D) + (int64_t)(i0 + row) * D + db * 32 + d4);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) sum += *reinterpret_cast<const f32x4*>(sums + (w * kLeaderRows + row) * SS + d4);
+      *reinterpret_cast<u32x2*>(p.dq + ((int64_t)(b * p.Hq + kvh * G) * N + i0 + row) * D + db * 32 + d4) =
+          u32x2{pack_elts(sum[0] * p.sm_scale, sum[1] * p.sm_scale), pack_elts(sum[2] * p.sm_scale, sum[3] * p.sm_scale)};
+    }
   }
 }
 
@@ -768,7 +790,7 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
                                                                      int shares) {
   constexpr int TS = D + 16, NDB = D / 32, NT = 4 * kWave, ROWS = kDvRows;
   constexpr int UNITS = G * ROWS * (D / 8), PER = (UNITS + NT - 1) / NT;   // 16-byte pieces of a dO tile, per thread
-  __shared__ __attribute__((aligned(16))) uint16_t tile[G * ROWS * TS];
+  __shared__ __attribute__((aligned(16))) uint16_t tile[std::max(G * ROWS * TS, CoropeLeaderCfg<D>::kElems)];
   __shared__ __attribute__((aligned(16))) float stat[2][2 * G * ROWS];   // two steps' [reference values, 1 / sums][head][row]
   static_assert(2 * G * ROWS <= NT, "one statistic per thread");
   const int n_groups = p.B * p.Hkv, leader_blocks = (p.N + kLeaderRows - 1) / kLeaderRows * n_groups;

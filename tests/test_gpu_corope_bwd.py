@@ -470,3 +470,14 @@ def test_corope_backward_slow_pairs(pkg, Hq, Hkv, N, theta, dtype, gates):
         print(f"  {name} relative error {err:.3e}")
         assert err <= bar, name
     assert torch.isnan(dk_bad[0, 0, : N - 59]).any() and torch.equal(dk_bad[0, 0, N - 59:], got[1][0, 0, N - 59:])
+
+
+@pytest.mark.parametrize("N", [15, 16, 17, 31, 32, 33, 63, 64, 65, 112, 113, 129, 177])
+@pytest.mark.parametrize("D", [64, 128])
+def test_corope_backward_leader_lengths(pkg, N, D):
+    """The leader's dq, whose gate path four waves sum in turn, 16 keys a step: lengths at which some of them have no step, or one fewer.  One head a
+    group, so that all of dQ is the leader's; small dO and sm_scale = 1 as where the gate path is material, with that test's bar."""
+    print(f"case N={N} D={D}", flush=True)
+    q, k, v, d_o = _inputs(1, 2, 2, N, D, seed=7)
+    q, k, d_o = bf16_round(q * 0.3), bf16_round(k * 0.3), d_o * 0.5
+    _compare(_gpu_grads(pkg, q, k, v, d_o, 1.0, 100.0), _oracle_grads(q, k, v, d_o, 1.0, 100.0), 1)

@@ -555,7 +555,7 @@ int corope_rope_attn_bwd_ws(const void* q, const void* k, const void* v, const v
 
 int64_t corope_rope_attn_bwd_rotated_parts_bytes(int B, int H, int Hkv, int N, int D, int causal) {
   if (Hkv <= 0 || H % Hkv != 0 || corope_rope_attn_check(B, H, N, D, D, 1.f, 1)) return -1;
-  return corope::bwd_dkdv_parts_bytes(B, H, Hkv, N, D, causal != 0);
+  return std::max(corope::bwd_dkdv_parts_bytes(B, H, Hkv, N, D, causal != 0), corope::bwd_dq_parts_bytes(B, H, N, D, causal != 0));
 }
 
 int corope_rope_attn_bwd_rotated(const void* q_rot, const void* k_rot, const void* v, const int64_t* v_strides, const void* o,
@@ -585,6 +585,7 @@ int corope_rope_attn_bwd_rotated(const void* q_rot, const void* k_rot, const voi
     if (parts_bytes < need)
       return fail(COROPE_E_BADARG, "%s: parts of %lld bytes, %lld needed", what, (long long)parts_bytes, (long long)need);
     p.parts = static_cast<float*>(parts);
+    if (parts_bytes >= corope::bwd_dq_parts_bytes(B, H, N, D, causal != 0)) p.dq_parts = p.parts;   // (used up before the dK+dV launch begins)
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   // the dQ kernel computes delta for the rows it owns, the dK+dV kernel reads it

@@ -164,6 +164,7 @@ struct BwdParams {
   int64_t v_sb, v_sh, do_sb, do_sh;
   int v_sn, do_sn;
   float* parts;    // partial sums of the dK+dV kernel's cut key blocks (bwd_dkdv_parts_bytes), or null: no block is cut
+  float* dq_parts; // the same for the dQ kernel's cut query blocks (bwd_dq_parts_bytes); may be the same memory, the launches follow one another
   void contiguous(int D) {
     v_sn = do_sn = D;
     v_sh = do_sh = (int64_t)N * D;
@@ -235,6 +236,7 @@ hipError_t launch_bwd_dkdv_fused(const BwdParams& p, int D, bool causal, hipStre
 // bytes of BwdParams::parts with which launch_bwd_dkdv_fused on rotated operands cuts key blocks; 0: it is faster without
 int64_t bwd_dkdv_parts_bytes(int B, int H, int Hkv, int N, int D, bool causal);
 hipError_t launch_bwd_dq(const BwdParams& p, int D, bool causal, hipStream_t stream);
+int64_t bwd_dq_parts_bytes(int B, int H, int N, int D, bool causal);   // of BwdParams::dq_parts, as above
 hipError_t launch_corope_gqa_fwd(const CoropeParams& p, int D, hipStream_t stream);
 int64_t corope_gqa_bwd_workspace_floats(int B, int Hq, int Hkv, int N, int D);
 hipError_t launch_corope_gqa_bwd(const CoropeBwdParams& p, int D, float* workspace, int64_t workspace_floats,

@@ -14,6 +14,7 @@
 // Operands that must be read "transposed" (contraction along the sequence axis of a row-major tile) use the
 // gfx950 transposing LDS read, so every tile is staged row-major exactly once.
 #include <algorithm>
+#include <cmath>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -499,10 +500,68 @@ struct DqCfg {
   static_assert(kLdsBytes <= 160 * 1024, "LDS of a compute unit");
 };
 
+// What a workgroup of the dQ kernel works on, as DkdvWork says for the other one: CUT = true cuts the list of the key tiles of all items, head after
+// head, into equal pieces.  Item i is query block num_blocks - 1 - i / BH of head i % BH.
+template <bool CUT>
+struct DqWork;
+
+template <>
+struct DqWork<false> {
+  ItemList items;
+  int total;
+  __device__ __forceinline__ DqWork(int num_blocks, int BH, int, int) : total(num_blocks * BH) {}
+  __device__ __forceinline__ int at(int round) const { return items.at(round); }   // >= total: no such item
+  __device__ __forceinline__ int begin(int) const { return 0; }
+  __device__ __forceinline__ int end(int, int tiles) const { return tiles; }
+  __device__ __forceinline__ int share() const { return 0; }
+};
+
+struct DqTiles {
+  int nb, heads, k_tiles, step, per_head, total_tiles;
+  // step: key tiles by which a query block sees more than the one before it (0 when every query sees every key)
+  __host__ __device__ DqTiles(int nb_, int heads_, int k_tiles_, int step_) : nb(nb_), heads(heads_), k_tiles(k_tiles_), step(step_) {
+    per_head = first(nb);
+    total_tiles = per_head * heads;
+  }
+  __host__ __device__ int first(int mb) const {   // tiles of a head before block mb
+    return step == 0 ? mb * k_tiles : mb == nb ? step * (nb * (nb - 1) / 2) + k_tiles : step * (mb * (mb + 1) / 2);
+  }
+  __device__ int start(int item) const { return (item % heads) * per_head + first(nb - 1 - item / heads); }
+  __device__ int begin_of_share(int w, int shares) const { return (int)((int64_t)w * total_tiles / shares); }
+  __device__ int share_of(int tile, int shares) const { return (int)((((int64_t)tile + 1) * shares - 1) / total_tiles); }
+};
+
+template <>
+struct DqWork<true> {
+  DqTiles t;
+  int total, t0, t1, li0, piece;
+  __device__ __forceinline__ DqWork(int num_blocks, int BH, int k_tiles, int step) : t(num_blocks, BH, k_tiles, step), total(num_blocks * BH) {
+    const int n = gridDim.x, id = blockIdx.x;   // (neighbouring pieces on one XCD)
+    piece = n % 8 == 0 ? (id % 8) * (n / 8) + id / 8 : id;
+    t0 = t.begin_of_share(piece, n);
+    t1 = t.begin_of_share(piece + 1, n);
+    const int head = t0 / t.per_head, rem = t0 % t.per_head;
+    int mb = 0;
+    while (mb + 1 < t.nb && t.first(mb + 1) <= rem) ++mb;
+    li0 = head * t.nb + mb;
+  }
+  __device__ __forceinline__ int at(int round) const {
+    const int li = li0 + round, head = li / t.nb, mb = li % t.nb;
+    return li < total && head * t.per_head + t.first(mb) < t1 ? (t.nb - 1 - mb) * t.heads + head : total;
+  }
+  __device__ __forceinline__ int begin(int item) const { return max(0, t0 - t.start(item)); }
+  __device__ __forceinline__ int end(int item, int tiles) const { return min(tiles, t1 - t.start(item)); }
+  __device__ __forceinline__ int share() const { return piece; }
+};
+
+// A slot of partial sums: NWAVES x 32 queries x D of dQ_r, as the accumulators lie ([32-row block][register quad][lane]).
+template <int D, int NWAVES>
+constexpr int64_t kDqSlotFloats = (int64_t)NWAVES * 32 * D;
+
 // Persistent, like the forward on a pre-rotated K: one workgroup per compute unit walks a balanced list of (head, query
 // block) items, the stream of K/V tiles runs on from item to item, and nothing at the change of items needs a workgroup
 // barrier (a wave's operand rows and its dQ rows go through an LDS tile of its own).
-template <int D, int NWAVES, int BLOCK_N, bool CAUSAL, bool PREROT>
+template <int D, int NWAVES, int BLOCK_N, bool CAUSAL, bool PREROT, bool CUT = false>
 __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<D>, kWavesPerSimd<D>))) void rope_attn_bwd_dq_kernel(BwdParams p) {
   using Cfg = DqCfg<D, NWAVES, BLOCK_N>;
   constexpr int NT = Cfg::kThreads;
@@ -520,9 +579,9 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   uint8_t* const wave_tile = smem + Cfg::kRingBytes + wave * Cfg::kWaveBytes;
   float* const wave_delta = reinterpret_cast<float*>(wave_tile + WaveTile<D>::kBytes);
 
-  const ItemList items;
-  const int total = p.num_blocks * p.BH;   // item i (heaviest first): query block num_blocks - 1 - i / BH of head i % BH
   const int n_k_tiles = (N + BLOCK_N - 1) / BLOCK_N;
+  const DqWork<CUT> items(p.num_blocks, p.BH, n_k_tiles, CAUSAL ? Cfg::kBlockM / BLOCK_N : 0);
+  const int total = items.total;   // item i (heaviest first): query block num_blocks - 1 - i / BH of head i % BH
   auto tiles_of = [&](int mb) {
     return CAUSAL ? min((mb * Cfg::kBlockM + Cfg::kBlockM + BLOCK_N - 1) / BLOCK_N, n_k_tiles) : n_k_tiles;
   };
@@ -538,7 +597,8 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     const int64_t kv_base = (int64_t)kv_slab(i % p.BH, p.H, p.Hkv) * N * D;
     l_kg = (PREROT ? p.k_rot : p.k) + kv_base;
     l_vg = v_slab_of<D, STRIDED>(p, kv_slab(i % p.BH, p.H, p.Hkv));
-    l_tiles = tiles_of(p.num_blocks - 1 - i / p.BH);
+    l_tile = items.begin(i);
+    l_tiles = items.end(i, tiles_of(p.num_blocks - 1 - i / p.BH));
     return true;
   };
   auto load_next_tile = [&]() __attribute__((always_inline)) {   // moves the cursor on and requests that tile
@@ -546,7 +606,6 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       ++l_tile;
     } else if (load_item(l_round + 1)) {
       ++l_round;
-      l_tile = 0;
     }   // else: past the last tile of the last item; the same tile is requested again and never used
     kst.load(l_kg, p.cos, p.sin, p.fstride, l_tile * BLOCK_N, N);
     vst.load(l_vg, l_tile * BLOCK_N, N, v_row_bytes<D, STRIDED>(p));
@@ -621,8 +680,8 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   int item = items.at(0);
   COROPE_ISTAMP(0);
   load_item(0);
-  kst.load(l_kg, p.cos, p.sin, p.fstride, 0, N);
-  vst.load(l_vg, 0, N, v_row_bytes<D, STRIDED>(p));
+  kst.load(l_kg, p.cos, p.sin, p.fstride, l_tile * BLOCK_N, N);
+  vst.load(l_vg, l_tile * BLOCK_N, N, v_row_bytes<D, STRIDED>(p));
   request_rows(item);
   take_rows(item);
   kst.store_rows(k_tile(0));
@@ -632,7 +691,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   for (int round = 0;; ++round) {
     const int bh = item % p.BH, mb = p.num_blocks - 1 - item / p.BH;
     const int m0 = mb * Cfg::kBlockM;
-    const int n_tiles = tiles_of(mb);
+    const int t_begin = items.begin(item), n_tiles = items.end(item, tiles_of(mb));   // of this workgroup's piece of the item
     const int q_row = m0 + rb * 32 + lq;
     const int wq_lo = m0 + rb * 32, wq_hi = wq_lo + 31;
     const int key_limit = CAUSAL ? q_row : N - 1;   // last key this lane's query attends to
@@ -666,7 +725,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       vst.store_rows(v_tile(cur ^ 1));
     };
 
-    for (int t = 0; t <= t_last; ++t) {
+    for (int t = t_begin; t <= t_last; ++t) {
       const int n0 = t * BLOCK_N;
 #ifdef COROPE_TRACE
       if (t == 1) COROPE_ISTAMP(3);
@@ -738,7 +797,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     const bool has_next = next_item < total;
     request_rows(has_next ? next_item : item);
     // of the tiles entirely above this wave's diagonal it only stages its share
-    for (int t = t_last + 1; t < n_tiles; ++t) {
+    for (int t = CUT ? max(t_begin, t_last + 1) : t_last + 1; t < n_tiles; ++t) {
       load_next_tile();
       stage_next();
       cur ^= 1;
@@ -746,13 +805,55 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     }
     // dQ_r -> dQ: scaled, un-rotated in fp32, rounded once, whole rows per store
     if constexpr (!PREROT) tb.load(p.cos, p.sin, p.fstride, wq_lo, N, opaque_lane());
-    store_unrotated_rows_via_wave_tile<D>(dqacc, tb, p.dq + (int64_t)bh * N * D, wq_lo, N, p.sm_scale, wave_tile, opaque_lane());
+    if (!CUT || (t_begin == 0 && n_tiles == tiles_of(mb))) {   // workgroup-uniform
+      store_unrotated_rows_via_wave_tile<D>(dqacc, tb, p.dq + (int64_t)bh * N * D, wq_lo, N, p.sm_scale, wave_tile, opaque_lane());
+    } else if constexpr (CUT) {   // a piece of the item: its partial sums
+      float* slot = p.dq_parts + dkdv_slot(items.share(), t_begin == 0) * kDqSlotFloats<D, NWAVES> + (int64_t)rb * 32 * D + 4 * opaque_lane();
+#pragma unroll
+      for (int i = 0; i < NDB * 4; ++i)
+        *reinterpret_cast<f32x4*>(slot + i * 4 * kWave) =
+            f32x4{dqacc[i / 4][4 * (i % 4)], dqacc[i / 4][4 * (i % 4) + 1], dqacc[i / 4][4 * (i % 4) + 2], dqacc[i / 4][4 * (i % 4) + 3]};
+    }
     COROPE_ISTAMP(6);
     if (!has_next) break;
     item = next_item;
     COROPE_ISTAMP(0);
     take_rows(item);
   }
+}
+
+// dQ of the items that were cut: a workgroup per 32 rows of an item, a wave per register quad and its partner (columns d and d + D / 2): adds the
+// pieces' accumulators, un-rotates, rounds.
+template <int D, int NWAVES, int BLOCK_N, bool CAUSAL>
+__global__ __launch_bounds__(D / 16 * kWave) void rope_attn_bwd_dq_sum_kernel(BwdParams p, int shares) {
+  constexpr int BLOCK_M = NWAVES * 32, PARTNER = D / 16 * 4 * kWave;
+  const int N = p.N;
+  const DqTiles t(p.num_blocks, p.BH, (N + BLOCK_N - 1) / BLOCK_N, CAUSAL ? BLOCK_M / BLOCK_N : 0);
+  const int item = blockIdx.x / NWAVES, rb = blockIdx.x % NWAVES, mb = p.num_blocks - 1 - item / p.BH;
+  const int start = t.start(item), w0 = t.share_of(start, shares), w1 = t.share_of(start + t.first(mb + 1) - t.first(mb) - 1, shares);
+  const int lane = threadIdx.x % kWave, i = threadIdx.x / kWave, row = mb * BLOCK_M + rb * 32 + lane % 32;
+  if (w0 == w1 || row >= N) return;   // one piece holds all of the item and has written it
+  const float* src = p.dq_parts + (int64_t)rb * 32 * D + 4 * (i * kWave + lane);
+  const int col = 8 * i + 4 * (lane / 32);
+  const f32x4 c = *reinterpret_cast<const f32x4*>(p.cos + row * p.fstride + col), s = *reinterpret_cast<const f32x4*>(p.sin + row * p.fstride + col);
+  f32x4 a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
+  for (int w = w0; w <= w1; w += 4) {   // eight loads in flight
+    f32x4 x[4], y[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float* slot = src + dkdv_slot(min(w + u, w1), min(w + u, w1) == w0) * kDqSlotFloats<D, NWAVES>;
+      x[u] = *reinterpret_cast<const f32x4*>(slot);
+      y[u] = *reinterpret_cast<const f32x4*>(slot + PARTNER);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (w + u <= w1) a += x[u], b += y[u];
+  }
+  a *= p.sm_scale, b *= p.sm_scale;
+  const f32x4 o1 = a * c + b * s, o2 = b * c - a * s;
+  uint16_t* out = p.dq + ((int64_t)(item % p.BH) * N + row) * D + col;
+  *reinterpret_cast<u32x2*>(out) = u32x2{pack_elts(o1[0], o1[1]), pack_elts(o1[2], o1[3])};
+  *reinterpret_cast<u32x2*>(out + D / 2) = u32x2{pack_elts(o2[0], o2[1]), pack_elts(o2[2], o2[3])};
 }
 
 // ===================================================================================== launchers
@@ -860,9 +961,13 @@ static hipError_t launch_dkdv_cfg(const BwdParams& p, hipStream_t stream) {
   }
 }
 
+template <int D>
+constexpr int kDqBlockN = D > 128 ? 32 : 64;   // what fits the LDS beside the waves' own tiles
+template <int D>
+constexpr int kDqCutWaves = D > 128 ? 4 : 8;
 template <int D, bool CAUSAL, bool PREROT, int NWAVES>
 static hipError_t launch_dq_waves(BwdParams p, hipStream_t stream) {
-  constexpr int BLOCK_N = D > 128 ? 32 : 64;   // what fits the LDS beside the waves' own tiles
+  constexpr int BLOCK_N = kDqBlockN<D>;
   using Cfg = DqCfg<D, NWAVES, BLOCK_N>;
   auto kern = rope_attn_bwd_dq_kernel<D, NWAVES, BLOCK_N, CAUSAL, PREROT>;
   static std::atomic<uint64_t> lds_ok{0};
@@ -876,8 +981,72 @@ static hipError_t launch_dq_waves(BwdParams p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// How many pieces the key tiles of the dQ launch on rotated operands are cut into; 0: whole items.  As dkdv_shares: with few heads the longest
+// whole item (a sequence's last queries, which see all of its keys) sets the time however many compute units are idle.  Measured
+// constants, in microseconds: a tile of a full chip, a change of items (at head dim 256, one wave per SIMD, nothing hides it), the launch; a
+// causal piece of T tiles crosses up to sqrt(2 T / step) of a head's lightest items.  dQ launch, whole / cut with its sums, B1 H N: D = 128: 8 4096 159 / 87, 4 8192
+// 296 / 132, 1 10000 330 / 66, 8 3000 not causal 119 / 80, and on the other side 16 4096 153 / 152, 40 1100 53 / 64; D = 64: 8 4096 63 / 50, 4 16384 276 / 239, 2 3000
+// not causal 46 / 27, 16 1500 27.5 / 28.2; D = 256: 2 2048 112 / 58, 4 4096 212 / 185, 8 2048 115 / 129, 16 2048 124 / 199.
+template <int D>
+static int dq_shares(int N, int BH, bool causal) {
+  constexpr int BN = kDqBlockN<D>, CW = kDqCutWaves<D>, kMost = 16;
+  if (g_tile_rows.load(std::memory_order_relaxed) != 0) return 0;   // a form was asked for
+  const int k_tiles = (N + BN - 1) / BN, cus = device_cu_count();
+  const bool small = D <= 128 && use_small_tiles(N, BH, DqCfg<D, 4, BN>::kLdsBytes);
+  const int block = small || D > 128 ? 128 : 256, nb = (N + block - 1) / block;
+  const int slots = cus * (small && fits_twice(DqCfg<D, 4, BN>::kLdsBytes) ? 2 : 1);
+  const int64_t n_items = (int64_t)nb * BH;
+  if (n_items > (int64_t)kMost * slots || n_items * k_tiles >= (1ll << 30)) return 0;   // many rounds even out
+  int64_t longest = 0;
+  const int grid = (int)std::min<int64_t>(n_items, slots);
+  for (int w = 0; w < grid; w += 8) {
+    int64_t sum = 0;
+    for (int r = 0; (int64_t)r * grid < n_items; ++r) {
+      const int64_t i = (int64_t)r * grid + ((r & 1) ? grid - 1 - w : w);
+      if (i < n_items) sum += causal ? std::min((nb - (int)(i / BH)) * (block / BN), k_tiles) : k_tiles;
+    }
+    longest = std::max(longest, sum);
+  }
+  const DqTiles t((N + CW * 32 - 1) / (CW * 32), BH, k_tiles, causal ? CW * 32 / BN : 0);
+  const int shares = std::max(1, std::min(cus, t.total_tiles / 4));
+  constexpr float kWholeTile = D == 64 ? 1.25f : D == 128 ? 2.8f : 1.75f, kTile = D == 64 ? 1.5f : D == 128 ? 2.9f : 1.6f;
+  constexpr float kChange = D == 64 ? 3.5f : D == 128 ? 5.f : 21.f;
+  const float busy = std::min(1.f, (float)t.total_tiles * (block == CW * 32 ? 1.f : 2.f) / ((float)longest * cus));
+  const float whole = (small ? 0.85f : 1.f) * longest * kWholeTile * (0.75f + 0.25f * busy) + kChange * ((n_items + grid - 1) / grid);
+  const float tiles = (float)t.total_tiles / shares, crossed = causal ? std::sqrt(2.f * tiles / (CW * 32 / BN)) : 1.f;
+  const float moved = (float)(shares + std::min<int64_t>(t.nb * (int64_t)BH, shares)) * kDqSlotFloats<D, CW> * 8;
+  const float cut = tiles * kTile + kChange * (1.f + crossed) + 9.f + moved / 12e6f;
+  return cut < 0.9f * whole ? shares : 0;
+}
+
+int64_t bwd_dq_parts_bytes(int B, int H, int N, int D, bool causal) {
+  if (D == 64) return 8 * dq_shares<64>(N, B * H, causal) * kDqSlotFloats<64, kDqCutWaves<64>>;
+  if (D == 128) return 8 * dq_shares<128>(N, B * H, causal) * kDqSlotFloats<128, kDqCutWaves<128>>;
+  return 8 * dq_shares<256>(N, B * H, causal) * kDqSlotFloats<256, kDqCutWaves<256>>;
+}
+
+template <int D, bool CAUSAL>
+static hipError_t launch_dq_cut(BwdParams p, int shares, hipStream_t stream) {
+  constexpr int NWAVES = kDqCutWaves<D>, BN = kDqBlockN<D>;
+  using Cfg = DqCfg<D, NWAVES, BN>;
+  auto kern = rope_attn_bwd_dq_kernel<D, NWAVES, BN, CAUSAL, true, true>;
+  static std::atomic<uint64_t> lds_ok{0};
+  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
+  p.num_blocks = (p.N + Cfg::kBlockM - 1) / Cfg::kBlockM;
+#ifdef COROPE_TRACE
+  p.trace = nullptr;
+#endif
+  hipLaunchKernelGGL(kern, dim3(shares), dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, p);
+  hipLaunchKernelGGL((rope_attn_bwd_dq_sum_kernel<D, NWAVES, BN, CAUSAL>), dim3((unsigned)p.num_blocks * p.BH * NWAVES), dim3(D / 16 * kWave), 0,
+                     stream, p, shares);
+  return hipGetLastError();
+}
+
 template <int D, bool CAUSAL, bool PREROT>
 static hipError_t launch_dq_cfg(const BwdParams& p, hipStream_t stream) {
+  if constexpr (PREROT)
+    if (p.dq_parts != nullptr)
+      if (const int shares = dq_shares<D>(p.N, p.BH, CAUSAL); shares > 0) return launch_dq_cut<D, CAUSAL>(p, shares, stream);
   if constexpr (D > 128) {
     return launch_dq_waves<D, CAUSAL, PREROT, 4>(p, stream);   // 4 waves x 512 registers
   } else {

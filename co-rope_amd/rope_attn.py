@@ -234,7 +234,7 @@ def _backward_rotated(lib, q_rot, k_rot, v, o, do, M, fc, fs, sm_scale, causal):
     dq, dk, dv = torch.empty_like(q_rot), torch.empty_like(k_rot), torch.empty_like(k_rot)
     delta = torch.empty_like(M)
     with _on_device(q_rot):
-        # scratch in which the dK+dV launch leaves the partial sums of key blocks it cuts among workgroups (0: none are cut); how
+        # scratch in which the dQ and the dK+dV launch leave the partial sums of blocks they cut among workgroups (0: none are cut); how
         # many pieces there are depends on the device (at most 128 MiB with 256 compute units).  Only speed needs it
         nbytes = lib.corope_rope_attn_bwd_rotated_parts_bytes(B, H, Hkv, N, D, int(causal))
         try:

@@ -286,8 +286,8 @@ int corope_rope_attn_bwd_gqa(const void *q, const void *k, int prerotated, const
 /* The whole backward on the rotated copies a two-launch forward kept (q_rot carries sm_scale * log2 e), bf16 or fp16 (fp16 != 0),
  * with or without grouped-query attention: the dQ kernel, which computes delta = rowsum(O o dO) on its way, then dK and dV in one
  * launch.  Up to D = 128 v and d_o may be strided views (batch, head and row strides in elements, as
- * corope_rope_attn_fwd_strided; NULL: contiguous); everything else is contiguous.  parts: scratch for partial sums, with which the dK+dV launch cuts its work into equal
- * pieces; corope_rope_attn_bwd_rotated_parts_bytes says how much, 0 where whole key blocks fill the chip as well (then, and if
+ * corope_rope_attn_fwd_strided; NULL: contiguous); everything else is contiguous.  parts: scratch for partial sums, with which the dQ and the dK+dV launch cut their work into equal
+ * pieces; corope_rope_attn_bwd_rotated_parts_bytes says how much, 0 where whole query and key blocks fill the chip as well (then, and if
  * NULL is passed, nothing is cut).  delta: (B,H,N) fp32 scratch.  Replaces _attention.backward
  * (fused-rope/fused_rope_attn.py:725-777; group sum: assets/flashattn-gqa/triton_gqa.py:605-666).  parts takes at most two slots per
  * compute unit: with 256 of them 64 MiB at D = 64, 128 MiB at D = 128 and 256, whatever the tensors' sizes. */

@@ -451,6 +451,36 @@ def test_backward_cut_key_blocks(pkg, B, Hq, Hkv, N, D, cut, causal, dtype):
         assert ok, name
 
 
+# Shapes whose dQ launch cuts query blocks into pieces: inside and across blocks and heads, a ragged last block and last key tile, waves whose rows see
+# none of a piece's keys, every head dim, v and dO as strided views.  What a cut changes is the order of a sum of fp32 values (the products are the same),
+# then one rounding: a step of the element type apart at most.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal", [(1, 2, 2, 2100, 128, True), (1, 3, 1, 1337, 128, False), (1, 1, 1, 4097, 128, True), (1, 2, 1, 3001, 64, False),
+                                                 (2, 1, 1, 4100, 64, True), (1, 2, 2, 2050, 256, True), (1, 1, 1, 1100, 256, False)])
+def test_backward_cut_query_blocks(pkg, B, Hq, Hkv, N, D, causal, dtype):
+    print(f"case B={B} Hq={Hq} Hkv={Hkv} N={N} D={D} causal={causal} {dtype}", flush=True)
+    lib, dev, scale = pkg._lib.load(), torch.device("cuda:0"), 1 / math.sqrt(D)
+    c, s = (t.to(dev) for t in O.precompute_freqs_cis(D, N))
+    q, k, v = (seeded((B, N, h, D), 110 + i).to(dev, dtype).transpose(1, 2).requires_grad_(True) for i, h in enumerate((Hq, Hkv, Hkv)))
+    g = seeded((B, N, Hq, D), 113).to(dev, dtype).transpose(1, 2)
+    out = pkg.attention(q, k, v, causal, scale, c, s)
+    qr, kr, vs, o, M, fc, fs = (t.detach() for t in out.grad_fn.saved_tensors)
+    dq = torch.autograd.grad(out, q, g)[0]
+    delta, gc = torch.empty_like(M), g.contiguous()
+    whole, dk, dv = (torch.empty_like(t) for t in (qr, kr, kr))
+    rc = lib.corope_rope_attn_bwd_rotated(*(t.data_ptr() for t in (qr, kr)), vs.data_ptr(), None, o.data_ptr(), gc.data_ptr(), None, M.data_ptr(),
+                                          delta.data_ptr(), fc.data_ptr(), fs.data_ptr(), fc.stride(0), whole.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, Hq,
+                                          Hkv, N, D, scale, int(causal), int(dtype == torch.float16), None, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    a, b = dq.float(), whole.float()
+    assert not torch.equal(a, b)   # (it was cut)
+    step = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    worst = ((a - b).abs() / b.abs().clamp_min(1e-2)).max().item()
+    print(f"  largest difference {worst:.2e} of the value")
+    assert torch.isfinite(a).all() and worst <= step * 1.01
+
+
 # Only the tables ask for a gradient: the operator has none for them, and its backward says so with the tensors its forward kept.
 @pytest.mark.parametrize("N", [130, 1024])
 def test_backward_when_only_the_tables_ask_for_a_gradient(pkg, N):

@@ -1,6 +1,7 @@
 // extern "C" surface of the library: argument validation (before any HIP call), error text, dispatch.
 #include "../../include/corope_amd.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -736,6 +737,19 @@ int corope_rope_attn_fwd_strided(const void* q, const int64_t* q_strides, const 
                                  const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin,
                                  int64_t freq_row_stride, void* o, float* lse, void* q_rot, void* k_rot, float* tile_kmax, int B,
                                  int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16, void* stream) {
+  return corope_rope_attn_fwd_cut(q, q_strides, k, k_strides, v, v_strides, freqs_cos, freqs_sin, freq_row_stride, o, lse, q_rot, k_rot, tile_kmax,
+                                  B, H, Hkv, N, D, sm_scale, causal, fp16, nullptr, 0, stream);
+}
+
+int64_t corope_rope_attn_fwd_parts_bytes(int B, int H, int N, int D, int causal) {
+  if (corope_rope_attn_check(B, H, N, D, D, 1.f, 0)) return -1;
+  return corope::fwd_parts_bytes(B, H, N, D, causal != 0);
+}
+
+int corope_rope_attn_fwd_cut(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,
+                             const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin, int64_t freq_row_stride, void* o, float* lse,
+                             void* q_rot, void* k_rot, float* tile_kmax, int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
+                             void* parts, int64_t parts_bytes, void* stream) {
   const char* what = "rope_attn_fwd_strided";
   if (Hkv <= 0 || H % Hkv != 0) return fail(COROPE_E_BADARG, "%s: H=%d is not a multiple of Hkv=%d", what, H, Hkv);
   int rc = corope_rope_attn_check(B, H, N, D, freq_row_stride, sm_scale, 0);
@@ -747,6 +761,13 @@ int corope_rope_attn_fwd_strided(const void* q, const int64_t* q_strides, const 
     if ((rc = check_strides(what, st, N, D))) return rc;
   if (k_rot == nullptr && q_rot != nullptr) return fail(COROPE_E_BADARG, "%s: q_rot without k_rot", what);
   corope::FwdParams p{};
+  if (parts != nullptr) {
+    if ((rc = check_ptrs(what, {parts}))) return rc;
+    const int64_t need = corope::fwd_parts_bytes(B, H, N, D, causal != 0);
+    if (parts_bytes < need)
+      return fail(COROPE_E_BADARG, "%s: parts of %lld bytes, %lld needed", what, (long long)parts_bytes, (long long)need);
+    p.parts = static_cast<float*>(parts);
+  }
   p.q = static_cast<const uint16_t*>(q);
   p.k = static_cast<const uint16_t*>(k);
   p.v = static_cast<const uint16_t*>(v);

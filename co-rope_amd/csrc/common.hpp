@@ -627,6 +627,63 @@ struct ItemList {
   __device__ __forceinline__ int at(int round) const { return round * G + ((round & 1) ? back : fwd); }
 };
 
+// What a workgroup of a kernel that owns query blocks works on.  CUT = false: whole items dealt in rounds.  CUT = true: the key tiles of all items,
+// head after head, form one list that the workgroups cut into equal pieces, so that few heads with long sequences keep every compute unit busy equally
+// long.  A piece that holds all of an item writes its result; others leave theirs in a slot of their own, at most one at each end of a
+// piece (piece_slot), and a second kernel joins an item's slots.  Item i is query block num_blocks - 1 - i / BH of head i % BH.
+template <bool CUT>
+struct QueryWork;
+
+template <>
+struct QueryWork<false> {
+  ItemList items;
+  int total;
+  __device__ __forceinline__ QueryWork(int num_blocks, int BH, int, int) : total(num_blocks * BH) {}
+  __device__ __forceinline__ int at(int round) const { return items.at(round); }   // >= total: no such item
+  __device__ __forceinline__ int begin(int) const { return 0; }
+  __device__ __forceinline__ int end(int, int tiles) const { return tiles; }
+  __device__ __forceinline__ int share() const { return 0; }
+};
+
+struct QueryTiles {
+  int nb, heads, k_tiles, step, per_head, total_tiles;
+  // step: key tiles by which a query block sees more than the one before it (0 when every query sees every key)
+  __host__ __device__ QueryTiles(int nb_, int heads_, int k_tiles_, int step_) : nb(nb_), heads(heads_), k_tiles(k_tiles_), step(step_) {
+    per_head = first(nb);
+    total_tiles = per_head * heads;
+  }
+  __host__ __device__ int first(int mb) const {   // tiles of a head before block mb
+    return step == 0 ? mb * k_tiles : mb == nb ? step * (nb * (nb - 1) / 2) + k_tiles : step * (mb * (mb + 1) / 2);
+  }
+  __device__ int start(int item) const { return (item % heads) * per_head + first(nb - 1 - item / heads); }
+  __device__ int begin_of_share(int w, int shares) const { return (int)((int64_t)w * total_tiles / shares); }
+  __device__ int share_of(int tile, int shares) const { return (int)((((int64_t)tile + 1) * shares - 1) / total_tiles); }
+};
+
+template <>
+struct QueryWork<true> {
+  QueryTiles t;
+  int total, t0, t1, li0, piece;
+  __device__ __forceinline__ QueryWork(int num_blocks, int BH, int k_tiles, int step) : t(num_blocks, BH, k_tiles, step), total(num_blocks * BH) {
+    const int n = gridDim.x, id = blockIdx.x;   // (neighbouring pieces on one XCD)
+    piece = n % 8 == 0 ? (id % 8) * (n / 8) + id / 8 : id;
+    t0 = t.begin_of_share(piece, n);
+    t1 = t.begin_of_share(piece + 1, n);
+    const int head = t0 / t.per_head, rem = t0 % t.per_head;
+    int mb = 0;
+    while (mb + 1 < t.nb && t.first(mb + 1) <= rem) ++mb;
+    li0 = head * t.nb + mb;
+  }
+  __device__ __forceinline__ int at(int round) const {
+    const int li = li0 + round, head = li / t.nb, mb = li % t.nb;
+    return li < total && head * t.per_head + t.first(mb) < t1 ? (t.nb - 1 - mb) * t.heads + head : total;
+  }
+  __device__ __forceinline__ int begin(int item) const { return max(0, t0 - t.start(item)); }
+  __device__ __forceinline__ int end(int item, int tiles) const { return min(tiles, t1 - t.start(item)); }
+  __device__ __forceinline__ int share() const { return piece; }
+};
+__device__ __forceinline__ int64_t piece_slot(int share, bool starts_item) { return 2 * (int64_t)share + (starts_item ? 1 : 0); }
+
 // Rows row0 .. row0 + 31 of a (n_rows, D) matrix of 16-bit elements from transposed fp32 accumulators (layout as for
 // store_rows_via_lds below), every value multiplied by `scale` (per lane = per row), one rounding, through a WaveTile:
 // 16-byte stores that cover whole rows.

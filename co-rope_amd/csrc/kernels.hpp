@@ -123,6 +123,7 @@ struct FwdParams {
   // rows; the last dimension is contiguous.  contiguous(D) fills in (B, H, N, D) row-major.
   int64_t q_sb, q_sh, k_sb, k_sh, v_sb, v_sh;
   int q_sn, k_sn, v_sn;
+  float* parts;      // scratch for the pieces of cut query blocks (fwd_parts_bytes), or null: none is cut
   void contiguous(int D) {
     q_sn = k_sn = v_sn = D;
     q_sh = k_sh = v_sh = (int64_t)N * D;
@@ -223,6 +224,8 @@ hipError_t launch_rope_attn_fwd_prerotated(const FwdParams& p, int D, bool causa
 // the same with 64 query rows per wave, one wave per SIMD (D = 128)
 hipError_t launch_rope_attn_fwd_prerotated_rows64(const FwdParams& p, int D, bool causal, hipStream_t stream);
 // head dim 256 (bf16): 32 query rows per wave, one wave per SIMD, 32-key tiles
+// bytes of FwdParams::parts with which the forward on rotated keys (with key-norm maxima) cuts query blocks; 0: it is faster without
+int64_t fwd_parts_bytes(int B, int H, int N, int D, bool causal);
 hipError_t launch_rope_attn_fwd_prerotated_pipe256(const FwdParams& p, bool causal, hipStream_t stream);
 // head dim 128 in that form (128-row items, 32-key tiles), two workgroups per compute unit
 hipError_t launch_rope_attn_fwd_prerotated_pipe32x2(const FwdParams& p, bool causal, hipStream_t stream);

@@ -137,7 +137,6 @@ struct DkdvWork<true> {
 // A slot of partial sums: NWAVES x 32 keys x D of dV, then of dK_r, as the accumulators lie ([32-key block][register quad][lane]).
 template <int D, int NWAVES>
 constexpr int64_t kDkdvSlotFloats = 2ll * NWAVES * 32 * D;
-__device__ __forceinline__ int64_t dkdv_slot(int share, bool starts_item) { return 2 * (int64_t)share + (starts_item ? 1 : 0); }
 
 // PREROT: Q and K come from copies that rope_rotate_kernel rotated beforehand (no table reads in the loop).
 template <int D, int NWAVES, int BLOCK_M, bool CAUSAL, bool DO_DV, bool DO_DK, bool PREROT, bool CUT = false>
@@ -422,7 +421,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
         store_unrotated_rows_via_wave_tile<D>(dkacc, tb, p.dk + base, wk_lo, N, 0.6931471805599453f, wave_slot, opaque_lane());
       }
     } else if constexpr (CUT) {   // a piece of the item: its partial sums
-      float* slot = p.parts + dkdv_slot(items.share(), it_begin == 0) * kDkdvSlotFloats<D, NWAVES> + (int64_t)rb * 32 * D + 4 * opaque_lane();
+      float* slot = p.parts + piece_slot(items.share(), it_begin == 0) * kDkdvSlotFloats<D, NWAVES> + (int64_t)rb * 32 * D + 4 * opaque_lane();
 #pragma unroll
       for (int i = 0; i < NDB * 4; ++i) {
         const int db = i / 4, g = i % 4;
@@ -458,7 +457,7 @@ __global__ __launch_bounds__(kWave) void rope_attn_bwd_dkdv_sum_kernel(BwdParams
   for (int db = 0; db < NDB; ++db) acc[db] = f32x16{0};
 #pragma unroll 1
   for (int w = w0; w <= w1; ++w) {
-    const float* slot = src + dkdv_slot(w, w == w0) * kDkdvSlotFloats<D, NWAVES>;
+    const float* slot = src + piece_slot(w, w == w0) * kDkdvSlotFloats<D, NWAVES>;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -500,60 +499,6 @@ struct DqCfg {
   static_assert(kLdsBytes <= 160 * 1024, "LDS of a compute unit");
 };
 
-// What a workgroup of the dQ kernel works on, as DkdvWork says for the other one: CUT = true cuts the list of the key tiles of all items, head after
-// head, into equal pieces.  Item i is query block num_blocks - 1 - i / BH of head i % BH.
-template <bool CUT>
-struct DqWork;
-
-template <>
-struct DqWork<false> {
-  ItemList items;
-  int total;
-  __device__ __forceinline__ DqWork(int num_blocks, int BH, int, int) : total(num_blocks * BH) {}
-  __device__ __forceinline__ int at(int round) const { return items.at(round); }   // >= total: no such item
-  __device__ __forceinline__ int begin(int) const { return 0; }
-  __device__ __forceinline__ int end(int, int tiles) const { return tiles; }
-  __device__ __forceinline__ int share() const { return 0; }
-};
-
-struct DqTiles {
-  int nb, heads, k_tiles, step, per_head, total_tiles;
-  // step: key tiles by which a query block sees more than the one before it (0 when every query sees every key)
-  __host__ __device__ DqTiles(int nb_, int heads_, int k_tiles_, int step_) : nb(nb_), heads(heads_), k_tiles(k_tiles_), step(step_) {
-    per_head = first(nb);
-    total_tiles = per_head * heads;
-  }
-  __host__ __device__ int first(int mb) const {   // tiles of a head before block mb
-    return step == 0 ? mb * k_tiles : mb == nb ? step * (nb * (nb - 1) / 2) + k_tiles : step * (mb * (mb + 1) / 2);
-  }
-  __device__ int start(int item) const { return (item % heads) * per_head + first(nb - 1 - item / heads); }
-  __device__ int begin_of_share(int w, int shares) const { return (int)((int64_t)w * total_tiles / shares); }
-  __device__ int share_of(int tile, int shares) const { return (int)((((int64_t)tile + 1) * shares - 1) / total_tiles); }
-};
-
-template <>
-struct DqWork<true> {
-  DqTiles t;
-  int total, t0, t1, li0, piece;
-  __device__ __forceinline__ DqWork(int num_blocks, int BH, int k_tiles, int step) : t(num_blocks, BH, k_tiles, step), total(num_blocks * BH) {
-    const int n = gridDim.x, id = blockIdx.x;   // (neighbouring pieces on one XCD)
-    piece = n % 8 == 0 ? (id % 8) * (n / 8) + id / 8 : id;
-    t0 = t.begin_of_share(piece, n);
-    t1 = t.begin_of_share(piece + 1, n);
-    const int head = t0 / t.per_head, rem = t0 % t.per_head;
-    int mb = 0;
-    while (mb + 1 < t.nb && t.first(mb + 1) <= rem) ++mb;
-    li0 = head * t.nb + mb;
-  }
-  __device__ __forceinline__ int at(int round) const {
-    const int li = li0 + round, head = li / t.nb, mb = li % t.nb;
-    return li < total && head * t.per_head + t.first(mb) < t1 ? (t.nb - 1 - mb) * t.heads + head : total;
-  }
-  __device__ __forceinline__ int begin(int item) const { return max(0, t0 - t.start(item)); }
-  __device__ __forceinline__ int end(int item, int tiles) const { return min(tiles, t1 - t.start(item)); }
-  __device__ __forceinline__ int share() const { return piece; }
-};
-
 // A slot of partial sums: NWAVES x 32 queries x D of dQ_r, as the accumulators lie ([32-row block][register quad][lane]).
 template <int D, int NWAVES>
 constexpr int64_t kDqSlotFloats = (int64_t)NWAVES * 32 * D;
@@ -580,7 +525,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   float* const wave_delta = reinterpret_cast<float*>(wave_tile + WaveTile<D>::kBytes);
 
   const int n_k_tiles = (N + BLOCK_N - 1) / BLOCK_N;
-  const DqWork<CUT> items(p.num_blocks, p.BH, n_k_tiles, CAUSAL ? Cfg::kBlockM / BLOCK_N : 0);
+  const QueryWork<CUT> items(p.num_blocks, p.BH, n_k_tiles, CAUSAL ? Cfg::kBlockM / BLOCK_N : 0);
   const int total = items.total;   // item i (heaviest first): query block num_blocks - 1 - i / BH of head i % BH
   auto tiles_of = [&](int mb) {
     return CAUSAL ? min((mb * Cfg::kBlockM + Cfg::kBlockM + BLOCK_N - 1) / BLOCK_N, n_k_tiles) : n_k_tiles;
@@ -808,7 +753,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     if (!CUT || (t_begin == 0 && n_tiles == tiles_of(mb))) {   // workgroup-uniform
       store_unrotated_rows_via_wave_tile<D>(dqacc, tb, p.dq + (int64_t)bh * N * D, wq_lo, N, p.sm_scale, wave_tile, opaque_lane());
     } else if constexpr (CUT) {   // a piece of the item: its partial sums
-      float* slot = p.dq_parts + dkdv_slot(items.share(), t_begin == 0) * kDqSlotFloats<D, NWAVES> + (int64_t)rb * 32 * D + 4 * opaque_lane();
+      float* slot = p.dq_parts + piece_slot(items.share(), t_begin == 0) * kDqSlotFloats<D, NWAVES> + (int64_t)rb * 32 * D + 4 * opaque_lane();
 #pragma unroll
       for (int i = 0; i < NDB * 4; ++i)
         *reinterpret_cast<f32x4*>(slot + i * 4 * kWave) =
@@ -828,7 +773,7 @@ template <int D, int NWAVES, int BLOCK_N, bool CAUSAL>
 __global__ __launch_bounds__(D / 16 * kWave) void rope_attn_bwd_dq_sum_kernel(BwdParams p, int shares) {
   constexpr int BLOCK_M = NWAVES * 32, PARTNER = D / 16 * 4 * kWave;
   const int N = p.N;
-  const DqTiles t(p.num_blocks, p.BH, (N + BLOCK_N - 1) / BLOCK_N, CAUSAL ? BLOCK_M / BLOCK_N : 0);
+  const QueryTiles t(p.num_blocks, p.BH, (N + BLOCK_N - 1) / BLOCK_N, CAUSAL ? BLOCK_M / BLOCK_N : 0);
   const int item = blockIdx.x / NWAVES, rb = blockIdx.x % NWAVES, mb = p.num_blocks - 1 - item / p.BH;
   const int start = t.start(item), w0 = t.share_of(start, shares), w1 = t.share_of(start + t.first(mb + 1) - t.first(mb) - 1, shares);
   const int lane = threadIdx.x % kWave, i = threadIdx.x / kWave, row = mb * BLOCK_M + rb * 32 + lane % 32;
@@ -841,7 +786,7 @@ __global__ __launch_bounds__(D / 16 * kWave) void rope_attn_bwd_dq_sum_kernel(Bw
     f32x4 x[4], y[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const float* slot = src + dkdv_slot(min(w + u, w1), min(w + u, w1) == w0) * kDqSlotFloats<D, NWAVES>;
+      const float* slot = src + piece_slot(min(w + u, w1), min(w + u, w1) == w0) * kDqSlotFloats<D, NWAVES>;
       x[u] = *reinterpret_cast<const f32x4*>(slot);
       y[u] = *reinterpret_cast<const f32x4*>(slot + PARTNER);
     }
@@ -1007,7 +952,7 @@ static int dq_shares(int N, int BH, bool causal) {
     }
     longest = std::max(longest, sum);
   }
-  const DqTiles t((N + CW * 32 - 1) / (CW * 32), BH, k_tiles, causal ? CW * 32 / BN : 0);
+  const QueryTiles t((N + CW * 32 - 1) / (CW * 32), BH, k_tiles, causal ? CW * 32 / BN : 0);
   const int shares = std::max(1, std::min(cus, t.total_tiles / 4));
   constexpr float kWholeTile = D == 64 ? 1.25f : D == 128 ? 2.8f : 1.75f, kTile = D == 64 ? 1.5f : D == 128 ? 2.9f : 1.6f;
   constexpr float kChange = D == 64 ? 3.5f : D == 128 ? 5.f : 21.f;

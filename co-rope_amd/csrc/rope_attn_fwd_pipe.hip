@@ -30,6 +30,8 @@
 #include "common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -58,6 +60,10 @@ struct FwdPipeCfg {
   static constexpr int kLdsBytes = kRingBytes + NW * WaveTile<D>::kBytes;
   static_assert(kLdsBytes <= 160 * 1024, "LDS of a compute unit");
 };
+
+// A slot of a piece's results: NW x 32 rows x D of O as the accumulators lie ([32-row block][register quad][lane]), then the rows' log-sum-exps.
+template <int D, int NW>
+constexpr int64_t kFwdSlotFloats = (int64_t)NW * 32 * (D + 1);
 
 // P^T is a bf16 operand in both builds (its unnormalised values span up to 2^kPipeMargin, more binary orders than fp16
 // has), so the product O^T += V^T P^T is a bf16 product in both: in the fp16 build the V tile is converted to bf16 while
@@ -107,7 +113,10 @@ __device__ __forceinline__ float wave_reduce_max(float x) { return wave_max(x); 
 // ring for its Q rows and O rows, so nothing at the change of items needs a workgroup barrier: a wave that is past its
 // causal diagonal normalises and stores its O rows and requests the next item's Q rows while the other waves still work
 // on the diagonal tiles, and only keeps staging its share of those tiles.
-template <int D, bool CAUSAL, int NW>
+//
+// CUT: a workgroup takes a piece of the list of all key tiles instead (QueryWork); a piece of an item starts its own softmax and leaves its
+// normalised O and log-sum-exp in a slot, which rope_attn_fwd_join_kernel weighs.
+template <int D, bool CAUSAL, int NW, bool CUT = false>
 __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) void rope_attn_fwd_pipe_kernel(FwdParams p) {
   using Cfg = FwdPipeCfg<D, NW>;
   constexpr int BLOCK_N = kPipeBlockN;
@@ -128,10 +137,10 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
   uint8_t* const wave_tile = smem + Cfg::kRingBytes + wave * WaveTile<D>::kBytes;
 
   // ---- the workgroup's list of items --------------------------------------------------------------------------------
-  const ItemList items;
-  const int total = p.num_m_blocks * p.BH;
-  auto item_at = [&](int r) { return items.at(r); };   // position in the heaviest-first order; >= total: none
   const int n_k_tiles = (N + BLOCK_N - 1) / BLOCK_N;
+  const QueryWork<CUT> items(p.num_m_blocks, p.BH, n_k_tiles, CAUSAL ? Cfg::kBlockM / BLOCK_N : 0);
+  const int total = items.total;
+  auto item_at = [&](int r) { return items.at(r); };   // position in the heaviest-first order; >= total: none
   auto tiles_of = [&](int mb) {
     return CAUSAL ? min((mb * Cfg::kBlockM + Cfg::kBlockM + BLOCK_N - 1) / BLOCK_N, n_k_tiles) : n_k_tiles;
   };
@@ -147,7 +156,8 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     const int kvs = kv_slab(i % p.BH, p.H, p.Hkv);
     l_kg = p.k_rot + (int64_t)kvs * N * D;
     l_vg = p.v_slab(kvs);
-    l_tiles = tiles_of(p.num_m_blocks - 1 - i / p.BH);
+    l_tile = items.begin(i);
+    l_tiles = items.end(i, tiles_of(p.num_m_blocks - 1 - i / p.BH));
     return true;
   };
   auto load_next_tile = [&]() __attribute__((always_inline)) {   // moves the cursor on and requests that tile
@@ -155,7 +165,6 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
       ++l_tile;
     } else if (load_item(l_round + 1)) {
       ++l_round;
-      l_tile = 0;
     }   // else: past the last tile of the last item; the same tile is requested again and never used
     kst.load(l_kg, l_tile * BLOCK_N, N);
     vst.load(l_vg, l_tile * BLOCK_N, N, (uint32_t)p.v_sn * 2);
@@ -207,7 +216,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     const int bh = i % p.BH, m0 = (p.num_m_blocks - 1 - i / p.BH) * Cfg::kBlockM;
     const int l = opaque_lane();
     qrows.load(p.q_slab(bh), p.cos, p.sin, p.fstride, m0 + rb * 32, N, l, (uint32_t)p.q_sn * 2);
-    kvec = reinterpret_cast<const uint32_t*>(p.tile_kmax)[(int64_t)kv_slab(bh, p.H, p.Hkv) * n_k_tiles + min(l, n_k_tiles - 1)];
+    kvec = reinterpret_cast<const uint32_t*>(p.tile_kmax)[(int64_t)kv_slab(bh, p.H, p.Hkv) * n_k_tiles + min(items.begin(i) + l, n_k_tiles - 1)];
   };
   auto take_q = [&](int i) __attribute__((always_inline)) {
     const int bh = i % p.BH, m0 = (p.num_m_blocks - 1 - i / p.BH) * Cfg::kBlockM;
@@ -219,8 +228,8 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
   int item = item_at(0);
   COROPE_ISTAMP(0);
   load_item(0);
-  kst.load(l_kg, 0, N);
-  vst.load(l_vg, 0, N, (uint32_t)p.v_sn * 2);
+  kst.load(l_kg, l_tile * BLOCK_N, N);
+  vst.load(l_vg, l_tile * BLOCK_N, N, (uint32_t)p.v_sn * 2);
   request_q(item);
   take_q(item);
   kst.store_rows(lds_at(koff_cur));
@@ -231,7 +240,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
   for (int round = 0;; ++round) {
     const int bh = item % p.BH, mb = p.num_m_blocks - 1 - item / p.BH;
     const int m0 = mb * Cfg::kBlockM;
-    const int n_tiles = tiles_of(mb);
+    const int t_begin = items.begin(item), n_tiles = items.end(item, tiles_of(mb));   // of this workgroup's piece of the item
     const int q_row = m0 + rb * 32 + lq;           // absolute query index of this lane
     const uint32_t* tile_kmax_bits = reinterpret_cast<const uint32_t*>(p.tile_kmax) + (int64_t)kv_slab(bh, p.H, p.Hkv) * n_k_tiles;
     COROPE_ISTAMP(1);
@@ -270,8 +279,8 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     // Reference value that puts every tile this wave will see within the margin.
     float lift_target;
     {
-      uint32_t kall = lane <= t_last ? kvec : 0u;   // non-negative floats order like their bit patterns
-      for (int t0 = kWave; t0 <= t_last; t0 += kWave) {
+      uint32_t kall = t_begin + lane <= t_last ? kvec : 0u;   // non-negative floats order like their bit patterns
+      for (int t0 = t_begin + kWave; t0 <= t_last; t0 += kWave) {
         const int tt = t0 + lane;
         kall = max(kall, tt <= t_last ? tile_kmax_bits[tt] : 0u);
       }
@@ -283,7 +292,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     // kmax_bits > thr_bits with thr = (min over rows of m_run + margin) / q_bound_wave, recomputed when the
     // reference moves.  Lane i of kvec holds the key-norm maximum of tile kvec_base + i.
     uint32_t thr_bits = 0;
-    int kvec_base = 0;
+    int kvec_base = t_begin;
 
     // v_lane: per-lane address of a V buffer (buffer offset + v_lane_off).  MFMA i of a PV half: block i % NDB, chunk i / NDB
     auto v_operand = [&](uint32_t v_lane, int half, int i) {
@@ -311,7 +320,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     uint64_t exact_passes = 0;   // tiles of this wave that were examined a second time to move the reference
 #endif
     // ---- tiles this wave's rows can see ------------------------------------------------------------------------------
-    for (int t = 0; t <= t_last; ++t) {
+    for (int t = t_begin; t <= t_last; ++t) {
       const int n0 = t * BLOCK_N;
 #ifdef COROPE_TRACE
       if (t == 1) COROPE_ISTAMP(3);
@@ -319,7 +328,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
 #endif
       // K(t), V(t), V(t-1); the first tile of an item has no predecessor: its "previous V" is multiplied by a zero P1 and
       // only has to be finite wherever V(0) is, so it is V(0) itself
-      uint32_t k_lane = k_lane_off + koff_cur, vt = v_lane_off + voff_cur, vprev = v_lane_off + (t == 0 ? voff_cur : voff_prev);
+      uint32_t k_lane = k_lane_off + koff_cur, vt = v_lane_off + voff_cur, vprev = v_lane_off + (t == t_begin ? voff_cur : voff_prev);
       asm volatile("" : "+v"(k_lane), "+v"(vt), "+v"(vprev));
       auto k_operand = [&](int half, int kc) {
         return *reinterpret_cast<const u32x4*>(lds_at(k_lane) + RowTile<D>::off(half * 32, 16 * kc));
@@ -383,11 +392,11 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
         asm volatile("" ::"v"(kvec));
       }
       const uint32_t kmax_bits = __builtin_amdgcn_readlane(kvec, t - kvec_base);
-      if (t == 0 || kmax_bits > thr_bits) {
+      if (t == t_begin || kmax_bits > thr_bits) {
 #ifdef COROPE_TRACE
         ++exact_passes;
 #endif
-        if (t > 0) drain();
+        if (t > t_begin) drain();
         f32x16 r0 = f32x16{0}, r1 = f32x16{0};
 #pragma unroll
         for (int kc = 0; kc < M; ++kc) {
@@ -407,7 +416,8 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
         // this block so far (m_true, a lower bound of the row's running maximum): the row's largest probability stays
         // above 2^-kPipeLift, far inside fp32 / bf16 range, however often the block runs.
         m_true = fmaxf(m_true, half_max(mt));
-        const float m_new = fmaxf(m_run, fmaxf(m_true, fminf(lift_target, m_true + kPipeLift)));
+        float m_new = fmaxf(m_run, fmaxf(m_true, fminf(lift_target, m_true + kPipeLift)));
+        if constexpr (CUT) m_new = fmaxf(m_new, -1e30f);   // (a row that sees no key of the piece so far)
         const float alpha = fast_exp2(m_run - m_new);   // m_new is finite: every row sees key 0 of tile 0
         l_run = (l_run + lsum) * alpha;
         lsum = 0.f;
@@ -441,7 +451,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     const int next_item = item_at(round + 1);
     const bool has_next = next_item < total;
     request_q(has_next ? next_item : item);
-    drain();
+    if (!CUT || t_last >= t_begin) drain();   // wave-uniform
     COROPE_ISTAMP(5);
 #ifdef COROPE_TRACE
     if (p.trace != nullptr && threadIdx.x == TT) {
@@ -452,12 +462,21 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
 
     // ---- of the tiles entirely above this wave's diagonal it only stages its share; then the item's O rows and statistic
     // leave, all waves at once, and the next item's Q rows are taken in -----------------------------------------------------
-    for (int t = t_last + 1; t < n_tiles; ++t) {
+    for (int t = CUT ? max(t_begin, t_last + 1) : t_last + 1; t < n_tiles; ++t) {
       stage_next();
       rotate_buffers();
       __syncthreads();
     }
-    {
+    if (CUT && !(t_begin == 0 && n_tiles == tiles_of(mb))) {   // workgroup-uniform: a piece of the item
+      const float l_tot = half_sum(l_run + lsum), inv = l_tot > 0.f ? 1.f / l_tot : 0.f;   // (0: no key seen)
+      const int l = opaque_lane();
+      float* slot = p.parts + piece_slot(items.share(), t_begin == 0) * kFwdSlotFloats<D, NW>;
+#pragma unroll
+      for (int i = 0; i < NDB * 4; ++i)
+        *reinterpret_cast<f32x4*>(slot + (rb * NDB * 4 + i) * 4 * kWave + 4 * l) =
+            f32x4{oacc[i / 4][4 * (i % 4)] * inv, oacc[i / 4][4 * (i % 4) + 1] * inv, oacc[i / 4][4 * (i % 4) + 2] * inv, oacc[i / 4][4 * (i % 4) + 3] * inv};
+      if (lh == 0) slot[NW * 32 * D + rb * 32 + lq] = m_run + fast_log2(l_tot);   // -inf where no key is seen
+    } else {
       const float l_tot = half_sum(l_run + lsum);
       store_rows_via_wave_tile<D>(oacc, p.o + (int64_t)bh * N * D, m0 + rb * 32, N, 1.f / l_tot, wave_tile, opaque_lane());
       if (q_row < N && lh == 0) p.lse[(int64_t)bh * N + q_row] = m_run + fast_log2(l_tot);
@@ -468,6 +487,44 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     COROPE_ISTAMP(0);
     take_q(item);
   }
+}
+
+// O and lse of the items that were cut: a workgroup per 32 rows of an item, a wave per two register quads.
+template <int D, bool CAUSAL, int NW>
+__global__ __launch_bounds__(D / 16 * kWave) void rope_attn_fwd_join_kernel(FwdParams p, int shares) {
+  constexpr int BLOCK_M = NW * 32, BLOCK_N = kPipeBlockN, QUADS = D / 16;
+  const int N = p.N;
+  const QueryTiles t(p.num_m_blocks, p.BH, (N + BLOCK_N - 1) / BLOCK_N, CAUSAL ? BLOCK_M / BLOCK_N : 0);
+  const int item = blockIdx.x / NW, rb = blockIdx.x % NW, mb = p.num_m_blocks - 1 - item / p.BH, bh = item % p.BH;
+  const int start = t.start(item), w0 = t.share_of(start, shares), w1 = t.share_of(start + t.first(mb + 1) - t.first(mb) - 1, shares);
+  const int lane = threadIdx.x % kWave, i = threadIdx.x / kWave, row = mb * BLOCK_M + rb * 32 + lane % 32;
+  if (w0 == w1 || row >= N) return;   // one piece holds all of the item and has written it
+  auto slot_of = [&](int w) { return p.parts + piece_slot(w, w == w0) * kFwdSlotFloats<D, NW>; };
+  auto lse_of = [&](int w) { return slot_of(w)[NW * 32 * D + rb * 32 + lane % 32]; };
+  float top = -INFINITY, sum = 0.f;   // (the first piece holds key 0, which every row sees: top is finite)
+  for (int w = w0; w <= w1; ++w) top = fmaxf(top, lse_of(w));
+  for (int w = w0; w <= w1; ++w) sum += fast_exp2(lse_of(w) - top);
+  const float lse = top + fast_log2(sum);
+  f32x4 a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
+  for (int w = w0; w <= w1; w += 4) {   // eight loads in flight
+    f32x4 x[4], y[4];
+    float f[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float* src = slot_of(min(w + u, w1)) + (rb * 2 * QUADS + i) * 4 * kWave + 4 * lane;
+      x[u] = *reinterpret_cast<const f32x4*>(src);
+      y[u] = *reinterpret_cast<const f32x4*>(src + QUADS * 4 * kWave);
+      f[u] = fast_exp2(lse_of(min(w + u, w1)) - lse);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (w + u <= w1) a += x[u] * f[u], b += y[u] * f[u];
+  }
+  const int col = 8 * i + 4 * (lane / 32);
+  uint16_t* out = p.o + ((int64_t)bh * N + row) * D + col;
+  *reinterpret_cast<u32x2*>(out) = u32x2{pack_elts(a[0], a[1]), pack_elts(a[2], a[3])};
+  *reinterpret_cast<u32x2*>(out + D / 2) = u32x2{pack_elts(b[0], b[1]), pack_elts(b[2], b[3])};
+  if (i == 0 && lane < 32) p.lse[(int64_t)bh * N + row] = lse;
 }
 
 // ---- host-side launch -----------------------------------------------------------------------------------------
@@ -486,8 +543,69 @@ static hipError_t launch_pipe_waves(FwdParams p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+constexpr int kCutWaves = 8;
+
+// How many pieces the key tiles of the launch are cut into; 0: whole items.  With few heads the longest whole item sets the time however many
+// compute units are idle.  Measured constants, in microseconds, as in dq_shares (a piece pays its first tile's second look and a change of items,
+// and the join a launch).  Whole / cut with its join, causal, B1 H N: D = 128: 8 4096 89 / 70, 4 8192 170 / 103, 1 10000 183 / 57, 3 20000 400 / 349, and on the
+// other side 16 4096 111 / 111, 32 1500 40 / 53; D = 64: 4 16384 217 / 189, 2 20000 220 / 145, 8 4096 49 / 46, 16 1500 23 / 30.
+template <int D>
+static int fwd_shares(int N, int BH, bool causal) {
+  constexpr int BN = kPipeBlockN, kMost = 16;
+  if (g_tile_rows.load(std::memory_order_relaxed) != 0 || g_fwd_wave_rows.load(std::memory_order_relaxed) != 0) return 0;   // a form was asked for
+  const int k_tiles = (N + BN - 1) / BN, cus = device_cu_count();
+  const bool small = use_small_tiles(N, BH, FwdPipeCfg<D, 4>::kLdsBytes);
+  const int block = small ? 128 : 256, nb = (N + block - 1) / block;
+  const int slots = cus * (small && fits_twice(FwdPipeCfg<D, 4>::kLdsBytes) ? 2 : 1);
+  const int64_t n_items = (int64_t)nb * BH;
+  if (n_items > (int64_t)kMost * slots || n_items * k_tiles >= (1ll << 30)) return 0;   // many rounds even out
+  int64_t longest = 0;
+  const int grid = (int)std::min<int64_t>(n_items, slots);
+  for (int w = 0; w < grid; w += 8) {
+    int64_t sum = 0;
+    for (int r = 0; (int64_t)r * grid < n_items; ++r) {
+      const int64_t i = (int64_t)r * grid + ((r & 1) ? grid - 1 - w : w);
+      if (i < n_items) sum += causal ? std::min((nb - (int)(i / BH)) * (block / BN), k_tiles) : k_tiles;
+    }
+    longest = std::max(longest, sum);
+  }
+  const QueryTiles t((N + kCutWaves * 32 - 1) / (kCutWaves * 32), BH, k_tiles, causal ? kCutWaves * 32 / BN : 0);
+  const int shares = std::max(1, std::min(cus, t.total_tiles / 4));
+  constexpr float kWholeTile = D == 64 ? 1.f : 1.75f, kTile = D == 64 ? 1.1f : 2.f, kChange = D == 64 ? 3.f : 4.f;
+  const float busy = std::min(1.f, (float)t.total_tiles * (small ? 2.f : 1.f) / ((float)longest * cus));
+  const float whole = (small ? 0.8f : 1.05f) * longest * kWholeTile * (0.75f + 0.25f * busy) + kChange * ((n_items + grid - 1) / grid) + 2.f;
+  const float tiles = (float)t.total_tiles / shares, crossed = causal ? std::sqrt(2.f * tiles / (kCutWaves * 32 / BN)) : 1.f;
+  const float moved = (float)(shares + std::min<int64_t>(t.nb * (int64_t)BH, shares)) * kFwdSlotFloats<D, kCutWaves> * 8;
+  const float cut = tiles * kTile + kChange * (1.f + crossed) + 9.f + moved / 12e6f;
+  return cut < 0.9f * whole ? shares : 0;
+}
+
+int64_t fwd_parts_bytes(int B, int H, int N, int D, bool causal) {
+  if (D == 64) return 8 * fwd_shares<64>(N, B * H, causal) * kFwdSlotFloats<64, kCutWaves>;
+  if (D == 128) return 8 * fwd_shares<128>(N, B * H, causal) * kFwdSlotFloats<128, kCutWaves>;
+  return 0;
+}
+
+template <int D, bool CAUSAL>
+static hipError_t launch_pipe_cut(FwdParams p, int shares, hipStream_t stream) {
+  using Cfg = FwdPipeCfg<D, kCutWaves>;
+  auto kern = rope_attn_fwd_pipe_kernel<D, CAUSAL, kCutWaves, true>;
+  static std::atomic<uint64_t> lds_ok{0};
+  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
+  p.num_m_blocks = (p.N + Cfg::kBlockM - 1) / Cfg::kBlockM;
+#ifdef COROPE_TRACE
+  p.trace = nullptr;
+#endif
+  hipLaunchKernelGGL(kern, dim3(shares), dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, p);
+  hipLaunchKernelGGL((rope_attn_fwd_join_kernel<D, CAUSAL, kCutWaves>), dim3((unsigned)p.num_m_blocks * p.BH * kCutWaves), dim3(D / 16 * kWave), 0, stream,
+                     p, shares);
+  return hipGetLastError();
+}
+
 template <int D, bool CAUSAL>
 static hipError_t launch_pipe_cfg(const FwdParams& p, hipStream_t stream) {
+  if (p.parts != nullptr)
+    if (const int shares = fwd_shares<D>(p.N, p.BH, CAUSAL); shares > 0) return launch_pipe_cut<D, CAUSAL>(p, shares, stream);
   return use_small_tiles(p.N, p.BH, FwdPipeCfg<D, 4>::kLdsBytes) ? launch_pipe_waves<D, CAUSAL, 4>(p, stream)
                                                                   : launch_pipe_waves<D, CAUSAL, 8>(p, stream);
 }

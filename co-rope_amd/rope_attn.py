@@ -151,6 +151,17 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
     rotated = None
     Hkv = k.shape[1]
     with _on_device(q):
+        # scratch for the pieces of query blocks that the kernel on rotated keys cuts among workgroups (0: none are cut).  Only speed needs it
+        parts, nbytes = None, 0
+        if two_launch and D <= 128 and not (q.dtype == torch.float16 and keep_rotated and FP16_TRAINING_FORWARD != "fast"):
+            nbytes = lib.corope_rope_attn_fwd_parts_bytes(B, H, N, D, int(bool(causal)))
+            if nbytes > 0:
+                try:
+                    parts = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
+                except torch.cuda.OutOfMemoryError:
+                    pass
+        if parts is not None and strides is None:
+            strides = tuple((ctypes.c_int64 * 3)(h * N * D, N * D, D) for h in (H, Hkv, Hkv))   # (contiguous; an axis of length 1 may say otherwise)
         if strides is not None:
             fp16 = q.dtype == torch.float16
             # fp16 with gradients: P and V stay fp16 (no key-norm maxima: the single-launch kernel, on the rotated copy)
@@ -158,13 +169,14 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
             q_rot = torch.empty(q.shape, device=q.device, dtype=q.dtype) if (two_launch and keep_rotated) else None
             k_rot = torch.empty(k.shape, device=q.device, dtype=q.dtype) if two_launch else None
             kmax = torch.empty((B, Hkv, (N + 63) // 64), device=q.device, dtype=torch.float32) if (two_launch and not exact) else None
-            rc = lib.corope_rope_attn_fwd_strided(q.data_ptr(), strides[0], k.data_ptr(), strides[1], v.data_ptr(), strides[2],
-                                                  fc.data_ptr(), fs.data_ptr(), fc.stride(0), o.data_ptr(), M.data_ptr(),
-                                                  q_rot.data_ptr() if q_rot is not None else None,
-                                                  k_rot.data_ptr() if k_rot is not None else None,
-                                                  kmax.data_ptr() if kmax is not None else None, B, H, Hkv, N, D,
-                                                  float(sm_scale), int(bool(causal)), int(fp16), _stream_ptr(q))
-            _lib.check(rc, "corope_rope_attn_fwd_strided")
+            rc = lib.corope_rope_attn_fwd_cut(q.data_ptr(), strides[0], k.data_ptr(), strides[1], v.data_ptr(), strides[2],
+                                              fc.data_ptr(), fs.data_ptr(), fc.stride(0), o.data_ptr(), M.data_ptr(),
+                                              q_rot.data_ptr() if q_rot is not None else None,
+                                              k_rot.data_ptr() if k_rot is not None else None,
+                                              kmax.data_ptr() if kmax is not None else None, B, H, Hkv, N, D,
+                                              float(sm_scale), int(bool(causal)), int(fp16),
+                                              parts.data_ptr() if parts is not None else None, nbytes, _stream_ptr(q))
+            _lib.check(rc, "corope_rope_attn_fwd_cut")
             if q_rot is not None:
                 rotated = (q_rot, k_rot)
         elif q.dtype == torch.float16:

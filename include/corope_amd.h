@@ -264,6 +264,18 @@ int corope_rope_attn_fwd_strided(const void *q, const int64_t *q_strides, const 
                                  void *o, float *lse, void *q_rot, void *k_rot, float *tile_kmax,
                                  int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16, void *stream);
 
+/* The same with scratch in which the kernel on rotated keys (k_rot and tile_kmax given) leaves the pieces of query blocks that it cuts among
+ * workgroups, so that few heads with long sequences fill the chip: corope_rope_attn_fwd_parts_bytes says how much, 0 where whole blocks fill it as
+ * well (then, and if parts is NULL, nothing is cut and this is corope_rope_attn_fwd_strided).  At most two slots per compute unit: with 256 of them
+ * 33 MiB at D = 64, 65 MiB at D = 128.  (fused-rope/fused_rope_attn.py:655-722 launches whole query blocks only.) */
+int64_t corope_rope_attn_fwd_parts_bytes(int B, int H, int N, int D, int causal);
+int corope_rope_attn_fwd_cut(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
+                             const void *v, const int64_t *v_strides,
+                             const float *freqs_cos, const float *freqs_sin, int64_t freq_row_stride,
+                             void *o, float *lse, void *q_rot, void *k_rot, float *tile_kmax,
+                             int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
+                             void *parts, int64_t parts_bytes, void *stream);
+
 /* Grouped-query form of the operator: q (B,Hq,N,D), k and v (B,Hkv,N,D), Hq a multiple of Hkv; query head h reads
  * key/value head h / (Hq/Hkv); dk and dv (B,Hkv,N,D) are sums over the query heads of their group (the key block's
  * workgroup sweeps all of them, no atomics).  The reference's RoPE operator requires Hq == Hkv

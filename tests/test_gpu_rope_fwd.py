@@ -1,6 +1,7 @@
 """GPU parity of the fused RoPE-attention forward against the CPU oracle (through the C ABI).
 
 Bar: max-abs <= 2e-2 for bf16 outputs against the fp32 oracle evaluated on the same bf16-rounded inputs."""
+import ctypes
 import math
 
 import pytest
@@ -327,3 +328,52 @@ def test_single_launch_kernel_on_a_rotated_key_copy(pkg, B, H, Hkv, N, D, causal
     if dtype == torch.bfloat16:   # (the Python wrapper of the rotation pass takes bf16 only)
         assert torch.equal(outs[1][3], pkg.rope_rotate(k, c, s))
         assert torch.equal(outs[1][2], pkg.rope_rotate(q, c, s, scale=scale * math.log2(math.e)))
+
+
+# Shapes whose forward cuts query blocks into pieces: inside and across blocks and heads, waves whose rows see none of a piece's keys, a ragged last
+# block and last key tile, strided views, logits hot enough to move the reference value.  Against the whole-block launch on the same inputs: O differs by
+# the rounding of P and of O to bf16 (2^-9 each, per row independent: 2-norm below 2^-8; in the fp16 build V is rounded to bf16 as well, alike in both), lse by
+# sums of up to N fp32 terms.  Against the oracle on rows around the cuts.  A query row that is not finite stays its own.
+@pytest.mark.parametrize("scale_mul", [1.0, 6.0])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal", [(1, 2, 2, 2100, 128, True), (1, 1, 1, 3000, 128, False), (1, 1, 1, 4097, 128, True), (1, 2, 1, 3001, 64, False),
+                                                 (2, 1, 1, 8200, 64, True)])
+def test_forward_cut_query_blocks(pkg, B, Hq, Hkv, N, D, causal, dtype, scale_mul):
+    print(f"case B={B} Hq={Hq} Hkv={Hkv} N={N} D={D} causal={causal} {dtype} x{scale_mul}", flush=True)
+    lib, dev, scale = pkg._lib.load(), torch.device("cuda:0"), scale_mul / math.sqrt(D)
+    assert lib.corope_rope_attn_fwd_parts_bytes(B, Hq, N, D, int(causal)) > 0
+    c, s = O.precompute_freqs_cis(D, N)
+    cd, sd = c.to(dev), s.to(dev)
+    q, k, v = (seeded((B, N, h, D), 130 + i).to(dtype).transpose(1, 2) for i, h in enumerate((Hq, Hkv, Hkv)))
+    qd, kd, vd = (t.to(dev) for t in (q, k, v))
+    o, M = pkg.rope_attn_forward_with_lse(qd, kd, vd, causal, scale, cd, sd)
+    qc, kc, vc = (t.contiguous() for t in (qd, kd, vd))
+    o1, M1 = pkg.rope_attn_forward_with_lse(qc, kc, vc, causal, scale, cd, sd)
+    assert torch.equal(o, o1) and torch.equal(M, M1)
+    whole, Mw, k_rot = torch.empty_like(o), torch.empty_like(M), torch.empty_like(kc)
+    kmax = torch.empty(B * Hkv * ((N + 63) // 64), device=dev)
+    st = [(ctypes.c_int64 * 3)(h * N * D, N * D, D) for h in (Hq, Hkv, Hkv)]
+    rc = lib.corope_rope_attn_fwd_strided(qc.data_ptr(), st[0], kc.data_ptr(), st[1], vc.data_ptr(), st[2], cd.data_ptr(), sd.data_ptr(), cd.stride(0),
+                                          whole.data_ptr(), Mw.data_ptr(), None, k_rot.data_ptr(), kmax.data_ptr(), B, Hq, Hkv, N, D, scale, int(causal),
+                                          int(dtype == torch.float16), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, pkg._lib.last_error()
+    torch.cuda.synchronize()
+    diff = ((o.float() - whole.float()).norm() / whole.float().norm()).item()
+    print(f"  O {diff:.2e} and lse {(M - Mw).abs().max().item():.2e} from the whole blocks'")
+    assert not torch.equal(o, whole) and diff <= 2.0 ** -8 and (M - Mw).abs().max() <= 1e-4
+    bad = qc.clone()
+    bad[0, 0, 1025] = float("nan")
+    ob = pkg.attention(bad, kc, vc, causal, scale, cd, sd)
+    rows = torch.ones(N, dtype=torch.bool, device=dev)
+    rows[1025] = False
+    assert torch.isnan(ob[0, 0, 1025]).all() and torch.isfinite(ob[0, :, rows]).all()
+    h = Hq - 1
+    pos = torch.cat([torch.arange(0, 3), torch.arange(250, 262), torch.arange(N // 2 - 4, N // 2 + 4), torch.arange(N - 70, N)])
+    qr, kr = O.apply_rotary_emb(q[-1:, h:h + 1].double(), c.double(), s.double()), O.apply_rotary_emb(k[-1:, -1:].double(), c.double(), s.double())
+    logits = (qr[:, :, pos] @ kr.transpose(-1, -2)) * scale
+    if causal:
+        logits = logits.masked_fill(torch.arange(N)[None, :] > pos[:, None], -math.inf)
+    ref = logits.softmax(-1) @ v[-1:, -1:].double()
+    err = (o[-1:, h:h + 1][:, :, pos.to(dev)].double().cpu() - ref).abs().max().item()
+    print(f"  O max-abs {err:.2e} from the oracle")
+    assert err <= (TOL if scale_mul == 1.0 else TOL_HOT)

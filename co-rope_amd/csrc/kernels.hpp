@@ -223,9 +223,9 @@ hipError_t launch_rope_rotate(const uint16_t* x, const float* cosp, const float*
 hipError_t launch_rope_attn_fwd_prerotated(const FwdParams& p, int D, bool causal, hipStream_t stream);  // needs k_rot
 // the same with 64 query rows per wave, one wave per SIMD (D = 128)
 hipError_t launch_rope_attn_fwd_prerotated_rows64(const FwdParams& p, int D, bool causal, hipStream_t stream);
-// head dim 256 (bf16): 32 query rows per wave, one wave per SIMD, 32-key tiles
 // bytes of FwdParams::parts with which the forward on rotated keys (with key-norm maxima) cuts query blocks; 0: it is faster without
 int64_t fwd_parts_bytes(int B, int H, int N, int D, bool causal);
+// head dim 256 (bf16): 32 query rows per wave, one wave per SIMD, 32-key tiles
 hipError_t launch_rope_attn_fwd_prerotated_pipe256(const FwdParams& p, bool causal, hipStream_t stream);
 // head dim 128 in that form (128-row items, 32-key tiles), two workgroups per compute unit
 hipError_t launch_rope_attn_fwd_prerotated_pipe32x2(const FwdParams& p, bool causal, hipStream_t stream);

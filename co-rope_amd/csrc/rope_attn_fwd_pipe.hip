@@ -417,7 +417,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
         // above 2^-kPipeLift, far inside fp32 / bf16 range, however often the block runs.
         m_true = fmaxf(m_true, half_max(mt));
         float m_new = fmaxf(m_run, fmaxf(m_true, fminf(lift_target, m_true + kPipeLift)));
-        if constexpr (CUT) m_new = fmaxf(m_new, -1e30f);   // (a row that sees no key of the piece so far)
+        if constexpr (CUT) m_new = m_new == -INFINITY ? 0.f : m_new;   // (a row that sees no key of this tile sees none of the piece's later ones)
         const float alpha = fast_exp2(m_run - m_new);   // m_new is finite: every row sees key 0 of tile 0
         l_run = (l_run + lsum) * alpha;
         lsum = 0.f;

@@ -330,6 +330,20 @@ def test_single_launch_kernel_on_a_rotated_key_copy(pkg, B, H, Hkv, N, D, causal
         assert torch.equal(outs[1][2], pkg.rope_rotate(q, c, s, scale=scale * math.log2(math.e)))
 
 
+def _whole_blocks(pkg, q, k, v, cos, sin, scale, causal):
+    """The forward on rotated keys without scratch for pieces: O and lse."""
+    (B, Hq, N, D), Hkv = q.shape, k.shape[1]
+    o, lse, k_rot = torch.empty_like(q), torch.empty((B, Hq, N), device=q.device), torch.empty_like(k)
+    kmax = torch.empty(B * Hkv * ((N + 63) // 64), device=q.device)
+    st = [(ctypes.c_int64 * 3)(h * N * D, N * D, D) for h in (Hq, Hkv, Hkv)]
+    rc = pkg._lib.load().corope_rope_attn_fwd_strided(q.data_ptr(), st[0], k.data_ptr(), st[1], v.data_ptr(), st[2], cos.data_ptr(), sin.data_ptr(), cos.stride(0),
+                                                      o.data_ptr(), lse.data_ptr(), None, k_rot.data_ptr(), kmax.data_ptr(), B, Hq, Hkv, N, D, scale, int(causal),
+                                                      int(q.dtype == torch.float16), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, pkg._lib.last_error()
+    torch.cuda.synchronize()
+    return o, lse
+
+
 # Shapes whose forward cuts query blocks into pieces: inside and across blocks and heads, waves whose rows see none of a piece's keys, a ragged last
 # block and last key tile, strided views, logits hot enough to move the reference value.  Against the whole-block launch on the same inputs: O differs by
 # the rounding of P and of O to bf16 (2^-9 each, per row independent: 2-norm below 2^-8; in the fp16 build V is rounded to bf16 as well, alike in both), lse by
@@ -350,14 +364,7 @@ def test_forward_cut_query_blocks(pkg, B, Hq, Hkv, N, D, causal, dtype, scale_mu
     qc, kc, vc = (t.contiguous() for t in (qd, kd, vd))
     o1, M1 = pkg.rope_attn_forward_with_lse(qc, kc, vc, causal, scale, cd, sd)
     assert torch.equal(o, o1) and torch.equal(M, M1)
-    whole, Mw, k_rot = torch.empty_like(o), torch.empty_like(M), torch.empty_like(kc)
-    kmax = torch.empty(B * Hkv * ((N + 63) // 64), device=dev)
-    st = [(ctypes.c_int64 * 3)(h * N * D, N * D, D) for h in (Hq, Hkv, Hkv)]
-    rc = lib.corope_rope_attn_fwd_strided(qc.data_ptr(), st[0], kc.data_ptr(), st[1], vc.data_ptr(), st[2], cd.data_ptr(), sd.data_ptr(), cd.stride(0),
-                                          whole.data_ptr(), Mw.data_ptr(), None, k_rot.data_ptr(), kmax.data_ptr(), B, Hq, Hkv, N, D, scale, int(causal),
-                                          int(dtype == torch.float16), torch.cuda.current_stream().cuda_stream)
-    assert rc == 0, pkg._lib.last_error()
-    torch.cuda.synchronize()
+    whole, Mw = _whole_blocks(pkg, qc, kc, vc, cd, sd, scale, causal)
     diff = ((o.float() - whole.float()).norm() / whole.float().norm()).item()
     print(f"  O {diff:.2e} and lse {(M - Mw).abs().max().item():.2e} from the whole blocks'")
     assert not torch.equal(o, whole) and diff <= 2.0 ** -8 and (M - Mw).abs().max() <= 1e-4
@@ -377,3 +384,21 @@ def test_forward_cut_query_blocks(pkg, B, Hq, Hkv, N, D, causal, dtype, scale_mu
     err = (o[-1:, h:h + 1][:, :, pos.to(dev)].double().cpu() - ref).abs().max().item()
     print(f"  O max-abs {err:.2e} from the oracle")
     assert err <= (TOL if scale_mul == 1.0 else TOL_HOT)
+
+
+# Every logit below -1e31 (base 2), one product each so that every difference of scores is exact, and one key ahead of all others by more than any exponent: a
+# row's reference value has to follow its scores down in every piece, and O is that key's v with nothing rounded for the rows that see it.  No rotation.
+@pytest.mark.parametrize("N,causal", [(4097, True), (3000, False)])
+def test_forward_cut_query_blocks_at_very_negative_logits(pkg, N, causal):
+    dev, D, best = torch.device("cuda:0"), 128, 5
+    assert pkg._lib.load().corope_rope_attn_fwd_parts_bytes(1, 1, N, D, int(causal)) > 0
+    c, s = torch.ones(N, D // 2, device=dev), torch.zeros(N, D // 2, device=dev)
+    q, k, v = torch.zeros(1, 1, N, D), torch.zeros(1, 1, N, D), seeded((1, 1, N, D), 140)
+    q[..., 3], k[..., 3] = 2.0 ** 52, -1.5 * 2.0 ** 51
+    k[:, :, best, 3] = -(2.0 ** 51)
+    q, k, v = (t.to(dev, torch.bfloat16) for t in (q, k, v))
+    o, lse = pkg.rope_attn_forward_with_lse(q, k, v, causal, 1.0, c, s)
+    whole, lse_w = _whole_blocks(pkg, q, k, v, c, s, 1.0, causal)
+    first = best if causal else 0
+    assert lse.max() < -1e31 and torch.equal(lse, lse_w)
+    assert torch.equal(o[:, :, first:], v[:, :, best:best + 1].expand(-1, -1, N - first, -1)) and torch.equal(o[:, :, :first], whole[:, :, :first])

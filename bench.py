@@ -423,24 +423,26 @@ def bench_corope(args):
         ws_bytes = groups * one
         by_workspace[f"{groups} of {B * Hkv} groups per pass, {ws_bytes / 2**30:.2f} GiB"] = round(time_bwd(), 4)
     ws_bytes = full_bytes
-    # VALU roofline: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz issue slots/s.  Issue slots per (sin, cos) pair, the same in the forward, the
-    # backward's scores kernel and its dk kernel: phase 1, reduced for half of the pairs at this N and theta (0.5), two
-    # transcendentals at half rate (measured on this chip: v_sin_f32 16.0 T lanes/s against 33.3 for v_fma_f32), so 2 slots
-    # each, and 4 to rotate; the dot products run on the matrix cores
-    fwd_instr, bwd_instr = pairs * 9.5, 2 * pairs * 9.5
+    # VALU roofline: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz issue slots/s.  Issue slots per (sin, cos) pair that is evaluated: phase 1, one
+    # more where it is reduced, two transcendentals at half rate (measured on this chip: v_sin_f32 16.0 T lanes/s against 33.3 for
+    # v_fma_f32), so 2 slots each, and 4 to rotate; the dot products run on the matrix cores.  The forward and the backward's dk
+    # kernel evaluate the half of the pairs that turns fast (the others are polynomials on the matrix cores), the scores kernel all;
+    # reduced are half of the forward's, all of dk's and half of the scores kernel's at this N and theta
+    fwd_pairs, bwd_pairs = pairs / 2, pairs + pairs / 2
+    fwd_instr, bwd_instr = fwd_pairs * 9.5, pairs * 9.5 + pairs / 2 * 10
     out = {"metric": "Co-RoPE GQA fwd, B2 Hq32 Hkv8 N4096 D128 causal", "value": round(flops / (ms * 1e-3) * 1e-12, 2),
            "unit": "TFLOP/s (attention-equivalent)", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
            "ms_per_step": round(ms, 4), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
            "settle_steps": settle_steps,
            "dtype": "bf16", "data": "synthetic",
            "config": {"workload": "C5: Co-RoPE GQA attention fwd B2 Hq32 Hkv8 N4096 D128 causal bf16", "theta": 10000.0},
-           "sincos_pairs_per_s": round(pairs / (kms * 1e-3), 1), "kernel_ms": round(kms, 4),
+           "sincos_pairs_per_s": round(fwd_pairs / (kms * 1e-3), 1), "kernel_ms": round(kms, 4),
            "roofline": {"bound": "valu", "kernel": "corope_gqa_fwd", "achieved": round(fwd_instr / (kms * 1e-3) * 1e-12, 3),
                         "peak": round(256 * 4 * 16 * 2.4e9 * 1e-12, 3), "unit": "T issue slots/s",
                         "frac": round(fwd_instr / (kms * 1e-3) / (256 * 4 * 16 * 2.4e9), 4),
                         "traffic": HBM_TRAFFIC_BYTES[("c5", "corope_gqa_fwd")]},
            "backward": {"ms": round(bms, 4), "steps": bsteps, "workspace_gib": round(ws_bytes / 2**30, 2), "ms_by_workspace": by_workspace,
-                        "sincos_pairs_per_s": round(2 * pairs / (bms * 1e-3), 1),
+                        "sincos_pairs_per_s": round(bwd_pairs / (bms * 1e-3), 1),
                         "tflops_attention_equivalent": round(2.5 * flops / (bms * 1e-3) * 1e-12, 2),
                         "roofline": {"bound": "valu", "kernel": "corope_gqa_bwd (5 launches)",
                                      "achieved": round(bwd_instr / (bms * 1e-3) * 1e-12, 3),

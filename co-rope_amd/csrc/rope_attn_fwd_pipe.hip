@@ -61,9 +61,11 @@ struct FwdPipeCfg {
   static_assert(kLdsBytes <= 160 * 1024, "LDS of a compute unit");
 };
 
-// A slot of a piece's results: NW x 32 rows x D of O as the accumulators lie ([32-row block][register quad][lane]), then the rows' log-sum-exps.
+// A slot of a piece's results: NW x 32 rows x D of the unnormalised O as the accumulators lie ([32-row block][register quad][lane]), then the rows'
+// reference values m (-inf where the piece shows the row no key), then their sums l.  (m + log2 l in one number would be rounded to the
+// spacing of floats at the logits' size, and a piece's weight with it.)
 template <int D, int NW>
-constexpr int64_t kFwdSlotFloats = (int64_t)NW * 32 * (D + 1);
+constexpr int64_t kFwdSlotFloats = (int64_t)NW * 32 * (D + 2);
 
 // P^T is a bf16 operand in both builds (its unnormalised values span up to 2^kPipeMargin, more binary orders than fp16
 // has), so the product O^T += V^T P^T is a bf16 product in both: in the fp16 build the V tile is converted to bf16 while
@@ -115,7 +117,7 @@ __device__ __forceinline__ float wave_reduce_max(float x) { return wave_max(x); 
 // on the diagonal tiles, and only keeps staging its share of those tiles.
 //
 // CUT: a workgroup takes a piece of the list of all key tiles instead (QueryWork); a piece of an item starts its own softmax and leaves its
-// normalised O and log-sum-exp in a slot, which rope_attn_fwd_join_kernel weighs.
+// O, reference values and sums in a slot, which rope_attn_fwd_join_kernel brings to one reference and adds.
 template <int D, bool CAUSAL, int NW, bool CUT = false>
 __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) void rope_attn_fwd_pipe_kernel(FwdParams p) {
   using Cfg = FwdPipeCfg<D, NW>;
@@ -418,7 +420,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
         m_true = fmaxf(m_true, half_max(mt));
         float m_new = fmaxf(m_run, fmaxf(m_true, fminf(lift_target, m_true + kPipeLift)));
         if constexpr (CUT) m_new = m_new == -INFINITY ? 0.f : m_new;   // (a row that sees no key of this tile sees none of the piece's later ones)
-        const float alpha = fast_exp2(m_run - m_new);   // m_new is finite: every row sees key 0 of tile 0
+        const float alpha = fast_exp2(m_run - m_new);   // m_new is finite: every row sees key 0 of tile 0, and a piece that starts later has the line above
         l_run = (l_run + lsum) * alpha;
         lsum = 0.f;
 #pragma unroll
@@ -468,14 +470,18 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
       __syncthreads();
     }
     if (CUT && !(t_begin == 0 && n_tiles == tiles_of(mb))) {   // workgroup-uniform: a piece of the item
-      const float l_tot = half_sum(l_run + lsum), inv = l_tot > 0.f ? 1.f / l_tot : 0.f;   // (0: no key seen)
+      const float l_tot = half_sum(l_run + lsum);
       const int l = opaque_lane();
       float* slot = p.parts + piece_slot(items.share(), t_begin == 0) * kFwdSlotFloats<D, NW>;
 #pragma unroll
       for (int i = 0; i < NDB * 4; ++i)
         *reinterpret_cast<f32x4*>(slot + (rb * NDB * 4 + i) * 4 * kWave + 4 * l) =
-            f32x4{oacc[i / 4][4 * (i % 4)] * inv, oacc[i / 4][4 * (i % 4) + 1] * inv, oacc[i / 4][4 * (i % 4) + 2] * inv, oacc[i / 4][4 * (i % 4) + 3] * inv};
-      if (lh == 0) slot[NW * 32 * D + rb * 32 + lq] = m_run + fast_log2(l_tot);   // -inf where no key is seen
+            f32x4{oacc[i / 4][4 * (i % 4)], oacc[i / 4][4 * (i % 4) + 1], oacc[i / 4][4 * (i % 4) + 2], oacc[i / 4][4 * (i % 4) + 3]};
+      if (lh == 0) {
+        float* stat = slot + NW * 32 * D + rb * 32 + lq;
+        stat[0] = l_tot == 0.f ? -INFINITY : m_run;
+        stat[NW * 32] = l_tot;
+      }
     } else {
       const float l_tot = half_sum(l_run + lsum);
       store_rows_via_wave_tile<D>(oacc, p.o + (int64_t)bh * N * D, m0 + rb * 32, N, 1.f / l_tot, wave_tile, opaque_lane());
@@ -500,31 +506,33 @@ __global__ __launch_bounds__(D / 16 * kWave) void rope_attn_fwd_join_kernel(FwdP
   const int lane = threadIdx.x % kWave, i = threadIdx.x / kWave, row = mb * BLOCK_M + rb * 32 + lane % 32;
   if (w0 == w1 || row >= N) return;   // one piece holds all of the item and has written it
   auto slot_of = [&](int w) { return p.parts + piece_slot(w, w == w0) * kFwdSlotFloats<D, NW>; };
-  auto lse_of = [&](int w) { return slot_of(w)[NW * 32 * D + rb * 32 + lane % 32]; };
+  auto stat_of = [&](int w) { return slot_of(w) + NW * 32 * D + rb * 32 + lane % 32; };
   float top = -INFINITY, sum = 0.f;   // (the first piece holds key 0, which every row sees: top is finite)
-  for (int w = w0; w <= w1; ++w) top = fmaxf(top, lse_of(w));
-  for (int w = w0; w <= w1; ++w) sum += fast_exp2(lse_of(w) - top);
-  const float lse = top + fast_log2(sum);
+  for (int w = w0; w <= w1; ++w) top = fmaxf(top, stat_of(w)[0]);
   f32x4 a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
   for (int w = w0; w <= w1; w += 4) {   // eight loads in flight
     f32x4 x[4], y[4];
-    float f[4];
+    float f[4], l[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const float* src = slot_of(min(w + u, w1)) + (rb * 2 * QUADS + i) * 4 * kWave + 4 * lane;
       x[u] = *reinterpret_cast<const f32x4*>(src);
       y[u] = *reinterpret_cast<const f32x4*>(src + QUADS * 4 * kWave);
-      f[u] = fast_exp2(lse_of(min(w + u, w1)) - lse);
+      const float* stat = stat_of(min(w + u, w1));
+      f[u] = fast_exp2(stat[0] - top);
+      l[u] = stat[NW * 32];
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (w + u <= w1) a += x[u] * f[u], b += y[u] * f[u];
+      if (w + u <= w1) a += x[u] * f[u], b += y[u] * f[u], sum += l[u] * f[u];
   }
+  const float inv = 1.f / sum;
+  a *= inv, b *= inv;
   const int col = 8 * i + 4 * (lane / 32);
   uint16_t* out = p.o + ((int64_t)bh * N + row) * D + col;
   *reinterpret_cast<u32x2*>(out) = u32x2{pack_elts(a[0], a[1]), pack_elts(a[2], a[3])};
   *reinterpret_cast<u32x2*>(out + D / 2) = u32x2{pack_elts(b[0], b[1]), pack_elts(b[2], b[3])};
-  if (i == 0 && lane < 32) p.lse[(int64_t)bh * N + row] = lse;
+  if (i == 0 && lane < 32) p.lse[(int64_t)bh * N + row] = top + fast_log2(sum);
 }
 
 // ---- host-side launch -----------------------------------------------------------------------------------------

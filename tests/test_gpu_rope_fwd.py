@@ -402,3 +402,30 @@ def test_forward_cut_query_blocks_at_very_negative_logits(pkg, N, causal):
     first = best if causal else 0
     assert lse.max() < -1e31 and torch.equal(lse, lse_w)
     assert torch.equal(o[:, :, first:], v[:, :, best:best + 1].expand(-1, -1, N - first, -1)) and torch.equal(o[:, :, :first], whole[:, :, :first])
+
+
+# Equal logits over several pieces, so large that a float holds them with no fraction: O is the mean of the v a row sees whatever the offset.  The pieces
+# of a row must be weighed by sums kept apart from their reference values.  P carries 2^-9 of rounding to bf16 (the sums do not), O another, and
+# N fp32 additions up to N 2^-24 of the mean |v|.
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("exponent", [8, 12, 52])   # logits of about 1.4e5, 3.6e7, 4.4e31 (base 2)
+@pytest.mark.parametrize("N,D,causal", [(4097, 128, True), (3000, 128, False), (3001, 64, False)])
+def test_forward_cut_query_blocks_at_equal_large_logits(pkg, N, D, causal, exponent, sign):
+    print(f"case N={N} D={D} causal={causal} 2^{exponent} {sign}", flush=True)
+    dev, H = torch.device("cuda:0"), 128 // D
+    assert pkg._lib.load().corope_rope_attn_fwd_parts_bytes(1, H, N, D, int(causal)) > 0
+    c, s = torch.ones(N, D // 2, device=dev), torch.zeros(N, D // 2, device=dev)
+    q, k, v = torch.zeros(1, H, N, D), torch.zeros(1, H, N, D), seeded((1, H, N, D), 150)
+    q[..., 3], k[..., 3] = 2.0 ** exponent, sign * 1.5 * 2.0 ** exponent
+    q, k, v = (t.to(dev, torch.bfloat16) for t in (q, k, v))
+    o, lse = pkg.rope_attn_forward_with_lse(q, k, v, causal, 1.0, c, s)
+    whole, lse_w = _whole_blocks(pkg, q, k, v, c, s, 1.0, causal)
+    n = torch.arange(1, N + 1, device=dev, dtype=torch.float64)[:, None] if causal else float(N)
+    sums = lambda t: t.cumsum(2) if causal else t.sum(2, keepdim=True).expand_as(t)
+    ref, size = sums(v.double()) / n, sums(v.double().abs()) / n
+    bar = 2.0 ** -8 * ref.abs() + N * 2.0 ** -24 * size
+    for name, x in (("whole", whole), ("cut", o)):
+        err = (x.double() - ref).abs()
+        print(f"  {name}: max-abs {err.max().item():.2e}, {(err / bar).max().item():.2f} of the bar")
+        assert (err <= bar).all(), name
+    assert ((lse - lse_w).abs() <= 2.0 ** -22 * lse_w.abs()).all()

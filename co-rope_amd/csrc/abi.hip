@@ -733,24 +733,14 @@ int corope_rope_attn_bwd_f16(const void* q, const void* k, int prerotated, const
   return launch_status(what, corope_f16::launch_bwd_dq(p, D, causal != 0, st));
 }
 
-int corope_rope_attn_fwd_strided(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,
-                                 const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin,
-                                 int64_t freq_row_stride, void* o, float* lse, void* q_rot, void* k_rot, float* tile_kmax, int B,
-                                 int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16, void* stream) {
-  return corope_rope_attn_fwd_cut(q, q_strides, k, k_strides, v, v_strides, freqs_cos, freqs_sin, freq_row_stride, o, lse, q_rot, k_rot, tile_kmax,
-                                  B, H, Hkv, N, D, sm_scale, causal, fp16, nullptr, 0, stream);
-}
+}  // extern "C" (reopened below)
 
-int64_t corope_rope_attn_fwd_parts_bytes(int B, int H, int N, int D, int causal) {
-  if (corope_rope_attn_check(B, H, N, D, D, 1.f, 0)) return -1;
-  return corope::fwd_parts_bytes(B, H, N, D, causal != 0);
-}
+namespace {
 
-int corope_rope_attn_fwd_cut(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,
-                             const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin, int64_t freq_row_stride, void* o, float* lse,
-                             void* q_rot, void* k_rot, float* tile_kmax, int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
-                             void* parts, int64_t parts_bytes, void* stream) {
-  const char* what = "rope_attn_fwd_strided";
+int rope_attn_fwd_strided_impl(const char* what, const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,
+                               const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin, int64_t freq_row_stride, void* o,
+                               float* lse, void* q_rot, void* k_rot, float* tile_kmax, int B, int H, int Hkv, int N, int D, float sm_scale,
+                               int causal, int fp16, void* parts, int64_t parts_bytes, void* stream) {
   if (Hkv <= 0 || H % Hkv != 0) return fail(COROPE_E_BADARG, "%s: H=%d is not a multiple of Hkv=%d", what, H, Hkv);
   int rc = corope_rope_attn_check(B, H, N, D, freq_row_stride, sm_scale, 0);
   if (rc) return rc;
@@ -805,6 +795,31 @@ int corope_rope_attn_fwd_cut(const void* q, const int64_t* q_strides, const void
   p.q_rot_out = static_cast<uint16_t*>(q_rot);
   return launch_status(what, fp16 ? corope_f16::launch_rope_attn_fwd_prerotated(p, D, causal != 0, st)
                                   : corope::launch_rope_attn_fwd_prerotated(p, D, causal != 0, st));
+}
+
+}  // namespace
+
+extern "C" {
+
+int corope_rope_attn_fwd_strided(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,
+                                 const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin,
+                                 int64_t freq_row_stride, void* o, float* lse, void* q_rot, void* k_rot, float* tile_kmax, int B,
+                                 int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16, void* stream) {
+  return rope_attn_fwd_strided_impl("rope_attn_fwd_strided", q, q_strides, k, k_strides, v, v_strides, freqs_cos, freqs_sin, freq_row_stride, o, lse,
+                                    q_rot, k_rot, tile_kmax, B, H, Hkv, N, D, sm_scale, causal, fp16, nullptr, 0, stream);
+}
+
+int64_t corope_rope_attn_fwd_parts_bytes(int B, int H, int N, int D, int causal) {
+  if (corope_rope_attn_check(B, H, N, D, D, 1.f, 0)) return -1;
+  return corope::fwd_parts_bytes(B, H, N, D, causal != 0);
+}
+
+int corope_rope_attn_fwd_cut(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,
+                             const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin, int64_t freq_row_stride, void* o, float* lse,
+                             void* q_rot, void* k_rot, float* tile_kmax, int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
+                             void* parts, int64_t parts_bytes, void* stream) {
+  return rope_attn_fwd_strided_impl("rope_attn_fwd_cut", q, q_strides, k, k_strides, v, v_strides, freqs_cos, freqs_sin, freq_row_stride, o, lse, q_rot,
+                                    k_rot, tile_kmax, B, H, Hkv, N, D, sm_scale, causal, fp16, parts, parts_bytes, stream);
 }
 
 int corope_rope_freqs(float* freqs_cos, float* freqs_sin, int n_pos, int D, int width, int64_t freq_row_stride, int pos0,

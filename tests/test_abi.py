@@ -267,6 +267,29 @@ def test_strided_forward_argument_checks(pkg):
     assert lib.corope_rope_attn_fwd_strided(ok, good, ok, good, ok + 2, good, *tail) == -3
 
 
+def test_cut_forward_argument_checks(pkg):
+    """Scratch that is too small or misaligned is refused before any launch (it is all that keeps the pieces' slots in range), under the
+    entry point's own name."""
+    lib = pkg._lib.load()
+    ok = 4096
+    B, H, N, D = 1, 8, 4096, 128   # few heads and long sequences: cut
+    need = lib.corope_rope_attn_fwd_parts_bytes(B, H, N, D, 1)
+    assert need > 0 and need % 16 == 0
+    assert lib.corope_rope_attn_fwd_parts_bytes(2, 32, 4096, 128, 1) == 0 and lib.corope_rope_attn_fwd_parts_bytes(1, 8, 4096, 96, 1) == -1
+    good = (ctypes.c_int64 * 3)(H * N * D, N * D, D)
+    narrow = (ctypes.c_int64 * 3)(H * N * D, N * D, D // 2)
+
+    def call(q_strides=good, q_rot=None, k_rot=ok, H=H, parts=ok, nbytes=need):
+        return lib.corope_rope_attn_fwd_cut(ok, q_strides, ok, good, ok, good, ok, ok, D, ok, ok, q_rot, k_rot, ok, B, H, 8, N, D, 1.0, 1, 0,
+                                            parts, nbytes, None)
+
+    for args, code, text in ((dict(nbytes=need - 1), -1, "parts"), (dict(nbytes=0), -1, "parts"), (dict(parts=ok + 8), -3, "aligned"),
+                             (dict(q_strides=None), -1, "null strides"), (dict(q_strides=narrow), -1, "stride"),
+                             (dict(k_rot=None, q_rot=ok), -1, "q_rot without k_rot"), (dict(H=9), -1, "multiple")):
+        assert call(**args) == code, args
+        assert text in pkg._lib.last_error() and pkg._lib.last_error().startswith("rope_attn_fwd_cut"), (args, pkg._lib.last_error())
+
+
 def test_alias_names_the_same_modules():
     """``corope_amd`` is an alias of the package in the directory ``co-rope_amd``: importing a submodule through either
     name gives the one module object whose globals the package's functions read (a second copy would have thresholds

@@ -1005,16 +1005,36 @@ __device__ __forceinline__ u32x4 pack_rest8(const float (&x)[8], u32x4 first) {
   return pack_elts8(r);
 }
 
+// The slow pairs' queries of a column, in its four lanes.  fp16: a query of 60000 would leave fp16's range on its way round, and the coefficients
+// of one of 1e-6 would have a handful of bits left; so they are scaled by the power of two that brings the largest of them to 2^14 .. 2^15.
+// Returns its inverse.
+template <int LOW>
+__device__ __forceinline__ float corope_low_queries(u32x4* raw) {
+  static_assert(kEltIsF16, "bf16 has the range");
+  uint32_t top = 0;   // (bit patterns of non-negative numbers order like the numbers)
+#pragma unroll
+  for (int u = 0; u < LOW; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) top = max(top, max(raw[u][e] & 0x7fffu, raw[u][e] >> 16 & 0x7fffu));
+  top = max(top, (uint32_t)__shfl_xor((int)top, 16));
+  top = max(top, (uint32_t)__shfl_xor((int)top, 32));
+  const int shift = 14 - max(-24, (int)(__builtin_bit_cast(uint32_t, elt_lo(top)) >> 23) - 127);   // (no query but zeros: any)
+#pragma unroll
+  for (int u = 0; u < LOW; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) raw[u][e] = pack_elts(ldexpf(elt_lo(raw[u][e]), shift), ldexpf(elt_hi(raw[u][e]), shift));
+  return ldexpf(1.f, -shift);
+}
+
 // B operands of the products above for one column (row, head) per lane, for LOW trailing groups of 16 pairs.
 template <int LOW>
 struct CoropeLowOps {
   static_assert(LOW == 1 || LOW == 2, "a class 0 group and perhaps a class 1 group behind it");
-  // (an fp16 query of 60000 would leave fp16's range on its way round: halved, and the scores doubled again)
-  static constexpr float kScale = kEltIsF16 ? 0.5f : 1.f;
   u32x4 c[5], c0r, c1r;   // class 0: powers 0..4, remainders of powers 0 and 1
   u32x4 d[3], d0r;        // class 1
 
-  // raw: the column's query, groups in operand order; turns: w / 2 pi of this lane's pairs; mid: the chunk's middle
+  // raw: the column's query (fp16: as corope_low_queries leaves it), groups in operand order; turns: w / 2 pi of this lane's pairs; mid: the
+  // chunk's middle
   __device__ __forceinline__ void build(const u32x4* raw, const float (*turns)[4], float mid) {
     static_for<LOW>([&](auto u_c) __attribute__((always_inline)) {
       constexpr int u = decltype(u_c)::value;
@@ -1022,7 +1042,7 @@ struct CoropeLowOps {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const uint32_t w1 = raw[u][e / 2], w2 = raw[u][2 + e / 2];
-        const float q1 = (e % 2 ? elt_hi(w1) : elt_lo(w1)) * kScale, q2 = (e % 2 ? elt_hi(w2) : elt_lo(w2)) * kScale;
+        const float q1 = e % 2 ? elt_hi(w1) : elt_lo(w1), q2 = e % 2 ? elt_hi(w2) : elt_lo(w2);
         const float x = __builtin_amdgcn_fractf(mid * turns[u][e]);
         const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
         v[e] = __builtin_fmaf(cs, q1, -(sn * q2));
@@ -1091,7 +1111,6 @@ struct CoropeLowOps {
       if constexpr (LOW > 1) s[b] = mfma16(kf[b][1], d0r, s[b]);
       s[b] = mfma16(kf[b][0], c[0], s[b]);
       if constexpr (LOW > 1) s[b] = mfma16(kf[b][1], d[0], s[b]);
-      if constexpr (kEltIsF16) s[b] *= 1.f / kScale;
     }
   }
 };

@@ -60,7 +60,8 @@ struct CoropeFwdCfg {
   static constexpr int kKStride = D + 8;    // K tile rows: 16 keys read at one column hit 16 different bank groups
   static constexpr int kVStride = D + 16;   // V tile rows: the 4 rows x 32 bytes of a transposing read cover 32 banks once
   static constexpr int kTileElems = kCoropeKeys * (kKStride + kVStride);
-  static constexpr int kDeltaFloats = 4 * R * 16 + (R + 3) / 4 * 4;          // per wave: [16-key block][row][key % 16], [row] the chunk's middle
+  static constexpr int kMids = 4 * R * 16, kUnscales = kMids + (R + 3) / 4 * 4;
+  static constexpr int kDeltaFloats = kUnscales + 16;   // per wave: [16-key block][row][key % 16], [row] the chunk's middle, [column] (corope_low_queries)
   static constexpr int kLdsBytes = 2 * kTileElems * 2 + kCoropeWaves * kDeltaFloats * 4;
   static_assert(2 * kLdsBytes <= 160 * 1024, "two workgroups per compute unit");
 };
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
       }
     }
   };
-  u32x4 qop[NG], lop[NG];   // B operand of the score product (fp16; the low groups' as they are), A operand of the logit product (element type)
+  u32x4 qop[NG], lop[NG];   // B operand of the score product (fp16; the low groups' in the element type), A operand of the logit product (element type)
   {
     const uint16_t* qrow = p.q + ((int64_t)(head0 + chead) * N + min(iw + crow, N - 1)) * D;
     const uint16_t* lrow = p.q + ((int64_t)head0 * N + min(iw + n * R / 16, N - 1)) * D;
@@ -126,6 +127,7 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
 #pragma unroll
       for (int e = 0; e < 4; ++e) qop[u][e] = n >= R * G ? 0u : u < NH ? pack_f16(elt_lo(qop[u][e]), elt_hi(qop[u][e])) : qop[u][e];
   }
+  if constexpr (LOW > 0 && kEltIsF16) dbuf[Cfg::kUnscales + n] = corope_low_queries<LOW>(qop + NH);   // (in LDS: the loop has no register left)
   float turns[NG * 4 / P][P];  // w_d / 2 pi of this lane's columns
 #pragma unroll
   for (int u = 0; u < NG * 4 / P; ++u)
@@ -214,7 +216,7 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
           dbuf[(b * R + r) * 16 + n] = right + (tot[b] - pre[b]);   // gates strictly to the right of the key, up to the diagonal
           right += tot[b];
         }
-        if constexpr (LOW > 0) dbuf[4 * R * 16 + r] = 0.5f * (carry[z] + right);
+        if constexpr (LOW > 0) dbuf[Cfg::kMids + r] = 0.5f * (carry[z] + right);
         carry[z] = right;
       }
     }
@@ -224,8 +226,8 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
     f32x4 sacc[4];
     if constexpr (LOW > 0) {
       CoropeLowOps<LOW> ops;
-      ops.build(qop + NH, turns + NH, dbuf[4 * R * 16 + crow]);
-      const float mid = dbuf[4 * R * 16 + crow];
+      ops.build(qop + NH, turns + NH, dbuf[Cfg::kMids + crow]);
+      const float mid = dbuf[Cfg::kMids + crow];
       constexpr int NB = 2;   // blocks at a time (with all four the kernel spills at D = 128)
 #pragma unroll
       for (int b0 = 0; b0 < 4; b0 += NB) {
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
         }
         ops.scores(kf, y, s);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) sacc[b0 + b] = s[b];
+        for (int b = 0; b < NB; ++b) sacc[b0 + b] = kEltIsF16 ? s[b] * dbuf[Cfg::kUnscales + n] : s[b];
       }
       if (c > 0) fetch(c - 1, std::false_type{});   // (behind the polynomial, which needs the registers)
     } else {

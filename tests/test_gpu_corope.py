@@ -187,3 +187,25 @@ def test_corope_forward_slow_pairs(pkg, B, Hq, Hkv, N, D, theta, gates):
         err = (o[hs].double().cpu() - ref).abs()
         print(f"  O max-abs {err.max():.3e} mean-abs {err.mean():.3e}")
         assert err.max() <= (4e-3 if theta > 9222 else TOL)
+
+
+@pytest.mark.parametrize("size", [1e-6, 3e-5, 1.1e4])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 32, 8, 385, 128), (1, 64, 16, 449, 128), (1, 32, 32, 260, 128), (2, 64, 16, 257, 64)])
+def test_corope_forward_fp16_query_sizes(pkg, B, Hq, Hkv, N, D, size):
+    """fp16 queries near either end of the type's range, with an sm_scale that makes the logits those of ordinary ones: the rotation must
+    keep fp16's bits whatever the queries' size.  Same bar as with ordinary queries (test_corope_forward_slow_pairs, |O - O64| <= 4e-3), on
+    the queries as fp16 holds them (1e-6: to five bits)."""
+    print(f"case B={B} Hq={Hq} Hkv={Hkv} N={N} D={D} size={size}", flush=True)
+    G, scale = Hq // Hkv, 1 / math.sqrt(D) / size
+    q, k, v = (torch.randn(B, h, N, D, generator=torch.Generator().manual_seed(60 + i)) for i, h in enumerate((Hq, Hkv, Hkv)))
+    q, k, v = (q * size).half(), k.half(), v.half()
+    assert torch.isfinite(q).all()
+    dev = torch.device("cuda:0")
+    o = pkg.corope_attention(q.to(dev), k.to(dev), v.to(dev), True, scale, 10000.0)
+    torch.cuda.synchronize()
+    for b, kv in ((0, 0), (B - 1, Hkv - 1)):
+        hs, sl = (slice(b, b + 1), slice(kv * G, (kv + 1) * G)), (slice(b, b + 1), slice(kv, kv + 1))
+        ref = C.corope_gqa_forward_rows(q[hs].double(), k[sl].double(), v[sl].double(), True, scale, 10000.0, torch.arange(N), torch.float64)
+        err = (o[hs].double().cpu() - ref).abs()
+        print(f"  O max-abs {err.max():.3e} mean-abs {err.mean():.3e}")
+        assert err.max() <= 4e-3

@@ -40,8 +40,7 @@
 // multiplies, two multiply-adds that round to fp16 -- and about 760 per chunk, wave and 16 columns for everything else, of which the slow
 // pairs take 350 where rotating them took 1220 with four rows per wave.
 // Measured, every pair rotated -> slow pairs as polynomials, the rows of a wave unrolled and the workgroups of a short launch dealt in turn:
-// B2 Hq32 Hkv8 N4096 D128 3.20 -> 2.26 ms, fp16 B1 Hq32 Hkv8 N1111 D128 143 -> 103 us, B2 Hq8 Hkv8 N3500 D64 1219 -> 780 us; of the first, 3.20 ->
-// 2.32 the polynomials, 2.32 -> 2.23 the unrolled rows.
+// B2 Hq32 Hkv8 N4096 D128 3.20 -> 2.23 ms (2.32 before the rows were unrolled), fp16 B1 Hq32 Hkv8 N1111 D128 143 -> 103 us, B2 Hq8 Hkv8 N3500 D64 1219 -> 780 us.
 #include <algorithm>
 
 #include "common.hpp"
@@ -268,18 +267,24 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
           k2[u][2 * e + 1] = elt_hi(w2);
         }
       const f32x4 low = sacc[b];
-      float delta[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) delta[r] = dbuf[(b * R + r) * 16 + n];
-#pragma unroll
+      // The rows are unrolled, which hides a row's chain behind the next row's: bf16 B2 Hq32 Hkv8 N4096 D128 2.32 -> 2.23 ms.  fp16 has no registers for
+      // that (84 to 134 of them went through scratch): with eight rows at D = 128 the scheduler is kept from mixing them, and where every pair
+      // is rotated they stay a loop, as do two rows in bf16.  All unrolled -> this, us: fp16 D128 N4096 Hq32 Hkv32 5523 -> 3674 and Hkv16 2787 -> 1865;
+      // theta = 1000 (every pair rotated) Hkv32 6815 -> 5770, Hkv8 1740 -> 1557, Hkv4 902 -> 880, bf16 Hkv4 918 -> 911.
+      constexpr bool kRowByRow = kEltIsF16 && D == 128 && LOW > 0 && R == 8;
+      constexpr int kUnroll = LOW == 0 && (kEltIsF16 || R == 2) ? 1 : R;
+      float delta = dbuf[b * R * 16 + n];
+#pragma unroll kUnroll
       for (int r = 0; r < R; ++r) {
+        const float delta_r = delta;
+        delta = dbuf[(b * R + min(r + 1, R - 1)) * 16 + n];
         f32x4 acc = low;
         static_for<UNITS>([&](auto u_c) __attribute__((always_inline)) {
           constexpr int u = decltype(u_c)::value;
           _Float16 y[2 * P];
 #pragma unroll
           for (int e = 0; e < P; ++e) {
-            const float x = corope_phase<(P / 4 * u < REDUCED)>(delta[r] * turns[u][e]);
+            const float x = corope_phase<(P / 4 * u < REDUCED)>(delta_r * turns[u][e]);
             const float sn = __builtin_amdgcn_sinf(x), cs = __builtin_amdgcn_cosf(x);
             y[e] = (_Float16)__builtin_fmaf(cs, k1[u][e], sn * k2[u][e]);
             y[P + e] = (_Float16)__builtin_fmaf(cs, k2[u][e], -(sn * k1[u][e]));
@@ -294,6 +299,7 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
         });
 #pragma unroll
         for (int e = 0; e < 4; ++e) sacc[b][e] = crow == r ? acc[e] : sacc[b][e];
+        if constexpr (kRowByRow) __builtin_amdgcn_sched_barrier(0);
       }
     });
 

@@ -1,5 +1,9 @@
-"""The build's check of asm-issued matrix-core instructions (co-rope_amd/check_isa.py), on small pieces of assembly."""
+"""The build's check of asm-issued matrix-core instructions (co-rope_amd/check_isa.py), on small pieces of assembly, and what the compiler noted
+of the kernels in the built library."""
 import importlib
+import re
+
+import pytest
 
 check = importlib.import_module("co-rope_amd.check_isa").check_asm_mfma
 
@@ -63,3 +67,26 @@ def test_sources_with_asm_matrix_instructions_are_found():
     checked = {s for s in build.SOURCES if build.isa_checked(s)}
     assert {"rope_attn_fwd_pipe.hip", "rope_attn_fwd_pipe_acc.hip", "rope_attn_bwd.hip"} <= checked
     assert "rope_rotate.hip" not in checked and "abi.hip" not in checked
+
+
+def _kernels_of_the_library(path):
+    """What the compiler noted of every kernel in a built library: the AMDGPU note (type 32) of each code object, a msgpack map."""
+    msgpack = pytest.importorskip("msgpack")
+    with open(path, "rb") as f:
+        data = f.read()
+    kernels = {}
+    for m in re.finditer(rb"\x07\0\0\0(....)\x20\0\0\0AMDGPU\0\0", data, re.S):
+        note = msgpack.unpackb(data[m.end():m.end() + int.from_bytes(m.group(1), "little")], strict_map_key=False)
+        for k in note["amdhsa.kernels"]:
+            kernels[k[".name"]] = k
+    return kernels
+
+
+def test_corope_forward_kernels_keep_their_registers():
+    """None of the Co-RoPE forward's forms sends more than a handful of registers through scratch memory (with 84 and more, in the loop over
+    rows, they took up to half as long again)."""
+    lib = importlib.import_module("co-rope_amd._lib").LIB_PATH
+    kernels = {n: k for n, k in _kernels_of_the_library(lib).items() if "corope_gqa_fwd_kernel" in n}
+    assert any("corope_f16" in n for n in kernels) and any("corope_f16" not in n for n in kernels)
+    spilled = {n: k[".vgpr_spill_count"] for n, k in kernels.items() if k[".vgpr_spill_count"] > 4}
+    assert not spilled, spilled

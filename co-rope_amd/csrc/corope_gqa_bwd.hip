@@ -919,8 +919,10 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
 //   dk_j = sum_i e^(i delta w) sum_h dS^h_ij q^h_i = sum_n sum_{i, h} (x_ij^n dS^h_ij) [ (i w)^n / n! e^(i mid_i w) q^h_i ] :
 // products that contract over rows and heads, one per power.  The bracket is shared by the block's keys: the four waves prepare it once per tile,
 // a wave per head.  Class 0 (|x w| <= 0.68) takes the powers 0 .. 5, class 1 (<= 0.08) 0 .. 2, the last coefficients lowered to spread the
-// remainder: below 1e-5 and 2.2e-5.  Operands are bf16 parts: two of dS and two of the bracket (16 bits) up to the power whose share is so small that
-// one keeps the sum as accurate.  Built for up to five heads a group, whose LDS leaves two workgroups to a compute unit.
+// remainder: below 1e-5 and 2.2e-5.  Operands are bf16 parts: two of dS and two of the bracket (16 bits) up to power 2 (fp16: 3) of class 0 and 1 of
+// class 1; one part of the powers above leaves an error of 4.8e-5 (fp16: 0.9e-5) and 1.6e-5 of dk for the fastest pair with every gate open, beside
+// 1.7e-3 (3e-4) of its rounding.  (With one part from power 2, fp16 3, and class 1's power 1 on it was 2.4e-4, 4.8e-5 and 1.1e-4.)  Built for up
+// to five heads a group (fp16: four), whose LDS leaves two workgroups to a compute unit.
 // What bounds it: the vector units, 9 or 10 issue slots per (row, key, pair) that is rotated.  Measured with the gate path moved: B2 Hq32 Hkv8 N4096 D128
 // forward + backward 15.0 -> 14.6 ms, B2 Hq8 Hkv2 N512 D64 133 -> 130.5 us; with the slow pairs as products the former 13.43 -> 12.70 ms, error of
 // dk against 64 bits 1.68e-3 (bf16) and 3.18e-4 (fp16) as before.
@@ -943,7 +945,7 @@ struct CoropeDkCfg {
   static constexpr int kMatBytes = kDkRows * kMats * kDkKeys * 4;
   static constexpr int kQBytes = kDkRows * D * 8 * 2;                       // [row][column][8 heads] bf16
   // slow pairs: [part][head][column][row] bf16, the parts of class 0, then of class 1; the rows' reference values of delta behind them
-  static constexpr int kParts0 = kEltIsF16 ? 9 : 8, kParts1 = kEltIsF16 ? 5 : 4;
+  static constexpr int kParts0 = kEltIsF16 ? 10 : 9, kParts1 = 5;
   static constexpr int kSlowElems = (LOW > 0 ? kParts0 : 0) * G * 32 * kDkRows + (LOW > 1 ? kParts1 : 0) * G * 32 * kDkRows;
   static constexpr int kLdsBytes = kMatBytes + kQBytes + kSlowElems * 2 + (LOW > 0 ? kDkRows * 4 : 0);
 };
@@ -1100,9 +1102,9 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
               times_iw(1.f);
               put(true);
               times_iw(a2);
-              put(kEltIsF16);
+              put(true);
               times_iw(1.f / (6.f * a2));
-              put(false);
+              put(kEltIsF16);
               times_iw(6.f * a4);
               put(false);
               times_iw(a5 / a4);
@@ -1110,7 +1112,7 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
             } else {                  // cos z ~ 1 - z^2 / 2, sin z ~ a1 z
               constexpr float a1 = 1.f - kDkLow1 * kDkLow1 / 8.f;
               times_iw(a1);
-              put(kEltIsF16);
+              put(true);
               times_iw(0.5f / a1);
               put(false);
             }
@@ -1186,27 +1188,27 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
             slow[u] = mfma32_bf16(lo, b, slow[u]);
             slow[u] = mfma32_bf16(hi, b, slow[u]);
           };
-          constexpr int F = kEltIsF16 ? 1 : 0, C1 = Cfg::kParts0;
+          constexpr int C1 = Cfg::kParts0, F = kEltIsF16 ? 1 : 0;
           split();
           full(0, 0);
           if constexpr (LOW > 1) full(1, C1);
           times_y();
           split();
           full(0, 2);
-          if constexpr (LOW > 1) {
-            if constexpr (kEltIsF16) full(1, C1 + 2);
-            else slow[1] = mfma32_bf16(hi, part(C1 + 2), slow[1]);
-          }
+          if constexpr (LOW > 1) full(1, C1 + 2);
           times_y();
           split();
-          if constexpr (kEltIsF16) full(0, 4);
-          else slow[0] = mfma32_bf16(hi, part(4), slow[0]);
-          if constexpr (LOW > 1) slow[1] = mfma32_bf16(hi, part(C1 + 3 + F), slow[1]);
+          full(0, 4);
+          if constexpr (LOW > 1) slow[1] = mfma32_bf16(hi, part(C1 + 4), slow[1]);
+          times_y();
+          split();
+          if constexpr (kEltIsF16) full(0, 6);
+          else slow[0] = mfma32_bf16(hi, part(6), slow[0]);
 #pragma unroll
-          for (int n = 3; n < 6; ++n) {
+          for (int n = 4; n < 6; ++n) {
             times_y();
             split();
-            slow[0] = mfma32_bf16(hi, part(n + 2 + F), slow[0]);
+            slow[0] = mfma32_bf16(hi, part(n + 3 + F), slow[0]);
           }
         }
       }
@@ -1345,7 +1347,7 @@ static hipError_t launch_corope_bwd_cfg(const CoropeBwdParams& p, const CoropeBw
   if (dv_shares > 1)
     hipLaunchKernelGGL((corope_bwd_sum_kernel<D, kDvRows>), dim3(n_blocks, n_groups, 8), dim3(256), 0, stream, parts, group_floats, p.dv,
                        p.N, dv_shares, 1.f);
-  constexpr int kLow = D == 128 && CoropeDkCfg<D, G, 2>::kLdsBytes <= 80 * 1024 ? 2 : 0;   // (two workgroups a compute unit: up to five heads)
+  constexpr int kLow = D == 128 && CoropeDkCfg<D, G, 2>::kLdsBytes <= 80 * 1024 ? 2 : 0;   // (two workgroups a compute unit: up to five heads, fp16: four)
   const hipError_t e = corope_low_groups(fr.turns, D) >= 2 ? launch_corope_bwd_dk<D, G, std::min(REDUCED, D / 64 - kLow / 2), kLow>(p, ws, fr, parts, dk_shares, stream)
                                                            : launch_corope_bwd_dk<D, G, REDUCED, 0>(p, ws, fr, parts, dk_shares, stream);
   if (e != hipSuccess) return e;

@@ -418,6 +418,20 @@ def test_seeded_sweep_over_shapes_and_paths(pkg, monkeypatch):
             assert within_bar(a, b, 1.5 * TOL * (math.sqrt(G) if name in ("dK", "dV") else 1.0))[0], (it, name)
 
 
+def _backward_on_whole_blocks(pkg, saved, g, scale, causal):
+    """(dQ, dK, dV) of the launches on rotated operands without scratch for pieces; ``saved``: what the operator's forward kept."""
+    qr, kr, v, o, M, fc, fs = saved
+    (B, Hq, N, D), Hkv = qr.shape, kr.shape[1]
+    g, delta, grads = g.contiguous(), torch.empty_like(M), [torch.empty_like(t) for t in (qr, kr, kr)]
+    rc = pkg._lib.load().corope_rope_attn_bwd_rotated(qr.data_ptr(), kr.data_ptr(), v.data_ptr(), None, o.data_ptr(), g.data_ptr(), None, M.data_ptr(),
+                                                      delta.data_ptr(), fc.data_ptr(), fs.data_ptr(), fc.stride(0), *(t.data_ptr() for t in grads), B, Hq,
+                                                      Hkv, N, D, scale, int(causal), int(qr.dtype == torch.float16), None, 0,
+                                                      torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, pkg._lib.last_error()
+    torch.cuda.synchronize()
+    return grads
+
+
 # Shapes whose dK+dV launch cuts key blocks into pieces (and, last, one that does not): cuts inside and across blocks and heads of
 # a group, a ragged last block, a last piece of one tile, every head dim, v and dO as strided views.
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -426,7 +440,6 @@ def test_seeded_sweep_over_shapes_and_paths(pkg, monkeypatch):
                                               (2, 2, 2, 2049, 128, True), (1, 8, 8, 600, 128, False)])
 def test_backward_cut_key_blocks(pkg, B, Hq, Hkv, N, D, cut, causal, dtype):
     dev = torch.device("cuda:0")
-    assert (pkg._lib.load().corope_rope_attn_bwd_rotated_parts_bytes(B, Hq, Hkv, N, D, int(causal)) > 0) == cut
     G, scale = Hq // Hkv, 1 / math.sqrt(D)
     q, g = (bf16_round(seeded((B, N, Hq, D), 30 + i)).transpose(1, 2) for i in range(2))
     k, v = (bf16_round(seeded((B, N, Hkv, D), 40 + i)).transpose(1, 2) for i in range(2))
@@ -434,8 +447,11 @@ def test_backward_cut_key_blocks(pkg, B, Hq, Hkv, N, D, cut, causal, dtype):
     qd, kd, vd = (t.to(dev, dtype).requires_grad_(True) for t in (q, k, v))
     assert Hkv == 1 or not vd.is_contiguous()
     o = pkg.attention(qd, kd, vd, causal, scale, c.to(dev), s.to(dev))
+    saved = [t.detach() for t in o.grad_fn.saved_tensors]
     grads = torch.autograd.grad(o, (qd, kd, vd), g.to(dev, dtype))
-    torch.cuda.synchronize()
+    # (the launch itself: cut, its sums are in another order)
+    whole = _backward_on_whole_blocks(pkg, saved, g.to(dev, dtype), scale, causal)
+    assert [torch.equal(a, b) for a, b in zip(grads[1:], whole[1:])] == [not cut, not cut]
     kx, vx = k.repeat_interleave(G, dim=1), v.repeat_interleave(G, dim=1)
     ref = O.rope_attn_fwd_bwd_blocked(q.contiguous(), kx, vx, g.contiguous(), causal, scale, c, s)
     rdq, rdk, rdv = ref[2], *(t.reshape(B, Hkv, G, N, D).sum(2) for t in ref[3:5])
@@ -459,20 +475,14 @@ def test_backward_cut_key_blocks(pkg, B, Hq, Hkv, N, D, cut, causal, dtype):
                                                  (2, 1, 1, 4100, 64, True), (1, 2, 2, 2050, 256, True), (1, 1, 1, 1100, 256, False)])
 def test_backward_cut_query_blocks(pkg, B, Hq, Hkv, N, D, causal, dtype):
     print(f"case B={B} Hq={Hq} Hkv={Hkv} N={N} D={D} causal={causal} {dtype}", flush=True)
-    lib, dev, scale = pkg._lib.load(), torch.device("cuda:0"), 1 / math.sqrt(D)
+    dev, scale = torch.device("cuda:0"), 1 / math.sqrt(D)
     c, s = (t.to(dev) for t in O.precompute_freqs_cis(D, N))
     q, k, v = (seeded((B, N, h, D), 110 + i).to(dev, dtype).transpose(1, 2).requires_grad_(True) for i, h in enumerate((Hq, Hkv, Hkv)))
     g = seeded((B, N, Hq, D), 113).to(dev, dtype).transpose(1, 2)
     out = pkg.attention(q, k, v, causal, scale, c, s)
-    qr, kr, vs, o, M, fc, fs = (t.detach() for t in out.grad_fn.saved_tensors)
+    saved = [t.detach() for t in out.grad_fn.saved_tensors]
     dq = torch.autograd.grad(out, q, g)[0]
-    delta, gc = torch.empty_like(M), g.contiguous()
-    whole, dk, dv = (torch.empty_like(t) for t in (qr, kr, kr))
-    rc = lib.corope_rope_attn_bwd_rotated(*(t.data_ptr() for t in (qr, kr)), vs.data_ptr(), None, o.data_ptr(), gc.data_ptr(), None, M.data_ptr(),
-                                          delta.data_ptr(), fc.data_ptr(), fs.data_ptr(), fc.stride(0), whole.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, Hq,
-                                          Hkv, N, D, scale, int(causal), int(dtype == torch.float16), None, 0, torch.cuda.current_stream().cuda_stream)
-    assert rc == 0
-    torch.cuda.synchronize()
+    whole = _backward_on_whole_blocks(pkg, saved, g, scale, causal)[0]
     a, b = dq.float(), whole.float()
     assert not torch.equal(a, b)   # (it was cut)
     step = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)

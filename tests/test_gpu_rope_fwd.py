@@ -345,13 +345,13 @@ def _whole_blocks(pkg, q, k, v, cos, sin, scale, causal):
 
 
 # Shapes whose forward cuts query blocks into pieces: inside and across blocks and heads, waves whose rows see none of a piece's keys, a ragged last
-# block and last key tile, strided views, logits hot enough to move the reference value.  Against the whole-block launch on the same inputs: O differs by
+# block and last key tile, pieces of more than 64 key tiles, strided views, logits hot enough to move the reference value.  Against the whole-block launch on the same inputs: O differs by
 # the rounding of P and of O to bf16 (2^-9 each, per row independent: 2-norm below 2^-8; in the fp16 build V is rounded to bf16 as well, alike in both), lse by
 # sums of up to N fp32 terms.  Against the oracle on rows around the cuts.  A query row that is not finite stays its own.
 @pytest.mark.parametrize("scale_mul", [1.0, 6.0])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,Hq,Hkv,N,D,causal", [(1, 2, 2, 2100, 128, True), (1, 1, 1, 3000, 128, False), (1, 1, 1, 4097, 128, True), (1, 2, 1, 3001, 64, False),
-                                                 (2, 1, 1, 8200, 64, True)])
+                                                 (2, 1, 1, 8200, 64, True), (1, 2, 1, 20000, 64, True), (1, 3, 3, 20000, 128, True)])
 def test_forward_cut_query_blocks(pkg, B, Hq, Hkv, N, D, causal, dtype, scale_mul):
     print(f"case B={B} Hq={Hq} Hkv={Hkv} N={N} D={D} causal={causal} {dtype} x{scale_mul}", flush=True)
     lib, dev, scale = pkg._lib.load(), torch.device("cuda:0"), scale_mul / math.sqrt(D)
@@ -402,6 +402,33 @@ def test_forward_cut_query_blocks_at_very_negative_logits(pkg, N, causal):
     first = best if causal else 0
     assert lse.max() < -1e31 and torch.equal(lse, lse_w)
     assert torch.equal(o[:, :, first:], v[:, :, best:best + 1].expand(-1, -1, N - first, -1)) and torch.equal(o[:, :, :first], whole[:, :, :first])
+
+
+# Pieces of more than 64 key tiles (the tiles' key norms come 64 at a time), and every 1489 keys one whose logit is 256 above all before it: a row follows
+# the last of them that it sees, so the reference value has to move on in the middle of a piece, also behind its 64th tile.  O is that key's v but for
+# the rounding of P, which need not be 1, and of O to bf16 (up to 2^-8 each); a reference that stays behind by 369 (base 2) overflows.  No rotation.
+@pytest.mark.parametrize("H,Hkv,N,D", [(2, 1, 20000, 64), (3, 3, 20000, 128)])
+def test_forward_cut_query_blocks_with_rising_logits_in_long_pieces(pkg, H, Hkv, N, D):
+    print(f"case H={H} Hkv={Hkv} N={N} D={D}", flush=True)
+    dev, every = torch.device("cuda:0"), 1489
+    assert pkg._lib.load().corope_rope_attn_fwd_parts_bytes(1, H, N, D, 1) > 0
+    tiles = H * sum(min(4 * (i + 1), (N + 63) // 64) for i in range((N + 255) // 256))
+    assert tiles / torch.cuda.get_device_properties(dev).multi_processor_count > 80
+    c, s = torch.ones(N, D // 2, device=dev), torch.zeros(N, D // 2, device=dev)
+    q, k, v = (seeded((1, h, N, D), 160 + i) * f for i, (h, f) in enumerate(((H, 0.25), (Hkv, 0.25), (Hkv, 1.0))))
+    top = torch.arange(every, N, every)
+    q[..., 3], k[..., 3] = 16.0, 0.0
+    k[:, :, top, 3] = 16.0 * torch.arange(1, len(top) + 1)
+    q, k, v = (t.to(dev, torch.bfloat16) for t in (q, k, v))
+    o, lse = pkg.rope_attn_forward_with_lse(q, k, v, True, 1.0, c, s)
+    whole, lse_w = _whole_blocks(pkg, q, k, v, c, s, 1.0, True)
+    rows = torch.arange(every, N, device=dev)
+    want = v.repeat_interleave(H // Hkv, dim=1)[:, :, rows // every * every].double()
+    for name, x in (("whole", whole), ("cut", o)):
+        err = (x[:, :, every:].double() - want).abs() / want.abs().clamp_min(2.0 ** -100)
+        print(f"  {name}: {err.max().item():.2e} of the value")
+        assert err.max() <= 2.0 ** -7 + 2.0 ** -16, name
+    assert ((lse - lse_w).abs() <= 1e-4 + 2.0 ** -22 * lse_w.abs()).all()
 
 
 # Equal logits over several pieces, so large that a float holds them with no fraction: O is the mean of the v a row sees whatever the offset.  The pieces

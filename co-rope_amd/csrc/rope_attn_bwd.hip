@@ -847,17 +847,8 @@ static int dkdv_shares(int N, int slabs, int group, bool causal) {
   const int slots = cus * (small && fits_twice(DkdvCfgOf<D, true, true, 4>::kLdsBytes) ? 2 : 1);
   const int64_t n_items = (int64_t)nb * slabs;
   if (n_items > (int64_t)kMost * slots || (int64_t)n_items * group * m_tiles >= (1ll << 30)) return 0;   // many rounds even out
-  // the heaviest item of every round goes to the workgroup that was dealt the lightest of the round before (ItemList)
-  int64_t longest = 0;
   const int grid = (int)std::min<int64_t>(n_items, slots);
-  for (int w = 0; w < grid; w += 8) {
-    int64_t sum = 0;
-    for (int r = 0; (int64_t)r * grid < n_items; ++r) {
-      const int64_t i = (int64_t)r * grid + ((r & 1) ? grid - 1 - w : w);
-      if (i < n_items) sum += group * (m_tiles - (causal ? (int)(i / slabs) * (block / BM) : 0));
-    }
-    longest = std::max(longest, sum);
-  }
+  const int64_t longest = most_tiles_dealt(n_items, grid, [&](int64_t i) -> int64_t { return group * (m_tiles - (causal ? (int)(i / slabs) * (block / BM) : 0)); });
   const DkdvTiles t((N + CW * 32 - 1) / (CW * 32), slabs, group, m_tiles, causal ? CW * 32 / BM : 0);
   const int shares = std::max(1, std::min(cus, t.total_tiles / 4));
   const float tile_us = D == 64 ? 1.7f : 3.3f;
@@ -942,16 +933,8 @@ static int dq_shares(int N, int BH, bool causal) {
   const int slots = cus * (small && fits_twice(DqCfg<D, 4, BN>::kLdsBytes) ? 2 : 1);
   const int64_t n_items = (int64_t)nb * BH;
   if (n_items > (int64_t)kMost * slots || n_items * k_tiles >= (1ll << 30)) return 0;   // many rounds even out
-  int64_t longest = 0;
   const int grid = (int)std::min<int64_t>(n_items, slots);
-  for (int w = 0; w < grid; w += 8) {
-    int64_t sum = 0;
-    for (int r = 0; (int64_t)r * grid < n_items; ++r) {
-      const int64_t i = (int64_t)r * grid + ((r & 1) ? grid - 1 - w : w);
-      if (i < n_items) sum += causal ? std::min((nb - (int)(i / BH)) * (block / BN), k_tiles) : k_tiles;
-    }
-    longest = std::max(longest, sum);
-  }
+  const int64_t longest = most_tiles_dealt(n_items, grid, [&](int64_t i) -> int64_t { return causal ? std::min((nb - (int)(i / BH)) * (block / BN), k_tiles) : k_tiles; });
   const QueryTiles t((N + CW * 32 - 1) / (CW * 32), BH, k_tiles, causal ? CW * 32 / BN : 0);
   const int shares = std::max(1, std::min(cus, t.total_tiles / 4));
   constexpr float kWholeTile = D == 64 ? 1.25f : D == 128 ? 2.8f : 1.75f, kTile = D == 64 ? 1.5f : D == 128 ? 2.9f : 1.6f;

@@ -567,16 +567,8 @@ static int fwd_shares(int N, int BH, bool causal) {
   const int slots = cus * (small && fits_twice(FwdPipeCfg<D, 4>::kLdsBytes) ? 2 : 1);
   const int64_t n_items = (int64_t)nb * BH;
   if (n_items > (int64_t)kMost * slots || n_items * k_tiles >= (1ll << 30)) return 0;   // many rounds even out
-  int64_t longest = 0;
   const int grid = (int)std::min<int64_t>(n_items, slots);
-  for (int w = 0; w < grid; w += 8) {
-    int64_t sum = 0;
-    for (int r = 0; (int64_t)r * grid < n_items; ++r) {
-      const int64_t i = (int64_t)r * grid + ((r & 1) ? grid - 1 - w : w);
-      if (i < n_items) sum += causal ? std::min((nb - (int)(i / BH)) * (block / BN), k_tiles) : k_tiles;
-    }
-    longest = std::max(longest, sum);
-  }
+  const int64_t longest = most_tiles_dealt(n_items, grid, [&](int64_t i) -> int64_t { return causal ? std::min((nb - (int)(i / BH)) * (block / BN), k_tiles) : k_tiles; });
   const QueryTiles t((N + kCutWaves * 32 - 1) / (kCutWaves * 32), BH, k_tiles, causal ? kCutWaves * 32 / BN : 0);
   const int shares = std::max(1, std::min(cus, t.total_tiles / 4));
   constexpr float kWholeTile = D == 64 ? 1.f : 1.75f, kTile = D == 64 ? 1.1f : 2.f, kChange = D == 64 ? 3.f : 4.f;

@@ -43,9 +43,9 @@ HBM_TRAFFIC_BYTES = {
     ("c4", "rope_attn_fwd"): int((1073484 * 2.0 + 243220) * 1024),
     # Co-RoPE at C5 (profiles/corope_gqa_c5_hbm_traffic.md): the forward kernel; the backward's launches together, with
     # the workspace for one pass
-    ("c5", "corope_gqa_fwd"): int((73773 * 2.0 + 65536) * 1024),
-    ("c5", "corope_gqa_bwd"): int(((3564006 + 1865385 + 2086161 + 26643 + 26649) * 2.0
-                                   + (9566621 + 74243 + 57856 + 11776 + 11776)) * 1024),
+    ("c5", "corope_gqa_fwd"): int((72701 * 2.0 + 65536) * 1024),
+    ("c5", "corope_gqa_bwd"): int(((3571091 + 1882246 + 2084760 + 26651 + 26650) * 2.0
+                                   + (9568497 + 74241 + 57856 + 11776 + 11776)) * 1024),
 }
 
 CONFIGS = {

@@ -79,7 +79,7 @@ def backward_min_workspace_bytes(B, Hq, Hkv, N, D):
 
 # The backward's scratch when the caller brings none: one buffer per device and stream, kept between calls and grown when
 # a call needs more, holding as many groups' matrices as fit BACKWARD_WORKSPACE_CAP_BYTES (never less than one group; all
-# groups in one pass is fastest: at B2 Hq32 Hkv8 N4096 D128 7.1 GiB and 11.1 ms, against 16.8 ms with a quarter of that).  The
+# groups in one pass is fastest: at B2 Hq32 Hkv8 N4096 D128 7.1 GiB and 9.8 ms, against 15.5 ms with a quarter of that).  The
 # size depends on the shape and the cap only, not on what else is resident.  Per stream, because calls on two streams of a
 # device may run at the same time and torch's allocator only orders a buffer's reuse on the stream it was allocated on.
 BACKWARD_WORKSPACE_CAP_BYTES = 8 << 30

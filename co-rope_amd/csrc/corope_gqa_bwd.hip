@@ -921,7 +921,7 @@ __global__ __launch_bounds__(4 * kWave) void corope_bwd_dv_kernel(CoropeBwdParam
 // a wave per head.  Class 0 (|x w| <= 0.68) takes the powers 0 .. 5, class 1 (<= 0.08) 0 .. 2, the last coefficients lowered to spread the
 // remainder: below 1e-5 and 2.2e-5.  Operands are bf16 parts: two of dS and two of the bracket (16 bits) up to power 2 (fp16: 3) of class 0 and 1 of
 // class 1; one part of the powers above leaves an error of 4.8e-5 (fp16: 0.9e-5) and 1.6e-5 of dk for the fastest pair with every gate open, beside
-// 1.7e-3 (3e-4) of its rounding.  (With one part from power 2, fp16 3, and class 1's power 1 on it was 2.4e-4, 4.8e-5 and 1.1e-4.)  Built for up
+// 1.7e-3 (3e-4) of its rounding.  (With one part from power 2, fp16 3, and class 1's power 1 on it was 2.4e-4, 4.8e-5 and 1.1e-4, and the kernel 3.06 instead of 3.15 ms.)  Built for up
 // to five heads a group (fp16: four), whose LDS leaves two workgroups to a compute unit.
 // What bounds it: the vector units, 9 or 10 issue slots per (row, key, pair) that is rotated.  Measured with the gate path moved: B2 Hq32 Hkv8 N4096 D128
 // forward + backward 15.0 -> 14.6 ms, B2 Hq8 Hkv2 N512 D64 133 -> 130.5 us; with the slow pairs as products the former 13.43 -> 12.70 ms, error of

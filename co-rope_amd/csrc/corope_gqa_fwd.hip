@@ -422,8 +422,9 @@ static hipError_t launch_corope_cfg(const CoropeParams& p, const CoropeFreqs& fr
   // Rows per wave: as many as fill the 16 columns, where the waves then still fill the chip; below that the longest rows, whose chunks
   // follow one after the other, set the time, and fewer rows per wave shorten it.
   // The slow pairs' products cost the same for one row as for all: they pay from two rows per wave on, and make more rows pay earlier.
-  // Whether they are used depends on the rows of one batch entry alone, so that an entry's result has the same bits whatever it is batched
-  // with; from `least` on, two rows per wave are no slower than one with every pair rotated.
+  // Whether they are used depends on the rows of one batch entry alone, so that an entry's scores are computed the same way whatever it is batched
+  // with (its bits may still differ: the rows of a wave, which depend on the whole batch, move their reference values together); from `least`
+  // on, two rows per wave are no slower than one with every pair rotated.
   // us with one (every pair rotated) / two / four rows, B1 Hq32 Hkv8, D = 64: N256 9.8 / 13.8 / 16.7, N512 26.5 / 24.9 / 29.8, N700 46 / 35 / 40, N900 73 / 54 / 53, N1024
   // 106 / 65 / 57; D = 128: N256 15.4 / 19.9 / 26.6, N400 34.5 / 33.0 / 43.0, N700 79 / 60 / 66, N900 126 / 92 / 87, N1300 273 / 175 / 139.  Every pair
   // rotated: fp16 B1 Hq32 Hkv8 N1111 D128 179 / 143 / 171, B2 Hq16 Hkv4 N2048 D128 582 / 466 / 418.

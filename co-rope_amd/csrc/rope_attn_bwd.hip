@@ -919,8 +919,8 @@ static hipError_t launch_dq_waves(BwdParams p, hipStream_t stream) {
 
 // How many pieces the key tiles of the dQ launch on rotated operands are cut into; 0: whole items.  As dkdv_shares: with few heads the longest
 // whole item (a sequence's last queries, which see all of its keys) sets the time however many compute units are idle.  Measured
-// constants, in microseconds: a tile of a full chip, a change of items (at head dim 256, one wave per SIMD, nothing hides it), the launch; a
-// causal piece of T tiles crosses up to sqrt(2 T / step) of a head's lightest items.  dQ launch, whole / cut with its sums, B1 H N: D = 128: 8 4096 159 / 87, 4 8192
+// constants, in microseconds: a tile of a full chip, a change of items (at head dim 256 nothing hides it with one wave per SIMD, and the cut kernel sends
+// 130 registers through scratch there, none in the tile loop), the launch; a causal piece of T tiles crosses up to sqrt(2 T / step) of a head's lightest items.  dQ launch, whole / cut with its sums, B1 H N: D = 128: 8 4096 159 / 87, 4 8192
 // 296 / 132, 1 10000 330 / 66, 8 3000 not causal 119 / 80, and on the other side 16 4096 153 / 152, 40 1100 53 / 64; D = 64: 8 4096 63 / 50, 4 16384 276 / 239, 2 3000
 // not causal 46 / 27, 16 1500 27.5 / 28.2; D = 256: 2 2048 112 / 58, 4 4096 212 / 185, 8 2048 115 / 129, 16 2048 124 / 199.
 template <int D>

@@ -1005,22 +1005,22 @@ __device__ __forceinline__ u32x4 pack_rest8(const float (&x)[8], u32x4 first) {
   return pack_elts8(r);
 }
 
-// The slow pairs' queries of a column, in its four lanes.  fp16: a query of 60000 would leave fp16's range on its way round, and the coefficients
-// of one of 1e-6 would have a handful of bits left; so they are scaled by the power of two that brings the largest of them to 2^14 .. 2^15.
-// Returns its inverse.
-template <int LOW>
-__device__ __forceinline__ float corope_low_queries(u32x4* raw) {
+// A column's query, in its four lanes, for the slow pairs' coefficients.  fp16: one of 60000 would leave fp16's range on its way round, and the
+// coefficients of one of 1e-6 would have a handful of bits left; so it is scaled by the power of two that brings its largest element to
+// 2^14 .. 2^15.  Returns the power's inverse.
+template <int NG>
+__device__ __forceinline__ float corope_scaled_query(u32x4 (&raw)[NG]) {
   static_assert(kEltIsF16, "bf16 has the range");
   uint32_t top = 0;   // (bit patterns of non-negative numbers order like the numbers)
 #pragma unroll
-  for (int u = 0; u < LOW; ++u)
+  for (int u = 0; u < NG; ++u)
 #pragma unroll
     for (int e = 0; e < 4; ++e) top = max(top, max(raw[u][e] & 0x7fffu, raw[u][e] >> 16 & 0x7fffu));
   top = max(top, (uint32_t)__shfl_xor((int)top, 16));
   top = max(top, (uint32_t)__shfl_xor((int)top, 32));
   const int shift = 14 - max(-24, (int)(__builtin_bit_cast(uint32_t, elt_lo(top)) >> 23) - 127);   // (no query but zeros: any)
 #pragma unroll
-  for (int u = 0; u < LOW; ++u)
+  for (int u = 0; u < NG; ++u)
 #pragma unroll
     for (int e = 0; e < 4; ++e) raw[u][e] = pack_elts(ldexpf(elt_lo(raw[u][e]), shift), ldexpf(elt_hi(raw[u][e]), shift));
   return ldexpf(1.f, -shift);
@@ -1033,7 +1033,7 @@ struct CoropeLowOps {
   u32x4 c[5], c0r, c1r;   // class 0: powers 0..4, remainders of powers 0 and 1
   u32x4 d[3], d0r;        // class 1
 
-  // raw: the column's query (fp16: as corope_low_queries leaves it), groups in operand order; turns: w / 2 pi of this lane's pairs; mid: the
+  // raw: the column's query (fp16: as corope_scaled_query leaves it), groups in operand order; turns: w / 2 pi of this lane's pairs; mid: the
   // chunk's middle
   __device__ __forceinline__ void build(const u32x4* raw, const float (*turns)[4], float mid) {
     static_for<LOW>([&](auto u_c) __attribute__((always_inline)) {

@@ -59,8 +59,7 @@ struct CoropeFwdCfg {
   static constexpr int kKStride = D + 8;    // K tile rows: 16 keys read at one column hit 16 different bank groups
   static constexpr int kVStride = D + 16;   // V tile rows: the 4 rows x 32 bytes of a transposing read cover 32 banks once
   static constexpr int kTileElems = kCoropeKeys * (kKStride + kVStride);
-  static constexpr int kMids = 4 * R * 16, kUnscales = kMids + (R + 3) / 4 * 4;
-  static constexpr int kDeltaFloats = kUnscales + 16;   // per wave: [16-key block][row][key % 16], [row] the chunk's middle, [column] (corope_low_queries)
+  static constexpr int kMids = 4 * R * 16, kDeltaFloats = kMids + (R + 3) / 4 * 4;   // per wave: [16-key block][row][key % 16], [row] the chunk's middle
   static constexpr int kLdsBytes = 2 * kTileElems * 2 + kCoropeWaves * kDeltaFloats * 4;
   static_assert(2 * kLdsBytes <= 160 * 1024, "two workgroups per compute unit");
 };
@@ -93,7 +92,6 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
   const uint16_t* kbase = p.k + (int64_t)grp * N * D;
   const uint16_t* vbase = p.v + (int64_t)grp * N * D;
   const int n_chunks = i0 / kCoropeKeys + 1;
-  const float scale2 = p.sm_scale * 1.4426950408889634f;               // scores in the base-2 domain
 
   // column n of the score product: (query row, head) = (iw + n / G, n % G); columns from R G on are idle
   const int crow = n < R * G ? n / G : 0, chead = n < R * G ? n % G : 0;
@@ -115,7 +113,7 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
       }
     }
   };
-  u32x4 qop[NG], lop[NG];   // B operand of the score product (fp16; the low groups' in the element type), A operand of the logit product (element type)
+  u32x4 qop[NG], lop[NG];   // B operand of the score product (fp16; the low groups' as they are), A operand of the logit product (element type)
   {
     const uint16_t* qrow = p.q + ((int64_t)(head0 + chead) * N + min(iw + crow, N - 1)) * D;
     const uint16_t* lrow = p.q + ((int64_t)head0 * N + min(iw + n * R / 16, N - 1)) * D;
@@ -126,7 +124,8 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
 #pragma unroll
       for (int e = 0; e < 4; ++e) qop[u][e] = n >= R * G ? 0u : u < NH ? pack_f16(elt_lo(qop[u][e]), elt_hi(qop[u][e])) : qop[u][e];
   }
-  if constexpr (LOW > 0 && kEltIsF16) dbuf[Cfg::kUnscales + n] = corope_low_queries<LOW>(qop + NH);   // (in LDS: the loop has no register left)
+  float scale2 = p.sm_scale * 1.4426950408889634f;   // scores in the base-2 domain, of this lane's column
+  if constexpr (LOW > 0 && kEltIsF16) scale2 *= corope_scaled_query(qop);
   float turns[NG * 4 / P][P];  // w_d / 2 pi of this lane's columns
 #pragma unroll
   for (int u = 0; u < NG * 4 / P; ++u)
@@ -241,7 +240,7 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
         }
         ops.scores(kf, y, s);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) sacc[b0 + b] = kEltIsF16 ? s[b] * dbuf[Cfg::kUnscales + n] : s[b];
+        for (int b = 0; b < NB; ++b) sacc[b0 + b] = s[b];
       }
       if (c > 0) fetch(c - 1, std::false_type{});   // (behind the polynomial, which needs the registers)
     } else {

@@ -421,15 +421,17 @@ static hipError_t launch_corope_cfg(const CoropeParams& p, const CoropeFreqs& fr
   // Rows per wave: as many as fill the 16 columns, where the waves then still fill the chip; below that the longest rows, whose chunks
   // follow one after the other, set the time, and fewer rows per wave shorten it.
   // The slow pairs' products cost the same for one row as for all: they pay from two rows per wave on, and make more rows pay earlier.
-  // Whether they are used depends on the rows of one batch entry alone, so that an entry's scores are computed the same way whatever it is batched
-  // with (its bits may still differ: the rows of a wave, which depend on the whole batch, move their reference values together); from `least`
-  // on, two rows per wave are no slower than one with every pair rotated.
+  // Whether they are used depends on the rows of one batch entry, so that an entry's scores are computed the same way whatever it is batched with (its
+  // bits may still differ: the rows of a wave, which depend on the whole batch, move their reference values together).  From `least` on, two rows
+  // per wave are no slower than one with every pair rotated; at D = 128 an entry alone needs 3.375 rows a SIMD for that, where the launch of
+  // one row per wave has just begun another round: us, every pair rotated / products, B1 Hq4 Hkv1 N3200 191 / 206, N3400 215 / 222, N3600 241 / 234; B2 Hq8 Hkv2 N1600
+  // (3200 rows an entry) 183 / 139.
   // us with one (every pair rotated) / two / four rows, B1 Hq32 Hkv8, D = 64: N256 9.8 / 13.8 / 16.7, N512 26.5 / 24.9 / 29.8, N700 46 / 35 / 40, N900 73 / 54 / 53, N1024
   // 106 / 65 / 57; D = 128: N256 15.4 / 19.9 / 26.6, N400 34.5 / 33.0 / 43.0, N700 79 / 60 / 66, N900 126 / 92 / 87, N1300 273 / 175 / 139.  Every pair
   // rotated: fp16 B1 Hq32 Hkv8 N1111 D128 179 / 143 / 171, B2 Hq16 Hkv4 N2048 D128 582 / 466 / 418.
   constexpr int kMost = G <= 2 ? 8 : G <= 4 ? 4 : 2, kLow = D / 64;
   const int64_t rows = (int64_t)p.N * p.B * p.Hkv, simds = 4 * device_cu_count(), least = (D == 64 ? 4 : 3) * simds;
-  if (low >= kLow && (int64_t)p.N * p.Hkv >= least) {
+  if (low >= kLow && (int64_t)p.N * p.Hkv >= least && rows >= (D == 64 ? least : least + 3 * simds / 8)) {
     if constexpr (kMost > 4) {
       if (rows >= 14 * simds) return launch_corope_reduced<D, G, kMost, kLow>(p, fr, reduced, stream);
     }

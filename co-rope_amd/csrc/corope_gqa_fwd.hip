@@ -124,8 +124,6 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
 #pragma unroll
       for (int e = 0; e < 4; ++e) qop[u][e] = n >= R * G ? 0u : u < NH ? pack_f16(elt_lo(qop[u][e]), elt_hi(qop[u][e])) : qop[u][e];
   }
-  float scale2 = p.sm_scale * 1.4426950408889634f;   // scores in the base-2 domain, of this lane's column
-  if constexpr (LOW > 0 && kEltIsF16) scale2 *= corope_scaled_query(qop);
   float turns[NG * 4 / P][P];  // w_d / 2 pi of this lane's columns
 #pragma unroll
   for (int u = 0; u < NG * 4 / P; ++u)
@@ -176,6 +174,8 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
   for (int z = 0; z < ZR; ++z) carry[z] = 0.f;
 
   fetch(n_chunks - 1, std::true_type{});
+  float scale2 = p.sm_scale * 1.4426950408889634f;   // scores in the base-2 domain, of this lane's column
+  if constexpr (LOW > 0 && kEltIsF16) scale2 *= corope_scaled_query(qop);   // (waits for the query under the first tiles' requests)
   park(0);
   __syncthreads();
   int buf = 0;
@@ -266,17 +266,19 @@ __global__ __launch_bounds__(kCoropeWaves* kWave) __attribute__((amdgpu_waves_pe
           k2[u][2 * e + 1] = elt_hi(w2);
         }
       const f32x4 low = sacc[b];
-      // The rows are unrolled, which hides a row's chain behind the next row's: bf16 B2 Hq32 Hkv8 N4096 D128 2.32 -> 2.23 ms.  fp16 has no registers for
-      // that (84 to 134 of them went through scratch): with eight rows at D = 128 the scheduler is kept from mixing them, and where every pair
-      // is rotated they stay a loop, as do two rows in bf16.  All unrolled -> this, us: fp16 D128 N4096 Hq32 Hkv32 5523 -> 3674 and Hkv16 2787 -> 1865;
-      // theta = 1000 (every pair rotated) Hkv32 6815 -> 5770, Hkv8 1740 -> 1557, Hkv4 902 -> 880, bf16 Hkv4 918 -> 911.
-      constexpr bool kRowByRow = kEltIsF16 && D == 128 && LOW > 0 && R == 8;
-      constexpr int kUnroll = LOW == 0 && (kEltIsF16 || R == 2) ? 1 : R;
-      float delta = dbuf[b * R * 16 + n];
+      // The rows are unrolled, which hides a row's chain behind the next row's: bf16 B2 Hq32 Hkv8 N4096 D128 2.32 -> 2.23 ms.  fp16 at D = 128 has no registers
+      // for that (84 to 134 of them went through scratch): with eight rows the scheduler is kept from mixing them, and where every pair is
+      // rotated they stay a loop.  All unrolled -> this, us: N4096 Hq32 Hkv32 5523 -> 3674 and Hkv16 2787 -> 1865; theta = 1000 (every pair
+      // rotated) Hkv32 6815 -> 5770, Hkv8 1740 -> 1557, Hkv4 902 -> 880.
+      constexpr bool kRowByRow = kEltIsF16 && D == 128 && LOW > 0 && R == 8, kLoop = kEltIsF16 && D == 128 && LOW == 0;
+      constexpr int kUnroll = kLoop ? 1 : R;
+      float delta[kLoop ? 1 : R];   // (in the loop: of the next row)
+#pragma unroll
+      for (int r = 0; r < (kLoop ? 1 : R); ++r) delta[r] = dbuf[(b * R + r) * 16 + n];
 #pragma unroll kUnroll
       for (int r = 0; r < R; ++r) {
-        const float delta_r = delta;
-        delta = dbuf[(b * R + min(r + 1, R - 1)) * 16 + n];
+        const float delta_r = delta[kLoop ? 0 : r];
+        if constexpr (kLoop) delta[0] = dbuf[(b * R + min(r + 1, R - 1)) * 16 + n];
         f32x4 acc = low;
         static_for<UNITS>([&](auto u_c) __attribute__((always_inline)) {
           constexpr int u = decltype(u_c)::value;

@@ -290,6 +290,20 @@ def test_cut_forward_argument_checks(pkg):
         assert text in pkg._lib.last_error() and pkg._lib.last_error().startswith("rope_attn_fwd_cut"), (args, pkg._lib.last_error())
 
 
+def test_where_launches_are_cut(pkg):
+    """The rules that cut query blocks, on either side of their lines (256 compute units, the figure taken without a device): where cutting was
+    measured to pay, and where whole blocks are as fast or faster."""
+    lib = pkg._lib.load()
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rules depend on the number of compute units")
+    fwd = lambda B, H, N, D, causal: lib.corope_rope_attn_fwd_parts_bytes(B, H, N, D, causal) > 0
+    assert fwd(1, 8, 4096, 128, 1) and fwd(1, 4, 8192, 128, 1) and fwd(1, 6, 2700, 64, 1) and fwd(1, 16, 9000, 128, 0)
+    assert not any(fwd(*s) for s in ((1, 16, 4096, 128, 1), (1, 32, 1500, 128, 1), (1, 16, 1500, 64, 1)))
+    # (key blocks are not cut at these shapes, so that the answer is the dQ launch's)
+    bwd = lambda B, H, Hkv, N, D, causal: lib.corope_rope_attn_bwd_rotated_parts_bytes(B, H, Hkv, N, D, causal) > 0
+    assert not bwd(1, 40, 10, 3000, 256, 0) and not bwd(1, 32, 32, 4096, 256, 0)
+
+
 def test_alias_names_the_same_modules():
     """``corope_amd`` is an alias of the package in the directory ``co-rope_amd``: importing a submodule through either
     name gives the one module object whose globals the package's functions read (a second copy would have thresholds

@@ -727,7 +727,7 @@ def main():
     dq, dk, dv = torch.empty_like(q), torch.empty_like(q), torch.empty_like(q)
     qp, kp, vp, dop = q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr()
     cp, sp, fs = cos.data_ptr(), sin.data_ptr(), cos.stride(0)
-    rotated = pkg.rope_attn.use_rotated_path(N, D, training=not fwd_only)
+    rotated = pkg.rope_attn.use_rotated_path(N, D, training=not fwd_only, slabs=B * H)
     if rotated:   # the forward the operator takes at this shape: rotate K, then attention
         k_rot, q_rot = torch.empty_like(k), torch.empty_like(q)
         kmax = torch.empty(B, H, (N + 63) // 64, device=dev, dtype=torch.float32)

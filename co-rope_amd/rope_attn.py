@@ -98,10 +98,18 @@ def _freq_table(f):
 
 # Shapes from which the operator rotates its operands ahead of the attention kernels: K once into a scratch buffer for
 # the forward (every K tile is otherwise rotated again by each query block of its head), and, when a gradient will be asked
-# for, q and k once for the backward (fused dK+dV, no tables in its loops).  Measured crossover on MI355X, the same for both:
-# N * D = 65536 (N = 512 at D = 128, N = 1024 at D = 64); below it every kernel rotates its own tiles.
+# for, q and k once for the backward (fused dK+dV, no tables in its loops, blocks cut into equal pieces where they are few).
+# Measured on MI355X, in us, unrotated -> rotated.  Forward and backward: always, B4 H8 N512 D64 52.1 -> 45.9, B1 H32 N96 D128
+# 64.3 -> 39.2, B3 Hq64 Hkv32 N64 D64 30.9 -> 26.7, B2 Hq32 Hkv4 N700 D64 299 -> 71, B2 Hq16 Hkv4 N400 D128 243 -> 77, B2 H8 N200
+# D256 133 -> 84 (from N * D = 65536 on it was before).  The forward alone pays the rotation pass's launch (3 to 4 us): D = 64, causal / not, H32 N600 16.7 -> 17.1 /
+# 15.9 -> 17.3 and N800 20.2 -> 19.4 / 19.9 -> 20.1; D = 256, H32 N128 26.1 -> 26.7 / 26.0 -> 24.8 and N160 35.5 -> 27.1; at D = 128 the
+# unrotated kernel's 256-row form holds out longer than its 128-row form: H32 N64 10.7 -> 13.2, N130 16.6 -> 15.4, N300 22.9 -> 19.0 (128 rows),
+# H128 N300 25.2 -> 26.6 / 22.5 -> 27.8 (256 rows).
 TWO_LAUNCH_MIN_N = 1024
-TRAIN_ROTATED_MIN_ND = 65536
+TRAIN_ROTATED_MIN_ND = 0
+_FWD_ROTATED_MIN_ND = 65536
+_FWD_ROTATED_MIN_N = {64: 768, 128: 129, 256: 129}
+_FWD_SMALL_ITEMS = 256   # 256-row items below this take the 128-row form: the compute units of an MI355X
 
 
 # fp16 tensors, forward of a call that will be differentiated: "exact" = the single-launch kernel's bookkeeping, which
@@ -113,9 +121,16 @@ TRAIN_ROTATED_MIN_ND = 65536
 FP16_TRAINING_FORWARD = "exact"
 
 
-def use_rotated_path(N, D, training):
-    """Whether the operator rotates the operands ahead of the attention kernels at this shape."""
-    return D <= _ROTATED_PATH_MAX_D and (N >= TWO_LAUNCH_MIN_N or N * D >= TRAIN_ROTATED_MIN_ND)
+def use_rotated_path(N, D, training, slabs=None):
+    """Whether the operator rotates the operands ahead of the attention kernels at this shape.  slabs: batch * query heads, or None
+    for an fp16 forward without gradients, whose kernel on rotated keys keeps P and V in bf16: it is left where it was."""
+    if N * D < TRAIN_ROTATED_MIN_ND or D > _ROTATED_PATH_MAX_D:
+        return N >= TWO_LAUNCH_MIN_N and D <= _ROTATED_PATH_MAX_D
+    if training or N >= TWO_LAUNCH_MIN_N or N * D >= _FWD_ROTATED_MIN_ND:
+        return True
+    if slabs is None or (D == 128 and (N + 255) // 256 * slabs >= _FWD_SMALL_ITEMS):
+        return False
+    return N >= _FWD_ROTATED_MIN_N[D]
 
 
 def _view_strides(t):
@@ -147,7 +162,7 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
     o = torch.empty(q.shape, device=q.device, dtype=q.dtype)
     M = torch.empty((B, H, N), device=q.device, dtype=torch.float32)
     if two_launch is None:
-        two_launch = use_rotated_path(N, D, training=keep_rotated)
+        two_launch = use_rotated_path(N, D, training=keep_rotated, slabs=B * H if q.dtype == torch.bfloat16 else None)
     rotated = None
     Hkv = k.shape[1]
     with _on_device(q):

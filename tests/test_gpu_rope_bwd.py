@@ -600,3 +600,21 @@ def test_entry_points_on_rotated_copies_agree(pkg, B, Hq, Hkv, N, D, causal):
             sv, sg = ((ctypes.c_int64 * 3)(*t.stride()[:3]) for t in (vv, gv))
             check("corope_rope_attn_bwd_rotated", qr, kr, vv, sv, o, gv, sg, *tables, fc.stride(0), *grads, B, Hq, Hkv, *scalars,
                   int(dtype == torch.float16), None, 0, st)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 2, 1, 1, 128), (2, 8, 2, 63, 64), (1, 8, 1, 65, 128), (3, 4, 4, 129, 64), (1, 6, 3, 129, 256), (2, 16, 4, 511, 128),
+                                          (1, 8, 2, 767, 64), (1, 4, 4, 768, 64)])
+def test_short_sequences_by_the_operators_own_rule(pkg, B, Hq, Hkv, N, D, causal):
+    """Training runs on rotated copies at every length, the forward alone from the lengths of use_rotated_path on (edges on both sides):
+    each against the oracle, and the two forwards within one bf16 step of each other."""
+    G, scale = Hq // Hkv, 1 / math.sqrt(D)
+    q, g = (bf16_round(seeded((B, Hq, N, D), 120 + i)) for i in range(2))
+    k, v = (bf16_round(seeded((B, Hkv, N, D), 130 + i)) for i in range(2))
+    c, s = O.precompute_freqs_cis(D, N)
+    got = _gpu_fwd_bwd(pkg, q, k, v, g, causal, scale, c, s)
+    alone = pkg.attention(*(t.cuda().bfloat16() for t in (q, k, v)), causal, scale, c.cuda(), s.cuda()).float().cpu()
+    ro, _, rdq, rdk, rdv, _ = O.rope_attn_fwd_bwd_blocked(q, k.repeat_interleave(G, 1), v.repeat_interleave(G, 1), g, causal, scale, c, s)
+    rdk, rdv = (t.reshape(B, Hkv, G, N, D).sum(2) for t in (rdk, rdv))
+    for name, a, b in (("O", got[0], ro), ("O alone", alone, ro), ("dQ", got[1], rdq), ("dK", got[2], rdk), ("dV", got[3], rdv)):
+        assert within_bar(a, b, TOL * (math.sqrt(G) if name in ("dK", "dV") else 1))[0], name

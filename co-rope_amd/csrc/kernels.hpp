@@ -139,6 +139,7 @@ struct FwdParams {
   // rows; the last dimension is contiguous.  contiguous(D) fills in (B, H, N, D) row-major.
   int64_t q_sb, q_sh, k_sb, k_sh, v_sb, v_sh;
   int q_sn, k_sn, v_sn;
+  bool exact;        // fp16, k_rot without tile_kmax, D <= 128: the pipelined kernel with P and V in fp16, not the single-launch one
   float* parts;      // scratch for the pieces of cut query blocks (fwd_parts_bytes), or null: none is cut
   void contiguous(int D) {
     q_sn = k_sn = v_sn = D;

@@ -27,6 +27,14 @@
 // made before the tile is touched.  Only then (and on the first tile) the pipeline is drained, the tile's scores are
 // computed once just for their row maxima, the reference moves there and the accumulators are rescaled; the tile is
 // then processed like any other.  Inside a tile there is no data-dependent branch.
+//
+// EXACT (fp16 only) keeps P and V in fp16, for a forward that will be differentiated.  fp16 ends at 65504, which no bound from key
+// norms tells from above (unit-variance inputs at 1/sqrt(D): scores of 7 base-2 units under a bound of 25), so the reference starts at the first tile's
+// true maximum and every half's sum of probabilities is looked at before they are multiplied: above kExactSumLimit the half is done
+// again against its true maximum.  The comparison is issued one MFMA ahead of the branch that waits for it.
+// Two branches a tile cost 1 to 3 % beside the form without; the single-launch kernel on rotated keys, whose comparisons the branches wait
+// for and which starts a workgroup per query block, took, with the rotation pass, B2 H32 N4096 D128 causal 387 us, this 330; B1 H13 N29504 D64
+// 1953 / 1610; few heads, whose blocks this one cuts, B1 H8 N4096 D128 143 / 78.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -45,6 +53,8 @@ constexpr int kPipeBlockN = 64;
 // scores actually seen before a tile has to be examined a second time (unit-variance inputs at sm_scale = 0.5 need ~110).
 constexpr float kPipeMargin = 64.f;
 constexpr float kPipeLift = 80.f;
+// EXACT: largest sum of a lane's 16 probabilities of a half; each of them is then far below fp16's 65504.
+constexpr float kExactSumLimit = 16384.f;
 
 template <int D, int NW>
 struct FwdPipeCfg {
@@ -67,7 +77,7 @@ struct FwdPipeCfg {
 template <int D, int NW>
 constexpr int64_t kFwdSlotFloats = (int64_t)NW * 32 * (D + 2);
 
-// P^T is a bf16 operand in both builds (its unnormalised values span up to 2^kPipeMargin, more binary orders than fp16
+// Without EXACT P^T is a bf16 operand in both builds (its unnormalised values span up to 2^kPipeMargin, more binary orders than fp16
 // has), so the product O^T += V^T P^T is a bf16 product in both: in the fp16 build the V tile is converted to bf16 while
 // it is staged (fp16's 11 significant bits become 8: the same rounding P itself carries).
 #ifdef COROPE_F16
@@ -79,26 +89,66 @@ __device__ __forceinline__ u32x4 v_operand_format(u32x4 x) {
 #else
 __device__ __forceinline__ u32x4 v_operand_format(u32x4 x) { return x; }
 #endif
-template <class Stage, class Tile>
+template <bool EXACT, class Stage, class Tile>
 __device__ __forceinline__ void store_v_rows(const Stage& st, uint16_t* lds, Tile) {
 #pragma unroll
   for (int it = 0; it < Stage::kIters; ++it) {
     const int u = threadIdx.x + it * (Stage::kUnits / Stage::kIters);
-    *reinterpret_cast<u32x4*>(lds + Tile::off(u / Stage::kChunks, (u % Stage::kChunks) * 8)) = v_operand_format(st.x[it]);
+    *reinterpret_cast<u32x4*>(lds + Tile::off(u / Stage::kChunks, (u % Stage::kChunks) * 8)) = EXACT ? st.x[it] : v_operand_format(st.x[it]);
   }
 }
 
 // One exponential pair of a 32-key half: scores 2j, 2j+1 of the lane (already relative to the reference value, base-2
-// units) -> one bf16x2 word of the P^T operand.
+// units) -> one word of the P^T operand (bf16; EXACT: the element type).
+template <bool EXACT>
 __device__ __forceinline__ void softmax_pair(int j, const f32x16& sacc, u32x4 (&pb)[2], float& lsum) {
   asm volatile("" : "+v"(lsum));  // the pair starts here, not wherever the optimiser would like to hoist it
   float p0 = fast_exp2(sacc[2 * j]);
   float p1 = fast_exp2(sacc[2 * j + 1]);
   // plain adds: the bf16 dot-product instruction would do this in one op but stalls the MFMA pipe
   lsum += p0 + p1;
-  uint32_t w = pack_bf16(p0, p1);
+  uint32_t w = EXACT ? pack_elts(p0, p1) : pack_bf16(p0, p1);
   asm volatile("" : "+v"(w), "+v"(lsum));   // ... and ends here, between the two MFMAs it is written between
   pb[j / 4][j % 4] = w;
+}
+
+template <bool EXACT>
+__device__ __forceinline__ f32x16 pv_mfma(u32x4 a, u32x4 b, f32x16 c) { return EXACT ? mfma32(a, b, c) : mfma32_bf16(a, b, c); }
+
+// EXACT, a half (scores sc, operand pb) before its product: its probabilities join the row's sum, or, where they outgrew fp16 (over, wave-uniform),
+// are computed again against the half's true maximum; pending(up): scores that were computed against the old reference and are still to come.
+__device__ __forceinline__ bool outgrown(float lsum) { return __builtin_amdgcn_ballot_w64(!(lsum <= kExactSumLimit)) != 0; }
+template <int NDB, class Pending>
+__device__ __forceinline__ void settle_half(const f32x16& sc, u32x4 (&pb)[2], bool over, f32x16 (&oacc)[NDB], f32x16& msb, float& m_run, float& l_run,
+                                            float& lsum, Pending&& pending) {
+  if (__builtin_expect(over, 0)) {
+    float mt = sc[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mt = fmaxf(mt, sc[i]);
+    const float m_new = m_run + fmaxf(half_max(mt), 0.f), up = m_new - m_run;
+    const float alpha = fast_exp2(-up);
+    l_run *= alpha;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) oacc[db][i] *= alpha;
+    m_run = m_new;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float x = -m_new;
+      asm volatile("" : "+v"(x));   // sixteen values of their own: one value in sixteen places is tied to the first of them
+      msb[i] = x;
+    }
+    lsum = 0.f;
+    f32x16 rel;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) rel[i] = sc[i] - up;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) softmax_pair<true>(j, rel, pb, lsum);
+    pending(up);
+  }
+  l_run += lsum;
+  lsum = 0.f;
 }
 
 __device__ __forceinline__ float wave_reduce_max(float x) { return wave_max(x); }   // data-parallel-primitive moves, no LDS round trips
@@ -118,7 +168,7 @@ __device__ __forceinline__ float wave_reduce_max(float x) { return wave_max(x); 
 //
 // CUT: a workgroup takes a piece of the list of all key tiles instead (QueryWork); a piece of an item starts its own softmax and leaves its
 // O, reference values and sums in a slot, which rope_attn_fwd_join_kernel brings to one reference and adds.
-template <int D, bool CAUSAL, int NW, bool CUT = false>
+template <int D, bool CAUSAL, int NW, bool CUT = false, bool EXACT = false>
 __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) void rope_attn_fwd_pipe_kernel(FwdParams p) {
   using Cfg = FwdPipeCfg<D, NW>;
   constexpr int BLOCK_N = kPipeBlockN;
@@ -198,7 +248,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     int ko = koff_next, vo = voff_next;
     asm volatile("" : "+s"(ko), "+s"(vo));
     kst.store_rows(lds_at(ko));
-    store_v_rows(vst, lds_at(vo), RowTile<D, Cfg::kVPad>{});
+    store_v_rows<EXACT>(vst, lds_at(vo), RowTile<D, Cfg::kVPad>{});
     load_next_tile();
   };
 
@@ -218,7 +268,8 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     const int bh = i % p.BH, m0 = (p.num_m_blocks - 1 - i / p.BH) * Cfg::kBlockM;
     const int l = opaque_lane();
     qrows.load(p.q_slab(bh), p.cos, p.sin, p.fstride, m0 + rb * 32, N, l, (uint32_t)p.q_sn * 2);
-    kvec = reinterpret_cast<const uint32_t*>(p.tile_kmax)[(int64_t)kv_slab(bh, p.H, p.Hkv) * n_k_tiles + min(items.begin(i) + l, n_k_tiles - 1)];
+    if constexpr (!EXACT)
+      kvec = reinterpret_cast<const uint32_t*>(p.tile_kmax)[(int64_t)kv_slab(bh, p.H, p.Hkv) * n_k_tiles + min(items.begin(i) + l, n_k_tiles - 1)];
   };
   auto take_q = [&](int i) __attribute__((always_inline)) {
     const int bh = i % p.BH, m0 = (p.num_m_blocks - 1 - i / p.BH) * Cfg::kBlockM;
@@ -235,7 +286,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
   request_q(item);
   take_q(item);
   kst.store_rows(lds_at(koff_cur));
-  store_v_rows(vst, lds_at(voff_cur), RowTile<D, Cfg::kVPad>{});
+  store_v_rows<EXACT>(vst, lds_at(voff_cur), RowTile<D, Cfg::kVPad>{});
   load_next_tile();
   __syncthreads();
 
@@ -249,8 +300,8 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
 
     // Largest |q_r| (scaled: base-2 units) of the wave's rows, a little generous: times a tile's largest key norm it
     // bounds the tile's scores.
-    float q_bound_wave;
-    {
+    [[maybe_unused]] float q_bound_wave;
+    if constexpr (!EXACT) {
       float ss = 0.f;
 #pragma unroll
       for (int kc = 0; kc < M; ++kc)
@@ -279,8 +330,8 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
     const int t_last = __builtin_amdgcn_readfirstlane(CAUSAL ? min(n_tiles - 1, wave_q_hi / BLOCK_N) : n_tiles - 1);
 
     // Reference value that puts every tile this wave will see within the margin.
-    float lift_target;
-    {
+    [[maybe_unused]] float lift_target;
+    if constexpr (!EXACT) {
       uint32_t kall = t_begin + lane <= t_last ? kvec : 0u;   // non-negative floats order like their bit patterns
       for (int t0 = t_begin + kWave; t0 <= t_last; t0 += kWave) {
         const int tt = t0 + lane;
@@ -305,16 +356,17 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
       uint32_t vp_lane = v_lane_off + voff_prev;
       asm volatile("" : "+v"(vp_lane));
 #pragma unroll
-      for (int j = 4; j < 8; ++j) softmax_pair(j, s1, pb1, lsum);
+      for (int j = 4; j < 8; ++j) softmax_pair<EXACT>(j, s1, pb1, lsum);
+      if constexpr (EXACT) settle_half(s1, pb1, outgrown(lsum), oacc, msb, m_run, l_run, lsum, [](float) {});
 #pragma unroll
-      for (int i = 0; i < M; ++i) oacc[i % NDB] = mfma32_bf16(v_operand(vp_lane, 1, i), pb1[i / NDB], oacc[i % NDB]);
+      for (int i = 0; i < M; ++i) oacc[i % NDB] = pv_mfma<EXACT>(v_operand(vp_lane, 1, i), pb1[i / NDB], oacc[i % NDB]);
     };
 
     // the Q operands and the first 64 key-norm maxima have landed before the loop on every path: left to their first use,
     // the wait would sit inside the loop and there also wait for the next tile's loads
 #pragma unroll
     for (int kc = 0; kc < M; ++kc) asm volatile("" ::"v"(qb[kc]));
-    asm volatile("" ::"v"(kvec));
+    if constexpr (!EXACT) asm volatile("" ::"v"(kvec));
     COROPE_ISTAMP(2);
 #ifdef COROPE_TRACE
     COROPE_ISTAMP_ID(n_tiles);
@@ -363,42 +415,57 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
         static_for<TOTAL>([&](auto n_c) __attribute__((always_inline)) {
           constexpr int n = decltype(n_c)::value;
           constexpr int slot = n / M, i = n % M;
+          [[maybe_unused]] bool over;
+          if constexpr (EXACT) {
+            if constexpr (slot % 2 == 0 && i == M - 1) over = outgrown(lsum);   // (the half's last pair is done)
+          }
           // MFMA
           if (slot == 0) t0 = i == 0 ? mfma32_from(ring[n % RING], qb[i], msb) : mfma32(ring[n % RING], qb[i], t0);
-          if (slot == 1) oacc[i % NDB] = mfma32_bf16(ring[n % RING], pb1[i / NDB], oacc[i % NDB]);
+          if (slot == 1) oacc[i % NDB] = pv_mfma<EXACT>(ring[n % RING], pb1[i / NDB], oacc[i % NDB]);
           if (slot == 2) s1 = i == 0 ? mfma32_from(ring[n % RING], qb[i], msb) : mfma32(ring[n % RING], qb[i], s1);
-          if (slot == 3) oacc[i % NDB] = mfma32_bf16(ring[n % RING], pb0[i / NDB], oacc[i % NDB]);
+          if (slot == 3) oacc[i % NDB] = pv_mfma<EXACT>(ring[n % RING], pb0[i / NDB], oacc[i % NDB]);
           if (n + RING < TOTAL) ring[n % RING] = operand(n + RING);
           if (n == 0) stage_next();
           // softmax on the side: four exponential pairs per slot
-          constexpr int jlo = i * 4 / M, jhi = (i + 1) * 4 / M;
+          // (EXACT: the second half's last pair ends one MFMA early, for the comparison above)
+          constexpr bool EARLY = EXACT && slot % 2 == 0;
+          constexpr int jlo = !EARLY ? i * 4 / M : i == 0 ? 0 : std::min(4, (4 * i + M - 2) / (M - 1));
+          constexpr int jhi = !EARLY ? (i + 1) * 4 / M : std::min(4, (4 * (i + 1) + M - 2) / (M - 1));
           if (slot == 1 && i == 0 && MASK) mask_scores(t0, 0);
           if (slot == 3 && i == 0 && MASK) mask_scores(s1, 1);
 #pragma unroll
           for (int j = jlo; j < jhi; ++j) {
-            if (slot == 0) softmax_pair(4 + j, s1, pb1, lsum);   // S1(t-1), second half
-            if (slot == 1) softmax_pair(j, t0, pb0, lsum);       // S0(t), first half
-            if (slot == 2) softmax_pair(4 + j, t0, pb0, lsum);   // S0(t), second half
-            if (slot == 3) softmax_pair(j, s1, pb1, lsum);       // S1(t), first half
+            if (slot == 0) softmax_pair<EXACT>(4 + j, s1, pb1, lsum);   // S1(t-1), second half
+            if (slot == 1) softmax_pair<EXACT>(j, t0, pb0, lsum);       // S0(t), first half
+            if (slot == 2) softmax_pair<EXACT>(4 + j, t0, pb0, lsum);   // S0(t), second half
+            if (slot == 3) softmax_pair<EXACT>(j, s1, pb1, lsum);       // S1(t), first half
+          }
+          if constexpr (EXACT) {
+            if constexpr (slot % 2 == 0 && i == M - 1)
+              settle_half(slot == 0 ? s1 : t0, slot == 0 ? pb1 : pb0, over, oacc, msb, m_run, l_run, lsum, [&](float up) __attribute__((always_inline)) {
+                f32x16& next = slot == 0 ? t0 : s1;
+#pragma unroll
+                for (int x = 0; x < 16; ++x) next[x] -= up;
+              });
           }
           __builtin_amdgcn_sched_barrier(0);
         });
       };
 
       // ---- does the reference have to move before this tile? ------------------------------------------------------
-      if (t - kvec_base == kWave) {
+      if (!EXACT && t - kvec_base == kWave) {
         kvec_base = t;
         kvec = tile_kmax_bits[min(t + lane, n_k_tiles - 1)];
         // waited for here, once in 64 tiles: left to the first use below, the wait would sit on the common path too and
         // there also wait for the next tile's loads, half a tile after they were issued instead of a whole one
         asm volatile("" ::"v"(kvec));
       }
-      const uint32_t kmax_bits = __builtin_amdgcn_readlane(kvec, t - kvec_base);
-      if (t == t_begin || kmax_bits > thr_bits) {
+      const uint32_t kmax_bits = EXACT ? 0u : __builtin_amdgcn_readlane(kvec, t - kvec_base);
+      if (t == t_begin || (!EXACT && kmax_bits > thr_bits)) {
 #ifdef COROPE_TRACE
         ++exact_passes;
 #endif
-        if (t > t_begin) drain();
+        if (!EXACT && t > t_begin) drain();
         f32x16 r0 = f32x16{0}, r1 = f32x16{0};
 #pragma unroll
         for (int kc = 0; kc < M; ++kc) {
@@ -418,7 +485,7 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
         // this block so far (m_true, a lower bound of the row's running maximum): the row's largest probability stays
         // above 2^-kPipeLift, far inside fp32 / bf16 range, however often the block runs.
         m_true = fmaxf(m_true, half_max(mt));
-        float m_new = fmaxf(m_run, fmaxf(m_true, fminf(lift_target, m_true + kPipeLift)));
+        float m_new = EXACT ? m_true : fmaxf(m_run, fmaxf(m_true, fminf(lift_target, m_true + kPipeLift)));
         if constexpr (CUT) m_new = m_new == -INFINITY ? 0.f : m_new;   // (a row that sees no key of this tile sees none of the piece's later ones)
         const float alpha = fast_exp2(m_run - m_new);   // m_new is finite: every row sees key 0 of tile 0, and a piece that starts later has the line above
         l_run = (l_run + lsum) * alpha;
@@ -434,9 +501,11 @@ __global__ __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(2, 2)
           asm volatile("" : "+v"(x));   // sixteen values of their own: one value in sixteen places is tied to the first of them
           msb[i] = x;
         }
-        const float m_min = -wave_reduce_max(-m_run);
-        const float thr = (m_min + kPipeMargin) / q_bound_wave;
-        thr_bits = __builtin_amdgcn_readfirstlane(thr > 0.f ? __builtin_bit_cast(uint32_t, thr) : 0u);
+        if constexpr (!EXACT) {
+          const float m_min = -wave_reduce_max(-m_run);
+          const float thr = (m_min + kPipeMargin) / q_bound_wave;
+          thr_bits = __builtin_amdgcn_readfirstlane(thr > 0.f ? __builtin_bit_cast(uint32_t, thr) : 0u);
+        }
         // nothing is pending now: an all-masked S1 and a zero P1 make the pending half of the tile body a no-op
 #pragma unroll
         for (int i = 0; i < 16; ++i) s1[i] = -INFINITY;
@@ -536,10 +605,10 @@ __global__ __launch_bounds__(D / 16 * kWave) void rope_attn_fwd_join_kernel(FwdP
 }
 
 // ---- host-side launch -----------------------------------------------------------------------------------------
-template <int D, bool CAUSAL, int NW>
+template <int D, bool CAUSAL, int NW, bool EXACT>
 static hipError_t launch_pipe_waves(FwdParams p, hipStream_t stream) {
   using Cfg = FwdPipeCfg<D, NW>;
-  auto kern = rope_attn_fwd_pipe_kernel<D, CAUSAL, NW>;
+  auto kern = rope_attn_fwd_pipe_kernel<D, CAUSAL, NW, false, EXACT>;
   static std::atomic<uint64_t> lds_ok{0};
   if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
   p.num_m_blocks = (p.N + Cfg::kBlockM - 1) / Cfg::kBlockM;
@@ -586,10 +655,10 @@ int64_t fwd_parts_bytes(int B, int H, int N, int D, bool causal) {
   return 0;
 }
 
-template <int D, bool CAUSAL>
+template <int D, bool CAUSAL, bool EXACT>
 static hipError_t launch_pipe_cut(FwdParams p, int shares, hipStream_t stream) {
   using Cfg = FwdPipeCfg<D, kCutWaves>;
-  auto kern = rope_attn_fwd_pipe_kernel<D, CAUSAL, kCutWaves, true>;
+  auto kern = rope_attn_fwd_pipe_kernel<D, CAUSAL, kCutWaves, true, EXACT>;
   static std::atomic<uint64_t> lds_ok{0};
   if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), Cfg::kLdsBytes, lds_ok); e != hipSuccess) return e;
   p.num_m_blocks = (p.N + Cfg::kBlockM - 1) / Cfg::kBlockM;
@@ -602,15 +671,25 @@ static hipError_t launch_pipe_cut(FwdParams p, int shares, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int D, bool CAUSAL>
+template <int D, bool CAUSAL, bool EXACT>
 static hipError_t launch_pipe_cfg(const FwdParams& p, hipStream_t stream) {
   if (p.parts != nullptr)
-    if (const int shares = fwd_shares<D>(p.N, p.BH, CAUSAL); shares > 0) return launch_pipe_cut<D, CAUSAL>(p, shares, stream);
-  return use_small_tiles(p.N, p.BH, FwdPipeCfg<D, 4>::kLdsBytes) ? launch_pipe_waves<D, CAUSAL, 4>(p, stream)
-                                                                  : launch_pipe_waves<D, CAUSAL, 8>(p, stream);
+    if (const int shares = fwd_shares<D>(p.N, p.BH, CAUSAL); shares > 0) return launch_pipe_cut<D, CAUSAL, EXACT>(p, shares, stream);
+  return use_small_tiles(p.N, p.BH, FwdPipeCfg<D, 4>::kLdsBytes) ? launch_pipe_waves<D, CAUSAL, 4, EXACT>(p, stream)
+                                                                  : launch_pipe_waves<D, CAUSAL, 8, EXACT>(p, stream);
+}
+
+template <bool EXACT>
+static hipError_t launch_pipe(const FwdParams& p, int D, bool causal, hipStream_t stream) {
+  if (D == 128) return causal ? launch_pipe_cfg<128, true, EXACT>(p, stream) : launch_pipe_cfg<128, false, EXACT>(p, stream);
+  return causal ? launch_pipe_cfg<64, true, EXACT>(p, stream) : launch_pipe_cfg<64, false, EXACT>(p, stream);
 }
 
 hipError_t launch_rope_attn_fwd_prerotated(const FwdParams& p, int D, bool causal, hipStream_t stream) {
+#ifdef COROPE_F16
+  // without key-norm maxima: P and V in fp16
+  if (p.tile_kmax == nullptr && p.exact && (D == 64 || D == 128)) return launch_pipe<true>(p, D, causal, stream);
+#endif
   // without key-norm maxima: the kernel that needs none
   if (p.tile_kmax == nullptr) return launch_rope_attn_fwd_single_prerotated(p, D, causal, stream);
 #ifndef COROPE_F16
@@ -625,8 +704,7 @@ hipError_t launch_rope_attn_fwd_prerotated(const FwdParams& p, int D, bool causa
   if (D == 128 && !use_small_tiles(p.N, p.BH) && g_fwd_wave_rows.load(std::memory_order_relaxed) == 64)
     return launch_rope_attn_fwd_prerotated_rows64(p, D, causal, stream);
 #endif
-  if (D == 128) return causal ? launch_pipe_cfg<128, true>(p, stream) : launch_pipe_cfg<128, false>(p, stream);
-  return causal ? launch_pipe_cfg<64, true>(p, stream) : launch_pipe_cfg<64, false>(p, stream);
+  return launch_pipe<false>(p, D, causal, stream);
 }
 
 }  // namespace COROPE_NS

@@ -112,9 +112,9 @@ _FWD_ROTATED_MIN_N = {64: 768, 128: 129, 256: 129}
 _FWD_SMALL_ITEMS = 256   # 256-row items below this take the 128-row form: the compute units of an MI355X
 
 
-# fp16 tensors, forward of a call that will be differentiated: "exact" = the single-launch kernel's bookkeeping, which
-# keeps P and V in fp16 (O within 1.2e-2 of the fp32 oracle at the reference's verification temperature sm_scale = 0.5,
-# gradients within its 0.15 / 5e-3 thresholds), from the rotated path's lengths on run on a key copy rotated beforehand;
+# fp16 tensors, forward of a call that will be differentiated: "exact" keeps P and V in fp16 (O within 1.2e-2 of the fp32 oracle at the
+# reference's verification temperature sm_scale = 0.5, gradients within its 0.15 / 5e-3 thresholds): the pipelined forward that looks at
+# each half tile's probabilities before it uses them, at D = 256 the single-launch kernel on a key copy rotated beforehand;
 # "fast" = the pipelined forward (bf16 probabilities against a V converted to bf16 on its way into LDS: as fast as with
 # bf16 tensors, O within one bf16 ulp), whose O carries bf16's rounding of V into delta = rowsum(O * dO) and through it
 # into dQ and dK: up to 0.24 there instead of 0.05.  A forward that will not be differentiated always takes the fast form.
@@ -122,8 +122,8 @@ FP16_TRAINING_FORWARD = "exact"
 
 
 def use_rotated_path(N, D, training, slabs=None):
-    """Whether the operator rotates the operands ahead of the attention kernels at this shape.  slabs: batch * query heads, or None
-    for an fp16 forward without gradients, whose kernel on rotated keys keeps P and V in bf16: it is left where it was."""
+    """Whether the operator rotates the operands ahead of the attention kernels at this shape.  slabs: batch * query heads; None leaves
+    out the lengths that depend on it (an fp16 forward at D = 256 has only the single-launch kernel there)."""
     if N * D < TRAIN_ROTATED_MIN_ND or D > _ROTATED_PATH_MAX_D:
         return N >= TWO_LAUNCH_MIN_N and D <= _ROTATED_PATH_MAX_D
     if training or N >= TWO_LAUNCH_MIN_N or N * D >= _FWD_ROTATED_MIN_ND:
@@ -161,26 +161,27 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
             q, k, v, strides = q.contiguous(), k.contiguous(), v.contiguous(), None
     o = torch.empty(q.shape, device=q.device, dtype=q.dtype)
     M = torch.empty((B, H, N), device=q.device, dtype=torch.float32)
-    if two_launch is None:
-        two_launch = use_rotated_path(N, D, training=keep_rotated, slabs=B * H if q.dtype == torch.bfloat16 else None)
+    asked = two_launch is not None
+    if not asked:
+        two_launch = use_rotated_path(N, D, training=keep_rotated, slabs=B * H if q.dtype == torch.bfloat16 or D <= 128 else None)
     rotated = None
     Hkv = k.shape[1]
     with _on_device(q):
         # scratch for the pieces of query blocks that the kernel on rotated keys cuts among workgroups (0: none are cut).  Only speed needs it
         parts, nbytes = None, 0
-        if two_launch and D <= 128 and not (q.dtype == torch.float16 and keep_rotated and FP16_TRAINING_FORWARD != "fast"):
+        # fp16 with gradients, or so short that the fast form's kernel never served it: P and V stay fp16 (no key-norm maxima)
+        fp16 = q.dtype == torch.float16
+        exact = fp16 and two_launch and (FP16_TRAINING_FORWARD != "fast" if keep_rotated else not asked and not use_rotated_path(N, D, False))
+        if two_launch and D <= 128:
             nbytes = lib.corope_rope_attn_fwd_parts_bytes(B, H, N, D, int(bool(causal)))
             if nbytes > 0:
                 try:
                     parts = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
                 except torch.cuda.OutOfMemoryError:
                     pass
-        if parts is not None and strides is None:
+        if strides is None and (parts is not None or (exact and D <= 128)):
             strides = tuple((ctypes.c_int64 * 3)(h * N * D, N * D, D) for h in (H, Hkv, Hkv))   # (contiguous; an axis of length 1 may say otherwise)
         if strides is not None:
-            fp16 = q.dtype == torch.float16
-            # fp16 with gradients: P and V stay fp16 (no key-norm maxima: the single-launch kernel, on the rotated copy)
-            exact = fp16 and keep_rotated and FP16_TRAINING_FORWARD != "fast"
             q_rot = torch.empty(q.shape, device=q.device, dtype=q.dtype) if (two_launch and keep_rotated) else None
             k_rot = torch.empty(k.shape, device=q.device, dtype=q.dtype) if two_launch else None
             kmax = torch.empty((B, Hkv, (N + 63) // 64), device=q.device, dtype=torch.float32) if (two_launch and not exact) else None
@@ -196,9 +197,8 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
                 rotated = (q_rot, k_rot)
         elif q.dtype == torch.float16:
             # the reference's dtype: one entry point covers the forms, grouped-query K/V included.  With key-norm maxima: the
-            # pipelined kernel (bf16 probabilities against a V converted to bf16 on its way into LDS); without, for a forward
-            # with gradients: the single-launch kernel on the rotated copy, P and V in fp16
-            exact = keep_rotated and FP16_TRAINING_FORWARD != "fast"
+            # pipelined kernel (bf16 probabilities against a V converted to bf16 on its way into LDS); without (here D = 256):
+            # the single-launch kernel on the rotated copy, P and V in fp16
             q_rot = torch.empty_like(q) if (two_launch and keep_rotated) else None
             k_rot = torch.empty_like(k) if two_launch else None
             kmax = torch.empty((B, Hkv, (N + 63) // 64), device=q.device, dtype=torch.float32) if (two_launch and not exact) else None

@@ -179,3 +179,50 @@ def test_fp16_grouped_query(pkg, monkeypatch, B, Hq, Hkv, N, D, causal, rotated)
         print(f"  {name}: max-abs {err.max():.3e} mean-abs {err.mean():.3e}")
         assert a.shape == b.shape and torch.isfinite(a).all(), name
         assert err.max() <= 2e-2 * (math.sqrt(G) if name in ("dK", "dV") else 1.0), name
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,H,Hkv,N,D,cut", [(2, 2, 1, 1, 64, False), (1, 2, 2, 64, 128, False), (1, 3, 3, 65, 64, False), (2, 4, 2, 257, 128, False),
+                                             (1, 40, 40, 1000, 64, False), (3, 60, 60, 500, 128, False), (1, 2, 1, 3001, 128, True), (1, 3, 3, 2500, 64, True)])
+def test_pipelined_forward_with_fp16_probabilities(pkg, monkeypatch, B, H, Hkv, N, D, cut, causal):
+    """The forward of a call that will be differentiated, on rotated keys, against the single launch on the original ones: the same
+    rounding points, so O may differ by the rounding of P (2^-11 of a weight, in either kernel) and of O, lse by that of fp32.  Some keys are
+    up to sixteen times as long as the others, so that rows meet scores more than 16 binary orders above their reference at any
+    place of a tile, also in the half that is still pending at the end of a row."""
+    lib = pkg._lib.load()
+    assert (lib.corope_rope_attn_fwd_parts_bytes(B, H, N, D, int(causal)) > 0) == cut
+    gen = torch.Generator().manual_seed(N + D)
+    q, k, v = (torch.randn(B, h, N, D, generator=gen) for h in (H, Hkv, Hkv))
+    k = k * torch.exp2(torch.randint(0, 5, (B, Hkv, N, 1), generator=gen) * (torch.rand(B, Hkv, N, 1, generator=gen) < 0.02))
+    if N > 64:
+        k[:, :, -1] *= 16
+    q, k, v = (t.cuda().half() for t in (q, k, v))
+    c, s = (t.cuda() for t in O.precompute_freqs_cis(D, N))
+    saved = {}
+    for rotated in (True, False):
+        monkeypatch.setattr(pkg.rope_attn, "TWO_LAUNCH_MIN_N", 1 if rotated else 1 << 30)
+        monkeypatch.setattr(pkg.rope_attn, "TRAIN_ROTATED_MIN_ND", 1 if rotated else 1 << 60)
+        out = pkg.attention(q.requires_grad_(True), k, v, causal, 1 / math.sqrt(D), c, s)
+        saved[rotated] = out.detach().float(), out.grad_fn.saved_tensors[4]
+    (o, M), (ro, rM) = saved[True], saved[False]
+    assert torch.isfinite(o).all() and torch.isfinite(M).all()
+    assert (o - ro).abs().max() <= 3 * 2.0 ** -11 * v.float().abs().max()
+    assert ((M - rM).abs() <= 1e-3 + 2.0 ** -20 * rM.abs()).all()
+
+
+def test_fp16_forward_of_inputs_that_are_not_finite(pkg):
+    """A query row that is NaN or infinite spoils its own output row and no other."""
+    B, H, N, D = 1, 2, 300, 128
+    q, k, v = (seeded((B, H, N, D), 60 + i).cuda().half() for i in range(3))
+    c, s = (t.cuda() for t in O.precompute_freqs_cis(D, N))
+    clean = pkg.attention(q.clone().requires_grad_(True), k, v, True, 1 / math.sqrt(D), c, s).detach()
+    for bad in (float("nan"), float("inf")):
+        x = q.clone()
+        x[0, 1, 170] = bad
+        out = pkg.attention(x.requires_grad_(True), k, v, True, 1 / math.sqrt(D), c, s).detach()
+        assert torch.isnan(out[0, 1, 170]).all()
+        keep = torch.ones(N, dtype=torch.bool)
+        keep[160:192] = False      # (rows that share a wave may be rescaled together: held to the rounding of P and O instead)
+        assert torch.equal(out[0, 0], clean[0, 0]) and torch.equal(out[0, 1][keep], clean[0, 1][keep])
+        near = [i for i in range(160, 192) if i != 170]
+        assert (out[0, 1, near].float() - clean[0, 1, near].float()).abs().max() <= 3 * 2.0 ** -11 * v.float().abs().max()

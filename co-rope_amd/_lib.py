@@ -5,6 +5,7 @@ the library is missing or a call fails, an exception is raised."""
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
@@ -62,12 +63,30 @@ SIGNATURES = {
     "corope_gqa_bwd_f16": (_I, [_P] * 8 + [_I] * 5 + [_F, _F, _P, _L, _P]),
 }
 
+# The operators' host side in native code (csrc/host_calls.cpp): one Python call per forward or backward instead of one per allocation
+# and a ctypes call.  Entry points it goes through, in its order.
+HOST_PATH = os.path.join(_HERE, "lib", "corope_host_calls.so")
+HOST_CALLS = ("corope_rope_attn_fwd_cut", "corope_rope_attn_bwd_rotated", "corope_gqa_fwd", "corope_gqa_fwd_f16", "corope_gqa_bwd", "corope_gqa_bwd_f16")
+
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 
 class CoRopeLibraryError(RuntimeError):
     """The native library is missing, stale, or a launch failed."""
+
+
+def _bind_host(lib):
+    """Sets lib.host to (native host module, its table of lib's entry points)."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise CoRopeLibraryError(f"{HOST_PATH} not found: build it with `python co-rope_amd/build.py`")
+        spec = importlib.util.spec_from_file_location("corope_host_calls", HOST_PATH)
+        _host = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(_host)
+    lib.host = _host, _host.make_table(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in HOST_CALLS))
 
 
 def load():
@@ -91,6 +110,7 @@ def load():
             fn.restype, fn.argtypes = res, args
         if lib.corope_amd_version() != ABI_VERSION:
             raise CoRopeLibraryError(f"{LIB_PATH} has ABI version {lib.corope_amd_version()}, expected {ABI_VERSION}")
+        _bind_host(lib)
         _lib = lib
     return _lib
 
@@ -113,6 +133,7 @@ def load_trace():
             fn.restype, fn.argtypes = res, args
         lib.corope_debug_trace.restype, lib.corope_debug_trace.argtypes = None, [_P]
         lib.corope_debug_set_forms.restype, lib.corope_debug_set_forms.argtypes = _I, [_I, _I]
+        _bind_host(lib)
         _trace_lib = lib
     return _trace_lib
 

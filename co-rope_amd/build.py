@@ -4,13 +4,14 @@ Run as ``python co-rope_amd/build.py`` or call ``build()``; the result lands in
 ``co-rope_amd/lib/libcorope_amd.so`` and is what ``_lib.load()`` opens.  Beside it, for measurement only:
 ``libcorope_amd_trace.so`` (the same sources with -DCOROPE_TRACE: the attention kernels stamp a clock at their phase
 boundaries into a buffer ``bench.py --phase-trace`` hands them, and a call forces kernel forms for the tests).
-``build_program`` compiles a stand-alone HIP program with the same flags (``bench.py --mfma-rate`` uses it)."""
+``corope_host_calls.so`` beside them is the Python binding's native half (host code only).  ``build_program`` compiles a stand-alone HIP program with the same flags (``bench.py --mfma-rate`` uses it)."""
 from __future__ import annotations
 
 import glob
 import os
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
@@ -25,6 +26,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libcorope_amd.so")
 TRACE_LIB = os.path.join(LIBDIR, "libcorope_amd_trace.so")
+HOST_LIB = os.path.join(LIBDIR, "corope_host_calls.so")
 
 # compiled a second time with -DCOROPE_F16 (fp16 elements, namespace corope_f16)
 F16_SOURCES = ["rope_rotate.hip", "rope_attn_fwd.hip", "rope_attn_fwd_pipe.hip", "rope_attn_bwd_pre.hip", "rope_attn_bwd.hip", "corope_gqa_fwd.hip",
@@ -88,6 +90,20 @@ def _link(objs, out, shared=True):
     return out
 
 
+def build_host():
+    """The native host side of the operators (csrc/host_calls.cpp): host code against torch's headers, no device code."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "host_calls.cpp"), "-o", HOST_LIB,
+           "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on host_calls.cpp:\n{r.stderr}")
+    return HOST_LIB
+
+
 def build(verbose=False, extra_flags=(), extras=True):
     """Compiles every source.  ``extras``: also the trace variant of the library."""
     os.makedirs(LIBDIR, exist_ok=True)
@@ -95,11 +111,13 @@ def build(verbose=False, extra_flags=(), extras=True):
     if extras:
         jobs += [(s, j[1] + ["-DCOROPE_TRACE"], j[2] + ".trace") for j in list(jobs) for s in [j[0]]]
     with ThreadPoolExecutor(max_workers=8) as ex:
+        host = ex.submit(build_host)
         results = list(ex.map(lambda j: _compile(*j), jobs))
     if verbose:
         for (_, err), j in zip(results, jobs):
             if err.strip():
                 print(f"--- {j[0]}{j[2]}\n{err}", file=sys.stderr)
+    host.result()
     n = len(SOURCES) + len(F16_SOURCES)
     _link([o for o, _ in results[:n]], LIB)
     if extras:

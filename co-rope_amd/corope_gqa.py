@@ -11,7 +11,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .rope_attn import _PADDED_D, gather_halves, spread_halves
+from .rope_attn import _PADDED_D, _on_device, _stream_ptr, gather_halves, spread_halves
 
 
 class _CoRopeGqaAttn(torch.autograd.Function):
@@ -38,11 +38,15 @@ class _CoRopeGqaAttn(torch.autograd.Function):
             raise ValueError(f"q, k, v must all be bfloat16 or all float16 (got {q.dtype}, {k.dtype}, {v.dtype})")
         lib = _lib.load()
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        o = torch.empty_like(q)
-        with torch.cuda.device(q.device):
-            fwd = lib.corope_gqa_fwd_f16 if q.dtype == torch.float16 else lib.corope_gqa_fwd
-            rc = fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, Hq, Hkv, N, D,
-                     float(sm_scale), float(theta), torch.cuda.current_stream(q.device).cuda_stream)
+        with _on_device(q):
+            host, table = lib.host
+            rc = host.gqa_forward(table, q, k, v, float(sm_scale), float(theta), q.device.index, _stream_ptr(q))
+            if type(rc) is tuple:
+                o, rc = rc[0], _lib.OK
+            elif rc is None:   # not plain tensors
+                o = torch.empty_like(q)
+                fwd = lib.corope_gqa_fwd_f16 if q.dtype == torch.float16 else lib.corope_gqa_fwd
+                rc = fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, Hq, Hkv, N, D, float(sm_scale), float(theta), _stream_ptr(q))
         _lib.check(rc, "corope_gqa_fwd")
         # what the reference keeps (:451), minus inv_freq (theta is enough), plus the output: the backward takes a
         # reference value for its row sums from it (accuracy of dQ on sharply peaked rows; not needed mathematically)
@@ -86,10 +90,10 @@ BACKWARD_WORKSPACE_CAP_BYTES = 8 << 30
 _workspaces = {}   # (device index, stream handle) -> uint8 tensor
 
 
-def _cached_workspace(device, B, Hq, Hkv, N, D):
+def _cached_workspace(device, stream, B, Hq, Hkv, N, D):
     one, full = backward_min_workspace_bytes(B, Hq, Hkv, N, D), backward_workspace_bytes(B, Hq, Hkv, N, D)
     want = min(full, max(1, BACKWARD_WORKSPACE_CAP_BYTES // one) * one)
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < want:
         _workspaces.pop(key, None)
@@ -135,14 +139,21 @@ def corope_gqa_backward(q, k, v, grad_output, sm_scale, theta, workspace=None, o
     out_c = None if out is None else out.contiguous()
     o_ptr = None if out_c is None else out_c.data_ptr()
     if workspace is None:
-        workspace = _cached_workspace(q.device, B, Hq, Hkv, N, D)
+        workspace = _cached_workspace(q.device, _stream_ptr(q), B, Hq, Hkv, N, D)
     have = workspace.numel() * workspace.element_size()
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    with torch.cuda.device(q.device):
+    with _on_device(q):
+        if out_c is not None:
+            host, table = lib.host
+            grads = host.gqa_backward(table, q, k, v, out_c, d_o, workspace, float(sm_scale), float(theta), q.device.index, _stream_ptr(q))
+            if type(grads) is int:
+                _lib.check(grads, "corope_gqa_bwd")
+            if grads is not None:
+                return grads
+        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         bwd = lib.corope_gqa_bwd_f16 if q.dtype == torch.float16 else lib.corope_gqa_bwd
         rc = bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o_ptr, d_o.data_ptr(), dq.data_ptr(), dk.data_ptr(),
                  dv.data_ptr(), B, Hq, Hkv, N, D, float(sm_scale), float(theta), workspace.data_ptr(),
-                 have, torch.cuda.current_stream(q.device).cuda_stream)
+                 have, _stream_ptr(q))
     _lib.check(rc, "corope_gqa_bwd")
     return dq, dk, dv
 

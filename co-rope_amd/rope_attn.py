@@ -144,6 +144,45 @@ def _view_strides(t):
     return (ctypes.c_int64 * 3)(sb, sh, sn)
 
 
+def _route(dtype, slabs, N, D, keep_rotated, two_launch=None):
+    """(rotate K ahead?, keep P and V in fp16 there?) for a forward."""
+    asked = two_launch is not None
+    if not asked:
+        two_launch = use_rotated_path(N, D, keep_rotated, slabs if dtype == torch.bfloat16 or D <= 128 else None)
+    # fp16 with gradients, or so short that the fast form's kernel never served it: P and V stay fp16 (no key-norm maxima)
+    return two_launch, (dtype == torch.float16 and two_launch and
+                        (FP16_TRAINING_FORWARD != "fast" if keep_rotated else not asked and not use_rotated_path(N, D, False)))
+
+
+def _scratch(nbytes, device):
+    """Scratch in which launches leave the partial sums of blocks that they cut among workgroups (0 bytes: none are cut), or None.  Only
+    speed needs it."""
+    try:
+        return torch.empty(nbytes, device=device, dtype=torch.uint8) if nbytes > 0 else None
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
+def _fwd_parts(lib, q, causal):
+    B, H, N, D = q.shape
+    nbytes = lib.corope_rope_attn_fwd_parts_bytes(B, H, N, D, int(bool(causal))) if D <= 128 else 0
+    return _scratch(nbytes, q.device), nbytes
+
+
+def _native_forward(lib, q, k, v, causal, sm_scale, fc, fs, keep):
+    """What _forward returns, by the native host side; None where this is not a plain call (then _check_inputs and _forward do it)."""
+    if q.dim() != 4 or not q.is_cuda or q.shape[3] not in _SUPPORTED_D or torch.cuda.current_device() != q.device.index:
+        return None
+    B, H, N, D = q.shape
+    rotated, exact = _route(q.dtype, B * H, N, D, keep)
+    host, table = lib.host
+    out = host.rope_forward(table, q, k, v, fc, fs, causal, float(sm_scale), rotated, exact, keep, q.device.index, _stream_ptr(q),
+                            _fwd_parts(lib, q, causal)[0] if rotated else None)
+    if type(out) is int:
+        _lib.check(out, "corope_rope_attn_fwd_cut")
+    return out and (out[0], out[1], fc, fs, out[2:] if out[2] is not None else None)
+
+
 def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, keep_rotated=False):
     """Runs the forward kernels; returns (o, M, fc, fs, rotated) with the tables in the form the kernels were given.
     ``rotated`` is (q_rot, k_rot) when ``keep_rotated`` was asked for and the two-launch path ran, else None.
@@ -161,24 +200,12 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
             q, k, v, strides = q.contiguous(), k.contiguous(), v.contiguous(), None
     o = torch.empty(q.shape, device=q.device, dtype=q.dtype)
     M = torch.empty((B, H, N), device=q.device, dtype=torch.float32)
-    asked = two_launch is not None
-    if not asked:
-        two_launch = use_rotated_path(N, D, training=keep_rotated, slabs=B * H if q.dtype == torch.bfloat16 or D <= 128 else None)
+    two_launch, exact = _route(q.dtype, B * H, N, D, keep_rotated, two_launch)
+    fp16 = q.dtype == torch.float16
     rotated = None
     Hkv = k.shape[1]
     with _on_device(q):
-        # scratch for the pieces of query blocks that the kernel on rotated keys cuts among workgroups (0: none are cut).  Only speed needs it
-        parts, nbytes = None, 0
-        # fp16 with gradients, or so short that the fast form's kernel never served it: P and V stay fp16 (no key-norm maxima)
-        fp16 = q.dtype == torch.float16
-        exact = fp16 and two_launch and (FP16_TRAINING_FORWARD != "fast" if keep_rotated else not asked and not use_rotated_path(N, D, False))
-        if two_launch and D <= 128:
-            nbytes = lib.corope_rope_attn_fwd_parts_bytes(B, H, N, D, int(bool(causal)))
-            if nbytes > 0:
-                try:
-                    parts = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-                except torch.cuda.OutOfMemoryError:
-                    pass
+        parts, nbytes = _fwd_parts(lib, q, causal) if two_launch else (None, 0)
         if strides is None and (parts is not None or (exact and D <= 128)):
             strides = tuple((ctypes.c_int64 * 3)(h * N * D, N * D, D) for h in (H, Hkv, Hkv))   # (contiguous; an axis of length 1 may say otherwise)
         if strides is not None:
@@ -254,20 +281,22 @@ def _backward_rotated(lib, q_rot, k_rot, v, o, do, M, fc, fs, sm_scale, causal):
     """(dq, dk, dv, ...) of the operator from the rotated q and k its forward kept."""
     B, H, N, D = q_rot.shape
     Hkv = k_rot.shape[1]
-    do_st = None
-    if not do.is_contiguous():
-        do_st = _view_strides(do) if D <= 128 else None
-        do = do if do_st is not None else do.contiguous()
-    dq, dk, dv = torch.empty_like(q_rot), torch.empty_like(k_rot), torch.empty_like(k_rot)
-    delta = torch.empty_like(M)
+    # (how many pieces there are depends on the device: at most 128 MiB with 256 compute units)
     with _on_device(q_rot):
-        # scratch in which the dQ and the dK+dV launch leave the partial sums of blocks they cut among workgroups (0: none are cut); how
-        # many pieces there are depends on the device (at most 128 MiB with 256 compute units).  Only speed needs it
         nbytes = lib.corope_rope_attn_bwd_rotated_parts_bytes(B, H, Hkv, N, D, int(causal))
-        try:
-            parts = torch.empty(nbytes, device=q_rot.device, dtype=torch.uint8) if nbytes > 0 else None
-        except torch.cuda.OutOfMemoryError:
-            parts = None
+        parts = _scratch(nbytes, q_rot.device)
+        host, table = lib.host
+        out = host.rope_backward(table, q_rot, k_rot, v, o, do, M, fc, fs, causal, sm_scale, q_rot.device.index, _stream_ptr(q_rot), parts)
+        if type(out) is int:
+            _lib.check(out, "corope_rope_attn_bwd_rotated")
+        if out is not None:
+            return *out, None, None, None, None, None
+        do_st = None
+        if not do.is_contiguous():
+            do_st = _view_strides(do) if D <= 128 else None
+            do = do if do_st is not None else do.contiguous()
+        dq, dk, dv = torch.empty_like(q_rot), torch.empty_like(k_rot), torch.empty_like(k_rot)
+        delta = torch.empty_like(M)
         rc = lib.corope_rope_attn_bwd_rotated(q_rot.data_ptr(), k_rot.data_ptr(), v.data_ptr(), None, o.data_ptr(), do.data_ptr(), do_st,
                                               M.data_ptr(), delta.data_ptr(), fc.data_ptr(), fs.data_ptr(), fc.stride(0), dq.data_ptr(),
                                               dk.data_ptr(), dv.data_ptr(), B, H, Hkv, N, D, sm_scale, int(causal),
@@ -281,9 +310,8 @@ class _FusedRopeAttn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, causal, sm_scale, freqs_cos, freqs_sin, warp_specialize=True):
-        _check_inputs(q, k, v, freqs_cos, freqs_sin)
-        B, H, N, D = q.shape
-        training = any(ctx.needs_input_grad[:3])
+        needs = ctx.needs_input_grad
+        training = needs[0] or needs[1] or needs[2]
         if training:
             # v is kept for the backward, and a view kept as it is would hold the fused projection it is cut from, and would be lost
             # if the caller overwrites that before the backward: a view is copied (377 -> 386 us forward and backward at B1 Hq32 Hkv8 N3001 D128), q and k are kept
@@ -291,10 +319,14 @@ class _FusedRopeAttn(torch.autograd.Function):
             v = v.contiguous()
         # when a gradient will be asked for, the forward keeps its rotated q and k for the backward and the originals
         # are not saved (the reference saves q and k, fused_rope_attn.py:718, and re-rotates them in its backward)
-        o, M, fc, fs, rotated = _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, keep_rotated=training)
+        out = _native_forward(_lib.load(), q, k, v, causal, sm_scale, freqs_cos, freqs_sin, training)
+        if out is None:
+            _check_inputs(q, k, v, freqs_cos, freqs_sin)
+            out = _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, keep_rotated=training)
+        o, M, fc, fs, rotated = out
         # nothing to differentiate, nothing kept: saving q and k would copy strided views of a fused projection.  (Tables that
         # ask for a gradient get None, but the backward that says so runs and wants its tensors.)
-        if not any(ctx.needs_input_grad):
+        if not any(needs):
             return o
         ctx.rotated = rotated is not None
         if ctx.rotated:
@@ -302,7 +334,7 @@ class _FusedRopeAttn(torch.autograd.Function):
         else:
             ctx.save_for_backward(q.contiguous(), k.contiguous(), v.contiguous(), o, M, fc, fs)
         ctx.sm_scale = float(sm_scale)
-        ctx.HEAD_DIM = D
+        ctx.HEAD_DIM = q.shape[-1]
         ctx.causal = bool(causal)
         return o
 

@@ -510,7 +510,7 @@ template <int D, int NWAVES, int BLOCK_N, bool CAUSAL, bool PREROT, bool CUT = f
 __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<D>, kWavesPerSimd<D>))) void rope_attn_bwd_dq_kernel(BwdParams p) {
   using Cfg = DqCfg<D, NWAVES, BLOCK_N>;
   constexpr int NT = Cfg::kThreads;
-  constexpr bool STRIDED = D <= 128;
+  constexpr bool STRIDED = D <= 128, DELTA_ACC = D == 64;
   constexpr int KC = D / 16, NDB = D / 32, NKB = BLOCK_N / 32;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
@@ -664,6 +664,16 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) asm volatile("" ::"v"(qb[kc]), "v"(dob[kc]));
     asm volatile("" ::"v"(delta_q));
+    // ... and dP - delta, where the registers for it are there (D = 64)
+    f32x16 mdb;
+    if constexpr (DELTA_ACC) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float x = -delta_q;
+        asm volatile("" : "+v"(x));
+        mdb[i] = x;
+      }
+    }
 
     auto stage_next = [&]() __attribute__((always_inline)) {
       kst.store_rows(k_tile(cur ^ 1));
@@ -695,7 +705,9 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
                                          : mfma32(*reinterpret_cast<const u32x4*>(krow), qb[0], msb);
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc)
-          dpacc = mfma32(*reinterpret_cast<const u32x4*>(vrow + 16 * kc), dob[kc], kc == 0 ? f32x16{0} : dpacc);
+          dpacc = kc > 0 ? mfma32(*reinterpret_cast<const u32x4*>(vrow + 16 * kc), dob[kc], dpacc)
+                  : DELTA_ACC ? mfma32_from(*reinterpret_cast<const u32x4*>(vrow), dob[0], mdb)
+                              : mfma32(*reinterpret_cast<const u32x4*>(vrow), dob[0], f32x16{0});
         // mask on the raw scores under a wave-uniform branch of its own; register i holds key
         // n0 + 32*kb + 8*(i/4) + 4*lh + i%4, the lane-dependent part of the threshold goes into one opaque value
         if (need_mask) {
@@ -711,7 +723,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
             float pv = fast_exp2(sacc[i + e]);
-            ds[e] = pv * (dpacc[i + e] - delta_q);
+            ds[e] = DELTA_ACC ? pv * dpacc[i + e] : pv * (dpacc[i + e] - delta_q);
           }
           dsb[2 * kb + i / 8][(i % 8) / 2] = pack_elts(ds[0], ds[1]);
         }

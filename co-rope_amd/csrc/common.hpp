@@ -384,6 +384,17 @@ __device__ __forceinline__ u32x4 load_a_trans_of(const uint16_t* tile, int kbase
   return u32x4{a[0], a[1], b[0], b[1]};
 }
 
+// The same with the per-lane part already in the pointer: what is left are immediates.
+template <class T>
+__device__ __forceinline__ u32x4 load_a_trans_lane(const uint16_t* lane_tile, int kbase, int m0) {
+  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+  const uint16_t* p = lane_tile + T::off(kbase, m0);
+  s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p));
+  s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + T::off(8, 0)));
+  u32x2 a = __builtin_bit_cast(u32x2, lo), b = __builtin_bit_cast(u32x2, hi);
+  return u32x4{a[0], a[1], b[0], b[1]};
+}
+
 // The same read with the address split into its per-lane part and the rest: a_trans_lane_offset(stride) elements are
 // added to the tile once (per lane), load_a_trans_at then needs only compile-time offsets on top of that pointer.
 __device__ __forceinline__ int a_trans_lane_offset(int stride) {

@@ -143,7 +143,7 @@ template <int D, int NWAVES, int BLOCK_M, bool CAUSAL, bool DO_DV, bool DO_DK, b
 __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<D>, kWavesPerSimd<D>))) void rope_attn_bwd_dkdv_kernel(BwdParams p) {
   constexpr int DO_PAD = DO_DK ? (DO_DV ? kDkdvBothWaysPad : 8) : 32;
   constexpr int Q_PAD = DO_DK ? kDkdvBothWaysPad : 8;
-  constexpr bool V_LDS = DO_DV && DO_DK, STRIDED = PREROT && D <= 128;
+  constexpr bool V_LDS = DO_DV && DO_DK && D <= 128, STRIDED = PREROT && D <= 128, PIPED = DO_DV && DO_DK && D > 128;
   using Cfg = DkdvCfg<D, NWAVES, BLOCK_M, DO_PAD, Q_PAD>;
   constexpr int NT = Cfg::kThreads;
   constexpr int KC = D / 16, NDB = D / 32, NQB = BLOCK_M / 32;
@@ -173,6 +173,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   qst.out_scale = p.qk_scale;
   CopyStage<D, BLOCK_M, NT, DO_PAD> dst;
   float st_lse = 0.f, st_delta = 0.f;
+  [[maybe_unused]] int st_row = 0;
   int l_round = 0, l_it, l_iters, l_slab0, l_mt0, l_tph;
   const uint16_t* l_do;
   auto load_item = [&](int r) {    // false: no such item
@@ -199,7 +200,16 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     const int qs = l_slab0 + l_it / l_tph, m0 = (l_mt0 + l_it % l_tph) * BLOCK_M;
     qst.load(q_all + (int64_t)qs * N * D, p.cos, p.sin, p.fstride, m0, N);
     dst.load(STRIDED ? l_do + (qs - l_slab0) * p.do_sh : p.d_o + (int64_t)qs * N * D, m0, N, do_row_bytes<D, STRIDED>(p));
-    if (threadIdx.x < BLOCK_M) {
+    if constexpr (PIPED) {
+      // As they lie in memory: a sign changed here waits for the loads, and for the tile's before them, on the spot.  With one wave per SIMD
+      // that was 0.6 us of a tile's 1.85; with two the other wave fills it, and this form is no faster (D = 128) or 2 % slower (64).
+      st_row = m0 + threadIdx.x;
+      if (threadIdx.x < BLOCK_M) {
+        const int64_t at = (int64_t)qs * N + min(st_row, N - 1);
+        st_lse = p.lse[at];
+        st_delta = p.delta[at];
+      }
+    } else if (threadIdx.x < BLOCK_M) {
       int qi = m0 + threadIdx.x;
       // -M and -delta: what the S and dP products start from.  Rows past the end: M = +inf makes P = 0, so they
       // contribute nothing
@@ -219,8 +229,8 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
     qst.store_rows(q_tile(buf));
     dst.store_rows(do_tile(buf));
     if (threadIdx.x < BLOCK_M) {
-      lse_tile(buf)[threadIdx.x] = st_lse;
-      if constexpr (DO_DK) delta_tile(buf)[threadIdx.x] = st_delta;
+      lse_tile(buf)[threadIdx.x] = !PIPED ? st_lse : st_row < N ? -st_lse : -INFINITY;
+      if constexpr (DO_DK) delta_tile(buf)[threadIdx.x] = !PIPED ? st_delta : st_row < N ? -st_delta : 0.f;
     }
   };
   int cur = 0;   // ring stage of the tile being consumed
@@ -307,8 +317,81 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       const uint16_t* dos = do_tile(cur);
       const float* lses = lse_tile(cur);
       const float* deltas = delta_tile(cur);
+      if constexpr (PIPED) {
+        // One wave per SIMD: nothing overlaps what the wave itself does not, so the tile is one stream of 4 x 16 products with its operands
+        // RING ahead, the exponentials between the dP products, dS between the dV products, and the next tile's staging between the dK products.
+        static_assert(NQB == 1 && kWavesPerSimd<D> == 1, "one 32-row block per tile");
+        if (CAUSAL && m0 + 31 < wk_lo) {   // queries that lie above every key of the wave: it only stages its share
+          store_tile(cur ^ 1);
+        } else {
+          constexpr int RING = 4, TOTAL = 4 * KC;
+          const uint32_t tr = (4 * lh + lane % 16 / 4) * RowTile<D, Q_PAD>::kStride + RowTile<D, Q_PAD>::stagger(4 * lh) + 16 * (lane / 16 % 2) + 4 * (lane % 4);
+          const uint16_t *q_l = qs + RowTile<D, Q_PAD>::off(lq, 8 * lh), *do_l = dos + RowTile<D, DO_PAD>::off(lq, 8 * lh), *q_t = qs + tr, *do_t = dos + tr;
+          auto operand = [&](int n) __attribute__((always_inline)) {
+            const int i = n % KC;
+            return n < KC       ? *reinterpret_cast<const u32x4*>(q_l + 16 * i)
+                   : n < 2 * KC ? *reinterpret_cast<const u32x4*>(do_l + 16 * i)
+                   : n < 3 * KC ? load_a_trans_lane<RowTile<D, DO_PAD>>(do_t, 16 * (i / NDB), i % NDB * 32)
+                                : load_a_trans_lane<RowTile<D, Q_PAD>>(q_t, 16 * (i / NDB), i % NDB * 32);
+          };
+          u32x4 ring[RING];
+          f32x16 sacc, dpacc;
 #pragma unroll
-      for (int qb = 0; qb < NQB; ++qb) {
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 m4 = *reinterpret_cast<const f32x4*>(lses + 8 * g + 4 * lh);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sacc[4 * g + e] = m4[e];
+          }
+#pragma unroll
+          for (int n = 0; n < RING; ++n) ring[n] = operand(n);
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 d4 = *reinterpret_cast<const f32x4*>(deltas + 8 * g + 4 * lh);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dpacc[4 * g + e] = d4[e];
+          }
+          u32x4 pb[2], dsb[2];
+          __builtin_amdgcn_sched_barrier(0);
+          static_for<TOTAL>([&](auto n_c) __attribute__((always_inline)) {
+            constexpr int n = decltype(n_c)::value, slot = n / KC, i = n % KC;
+            const u32x4 a = ring[n % RING];
+            if constexpr (slot == 0) mfma32_acc_v(sacc, a, kb[i]);
+            if constexpr (slot == 1) mfma32_acc_v(dpacc, a, vb[i]);
+            if constexpr (slot == 2) dvacc[i % NDB] = mfma32(a, pb[i / NDB], dvacc[i % NDB]);
+            if constexpr (slot == 3) dkacc[i % NDB] = mfma32(a, dsb[i / NDB], dkacc[i % NDB]);
+            if constexpr (n + RING < TOTAL) ring[n % RING] = operand(n + RING);
+            if constexpr (n == 3 * KC + 1) store_tile(cur ^ 1);
+            // what the asm statements of the slot before left: nothing reads it behind product 0, which waits a little instead
+            if constexpr ((slot == 1 || slot == 2) && i == 0) asm volatile("s_nop 7");
+            if constexpr (slot == 1 && i == 1) {
+              if (CAUSAL && m0 < wk_hi) {
+                int rel = key - m0 - 4 * lh;
+                asm volatile("" : "+v"(rel));
+#pragma unroll
+                for (int x = 0; x < 16; ++x)
+                  if (8 * (x / 4) + x % 4 < rel) sacc[x] = -INFINITY;
+              }
+            }
+            // eight pairs over the products 1 .. KC - 1 of a slot
+            constexpr int lo = i == 0 ? 0 : (i - 1) * 8 / (KC - 1), hi = i == 0 ? 0 : i * 8 / (KC - 1);
+            if constexpr (slot == 1) {
+#pragma unroll
+              for (int j = lo; j < hi; ++j) {
+                sacc[2 * j] = fast_exp2(sacc[2 * j]);
+                sacc[2 * j + 1] = fast_exp2(sacc[2 * j + 1]);
+                pb[j / 4][j % 4] = pack_elts(sacc[2 * j], sacc[2 * j + 1]);
+              }
+            }
+            if constexpr (slot == 2) {
+#pragma unroll
+              for (int j = lo; j < hi; ++j) dsb[j / 4][j % 4] = pack_elts(sacc[2 * j] * dpacc[2 * j], sacc[2 * j + 1] * dpacc[2 * j + 1]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          });
+        }
+      }
+#pragma unroll
+      for (int qb = 0; qb < (PIPED ? 0 : NQB); ++qb) {
         const int mq0 = m0 + qb * 32;
         // queries of this 32-row block that lie above every key of the wave see none of them
         if (CAUSAL && mq0 + 31 < wk_lo) continue;
@@ -395,7 +478,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
           if constexpr (DO_DK) asm volatile("" : "+a"(dkacc[db]));
         }
       }
-      store_tile(cur ^ 1);
+      if constexpr (!PIPED) store_tile(cur ^ 1);
       cur ^= 1;
       __syncthreads();
     }

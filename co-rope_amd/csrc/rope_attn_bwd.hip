@@ -593,6 +593,8 @@ template <int D, int NWAVES, int BLOCK_N, bool CAUSAL, bool PREROT, bool CUT = f
 __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<D>, kWavesPerSimd<D>))) void rope_attn_bwd_dq_kernel(BwdParams p) {
   using Cfg = DqCfg<D, NWAVES, BLOCK_N>;
   constexpr int NT = Cfg::kThreads;
+  // (A causal launch that is cut changes items often, and more of a change goes through scratch memory in this form: B1 H2 N8000 270 -> 324 us.)
+  constexpr bool PIPED = D > 128 && PREROT && !(CUT && CAUSAL);
   constexpr bool STRIDED = D <= 128, DELTA_ACC = D == 64;
   constexpr int KC = D / 16, NDB = D / 32, NKB = BLOCK_N / 32;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -758,6 +760,13 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       }
     }
 
+    if constexpr (PIPED) {   // the operand rows' home, and the accumulators', is the accumulation half of the register file
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) asm volatile("" : "+a"(qb[kc]), "+a"(dob[kc]));
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) asm volatile("" : "+a"(dqacc[db]));
+    }
+
     auto stage_next = [&]() __attribute__((always_inline)) {
       kst.store_rows(k_tile(cur ^ 1));
       vst.store_rows(v_tile(cur ^ 1));
@@ -774,8 +783,64 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       const uint16_t* vs = v_tile(cur);
       const bool need_mask = (CAUSAL && n0 + BLOCK_N - 1 > wq_lo) || (!CAUSAL && n0 + BLOCK_N > N);
       u32x4 dsb[BLOCK_N / 16];
+      if constexpr (PIPED) {
+        // One stream of 3 x 16 products as in the dK+dV kernel at this head dim: the exponentials between the dP products, the second half of dS
+        // between the first half of the dQ products (the first half of dS is all that waits), then the next tile's staging.
+        static_assert(NKB == 1, "one 32-key block per tile");
+        constexpr int RING = 4, TOTAL = 3 * KC;
+        using KT = RowTile<D, kBothWaysPad>;
+        const uint16_t *k_l = ks + KT::off(lq, 8 * lh), *v_l = vs + RowTile<D>::off(lq, 8 * lh);
+        const uint16_t* k_t = ks + KT::off(4 * lh + lane % 16 / 4, 16 * (lane / 16 % 2) + 4 * (lane % 4));
+        auto operand = [&](int n) __attribute__((always_inline)) {
+          const int i = n % KC;
+          return n < KC       ? *reinterpret_cast<const u32x4*>(k_l + 16 * i)
+                 : n < 2 * KC ? *reinterpret_cast<const u32x4*>(v_l + 16 * i)
+                              : load_a_trans_lane<KT>(k_t, 16 * (i / NDB), i % NDB * 32);
+        };
+        u32x4 ring[RING];
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
+        for (int n = 0; n < RING; ++n) ring[n] = operand(n);
+        f32x16 sacc, dpacc;
+        auto ds_pair = [&](int j) __attribute__((always_inline)) {
+          dsb[j / 4][j % 4] = pack_elts(sacc[2 * j] * (dpacc[2 * j] - delta_q), sacc[2 * j + 1] * (dpacc[2 * j + 1] - delta_q));
+        };
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<TOTAL>([&](auto n_c) __attribute__((always_inline)) {
+          constexpr int n = decltype(n_c)::value, slot = n / KC, i = n % KC;
+          if constexpr (slot == 2 && i == 0) {
+            mfma32_settle(dpacc);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) ds_pair(j);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          const u32x4 a = ring[n % RING];
+          if constexpr (slot == 0) { if constexpr (i == 0) sacc = mfma32_from_aq(a, qb[0], msb); else mfma32_acc_aq(sacc, a, qb[i]); }
+          if constexpr (slot == 1) { if constexpr (i == 0) dpacc = mfma32_zero_aq(a, dob[0]); else mfma32_acc_aq(dpacc, a, dob[i]); }
+          if constexpr (slot == 2) dqacc[i % NDB] = mfma32(a, dsb[i / NDB], dqacc[i % NDB]);
+          if constexpr (n + RING < TOTAL) ring[n % RING] = operand(n + RING);
+          if constexpr (slot == 1 && i == 0) asm volatile("s_nop 7");   // (nothing reads the scores behind product 0, which waits a little instead)
+          if constexpr (slot == 1 && i == 1) {
+            if (need_mask) {
+              int rel = key_limit - n0 - 4 * lh;
+              asm volatile("" : "+v"(rel));
+#pragma unroll
+              for (int x = 0; x < 16; ++x)
+                if (8 * (x / 4) + x % 4 > rel) sacc[x] = -INFINITY;
+            }
+          }
+          if constexpr (slot == 1) {
+#pragma unroll
+            for (int e = (i == 0 ? 0 : (i - 1) * 16 / (KC - 1)); e < (i == 0 ? 0 : i * 16 / (KC - 1)); ++e) sacc[e] = fast_exp2(sacc[e]);
+          }
+          if constexpr (slot == 2 && i < 4) ds_pair(4 + i);
+          if constexpr (slot == 2 && i == KC - 2) stage_next();
+          __builtin_amdgcn_sched_barrier(0);
+        });
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) asm volatile("" : "+a"(dqacc[db]));
+      }
+#pragma unroll
+      for (int kb = 0; kb < (PIPED ? 0 : NKB); ++kb) {
         f32x16 sacc, dpacc;   // dP starts from a literal zero, S from -M
         const uint16_t* krow = ks + RowTile<D, kBothWaysPad>::off(kb * 32 + lq, 8 * lh);
         const uint16_t* vrow = vs + RowTile<D>::off(kb * 32 + lq, 8 * lh);
@@ -812,11 +877,11 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
         }
       }
 #pragma unroll
-      for (int c = 0; c < BLOCK_N / 16; ++c)
+      for (int c = 0; c < (PIPED ? 0 : BLOCK_N / 16); ++c)
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
           dqacc[db] = mfma32(load_a_trans_of<RowTile<D, kBothWaysPad>>(ks, 16 * c, db * 32), dsb[c], dqacc[db]);
-      stage_next();
+      if constexpr (!PIPED) stage_next();
       cur ^= 1;
       __syncthreads();
     }

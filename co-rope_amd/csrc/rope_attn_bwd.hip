@@ -144,6 +144,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   constexpr int DO_PAD = DO_DK ? (DO_DV ? kDkdvBothWaysPad : 8) : 32;
   constexpr int Q_PAD = DO_DK ? kDkdvBothWaysPad : 8;
   constexpr bool V_LDS = DO_DV && DO_DK && D <= 128, STRIDED = PREROT && D <= 128, PIPED = DO_DV && DO_DK && D > 128;
+  constexpr bool LATE = CUT && PIPED;
   using Cfg = DkdvCfg<D, NWAVES, BLOCK_M, DO_PAD, Q_PAD>;
   constexpr int NT = Cfg::kThreads;
   constexpr int KC = D / 16, NDB = D / 32, NQB = BLOCK_M / 32;
@@ -497,7 +498,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       UnrotateTables<D> tb;
       if constexpr (DO_DK && PREROT) tb.load(p.cos, p.sin, p.fstride, wk_lo, N, opaque_lane());
       if constexpr (DO_DV) store_rows_via_wave_tile<D>(dvacc, p.dv + base, wk_lo, N, 1.f, wave_slot, opaque_lane());
-      request_rows(has_next ? next_item : item);
+      if constexpr (!LATE) request_rows(has_next ? next_item : item);
       if constexpr (DO_DK) {
         if constexpr (!PREROT) tb.load(p.cos, p.sin, p.fstride, wk_lo, N, opaque_lane());
         // the Q_r operand carried sm_scale * log2(e): ln 2 is what is left of sm_scale
@@ -512,8 +513,9 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
         *reinterpret_cast<f32x4*>(slot + NWAVES * 32 * D + i * 4 * kWave) = f32x4{dkacc[db][4 * g], dkacc[db][4 * g + 1], dkacc[db][4 * g + 2], dkacc[db][4 * g + 3]};
       }
       __builtin_amdgcn_sched_barrier(0);
-      request_rows(has_next ? next_item : item);
+      if constexpr (!LATE) request_rows(has_next ? next_item : item);
     }
+    if constexpr (LATE) request_rows(has_next ? next_item : item);
     COROPE_ISTAMP(6);
     if (!has_next) break;
     item = next_item;

@@ -562,6 +562,51 @@ __global__ __launch_bounds__(kWave) void rope_attn_bwd_dkdv_sum_kernel(BwdParams
   }
 }
 
+// The same for few items, whose many pieces one wave would fetch one after the other: a workgroup per 32 keys, output and 64 columns
+// (blockIdx.z), a wave per register quad and its partner (columns d and d + D / 2), four pieces in flight.
+constexpr int kDkdvSumThreads = 4 * kWave;
+constexpr unsigned kSplitSumBlocks = 512;
+
+template <int D, int NWAVES, int BLOCK_M, bool CAUSAL>
+__global__ __launch_bounds__(kDkdvSumThreads) void rope_attn_bwd_dkdv_sum_split_kernel(BwdParams p, int shares) {
+  constexpr int BLOCK_N = NWAVES * 32, PARTNER = D / 16 * 4 * kWave;
+  const int N = p.N, slabs = p.BH / p.H * p.Hkv, GQ = p.H / p.Hkv, m_tiles = (N + BLOCK_M - 1) / BLOCK_M;
+  const DkdvTiles t(p.num_blocks, slabs, GQ, m_tiles, CAUSAL ? BLOCK_N / BLOCK_M : 0);
+  const int item = blockIdx.x / NWAVES, rb = blockIdx.x % NWAVES, kb = item / slabs, slab = item % slabs;
+  const int start = t.start(item), w0 = t.share_of(start, shares), w1 = t.share_of(start + t.first(kb + 1) - t.first(kb) - 1, shares);
+  const int lane = threadIdx.x % kWave, i = blockIdx.z * 4 + threadIdx.x / kWave, row = kb * BLOCK_N + rb * 32 + lane % 32;
+  if (w0 == w1 || row >= N) return;   // one piece holds all of the item and has written it
+  const float* src = p.parts + blockIdx.y * (NWAVES * 32 * D) + (int64_t)rb * 32 * D + 4 * (i * kWave + lane);
+  f32x4 a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
+  int w = w0;
+  auto add = [&](auto count_c) __attribute__((always_inline)) {   // that many pieces
+    constexpr int COUNT = decltype(count_c)::value;
+    f32x4 x[COUNT], y[COUNT];
+#pragma unroll
+    for (int u = 0; u < COUNT; ++u) {
+      const float* slot = src + piece_slot(w + u, w + u == w0) * kDkdvSlotFloats<D, NWAVES>;
+      x[u] = *reinterpret_cast<const f32x4*>(slot);
+      y[u] = *reinterpret_cast<const f32x4*>(slot + PARTNER);
+    }
+#pragma unroll
+    for (int u = 0; u < COUNT; ++u) a += x[u], b += y[u];
+    w += COUNT;
+  };
+  while (w + 3 <= w1) add(std::integral_constant<int, 4>{});
+  if (w + 1 <= w1) add(std::integral_constant<int, 2>{});
+  if (w <= w1) add(std::integral_constant<int, 1>{});
+  const int col = 8 * i + 4 * (lane / 32);
+  f32x4 o1 = a, o2 = b;
+  if (blockIdx.y == 1) {   // (the Q_r operand carried sm_scale * log2(e): ln 2 is what is left of sm_scale)
+    const f32x4 c = *reinterpret_cast<const f32x4*>(p.cos + row * p.fstride + col), s = *reinterpret_cast<const f32x4*>(p.sin + row * p.fstride + col);
+    a *= 0.6931471805599453f, b *= 0.6931471805599453f;
+    o1 = a * c + b * s, o2 = b * c - a * s;
+  }
+  uint16_t* out = (blockIdx.y == 0 ? p.dv : p.dk) + ((int64_t)slab * N + row) * D + col;
+  *reinterpret_cast<u32x2*>(out) = u32x2{pack_elts(o1[0], o1[1]), pack_elts(o1[2], o1[3])};
+  *reinterpret_cast<u32x2*>(out + D / 2) = u32x2{pack_elts(o2[0], o2[1]), pack_elts(o2[2], o2[3])};
+}
+
 // ===================================================================================== dQ
 // Workgroup = NWAVES waves x 32 queries.  Rotated Q rows and dO rows of the wave stay in registers.
 // Per key tile (BLOCK_N rows, staged: rotated K and V):
@@ -1041,7 +1086,13 @@ static hipError_t launch_dkdv_cut(BwdParams p, int shares, hipStream_t stream) {
 #endif
   hipLaunchKernelGGL(kern, dim3(shares), dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, p);
   const unsigned blocks = (unsigned)p.num_blocks * (p.BH / p.H * p.Hkv) * NWAVES;
-  hipLaunchKernelGGL((rope_attn_bwd_dkdv_sum_kernel<D, NWAVES, BM, CAUSAL>), dim3(blocks, 2), dim3(kWave), 0, stream, p, shares);
+  // One wave per 32 keys reads its pieces at the memory's rate once there are waves enough; below that the pieces' latencies set the time.
+  // us, one wave / split, by blocks of 32 keys: 24 (B1 Hq8 Hkv1 N700 D128) 12.8 / 5.4, 64 (B2 Hq16 Hkv2 N512 D256) 28.0 / 12.2, 128 (B1 Hq16 Hkv4 N1024 D128)
+  // 11.4 / 8.5, 496 (B1 H4 N3900 D256) 21.4 / 19.2, 512 (B1 H8 N2048 D128) 15.3 / 15.3, 768 (B1 Hq32 Hkv8 N3001 D128) 17.7 / 18.9, 1536 (B2 H8 N3000 D256) 19.3 / 25.5.
+  if (blocks < kSplitSumBlocks)
+    hipLaunchKernelGGL((rope_attn_bwd_dkdv_sum_split_kernel<D, NWAVES, BM, CAUSAL>), dim3(blocks, 2, D / 64), dim3(kDkdvSumThreads), 0, stream, p, shares);
+  else
+    hipLaunchKernelGGL((rope_attn_bwd_dkdv_sum_kernel<D, NWAVES, BM, CAUSAL>), dim3(blocks, 2), dim3(kWave), 0, stream, p, shares);
   return hipGetLastError();
 }
 

@@ -618,3 +618,20 @@ def test_short_sequences_by_the_operators_own_rule(pkg, B, Hq, Hkv, N, D, causal
     rdk, rdv = (t.reshape(B, Hkv, G, N, D).sum(2) for t in (rdk, rdv))
     for name, a, b in (("O", got[0], ro), ("O alone", alone, ro), ("dQ", got[1], rdq), ("dK", got[2], rdk), ("dV", got[3], rdv)):
         assert within_bar(a, b, TOL * (math.sqrt(G) if name in ("dK", "dV") else 1))[0], name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 8, 1, 65, 128), (1, 8, 1, 700, 64), (2, 16, 2, 509, 256), (1, 8, 8, 2017, 128), (1, 9, 9, 2048, 128), (2, 8, 8, 1999, 256)])
+def test_sums_of_cut_key_blocks(pkg, B, Hq, Hkv, N, D, dtype):
+    """dK and dV of key blocks that were cut, few blocks with many pieces (added by several waves) and many (by one each), against whole blocks: the
+    same products summed in another order in fp32, then one rounding."""
+    dev = torch.device("cuda:0")
+    q, g = (seeded((B, Hq, N, D), 140 + i).to(dev, dtype) for i in range(2))
+    k, v = (seeded((B, Hkv, N, D), 142 + i).to(dev, dtype) for i in range(2))
+    c, s = (t.to(dev) for t in O.precompute_freqs_cis(D, N))
+    out = pkg.attention(q.requires_grad_(True), k.requires_grad_(True), v.requires_grad_(True), True, 1 / math.sqrt(D), c, s)
+    saved = [t.detach() for t in out.grad_fn.saved_tensors]
+    whole = _backward_on_whole_blocks(pkg, saved, g, 1 / math.sqrt(D), True)
+    step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for a, b in zip(torch.autograd.grad(out, (q, k, v), g)[1:], whole[1:]):
+        assert (a.float() - b.float()).abs().max() <= 2 * step * b.float().abs().max() + 1e-5

@@ -983,6 +983,24 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
   constexpr int kTileElems = kDkRows * MATS * kDkKeys, TI = kTileElems / NT;      // fp32 values per thread and tile
   constexpr int kRowItems = kDkRows * G * (D / 8), RI = (kRowItems + NT - 1) / NT;  // 16-byte pieces of q rows
   static_assert(kTileElems % (4 * NT) == 0, "tile elements divide evenly over the threads, four keys at a time");
+  // A thread fetches four keys of (row, matrix) number first_unit + k STEP, k = 0 .. MATS - 1; the matrices come round with period PERIOD and the rows
+  // then lie ROWS_ON further, so what depends on the matrix is looked up once (per tile it was a tenth of the kernel's instructions), and keys are
+  // looked at one by one only where a row of the tile does not see all of them: B2 Hq32 Hkv8 N4096 D128 3.18 -> 3.06 ms.  (One head a group has few
+  // matrices, and the registers cost it more: B2 H16 N2000 D64 fp16 930 -> 960 us.)
+  constexpr bool KEPT = G > 1;
+  constexpr int STEP = 4 * NT / kDkKeys, PERIOD = MATS % 8 == 0 ? MATS / 8 : MATS % 4 == 0 ? MATS / 4 : MATS % 2 == 0 ? MATS / 2 : MATS;
+  constexpr int ROWS_ON = STEP * PERIOD / MATS;
+  static_assert(STEP == 8 && STEP * PERIOD % MATS == 0, "period of the matrices");
+  const int key0 = 4 * (threadIdx.x % (kDkKeys / 4));
+  const float* mat_at[PERIOD];
+  int row_at[PERIOD];
+#pragma unroll
+  for (int j = 0; j < (KEPT ? PERIOD : 0); ++j) {
+    const int unit = threadIdx.x / (kDkKeys / 4) + j * STEP;
+    row_at[j] = unit / MATS;
+    const int m = unit % MATS, mat = m == 0 ? g : m == 1 ? ws.n_groups + g : 2 * ws.n_groups + ws.n_heads + head0 + m - 2;   // (as CoropeBwdWs counts them)
+    mat_at[j] = ws.base + mat * ws.NN;
+  }
 
   int kb = 0;
 #pragma unroll 1
@@ -1000,13 +1018,18 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
       const int row_len = 64 * (i0 / 64 + 1);
       static_for<TI / 4>([&](auto k_c) __attribute__((always_inline)) {
         constexpr int k = decltype(k_c)::value;
-        const int e = 4 * (threadIdx.x + k * NT);
-        const int key = e % kDkKeys, m = (e / kDkKeys) % MATS, r = e / (kDkKeys * MATS);
-        const int mat = m == 0 ? g : m == 1 ? ws.n_groups + g : 2 * ws.n_groups + ws.n_heads + head0 + m - 2;   // (as CoropeBwdWs counts them)
-        const float* src = ws.base + mat * ws.NN;
         // four keys with one load, always inside the padded row (no branch); what is not defined there becomes zero on its way into
         // LDS (here the select would wait for the load)
-        mv[k] = *reinterpret_cast<const f32x4*>(src + tile0 + (int64_t)row_len * min(r, N - 1 - i0) + min(jb + key, row_len - 4));
+        if constexpr (KEPT) {
+          const uint32_t off = (uint32_t)row_len * min(row_at[k % PERIOD] + k / PERIOD * ROWS_ON, N - 1 - i0) + min(jb + key0, row_len - 4);
+          mv[k] = *reinterpret_cast<const f32x4*>(mat_at[k % PERIOD] + tile0 + off);
+        } else {
+          const int e = 4 * (threadIdx.x + k * NT);
+          const int key = e % kDkKeys, m = (e / kDkKeys) % MATS, r = e / (kDkKeys * MATS);
+          const int mat = m == 0 ? g : m == 1 ? ws.n_groups + g : 2 * ws.n_groups + ws.n_heads + head0 + m - 2;
+          const float* src = ws.base + mat * ws.NN;
+          mv[k] = *reinterpret_cast<const f32x4*>(src + tile0 + (int64_t)row_len * min(r, N - 1 - i0) + min(jb + key, row_len - 4));
+        }
       });
       static_for<RI>([&](auto k_c) __attribute__((always_inline)) {
         constexpr int k = decltype(k_c)::value;
@@ -1030,12 +1053,16 @@ __global__ __launch_bounds__(kDkWaves* kWave) __attribute__((amdgpu_waves_per_eu
 #pragma unroll 1
     for (int i0 = row_begin; i0 < row_end; i0 += kDkRows) {
       __syncthreads();   // the previous tile has been consumed
+      const bool inside = i0 >= jb + kDkKeys - 1 && i0 + kDkRows <= N;   // every row of the tile sees every key of the block
       static_for<TI / 4>([&](auto k_c) __attribute__((always_inline)) {
         constexpr int k = decltype(k_c)::value;
-        const int e = 4 * (threadIdx.x + k * NT), i = i0 + e / (kDkKeys * MATS), j = jb + e % kDkKeys;
-        f32x4 v;
+        const int e = 4 * (threadIdx.x + k * NT), j = jb + (KEPT ? key0 : e % kDkKeys);
+        const int i = i0 + (KEPT ? row_at[k % PERIOD] + k / PERIOD * ROWS_ON : e / (kDkKeys * MATS));
+        f32x4 v = mv[k];
+        if (!KEPT || !inside) {   // wave-uniform
 #pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] = (i < N && j + x <= i) ? mv[k][x] : 0.f;   // outside the causal triangle or past N
+          for (int x = 0; x < 4; ++x) v[x] = (i < N && j + x <= i) ? mv[k][x] : 0.f;   // outside the causal triangle or past N
+        }
         *reinterpret_cast<f32x4*>(tile + e) = v;
       });
       static_for<RI>([&](auto k_c) __attribute__((always_inline)) {

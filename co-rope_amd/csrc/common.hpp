@@ -501,11 +501,13 @@ struct WaveRows<D, true> {
   f32x4 c[IT][2], s[IT][2];
   // l: the lane (callers inside a loop over work items pass a value the optimiser cannot see through, so that the
   // per-lane address parts are recomputed per item instead of being kept in registers across the whole loop)
+  // FROM .. TO: of the IT loads (a kernel without registers for all of them requests them in two parts)
+  template <int FROM = 0, int TO = IT>
   __device__ __forceinline__ void load(const uint16_t* __restrict__ src, const float* __restrict__ cosp,
                                        const float* __restrict__ sinp, int64_t fstride, int row0, int n_rows,
                                        int l = threadIdx.x % kWave, uint32_t row_bytes = D * 2) {
 #pragma unroll
-    for (int i = 0; i < IT; ++i) {
+    for (int i = FROM; i < TO; ++i) {
       const int row = min(row0 + RPI * i + l / UPR, n_rows - 1), u = l % UPR;
       const uint16_t* xp = byte_offset(src, (uint32_t)row * row_bytes + u * 16);
       x1[i] = *reinterpret_cast<const u32x4*>(xp);

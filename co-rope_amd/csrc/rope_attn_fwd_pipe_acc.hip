@@ -597,9 +597,20 @@ __global__ __launch_bounds__(pipe64::Cfg32<D_>::kThreads)
     asm volatile("" : "+v"(l));
     return l;
   };
-  auto request_q = [&](int i) __attribute__((always_inline)) {
+  // At head dim 256 the rows and their table values take 192 registers: requested all at once, beside the accumulators, some of the loads went to
+  // scratch memory one by one, each waiting for the memory's full latency.  The second part is requested when the item's O rows have left.
+  // B7 Hq10 N2371 374 -> 354 us, B1 H16 N300 26.6 -> 24.7; not causal, where other registers then go that way, B2 H8 N3000 228 -> 237: not there.
+  constexpr int kQFirst = D > 128 && CAUSAL ? WaveRows<D, true>::IT / 2 : WaveRows<D, true>::IT;
+  auto request_q_part = [&](int i, auto from_c, auto to_c) __attribute__((always_inline)) {
     const int bh = i % p.BH, m0 = (p.num_m_blocks - 1 - i / p.BH) * C::kBlockM;
-    qrows.load(p.q_slab(bh), p.cos, p.sin, p.fstride, m0 + wave * 32, N, opaque_lane(), (uint32_t)p.q_sn * 2);
+    qrows.template load<decltype(from_c)::value, decltype(to_c)::value>(p.q_slab(bh), p.cos, p.sin, p.fstride, m0 + wave * 32, N, opaque_lane(),
+                                                                        (uint32_t)p.q_sn * 2);
+  };
+  auto request_q = [&](int i) __attribute__((always_inline)) {
+    request_q_part(i, std::integral_constant<int, 0>{}, std::integral_constant<int, kQFirst>{});
+  };
+  auto request_q_rest = [&](int i) __attribute__((always_inline)) {
+    request_q_part(i, std::integral_constant<int, kQFirst>{}, std::integral_constant<int, WaveRows<D, true>::IT>{});
   };
   auto request_kvec = [&](int i) __attribute__((always_inline)) {
     const int bh = i % p.BH;
@@ -618,6 +629,7 @@ __global__ __launch_bounds__(pipe64::Cfg32<D_>::kThreads)
   kst.load(l_kg, 0, N);
   vst.load(l_vg, 0, N, (uint32_t)p.v_sn * 2);
   request_q(item);
+  request_q_rest(item);
   request_kvec(item);
   take_q(item);
   kst.store_rows(lds_at(koff_cur));
@@ -857,6 +869,7 @@ __global__ __launch_bounds__(pipe64::Cfg32<D_>::kThreads)
     if (!has_next) break;
     item = next_item;
     COROPE_ISTAMP(0);
+    request_q_rest(item);
     take_q(item);
   }
 }

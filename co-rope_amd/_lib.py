@@ -51,6 +51,7 @@ SIGNATURES = {
     "corope_rope_attn_fwd_strided": (_I, [_P] * 8 + [_L] + [_P] * 5 + [_I] * 5 + [_F, _I, _I, _P]),
     "corope_rope_attn_fwd_parts_bytes": (_L, [_I] * 5),
     "corope_rope_attn_fwd_cut": (_I, [_P] * 8 + [_L] + [_P] * 5 + [_I] * 5 + [_F, _I, _I, _P, _L, _P]),
+    "corope_rope_attn_fwd_keep": (_I, [_P] * 8 + [_L] + [_P] * 5 + [_I] * 5 + [_F, _I, _I, _P, _L, _P, _P]),
     "corope_rope_attn_fwd_gqa": (_I, [_P] * 5 + [_L] + [_P] * 5 + [_I] * 5 + [_F, _I, _P]),
     "corope_rope_attn_bwd_gqa": (_I, [_P, _P, _I] + [_P] * 7 + [_L, _P, _P, _P] + [_I] * 5 + [_F, _I, _P]),
     "corope_rope_attn_bwd_rotated_parts_bytes": (_L, [_I] * 6),
@@ -66,7 +67,7 @@ SIGNATURES = {
 # The operators' host side in native code (csrc/host_calls.cpp): one Python call per forward or backward instead of one per allocation
 # and a ctypes call.  Entry points it goes through, in its order.
 HOST_PATH = os.path.join(_HERE, "lib", "corope_host_calls.so")
-HOST_CALLS = ("corope_rope_attn_fwd_cut", "corope_rope_attn_bwd_rotated", "corope_gqa_fwd", "corope_gqa_fwd_f16", "corope_gqa_bwd", "corope_gqa_bwd_f16")
+HOST_CALLS = ("corope_rope_attn_fwd_keep", "corope_rope_attn_bwd_rotated", "corope_gqa_fwd", "corope_gqa_fwd_f16", "corope_gqa_bwd", "corope_gqa_bwd_f16")
 
 _lock = threading.Lock()
 _lib = None

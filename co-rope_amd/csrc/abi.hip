@@ -680,7 +680,7 @@ int corope_rope_attn_fwd_f16(const void* q, const void* k, const void* v, const 
   // tile_kmax null: the attention kernel is the single-launch one on the rotated copy (probabilities in fp16 against an fp16 V)
   if (reinterpret_cast<uintptr_t>(tile_kmax) & 3u) return fail(COROPE_E_ALIGN, "%s: tile_kmax %p is misaligned", what, (const void*)tile_kmax);
   rc = launch_status(what, corope_f16::launch_rope_rotate(p.k, p.cos, p.sin, p.fstride, static_cast<uint16_t*>(k_rot), tile_kmax,
-                                                          B * Hkv, N, D, st, 1.f, 1, 0, 0, 0));
+                                                          B * Hkv, N, D, st, 1.f, 1, 0, 0, 0, nullptr, 0, 0, 0, nullptr));
   if (rc) return rc;
   p.k_rot = static_cast<const uint16_t*>(k_rot);
   p.tile_kmax = tile_kmax;
@@ -713,9 +713,10 @@ int corope_rope_attn_bwd_f16(const void* q, const void* k, int prerotated, const
     uint16_t* q_rot = static_cast<uint16_t*>(workspace);
     uint16_t* k_rot = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + each);
     rc = launch_status(what, corope_f16::launch_rope_rotate(p.q, p.cos, p.sin, p.fstride, q_rot, nullptr, p.BH, N, D, st,
-                                                            p.qk_scale, 1, 0, 0, 0));
+                                                            p.qk_scale, 1, 0, 0, 0, nullptr, 0, 0, 0, nullptr));
     if (rc) return rc;
-    rc = launch_status(what, corope_f16::launch_rope_rotate(p.k, p.cos, p.sin, p.fstride, k_rot, nullptr, B * Hkv, N, D, st, 1.f, 1, 0, 0, 0));
+    rc = launch_status(what, corope_f16::launch_rope_rotate(p.k, p.cos, p.sin, p.fstride, k_rot, nullptr, B * Hkv, N, D, st, 1.f,
+                                                            1, 0, 0, 0, nullptr, 0, 0, 0, nullptr));
     if (rc) return rc;
     p.q = p.q_rot = q_rot;
     p.k = p.k_rot = k_rot;
@@ -740,7 +741,7 @@ namespace {
 int rope_attn_fwd_strided_impl(const char* what, const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,
                                const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin, int64_t freq_row_stride, void* o,
                                float* lse, void* q_rot, void* k_rot, float* tile_kmax, int B, int H, int Hkv, int N, int D, float sm_scale,
-                               int causal, int fp16, bool cut, void* parts, int64_t parts_bytes, void* stream) {
+                               int causal, int fp16, bool cut, void* parts, int64_t parts_bytes, void* v_keep, void* stream) {
   if (Hkv <= 0 || H % Hkv != 0) return fail(COROPE_E_BADARG, "%s: H=%d is not a multiple of Hkv=%d", what, H, Hkv);
   int rc = corope_rope_attn_check(B, H, N, D, freq_row_stride, sm_scale, 0);
   if (rc) return rc;
@@ -750,6 +751,11 @@ int rope_attn_fwd_strided_impl(const char* what, const void* q, const int64_t* q
   for (const int64_t* st : {q_strides, k_strides, v_strides})
     if ((rc = check_strides(what, st, N, D))) return rc;
   if (k_rot == nullptr && q_rot != nullptr) return fail(COROPE_E_BADARG, "%s: q_rot without k_rot", what);
+  if (v_keep != nullptr) {
+    if (k_rot == nullptr) return fail(COROPE_E_BADARG, "%s: v_keep without k_rot", what);
+    if ((rc = check_ptrs(what, {v_keep}))) return rc;
+    if ((int64_t)B * Hkv * ((N + 63) / 64) >= ((int64_t)1 << 30)) return fail(COROPE_E_UNSUPPORTED, "%s: too many tiles for one launch", what);
+  }
   corope::FwdParams p{};
   if (parts != nullptr) {
     if ((rc = check_ptrs(what, {parts}))) return rc;
@@ -786,9 +792,9 @@ int rope_attn_fwd_strided_impl(const char* what, const void* q, const int64_t* q
   if (reinterpret_cast<uintptr_t>(tile_kmax) & 3u) return fail(COROPE_E_ALIGN, "%s: tile_kmax %p is misaligned", what, (const void*)tile_kmax);
   uint16_t* kr = static_cast<uint16_t*>(k_rot);
   rc = launch_status(what, fp16 ? corope_f16::launch_rope_rotate(p.k, p.cos, p.sin, p.fstride, kr, tile_kmax, B * Hkv, N, D, st, 1.f,
-                                                                 Hkv, p.k_sb, p.k_sh, p.k_sn)
+                                                                 Hkv, p.k_sb, p.k_sh, p.k_sn, p.v, p.v_sb, p.v_sh, p.v_sn, static_cast<uint16_t*>(v_keep))
                                 : corope::launch_rope_rotate(p.k, p.cos, p.sin, p.fstride, kr, tile_kmax, B * Hkv, N, D, st, 1.f, Hkv,
-                                                             p.k_sb, p.k_sh, p.k_sn));
+                                                             p.k_sb, p.k_sh, p.k_sn, p.v, p.v_sb, p.v_sh, p.v_sn, static_cast<uint16_t*>(v_keep)));
   if (rc) return rc;
   p.k_rot = kr;
   p.tile_kmax = tile_kmax;
@@ -807,7 +813,7 @@ int corope_rope_attn_fwd_strided(const void* q, const int64_t* q_strides, const 
                                  int64_t freq_row_stride, void* o, float* lse, void* q_rot, void* k_rot, float* tile_kmax, int B,
                                  int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16, void* stream) {
   return rope_attn_fwd_strided_impl("rope_attn_fwd_strided", q, q_strides, k, k_strides, v, v_strides, freqs_cos, freqs_sin, freq_row_stride, o, lse,
-                                    q_rot, k_rot, tile_kmax, B, H, Hkv, N, D, sm_scale, causal, fp16, false, nullptr, 0, stream);
+                                    q_rot, k_rot, tile_kmax, B, H, Hkv, N, D, sm_scale, causal, fp16, false, nullptr, 0, nullptr, stream);
 }
 
 int64_t corope_rope_attn_fwd_parts_bytes(int B, int H, int N, int D, int causal) {
@@ -820,7 +826,15 @@ int corope_rope_attn_fwd_cut(const void* q, const int64_t* q_strides, const void
                              void* q_rot, void* k_rot, float* tile_kmax, int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
                              void* parts, int64_t parts_bytes, void* stream) {
   return rope_attn_fwd_strided_impl("rope_attn_fwd_cut", q, q_strides, k, k_strides, v, v_strides, freqs_cos, freqs_sin, freq_row_stride, o, lse, q_rot,
-                                    k_rot, tile_kmax, B, H, Hkv, N, D, sm_scale, causal, fp16, true, parts, parts_bytes, stream);
+                                    k_rot, tile_kmax, B, H, Hkv, N, D, sm_scale, causal, fp16, true, parts, parts_bytes, nullptr, stream);
+}
+
+int corope_rope_attn_fwd_keep(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,
+                              const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin, int64_t freq_row_stride, void* o, float* lse,
+                              void* q_rot, void* k_rot, float* tile_kmax, int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
+                              void* parts, int64_t parts_bytes, void* v_keep, void* stream) {
+  return rope_attn_fwd_strided_impl("rope_attn_fwd_keep", q, q_strides, k, k_strides, v, v_strides, freqs_cos, freqs_sin, freq_row_stride, o, lse, q_rot,
+                                    k_rot, tile_kmax, B, H, Hkv, N, D, sm_scale, causal, fp16, true, parts, parts_bytes, v_keep, stream);
 }
 
 int corope_rope_freqs(float* freqs_cos, float* freqs_sin, int n_pos, int D, int width, int64_t freq_row_stride, int pos0,

@@ -16,7 +16,7 @@ namespace {
 
 // Entry points of the library in use, by address (the order of host_calls in _lib.py).
 struct Table {
-  decltype(&corope_rope_attn_fwd_cut) fwd_cut;
+  decltype(&corope_rope_attn_fwd_keep) fwd_keep;
   decltype(&corope_rope_attn_bwd_rotated) bwd;
   decltype(&corope_gqa_fwd) gqa_fwd, gqa_fwd_f16;
   decltype(&corope_gqa_bwd) gqa_bwd, gqa_bwd_f16;
@@ -114,7 +114,7 @@ PyObject* make_table(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 // rope_forward(table, q, k, v, cos, sin, causal, sm_scale, rotated, exact, keep, device, stream, parts)
-//   -> None | status | (o, lse, q_rot or None, k_rot or None)
+//   -> None | status | (o, lse, q_rot or None, k_rot or None, v: a contiguous one where keep asks for it)
 PyObject* rope_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   COROPE_ARGS(14)
@@ -134,24 +134,26 @@ PyObject* rope_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if ((D != 64 && D != 128 && D != 256) || !table_ok(fc, N, D) || !table_ok(fs, N, D) || fc.stride(0) != fs.stride(0) || !strides_of(q, qs) ||
       !strides_of(k, ks) || !strides_of(v, vs))
     Py_RETURN_NONE;
+  if (keep && !rotated && !v.is_contiguous()) Py_RETURN_NONE;
   const auto opts = q.options().requires_grad(false), fopts = opts.dtype(at::kFloat);
-  at::Tensor o, lse, q_rot, k_rot, kmax, parts;
+  at::Tensor o, lse, v_keep, q_rot, k_rot, kmax, parts;
   if (!parts_of(args[13], device, parts)) Py_RETURN_NONE;
   o = at::empty({B, H, N, D}, opts);
   lse = at::empty({B, H, N}, fopts);
   if (rotated) {
     k_rot = at::empty({B, Hkv, N, D}, opts);
     if (keep) q_rot = at::empty({B, H, N, D}, opts);
+    if (keep && !v.is_contiguous()) v_keep = at::empty({B, Hkv, N, D}, opts);
     if (!exact) kmax = at::empty({B, Hkv, (N + 63) / 64}, fopts);
   }
   int rc;
   {
     NoGil free;
-    rc = tab->fwd_cut(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs, floats(fc), floats(fs), fc.stride(0), o.data_ptr(), floats(lse), data(q_rot),
-                      data(k_rot), floats(kmax), B, H, Hkv, N, D, (float)sm_scale, causal, q.scalar_type() == at::kHalf, data(parts), parts.defined() ? (int64_t)parts.nbytes() : 0, stream);
+    rc = tab->fwd_keep(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs, floats(fc), floats(fs), fc.stride(0), o.data_ptr(), floats(lse), data(q_rot),
+                      data(k_rot), floats(kmax), B, H, Hkv, N, D, (float)sm_scale, causal, q.scalar_type() == at::kHalf, data(parts), parts.defined() ? (int64_t)parts.nbytes() : 0, data(v_keep), stream);
   }
   if (rc != 0) return PyLong_FromLong(rc);
-  return pack({o, lse, q_rot, keep ? k_rot : at::Tensor()});
+  return pack({o, lse, q_rot, keep ? k_rot : at::Tensor(), v_keep.defined() ? v_keep : v});
   END_HANDLE_TH_ERRORS
 }
 

@@ -234,9 +234,11 @@ using namespace corope;
 
 // y = out_scale * rotated x for a (BH, N, D) tensor; tile_max (may be null) receives [BH][ceil(N / 64)] largest row norms.
 // (x_sb, x_sh, x_sn: elements between batches, heads and rows of x, with H heads per batch; 0, 0, 0: contiguous)
+// v_out: receives a contiguous copy of v, of x's shape at strides of its own (the strided form only).
 hipError_t launch_rope_rotate(const uint16_t* x, const float* cosp, const float* sinp, int64_t fstride, uint16_t* y,
                               float* tile_max, int BH, int N, int D, hipStream_t stream, float out_scale = 1.f, int H = 1,
-                              int64_t x_sb = 0, int64_t x_sh = 0, int x_sn = 0);
+                              int64_t x_sb = 0, int64_t x_sh = 0, int x_sn = 0, const uint16_t* v = nullptr, int64_t v_sb = 0, int64_t v_sh = 0,
+                              int v_sn = 0, uint16_t* v_out = nullptr);
 hipError_t launch_rope_attn_fwd_prerotated(const FwdParams& p, int D, bool causal, hipStream_t stream);  // needs k_rot
 // the same with 64 query rows per wave, one wave per SIMD (D = 128)
 hipError_t launch_rope_attn_fwd_prerotated_rows64(const FwdParams& p, int D, bool causal, hipStream_t stream);
@@ -278,7 +280,7 @@ hipError_t launch_bwd_dq(const corope::BwdParams& p, int D, bool causal, hipStre
 hipError_t launch_bwd_dkdv_fused(const corope::BwdParams& p, int D, bool causal, hipStream_t stream);
 hipError_t launch_rope_rotate(const uint16_t* x, const float* cosp, const float* sinp, int64_t fstride, uint16_t* y,
                               float* tile_max, int BH, int N, int D, hipStream_t stream, float out_scale, int H, int64_t x_sb,
-                              int64_t x_sh, int x_sn);
+                              int64_t x_sh, int x_sn, const uint16_t* v, int64_t v_sb, int64_t v_sh, int v_sn, uint16_t* v_out);
 hipError_t launch_corope_gqa_fwd(const corope::CoropeParams& p, int D, hipStream_t stream);
 hipError_t launch_corope_gqa_bwd(const corope::CoropeBwdParams& p, int D, float* workspace, int64_t workspace_floats,
                                  hipStream_t stream);

@@ -11,6 +11,9 @@
 // out_scale != 1: y = out_scale * rotated x, still one rounding -- the form in which the backward kernels and the
 // two-launch forward take a pre-rotated Q (out_scale = sm_scale * log2(e)).
 //
+// v_out (may be null): receives a contiguous copy of the strided v, which a forward keeps for its backward; its tiles are further workgroups of the
+// launch.  What bounds either is memory, and on short sequences the launch: a copy by itself was one more (forward + backward B1 Hq32 Hkv8 N3001 D128 381 -> 375 us).
+//
 // tile_max[bh][t] = max over the rows of tile t of |y| (norm of the ROUNDED row).  With the norm of a query this
 // bounds every score of the tile, which lets the forward kernel pick its softmax mode per tile up front.
 #include "common.hpp"
@@ -27,7 +30,19 @@ __global__ __launch_bounds__(kRotThreads) void rope_rotate_kernel(const uint16_t
                                                                   const float* __restrict__ sinp, int64_t fstride,
                                                                   uint16_t* __restrict__ y, float* __restrict__ tile_max,
                                                                   int N, int n_tiles, float out_scale, int H, int64_t x_sb,
-                                                                  int64_t x_sh, int x_sn) {
+                                                                  int64_t x_sh, int x_sn, const uint16_t* __restrict__ v,
+                                                                  int64_t v_sb, int64_t v_sh, int v_sn, uint16_t* __restrict__ v_out) {
+  if (v_out != nullptr && blockIdx.x >= gridDim.x / 2) {   // workgroup-uniform
+    const int at = blockIdx.x - gridDim.x / 2, row0 = at % n_tiles * kRotRows, bh = at / n_tiles;
+    const uint16_t* src = v + (bh / H) * v_sb + (bh % H) * v_sh;
+    uint16_t* dst = v_out + (int64_t)bh * N * D;
+#pragma unroll
+    for (int it = 0; it < kRotRows * (D / 8) / kRotThreads; ++it) {
+      const int u = threadIdx.x + it * kRotThreads, row = row0 + u / (D / 8), col = u % (D / 8) * 8;
+      if (row < N) *reinterpret_cast<u32x4*>(dst + (int64_t)row * D + col) = *reinterpret_cast<const u32x4*>(src + (int64_t)row * v_sn + col);
+    }
+    return;
+  }
   using Stage = RotStage<D, kRotRows, kRotThreads, SCALED>;
   constexpr int kChunks = Stage::kChunks;
   __shared__ float wave_max[kRotThreads / kWave];
@@ -77,7 +92,8 @@ __global__ __launch_bounds__(kRotThreads) void rope_rotate_kernel(const uint16_t
 
 hipError_t launch_rope_rotate(const uint16_t* x, const float* cosp, const float* sinp, int64_t fstride, uint16_t* y,
                               float* tile_max, int BH, int N, int D, hipStream_t stream, float out_scale, int H, int64_t x_sb,
-                              int64_t x_sh, int x_sn) {
+                              int64_t x_sh, int x_sn, const uint16_t* v, int64_t v_sb, int64_t v_sh, int v_sn, uint16_t* v_out) {
+  if (v_out != nullptr && x_sn == 0) return hipErrorInvalidValue;   // (a copy comes with the strided form, whose H it shares)
   if (D != 64 && D != 128 && D != 256) return hipErrorInvalidValue;
   if (x_sn == 0) {   // contiguous (BH, N, D)
     H = 1;
@@ -86,10 +102,10 @@ hipError_t launch_rope_rotate(const uint16_t* x, const float* cosp, const float*
     x_sn = D;
   }
   const int n_tiles = (N + kRotRows - 1) / kRotRows;
-  dim3 grid((unsigned)n_tiles * BH);   // one axis: the second grid axis stops at 65535 slabs
+  dim3 grid((unsigned)n_tiles * BH * (v_out != nullptr ? 2 : 1));   // one axis: the second grid axis stops at 65535 slabs
 #define COROPE_ROT(DD, SS)                                                                                             \
   hipLaunchKernelGGL((rope_rotate_kernel<DD, SS>), grid, dim3(kRotThreads), 0, stream, x, cosp, sinp, fstride, y, tile_max, \
-                     N, n_tiles, out_scale, H, x_sb, x_sh, x_sn)
+                     N, n_tiles, out_scale, H, x_sb, x_sh, x_sn, v, v_sb, v_sh, v_sn, v_out)
   if (D == 256) {
     if (out_scale == 1.f) COROPE_ROT(256, false); else COROPE_ROT(256, true);
   } else if (D == 128) {

@@ -170,7 +170,8 @@ def _fwd_parts(lib, q, causal):
 
 
 def _native_forward(lib, q, k, v, causal, sm_scale, fc, fs, keep):
-    """What _forward returns, by the native host side; None where this is not a plain call (then _check_inputs and _forward do it)."""
+    """What _forward returns, and the v to keep, by the native host side; None where this is not a plain call (then _check_inputs and
+    _forward do it)."""
     if q.dim() != 4 or not q.is_cuda or q.shape[3] not in _SUPPORTED_D or torch.cuda.current_device() != q.device.index:
         return None
     B, H, N, D = q.shape
@@ -179,8 +180,8 @@ def _native_forward(lib, q, k, v, causal, sm_scale, fc, fs, keep):
     out = host.rope_forward(table, q, k, v, fc, fs, causal, float(sm_scale), rotated, exact, keep, q.device.index, _stream_ptr(q),
                             _fwd_parts(lib, q, causal)[0] if rotated else None)
     if type(out) is int:
-        _lib.check(out, "corope_rope_attn_fwd_cut")
-    return out and (out[0], out[1], fc, fs, out[2:] if out[2] is not None else None)
+        _lib.check(out, "corope_rope_attn_fwd_keep")
+    return out and (out[0], out[1], fc, fs, out[2:4] if out[2] is not None else None, out[4])
 
 
 def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, keep_rotated=False):
@@ -312,18 +313,18 @@ class _FusedRopeAttn(torch.autograd.Function):
     def forward(ctx, q, k, v, causal, sm_scale, freqs_cos, freqs_sin, warp_specialize=True):
         needs = ctx.needs_input_grad
         training = needs[0] or needs[1] or needs[2]
-        if training:
-            # v is kept for the backward, and a view kept as it is would hold the fused projection it is cut from, and would be lost
-            # if the caller overwrites that before the backward: a view is copied (377 -> 386 us forward and backward at B1 Hq32 Hkv8 N3001 D128), q and k are kept
-            # rotated, in tensors of their own
-            v = v.contiguous()
+        # v is kept for the backward, and a view kept as it is would hold the fused projection it is cut from, and would be lost
+        # if the caller overwrites that before the backward: a view is copied (by the launch that rotates K), q and k are kept
+        # rotated, in tensors of their own
         # when a gradient will be asked for, the forward keeps its rotated q and k for the backward and the originals
         # are not saved (the reference saves q and k, fused_rope_attn.py:718, and re-rotates them in its backward)
         out = _native_forward(_lib.load(), q, k, v, causal, sm_scale, freqs_cos, freqs_sin, training)
         if out is None:
             _check_inputs(q, k, v, freqs_cos, freqs_sin)
-            out = _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, keep_rotated=training)
-        o, M, fc, fs, rotated = out
+            if training:
+                v = v.contiguous()
+            out = *_forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, keep_rotated=training), v
+        o, M, fc, fs, rotated, v = out
         # nothing to differentiate, nothing kept: saving q and k would copy strided views of a fused projection.  (Tables that
         # ask for a gradient get None, but the backward that says so runs and wants its tensors.)
         if not any(needs):

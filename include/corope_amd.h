@@ -277,6 +277,14 @@ int corope_rope_attn_fwd_cut(const void *q, const int64_t *q_strides, const void
                              void *o, float *lse, void *q_rot, void *k_rot, float *tile_kmax,
                              int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
                              void *parts, int64_t parts_bytes, void *stream);
+/* The same, and v_keep ((B,Hkv,N,D), may be NULL; needs k_rot) receives a contiguous copy of v, made by the launch that rotates K: what a caller that must
+ * not hold on to a view of its projection keeps for the backward (the reference saves v itself, fused-rope/fused_rope_attn.py:718). */
+int corope_rope_attn_fwd_keep(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
+                              const void *v, const int64_t *v_strides,
+                              const float *freqs_cos, const float *freqs_sin, int64_t freq_row_stride,
+                              void *o, float *lse, void *q_rot, void *k_rot, float *tile_kmax,
+                              int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
+                              void *parts, int64_t parts_bytes, void *v_keep, void *stream);
 
 /* Grouped-query form of the operator: q (B,Hq,N,D), k and v (B,Hkv,N,D), Hq a multiple of Hkv; query head h reads
  * key/value head h / (Hq/Hkv); dk and dv (B,Hkv,N,D) are sums over the query heads of their group (the key block's

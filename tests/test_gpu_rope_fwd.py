@@ -456,3 +456,29 @@ def test_forward_cut_query_blocks_at_equal_large_logits(pkg, N, D, causal, expon
         print(f"  {name}: max-abs {err.max().item():.2e}, {(err / bar).max().item():.2f} of the bar")
         assert (err <= bar).all(), name
     assert ((lse - lse_w).abs() <= 2.0 ** -22 * lse_w.abs()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,Hkv,N,D", [(1, 2, 1, 1, 64), (2, 4, 2, 63, 128), (1, 3, 3, 65, 256), (3, 4, 4, 130, 64), (2, 6, 3, 1025, 128)])
+def test_kept_copy_of_v(pkg, B, H, Hkv, N, D, dtype):
+    """corope_rope_attn_fwd_keep leaves a contiguous copy of a strided v, bit for bit and no further than its end, beside what corope_rope_attn_fwd_cut gives."""
+    import ctypes
+    dev, lib = torch.device("cuda:0"), pkg._lib.load()
+    q = seeded((B, N, H, D), 31).to(dev, dtype).transpose(1, 2)
+    kv = seeded((B, N, 2, Hkv, D), 32).to(dev, dtype)
+    k, v = kv[:, :, 0].transpose(1, 2), kv[:, :, 1].transpose(1, 2)
+    c, s = (t.to(dev) for t in O.precompute_freqs_cis(D, N))
+    st3, fp16 = (lambda t: (ctypes.c_int64 * 3)(t.stride(0), t.stride(1), t.stride(2))), int(dtype == torch.float16)
+    outs = []
+    kept = torch.full((v.numel() + 64,), 7.0, device=dev, dtype=dtype)
+    for name, extra in (("corope_rope_attn_fwd_cut", ()), ("corope_rope_attn_fwd_keep", (kept.data_ptr(),))):
+        o, M, kr = torch.empty(B, H, N, D, device=dev, dtype=dtype), torch.empty(B, H, N, device=dev), torch.empty(B, Hkv, N, D, device=dev, dtype=dtype)
+        kmax = torch.empty(B, Hkv, (N + 63) // 64, device=dev)
+        rc = getattr(lib, name)(q.data_ptr(), st3(q), k.data_ptr(), st3(k), v.data_ptr(), st3(v), c.data_ptr(), s.data_ptr(), c.stride(0), o.data_ptr(),
+                                M.data_ptr(), None, kr.data_ptr(), kmax.data_ptr(), B, H, Hkv, N, D, 0.125, 1, fp16, None, 0, *extra,
+                                torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, pkg._lib.last_error()
+        outs.append((o, M, kr, kmax))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+    assert torch.equal(kept[:v.numel()].view(B, Hkv, N, D), v) and (kept[v.numel():] == 7).all()

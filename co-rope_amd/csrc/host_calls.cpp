@@ -3,7 +3,7 @@
 // binding that called does it (and raises what it always raised).  No kernel and no rule lives here.
 //
 // What bounds the smallest calls is the host: torch.empty takes 2 us, a ctypes call of 25 arguments 4, beside 3 for a launch.  A forward without
-// gradients 15.4 -> 10.0 us of the host's time; forward and backward, on a box where the autograd engine's hand-over to its thread is slow:
+// gradients 15.4 -> 10.0 us of the host's time; forward and backward, on a machine where the autograd engine's hand-over to its thread is slow:
 // B4 H8 N512 D64 117 -> 110 us, Co-RoPE B2 Hq8 Hkv2 N512 D64 134 -> 105, B2 Hq16 Hkv8 N82 D128 127 -> 104.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>

@@ -144,6 +144,8 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
   constexpr int DO_PAD = DO_DK ? (DO_DV ? kDkdvBothWaysPad : 8) : 32;
   constexpr int Q_PAD = DO_DK ? kDkdvBothWaysPad : 8;
   constexpr bool V_LDS = DO_DV && DO_DK && D <= 128, STRIDED = PREROT && D <= 128, PIPED = DO_DV && DO_DK && D > 128;
+  // The next rows are requested behind a cut block's partial sums: in both branches of the change of items, 27 of the loads went to scratch memory one
+  // by one, each waiting for the memory's full latency (B1 H4 N4096 154 -> 104 us, B1 H1 N30000 fp16 1585 -> 990).
   constexpr bool LATE = CUT && PIPED;
   using Cfg = DkdvCfg<D, NWAVES, BLOCK_M, DO_PAD, Q_PAD>;
   constexpr int NT = Cfg::kThreads;
@@ -321,6 +323,8 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       if constexpr (PIPED) {
         // One wave per SIMD: nothing overlaps what the wave itself does not, so the tile is one stream of 4 x 16 products with its operands
         // RING ahead, the exponentials between the dP products, dS between the dV products, and the next tile's staging between the dK products.
+        // What bounds it: LDS reads (64 KB a tile) and products in about equal parts, and what of the latencies is still seen.  As the compiler scheduled it, V
+        // read from the LDS for every product: B2 H16 N2048 245 -> 187 us, B7 Hq10 Hkv5 N2371 700 -> 487 (RING 6 or later staging: no difference).
         static_assert(NQB == 1 && kWavesPerSimd<D> == 1, "one 32-row block per tile");
         if (CAUSAL && m0 + 31 < wk_lo) {   // queries that lie above every key of the wave: it only stages its share
           store_tile(cur ^ 1);
@@ -796,7 +800,7 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) asm volatile("" ::"v"(qb[kc]), "v"(dob[kc]));
     asm volatile("" ::"v"(delta_q));
-    // ... and dP - delta, where the registers for it are there (D = 64)
+    // ... and dP - delta, where the registers for it are there (D = 64: B2 H16 N4096 128 -> 122.5 us; at D = 128, with -delta from the LDS, 440 -> 460)
     f32x16 mdb;
     if constexpr (DELTA_ACC) {
 #pragma unroll
@@ -832,7 +836,8 @@ __global__ __launch_bounds__(NWAVES* kWave) __attribute__((amdgpu_waves_per_eu(k
       u32x4 dsb[BLOCK_N / 16];
       if constexpr (PIPED) {
         // One stream of 3 x 16 products as in the dK+dV kernel at this head dim: the exponentials between the dP products, the second half of dS
-        // between the first half of the dQ products (the first half of dS is all that waits), then the next tile's staging.
+        // between the first half of the dQ products (the first half of dS is all that waits), then the next tile's staging.  As the compiler scheduled
+        // it: B2 H16 N2048 171 -> 158 us, B2 H8 N3000 not causal 285 -> 253.
         static_assert(NKB == 1, "one 32-key block per tile");
         constexpr int RING = 4, TOTAL = 3 * KC;
         using KT = RowTile<D, kBothWaysPad>;

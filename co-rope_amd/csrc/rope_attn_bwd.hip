@@ -1138,8 +1138,8 @@ static hipError_t launch_dq_waves(BwdParams p, hipStream_t stream) {
 // How many pieces the key tiles of the dQ launch on rotated operands are cut into; 0: whole items.  As dkdv_shares: with few heads the longest
 // whole item (a sequence's last queries, which see all of its keys) sets the time however many compute units are idle.  Measured
 // constants, in microseconds: a tile of a full chip, a change of items (at head dim 256 nothing hides it with one wave per SIMD, and the cut kernel sends
-// 130 registers through scratch there, none in the tile loop), the launch; a causal piece of T tiles crosses up to sqrt(2 T / step) of a head's lightest items,
-// one that is not T / k_tiles (at head dims up to 128, where a change is short, the constants hold with one for it).  dQ launch, whole / cut
+// 130 registers through scratch there, none in the tile loop), the launch; a causal piece of T tiles crosses up to sqrt(2 T / step) of a head's lightest items
+// (items_crossed), one that is not T / k_tiles (at head dims up to 128, where a change is short, the constants hold with one for less than one).  dQ launch, whole / cut
 // with its sums, B1 H N: D = 128: 8 4096 159 / 87, 4 8192 296 / 132, 1 10000 330 / 66, 8 3000 not causal 119 / 80, and on the other side 16 4096 153 / 152, 40 1100 53 / 64; D = 64: 8 4096 63 / 50, 4 16384 276 / 239, 2 3000
 // not causal 46 / 27, 16 1500 27.5 / 28.2; D = 256: 2 2048 112 / 58, 4 4096 212 / 185, 8 2048 115 / 129, 16 2048 124 / 199,
 // not causal 12 4096 435 / 377, 8 1024 66 / 47, and on the other side 40 2304 397 / 451, 32 4096 888 / 973.
@@ -1161,7 +1161,7 @@ static int dq_shares(int N, int BH, bool causal) {
   constexpr float kChange = D == 64 ? 3.5f : D == 128 ? 5.f : 21.f;
   const float busy = std::min(1.f, (float)t.total_tiles * (block == CW * 32 ? 1.f : 2.f) / ((float)longest * cus));
   const float whole = (small ? 0.85f : 1.f) * longest * kWholeTile * (0.75f + 0.25f * busy) + kChange * ((n_items + grid - 1) / grid);
-  const float tiles = (float)t.total_tiles / shares, crossed = causal ? std::sqrt(2.f * tiles / (CW * 32 / BN)) : D > 128 ? tiles / k_tiles : 1.f;
+  const float tiles = (float)t.total_tiles / shares, crossed = D > 128 && !causal ? tiles / k_tiles : items_crossed(t, tiles);
   const float moved = (float)(shares + std::min<int64_t>(t.nb * (int64_t)BH, shares)) * kDqSlotFloats<D, CW> * 8;
   const float cut = tiles * kTile + kChange * (1.f + crossed) + 9.f + moved / 12e6f;
   return cut < 0.9f * whole ? shares : 0;

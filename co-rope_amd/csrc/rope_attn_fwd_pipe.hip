@@ -643,7 +643,7 @@ static int fwd_shares(int N, int BH, bool causal) {
   constexpr float kWholeTile = D == 64 ? 1.f : 1.75f, kTile = D == 64 ? 1.1f : 2.f, kChange = D == 64 ? 3.f : 4.f;
   const float busy = std::min(1.f, (float)t.total_tiles * (small ? 2.f : 1.f) / ((float)longest * cus));
   const float whole = (small ? 0.8f : 1.05f) * longest * kWholeTile * (0.75f + 0.25f * busy) + kChange * ((n_items + grid - 1) / grid) + 2.f;
-  const float tiles = (float)t.total_tiles / shares, crossed = causal ? std::sqrt(2.f * tiles / (kCutWaves * 32 / BN)) : 1.f;
+  const float tiles = (float)t.total_tiles / shares, crossed = items_crossed(t, tiles);
   const float moved = (float)(shares + std::min<int64_t>(t.nb * (int64_t)BH, shares)) * kFwdSlotFloats<D, kCutWaves> * 8;
   const float cut = tiles * kTile + kChange * (1.f + crossed) + 9.f + moved / 12e6f;
   return cut < 0.9f * whole ? shares : 0;

@@ -304,6 +304,19 @@ def test_where_launches_are_cut(pkg):
     assert not bwd(1, 40, 10, 3000, 256, 0) and not bwd(1, 32, 32, 4096, 256, 0)
 
 
+def test_short_items_are_not_cut(pkg):
+    """Launches of many short items: a piece would change items at every tile or two (measured slower by a sixth to a half; 256 compute units)."""
+    lib = pkg._lib.load()
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rules depend on the number of compute units")
+    fwd = lambda B, H, N, D, causal: lib.corope_rope_attn_fwd_parts_bytes(B, H, N, D, causal) > 0
+    bwd = lambda B, H, N, D, causal: lib.corope_rope_attn_bwd_rotated_parts_bytes(B, H, H, N, D, causal) > 0
+    for D in (64, 128):
+        for causal in (0, 1):
+            assert not any(f(B, 32, N, D, causal) for f in (fwd, bwd) for B in (48, 64, 96, 128) for N in (16, 64, 100, 128, 200, 300)), (D, causal)
+    assert not fwd(16, 128, 512, 64, 0) and not bwd(16, 96, 300, 128, 0)
+
+
 def test_alias_names_the_same_modules():
     """``corope_amd`` is an alias of the package in the directory ``co-rope_amd``: importing a submodule through either
     name gives the one module object whose globals the package's functions read (a second copy would have thresholds

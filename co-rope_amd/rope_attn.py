@@ -130,7 +130,7 @@ def use_rotated_path(N, D, training, slabs=None):
         return True
     if slabs is None or (D == 128 and (N + 255) // 256 * slabs >= _FWD_SMALL_ITEMS):
         return False
-    return N >= _FWD_ROTATED_MIN_N[D]
+    return N >= _FWD_ROTATED_MIN_N.get(D, TWO_LAUNCH_MIN_N)
 
 
 def _view_strides(t):

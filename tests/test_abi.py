@@ -317,6 +317,16 @@ def test_short_items_are_not_cut(pkg):
     assert not fwd(16, 128, 512, 64, 0) and not bwd(16, 96, 300, 128, 0)
 
 
+def test_rotated_path_rule_answers_for_every_head_dim(pkg):
+    """The rule is also asked about head dims that no kernel is built for (they take the length rule alone)."""
+    rule = pkg.rope_attn.use_rotated_path
+    for D in (16, 32, 64, 96, 128, 192, 256, 512):
+        for N in (1, 300, 1023, 1024, 5000):
+            for slabs in (None, 1, 40, 100000):
+                assert rule(N, D, False, slabs) in (True, False)
+    assert not rule(300, 96, False, 4) and rule(1024, 96, False, 4) and not rule(5000, 512, False, 4)
+
+
 def test_alias_names_the_same_modules():
     """``corope_amd`` is an alias of the package in the directory ``co-rope_amd``: importing a submodule through either
     name gives the one module object whose globals the package's functions read (a second copy would have thresholds

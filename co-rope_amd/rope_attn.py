@@ -101,15 +101,34 @@ def _freq_table(f):
 # for, q and k once for the backward (fused dK+dV, no tables in its loops, blocks cut into equal pieces where they are few).
 # Measured on MI355X, in us, unrotated -> rotated.  Forward and backward: always, B4 H8 N512 D64 52.1 -> 45.9, B1 H32 N96 D128
 # 64.3 -> 39.2, B3 Hq64 Hkv32 N64 D64 30.9 -> 26.7, B2 Hq32 Hkv4 N700 D64 299 -> 71, B2 Hq16 Hkv4 N400 D128 243 -> 77, B2 H8 N200
-# D256 133 -> 84 (from N * D = 65536 on it was before).  The forward alone pays the rotation pass's launch (3 to 4 us): D = 64, causal / not, H32 N600 16.7 -> 17.1 /
-# 15.9 -> 17.3 and N800 20.2 -> 19.4 / 19.9 -> 20.1; D = 256, H32 N128 26.1 -> 26.7 / 26.0 -> 24.8 and N160 35.5 -> 27.1; at D = 128 the
-# unrotated kernel's 256-row form holds out longer than its 128-row form: H32 N64 10.7 -> 13.2, N130 16.6 -> 15.4, N300 22.9 -> 19.0 (128 rows),
-# H128 N300 25.2 -> 26.6 / 22.5 -> 27.8 (256 rows).
+# D256 133 -> 84, B128 H32 N64 D64 265 -> 249, B512 H32 N16 D64 920 -> 869, B128 H32 N16 D256 1013 -> 571 (from N * D = 65536 on it was before).
+# The forward alone pays the rotation pass's launch (3 to 4 us) and its way through memory (_forward_pays_rotation).
 TWO_LAUNCH_MIN_N = 1024
 TRAIN_ROTATED_MIN_ND = 0
 _FWD_ROTATED_MIN_ND = 65536
-_FWD_ROTATED_MIN_N = {64: 768, 128: 129, 256: 129}
-_FWD_SMALL_ITEMS = 256   # 256-row items below this take the 128-row form: the compute units of an MI355X
+_COMPUTE_UNITS = 256   # of an MI355X
+
+
+def _forward_pays_rotation(N, D, slabs, kv_slabs, causal, cus):
+    """Whether a forward alone that is shorter than 1024 rows and 65536 elements a head takes rotated keys.  Both sides measured on MI355X, in us,
+    unrotated -> rotated, B1, 256 compute units:
+
+    D = 64, causal: the unrotated kernel rotates its tiles beside the products of other waves.  H16 N832 19.0 -> 17.4, H32 N832 19.2 -> 18.5, grouped Hq192
+    Hkv24 N1000 56.6 -> 54.2; beyond, H48 N896 20.5 -> 21.6, H80 N768 19.3 -> 23.3, H192 N768 40.3 -> 45.9, H224 N960 65.4 -> 71.7.
+    D = 64, not causal: H112 N832 46.5 -> 44.3, H256 N896 101.9 -> 91.4; not where the 256-row items are just one round or a little less
+    (H64 N832 25.2 -> 27.3, H80 N768 24.8 -> 27.5).
+    D = 128, fewer 256-row items than compute units (from there on the unrotated kernel's 256-row form holds out: H128 N300 25.2 -> 26.6): H8 N129
+    15.4 -> 14.4, H96 N257 27.4 -> 26.1, H255 N129 not causal 33.0 -> 31.4; causal, up to three blocks of 128 rows, only while those are about one
+    round: H128 N160 18.1 -> 18.2; beyond, H160 N160 23.0 -> 26.6, H192 N256 28.4 -> 31.2, H112 N320 28.4 -> 29.9.
+    D = 256: H32 N128 26.1 -> 26.7, N160 35.5 -> 27.1, H255 N129 75.9 -> 48.9."""
+    items = (N + 255) // 256 * slabs
+    if D == 256:
+        return N > 128
+    if D == 128:
+        return N > 128 and items < cus and not (causal and N <= 384 and (N + 127) // 128 * slabs * 8 > cus * 9)
+    if D == 64 and causal:
+        return N >= 768 and kv_slabs * 8 <= cus
+    return D == 64 and N > 768 and not cus * 3 < items * 4 <= cus * 4
 
 
 # fp16 tensors, forward of a call that will be differentiated: "exact" keeps P and V in fp16 (O within 1.2e-2 of the fp32 oracle at the
@@ -121,16 +140,14 @@ _FWD_SMALL_ITEMS = 256   # 256-row items below this take the 128-row form: the c
 FP16_TRAINING_FORWARD = "exact"
 
 
-def use_rotated_path(N, D, training, slabs=None):
-    """Whether the operator rotates the operands ahead of the attention kernels at this shape.  slabs: batch * query heads; None leaves
-    out the lengths that depend on it (an fp16 forward at D = 256 has only the single-launch kernel there)."""
+def use_rotated_path(N, D, training, slabs=None, kv_slabs=None, causal=True, cus=_COMPUTE_UNITS):
+    """Whether the operator rotates the operands ahead of the attention kernels at this shape.  slabs, kv_slabs: batch times query and key/value heads;
+    None leaves out the lengths that depend on them (an fp16 forward at D = 256 has only the single-launch kernel there).  cus: compute units."""
     if N * D < TRAIN_ROTATED_MIN_ND or D > _ROTATED_PATH_MAX_D:
         return N >= TWO_LAUNCH_MIN_N and D <= _ROTATED_PATH_MAX_D
     if training or N >= TWO_LAUNCH_MIN_N or N * D >= _FWD_ROTATED_MIN_ND:
         return True
-    if slabs is None or (D == 128 and (N + 255) // 256 * slabs >= _FWD_SMALL_ITEMS):
-        return False
-    return N >= _FWD_ROTATED_MIN_N.get(D, TWO_LAUNCH_MIN_N)
+    return slabs is not None and _forward_pays_rotation(N, D, slabs, slabs if kv_slabs is None else kv_slabs, causal, cus)
 
 
 def _view_strides(t):
@@ -144,13 +161,14 @@ def _view_strides(t):
     return (ctypes.c_int64 * 3)(sb, sh, sn)
 
 
-def _route(dtype, slabs, N, D, keep_rotated, two_launch=None):
+def _route(q, k, causal, keep_rotated, two_launch=None):
     """(rotate K ahead?, keep P and V in fp16 there?) for a forward."""
+    B, H, N, D = q.shape
     asked = two_launch is not None
     if not asked:
-        two_launch = use_rotated_path(N, D, keep_rotated, slabs if dtype == torch.bfloat16 or D <= 128 else None)
+        two_launch = use_rotated_path(N, D, keep_rotated, B * H if q.dtype == torch.bfloat16 or D <= 128 else None, B * k.shape[1], causal)
     # fp16 with gradients, or so short that the fast form's kernel never served it: P and V stay fp16 (no key-norm maxima)
-    return two_launch, (dtype == torch.float16 and two_launch and
+    return two_launch, (q.dtype == torch.float16 and two_launch and
                         (FP16_TRAINING_FORWARD != "fast" if keep_rotated else not asked and not use_rotated_path(N, D, False)))
 
 
@@ -172,10 +190,9 @@ def _fwd_parts(lib, q, causal):
 def _native_forward(lib, q, k, v, causal, sm_scale, fc, fs, keep):
     """What _forward returns, and the v to keep, by the native host side; None where this is not a plain call (then _check_inputs and
     _forward do it)."""
-    if q.dim() != 4 or not q.is_cuda or q.shape[3] not in _SUPPORTED_D or torch.cuda.current_device() != q.device.index:
+    if q.dim() != 4 or k.dim() != 4 or not q.is_cuda or q.shape[3] not in _SUPPORTED_D or torch.cuda.current_device() != q.device.index:
         return None
-    B, H, N, D = q.shape
-    rotated, exact = _route(q.dtype, B * H, N, D, keep)
+    rotated, exact = _route(q, k, causal, keep)
     host, table = lib.host
     out = host.rope_forward(table, q, k, v, fc, fs, causal, float(sm_scale), rotated, exact, keep, q.device.index, _stream_ptr(q),
                             _fwd_parts(lib, q, causal)[0] if rotated else None)
@@ -201,7 +218,7 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
             q, k, v, strides = q.contiguous(), k.contiguous(), v.contiguous(), None
     o = torch.empty(q.shape, device=q.device, dtype=q.dtype)
     M = torch.empty((B, H, N), device=q.device, dtype=torch.float32)
-    two_launch, exact = _route(q.dtype, B * H, N, D, keep_rotated, two_launch)
+    two_launch, exact = _route(q, k, causal, keep_rotated, two_launch)
     fp16 = q.dtype == torch.float16
     rotated = None
     Hkv = k.shape[1]

@@ -327,6 +327,17 @@ def test_rotated_path_rule_answers_for_every_head_dim(pkg):
     assert not rule(300, 96, False, 4) and rule(1024, 96, False, 4) and not rule(5000, 512, False, 4)
 
 
+def test_where_a_forward_alone_takes_rotated_keys(pkg):
+    """Both sides of the rule for forwards alone below 1024 rows, at shapes where one path was measured to be the faster (256 compute units)."""
+    rule = lambda N, D, slabs, causal=True, kv=None: pkg.rope_attn.use_rotated_path(N, D, False, slabs, kv, causal)
+    rotated = [(832, 64, 16), (1000, 64, 32), (1000, 64, 192, True, 24), (832, 64, 112, False), (900, 64, 1000, False), (129, 128, 8), (160, 128, 128), (257, 128, 96),
+               (511, 128, 127), (129, 128, 255, False), (300, 128, 112, False), (129, 256, 2048)]
+    unrotated = [(767, 64, 8), (768, 64, 80), (900, 64, 48), (1000, 64, 128), (768, 64, 80, False), (832, 64, 64, False), (128, 128, 8), (160, 128, 160), (256, 128, 192),
+                 (320, 128, 112), (300, 128, 128), (300, 128, 128, False), (128, 256, 32)]
+    assert all(rule(*s) for s in rotated) and not any(rule(*s) for s in unrotated)
+    assert all(rule(N, D, slabs, causal) for N, D in ((1024, 64), (512, 128), (256, 256)) for slabs in (1, 64, 4096) for causal in (True, False))
+
+
 def test_alias_names_the_same_modules():
     """``corope_amd`` is an alias of the package in the directory ``co-rope_amd``: importing a submodule through either
     name gives the one module object whose globals the package's functions read (a second copy would have thresholds

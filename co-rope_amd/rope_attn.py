@@ -10,6 +10,7 @@ the same kernel sources built for fp16 elements)."""
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -106,7 +107,6 @@ def _freq_table(f):
 TWO_LAUNCH_MIN_N = 1024
 TRAIN_ROTATED_MIN_ND = 0
 _FWD_ROTATED_MIN_ND = 65536
-_COMPUTE_UNITS = 256   # of an MI355X
 
 
 def _forward_pays_rotation(N, D, slabs, kv_slabs, causal, cus):
@@ -131,6 +131,12 @@ def _forward_pays_rotation(N, D, slabs, kv_slabs, causal, cus):
     return D == 64 and N > 768 and not cus * 3 < items * 4 <= cus * 4
 
 
+@functools.lru_cache(maxsize=None)
+def _compute_units(device_index):
+    """As the library asks for its own rules: a partition of the card has fewer than its 256."""
+    return torch.cuda.get_device_properties(device_index).multi_processor_count
+
+
 # fp16 tensors, forward of a call that will be differentiated: "exact" keeps P and V in fp16 (O within 1.2e-2 of the fp32 oracle at the
 # reference's verification temperature sm_scale = 0.5, gradients within its 0.15 / 5e-3 thresholds): the pipelined forward that looks at
 # each half tile's probabilities before it uses them, at D = 256 the single-launch kernel on a key copy rotated beforehand;
@@ -140,7 +146,7 @@ def _forward_pays_rotation(N, D, slabs, kv_slabs, causal, cus):
 FP16_TRAINING_FORWARD = "exact"
 
 
-def use_rotated_path(N, D, training, slabs=None, kv_slabs=None, causal=True, cus=_COMPUTE_UNITS):
+def use_rotated_path(N, D, training, slabs=None, kv_slabs=None, causal=True, cus=256):
     """Whether the operator rotates the operands ahead of the attention kernels at this shape.  slabs, kv_slabs: batch times query and key/value heads;
     None leaves out the lengths that depend on them (an fp16 forward at D = 256 has only the single-launch kernel there).  cus: compute units."""
     if N * D < TRAIN_ROTATED_MIN_ND or D > _ROTATED_PATH_MAX_D:
@@ -166,7 +172,8 @@ def _route(q, k, causal, keep_rotated, two_launch=None):
     B, H, N, D = q.shape
     asked = two_launch is not None
     if not asked:
-        two_launch = use_rotated_path(N, D, keep_rotated, B * H if q.dtype == torch.bfloat16 or D <= 128 else None, B * k.shape[1], causal)
+        two_launch = use_rotated_path(N, D, keep_rotated, B * H if q.dtype == torch.bfloat16 or D <= 128 else None, B * k.shape[1], causal,
+                                      _compute_units(q.device.index))
     # fp16 with gradients, or so short that the fast form's kernel never served it: P and V stay fp16 (no key-norm maxima)
     return two_launch, (q.dtype == torch.float16 and two_launch and
                         (FP16_TRAINING_FORWARD != "fast" if keep_rotated else not asked and not use_rotated_path(N, D, False)))

@@ -338,6 +338,19 @@ def test_where_a_forward_alone_takes_rotated_keys(pkg):
     assert all(rule(N, D, slabs, causal) for N, D in ((1024, 64), (512, 128), (256, 256)) for slabs in (1, 64, 4096) for causal in (True, False))
 
 
+def test_forward_route_asks_the_device_for_its_compute_units(pkg, monkeypatch):
+    """The line between the forward's kernel forms moves with the compute units, as the library's own does (a partition of a card has fewer)."""
+    R = pkg.rope_attn
+    monkeypatch.setattr(R, "_compute_units", lambda index: 64)
+
+    class Q:
+        shape, dtype, device = (1, 100, 200, 128), torch.bfloat16, torch.device("cuda", 0)
+
+    assert R._route(Q, Q, True, False) == (False, False)
+    monkeypatch.setattr(R, "_compute_units", lambda index: 256)
+    assert R._route(Q, Q, True, False) == (True, False)
+
+
 def test_alias_names_the_same_modules():
     """``corope_amd`` is an alias of the package in the directory ``co-rope_amd``: importing a submodule through either
     name gives the one module object whose globals the package's functions read (a second copy would have thresholds

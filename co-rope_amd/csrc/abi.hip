@@ -741,7 +741,7 @@ namespace {
 int rope_attn_fwd_strided_impl(const char* what, const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,
                                const int64_t* v_strides, const float* freqs_cos, const float* freqs_sin, int64_t freq_row_stride, void* o,
                                float* lse, void* q_rot, void* k_rot, float* tile_kmax, int B, int H, int Hkv, int N, int D, float sm_scale,
-                               int causal, int fp16, bool cut, void* parts, int64_t parts_bytes, void* v_keep, void* stream) {
+                               int causal, int fp16, bool pipe_exact, void* parts, int64_t parts_bytes, void* v_keep, void* stream) {
   if (Hkv <= 0 || H % Hkv != 0) return fail(COROPE_E_BADARG, "%s: H=%d is not a multiple of Hkv=%d", what, H, Hkv);
   int rc = corope_rope_attn_check(B, H, N, D, freq_row_stride, sm_scale, 0);
   if (rc) return rc;
@@ -788,7 +788,7 @@ int rope_attn_fwd_strided_impl(const char* what, const void* q, const int64_t* q
   if (rc) return rc;
   if (q_rot != nullptr && !aligned16(q_rot)) return fail(COROPE_E_ALIGN, "%s: q_rot %p is not 16-byte aligned", what, q_rot);
   // tile_kmax null: the attention kernel is the single-launch one on the rotated copy (no lazy reference value; for fp16
-  // tensors: probabilities in fp16 against an fp16 V); for fp16 and with the right to cut the pipelined one that keeps them so
+  // tensors: probabilities in fp16 against an fp16 V), or, where pipe_exact asks for it, the pipelined one that keeps them so
   if (reinterpret_cast<uintptr_t>(tile_kmax) & 3u) return fail(COROPE_E_ALIGN, "%s: tile_kmax %p is misaligned", what, (const void*)tile_kmax);
   uint16_t* kr = static_cast<uint16_t*>(k_rot);
   rc = launch_status(what, fp16 ? corope_f16::launch_rope_rotate(p.k, p.cos, p.sin, p.fstride, kr, tile_kmax, B * Hkv, N, D, st, 1.f,
@@ -798,7 +798,7 @@ int rope_attn_fwd_strided_impl(const char* what, const void* q, const int64_t* q
   if (rc) return rc;
   p.k_rot = kr;
   p.tile_kmax = tile_kmax;
-  p.exact = cut && fp16;
+  p.exact = pipe_exact && fp16;
   p.q_rot_out = static_cast<uint16_t*>(q_rot);
   return launch_status(what, fp16 ? corope_f16::launch_rope_attn_fwd_prerotated(p, D, causal != 0, st)
                                   : corope::launch_rope_attn_fwd_prerotated(p, D, causal != 0, st));
@@ -826,7 +826,7 @@ int corope_rope_attn_fwd_cut(const void* q, const int64_t* q_strides, const void
                              void* q_rot, void* k_rot, float* tile_kmax, int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
                              void* parts, int64_t parts_bytes, void* stream) {
   return rope_attn_fwd_strided_impl("rope_attn_fwd_cut", q, q_strides, k, k_strides, v, v_strides, freqs_cos, freqs_sin, freq_row_stride, o, lse, q_rot,
-                                    k_rot, tile_kmax, B, H, Hkv, N, D, sm_scale, causal, fp16, true, parts, parts_bytes, nullptr, stream);
+                                    k_rot, tile_kmax, B, H, Hkv, N, D, sm_scale, causal, fp16, false, parts, parts_bytes, nullptr, stream);
 }
 
 int corope_rope_attn_fwd_keep(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides, const void* v,

@@ -237,14 +237,14 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
             q_rot = torch.empty(q.shape, device=q.device, dtype=q.dtype) if (two_launch and keep_rotated) else None
             k_rot = torch.empty(k.shape, device=q.device, dtype=q.dtype) if two_launch else None
             kmax = torch.empty((B, Hkv, (N + 63) // 64), device=q.device, dtype=torch.float32) if (two_launch and not exact) else None
-            rc = lib.corope_rope_attn_fwd_cut(q.data_ptr(), strides[0], k.data_ptr(), strides[1], v.data_ptr(), strides[2],
+            rc = lib.corope_rope_attn_fwd_keep(q.data_ptr(), strides[0], k.data_ptr(), strides[1], v.data_ptr(), strides[2],
                                               fc.data_ptr(), fs.data_ptr(), fc.stride(0), o.data_ptr(), M.data_ptr(),
                                               q_rot.data_ptr() if q_rot is not None else None,
                                               k_rot.data_ptr() if k_rot is not None else None,
                                               kmax.data_ptr() if kmax is not None else None, B, H, Hkv, N, D,
                                               float(sm_scale), int(bool(causal)), int(fp16),
-                                              parts.data_ptr() if parts is not None else None, nbytes, _stream_ptr(q))
-            _lib.check(rc, "corope_rope_attn_fwd_cut")
+                                              parts.data_ptr() if parts is not None else None, nbytes, None, _stream_ptr(q))
+            _lib.check(rc, "corope_rope_attn_fwd_keep")
             if q_rot is not None:
                 rotated = (q_rot, k_rot)
         elif q.dtype == torch.float16:

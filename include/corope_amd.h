@@ -264,11 +264,9 @@ int corope_rope_attn_fwd_strided(const void *q, const int64_t *q_strides, const 
                                  void *o, float *lse, void *q_rot, void *k_rot, float *tile_kmax,
                                  int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16, void *stream);
 
-/* The same with scratch in which the kernel on rotated keys leaves the pieces of query blocks that it cuts among
+/* The same with scratch in which the kernel on rotated keys (k_rot and tile_kmax given) leaves the pieces of query blocks that it cuts among
  * workgroups, so that few heads with long sequences fill the chip: corope_rope_attn_fwd_parts_bytes says how much, 0 where whole blocks fill it as
- * well (then, and if parts is NULL, nothing is cut).  With tile_kmax given, or k_rot NULL, it is otherwise corope_rope_attn_fwd_strided; fp16 tensors
- * with k_rot and without tile_kmax run (D = 64, 128) the pipelined kernel with P and V in fp16: that of corope_rope_attn_fwd_strided keeps the bits of
- * the single launch, this one is up to a third faster, and more with few heads.  (bf16 with k_rot and without tile_kmax is never cut.)  At most two slots per compute unit: with 256 of them
+ * well (then, and if parts is NULL, nothing is cut and this is corope_rope_attn_fwd_strided).  At most two slots per compute unit: with 256 of them
  * 33 MiB at D = 64, 65 MiB at D = 128.  (fused-rope/fused_rope_attn.py:655-722 launches whole query blocks only.) */
 int64_t corope_rope_attn_fwd_parts_bytes(int B, int H, int N, int D, int causal);
 int corope_rope_attn_fwd_cut(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
@@ -278,7 +276,9 @@ int corope_rope_attn_fwd_cut(const void *q, const int64_t *q_strides, const void
                              int B, int H, int Hkv, int N, int D, float sm_scale, int causal, int fp16,
                              void *parts, int64_t parts_bytes, void *stream);
 /* The same, and v_keep ((B,Hkv,N,D), may be NULL; needs k_rot) receives a contiguous copy of v, made by the launch that rotates K: what a caller that must
- * not hold on to a view of its projection keeps for the backward (the reference saves v itself, fused-rope/fused_rope_attn.py:718). */
+ * not hold on to a view of its projection keeps for the backward (the reference saves v itself, fused-rope/fused_rope_attn.py:718).  And fp16 tensors with
+ * k_rot and without tile_kmax run (D = 64, 128) the pipelined kernel with P and V in fp16, whose blocks may be cut: up to a third faster than the single
+ * launch, whose bits the two entry points above keep, and more with few heads.  (bf16 with k_rot and without tile_kmax is never cut.) */
 int corope_rope_attn_fwd_keep(const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
                               const void *v, const int64_t *v_strides,
                               const float *freqs_cos, const float *freqs_sin, int64_t freq_row_stride,

@@ -210,6 +210,34 @@ def test_pipelined_forward_with_fp16_probabilities(pkg, monkeypatch, B, H, Hkv, 
     assert ((M - rM).abs() <= 1e-3 + 2.0 ** -20 * rM.abs()).all()
 
 
+@pytest.mark.parametrize("B,H,Hkv,N,D", [(1, 2, 1, 70, 64), (1, 2, 2, 257, 128), (1, 8, 8, 4096, 128), (2, 3, 1, 130, 256)])
+def test_forward_entry_points_without_key_norm_maxima(pkg, B, H, Hkv, N, D):
+    """fp16, k_rot without tile_kmax: corope_rope_attn_fwd_cut keeps the bits of corope_rope_attn_fwd_strided, with scratch and without, and
+    corope_rope_attn_fwd_keep runs the pipelined kernel (other sums of the same rounded weights)."""
+    import ctypes
+    lib = pkg._lib.load()
+    q, k, v = (seeded((B, h, N, D), 90 + h).cuda().half() for h in (H, Hkv, Hkv))
+    c, s = (t.cuda() for t in O.precompute_freqs_cis(D, N))
+    st3 = lambda t: (ctypes.c_int64 * 3)(*t.stride()[:3])
+    nbytes = max(0, lib.corope_rope_attn_fwd_parts_bytes(B, H, N, D, 1)) if D <= 128 else 0
+    parts = torch.empty(nbytes, device="cuda", dtype=torch.uint8) if nbytes else None
+    assert (nbytes > 0) == (N == 4096)
+
+    def run(name, *tail):
+        o, M, kr = torch.empty_like(q), torch.empty(B, H, N, device="cuda"), torch.empty_like(k)
+        rc = getattr(lib, name)(q.data_ptr(), st3(q), k.data_ptr(), st3(k), v.data_ptr(), st3(v), c.data_ptr(), s.data_ptr(), c.stride(0), o.data_ptr(),
+                                M.data_ptr(), None, kr.data_ptr(), None, B, H, Hkv, N, D, 1 / math.sqrt(D), 1, 1, *tail, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, pkg._lib.last_error()
+        return o, M
+
+    single = run("corope_rope_attn_fwd_strided")
+    for scratch in ((None, 0), (parts.data_ptr() if nbytes else None, nbytes)):
+        assert all(torch.equal(a, b) for a, b in zip(run("corope_rope_attn_fwd_cut", *scratch), single))
+        o, M = run("corope_rope_attn_fwd_keep", *scratch, None)
+        assert (o.float() - single[0].float()).abs().max() <= 3 * 2.0 ** -11 * v.float().abs().max() and (M - single[1]).abs().max() <= 1e-3
+        assert D == 256 or not torch.equal(M, single[1])
+
+
 def test_fp16_forward_of_inputs_that_are_not_finite(pkg):
     """A query row that is NaN or infinite spoils its own output row and no other."""
     B, H, N, D = 1, 2, 300, 128

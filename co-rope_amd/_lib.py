@@ -8,6 +8,7 @@ import ctypes
 import importlib.util
 import os
 import threading
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libcorope_amd.so")
@@ -65,7 +66,7 @@ SIGNATURES = {
 }
 
 # The operators' host side in native code (csrc/host_calls.cpp): one Python call per forward or backward instead of one per allocation
-# and a ctypes call.  Entry points it goes through, in its order.
+# and a ctypes call; without it the Python binding does the same.  Entry points it goes through, in its order.
 HOST_PATH = os.path.join(_HERE, "lib", "corope_host_calls.so")
 HOST_CALLS = ("corope_rope_attn_fwd_keep", "corope_rope_attn_bwd_rotated", "corope_gqa_fwd", "corope_gqa_fwd_f16", "corope_gqa_bwd", "corope_gqa_bwd_f16")
 
@@ -78,15 +79,36 @@ class CoRopeLibraryError(RuntimeError):
     """The native library is missing, stale, or a launch failed."""
 
 
+class _NoHost:
+    """In the place of the native host side where it cannot be loaded: takes no call, so that the Python binding does every one."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _load_host():
+    """The native host side.  It only saves host time, so where it was not built, or was built against another torch, calls go without it."""
+    import torch
+    try:
+        if not os.path.exists(HOST_PATH):
+            raise ImportError("not found")
+        spec = importlib.util.spec_from_file_location("corope_host_calls", HOST_PATH)
+        host = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(host)
+        if host.torch_version != torch.__version__.split("+")[0]:
+            raise ImportError(f"built against torch {host.torch_version}, this is {torch.__version__}")
+        return host
+    except (ImportError, OSError, AttributeError) as e:
+        warnings.warn(f"{HOST_PATH}: {e}; every call goes through the Python binding, which takes up to twice the host time "
+                      "(`python co-rope_amd/build.py` builds it where torch, its headers and g++ are)", RuntimeWarning, stacklevel=4)
+        return _NoHost()
+
+
 def _bind_host(lib):
     """Sets lib.host to (native host module, its table of lib's entry points)."""
     global _host
     if _host is None:
-        if not os.path.exists(HOST_PATH):
-            raise CoRopeLibraryError(f"{HOST_PATH} not found: build it with `python co-rope_amd/build.py`")
-        spec = importlib.util.spec_from_file_location("corope_host_calls", HOST_PATH)
-        _host = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(_host)
+        _host = _load_host()
     lib.host = _host, _host.make_table(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in HOST_CALLS))
 
 

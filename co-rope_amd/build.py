@@ -4,11 +4,14 @@ Run as ``python co-rope_amd/build.py`` or call ``build()``; the result lands in
 ``co-rope_amd/lib/libcorope_amd.so`` and is what ``_lib.load()`` opens.  Beside it, for measurement only:
 ``libcorope_amd_trace.so`` (the same sources with -DCOROPE_TRACE: the attention kernels stamp a clock at their phase
 boundaries into a buffer ``bench.py --phase-trace`` hands them, and a call forces kernel forms for the tests).
-``corope_host_calls.so`` beside them is the Python binding's native half (host code only).  ``build_program`` compiles a stand-alone HIP program with the same flags (``bench.py --mfma-rate`` uses it)."""
+``corope_host_calls.so`` beside them is the Python binding's native half (host code only, built where torch's headers are).
+``build_program`` compiles a stand-alone HIP program with the same flags (``bench.py --mfma-rate`` uses it)."""
 from __future__ import annotations
 
 import glob
+import importlib.util
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -90,8 +93,24 @@ def _link(objs, out, shared=True):
     return out
 
 
+def host_lacks():
+    """What build_host needs and is not there (the kernels need only hipcc)."""
+    missing = [] if importlib.util.find_spec("torch") else ["torch"]
+    if shutil.which("g++") is None:
+        missing.append("g++")
+    if not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")):
+        missing.append("Python.h")
+    return missing
+
+
 def build_host():
-    """The native host side of the operators (csrc/host_calls.cpp): host code against torch's headers, no device code."""
+    """The native host side of the operators (csrc/host_calls.cpp): host code against torch's headers, no device code.  Where what it needs is
+    not there it is left out (the Python binding serves every call without it)."""
+    if host_lacks():
+        print(f"corope_host_calls.so is not built: no {', '.join(host_lacks())}", file=sys.stderr)
+        if os.path.exists(HOST_LIB):
+            os.remove(HOST_LIB)   # (of another state of the sources)
+        return None
     import torch
     root = os.path.dirname(torch.__file__)
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",

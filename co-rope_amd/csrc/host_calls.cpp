@@ -9,6 +9,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pycfunction_helpers.h>
 #include <ATen/ATen.h>
+#include <torch/version.h>
 
 #include "../../include/corope_amd.h"
 
@@ -263,4 +264,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "corope_host_calls", nullptr, -1, m
 
 }  // namespace
 
-extern "C" __attribute__((visibility("default"))) PyObject* PyInit_corope_host_calls(void) { return PyModule_Create(&module); }
+extern "C" __attribute__((visibility("default"))) PyObject* PyInit_corope_host_calls(void) {
+  PyObject* m = PyModule_Create(&module);
+  // (the tensors' layout is that of the torch this was built against: the loader compares)
+  if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}

@@ -252,6 +252,36 @@ def test_missing_library_fails_loudly(pkg, monkeypatch):
         pkg._lib.load()
 
 
+@pytest.mark.parametrize("form", ["missing", "not a module", "other torch"])
+def test_library_loads_without_its_native_host_side(pkg, monkeypatch, tmp_path, form):
+    """The host side only saves host time: without it the library loads, says so, and no call goes through it."""
+    L = pkg._lib
+    path = tmp_path / "corope_host_calls.so"
+    if form == "not a module":
+        path.write_bytes(b"no shared object")
+    monkeypatch.setattr(L, "_lib", None)
+    monkeypatch.setattr(L, "_host", None)
+    if form == "other torch":
+        monkeypatch.setattr(torch, "__version__", "1.0.0+other")
+    else:
+        monkeypatch.setattr(L, "HOST_PATH", str(path))
+    with pytest.warns(RuntimeWarning, match="corope_host_calls.so.*Python binding"):
+        lib = L.load()
+    host, table = lib.host
+    assert lib.corope_amd_version() == L.ABI_VERSION and host.rope_forward(table, 1, 2) is None and host.gqa_backward(table) is None
+
+
+def test_kernels_build_without_what_the_host_side_needs(monkeypatch, tmp_path, capsys):
+    from importlib import import_module
+    build = import_module("co-rope_amd.build")
+    assert build.host_lacks() == []
+    stale = tmp_path / "corope_host_calls.so"
+    stale.write_bytes(b"")
+    monkeypatch.setattr(build, "HOST_LIB", str(stale))
+    monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    assert build.build_host() is None and not stale.exists() and "g++" in capsys.readouterr().err
+
+
 def test_strided_forward_argument_checks(pkg):
     """Strides are checked before any launch: multiples of 8 elements, rows at least D apart, slices below 4 GiB."""
     import ctypes

@@ -181,8 +181,12 @@ PyObject* rope_backward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   at::Tensor d_o = *x[4];
   int64_t ds[3];
-  const bool view = !d_o.is_contiguous();
-  if (!aligned16(d_o) || (view && (D > 128 || !strides_of(d_o, ds)))) Py_RETURN_NONE;
+  bool view = !d_o.is_contiguous();
+  if (view && (D > 128 || !strides_of(d_o, ds))) {   // what the kernels cannot read where it lies is copied
+    d_o = d_o.contiguous();
+    view = false;
+  }
+  if (!aligned16(d_o)) Py_RETURN_NONE;
   at::Tensor parts;
   if (!parts_of(args[13], device, parts)) Py_RETURN_NONE;
   const auto opts = q.options().requires_grad(false);

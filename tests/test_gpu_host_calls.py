@@ -88,14 +88,16 @@ def test_rope_same_bits_both_ways(pkg, both_ways, layout, B, H, Hkv, N, D, dtype
         out = pkg.attention(*x, False, scale, c, s)
         return [out.detach(), *torch.autograd.grad(out, x, g)]
 
+    plain = layout in ("bhnd", "bnhd", "qkv", "narrow") or (layout == "transposed" and N == 1)
     for f in (forward, train):
+        both_ways.seen.clear()
         a, b = both_ways(f)
+        # (what a forward keeps is plain in any case, and a gradient of another layout is copied)
+        assert both_ways.seen == [("rope_forward", plain)] + [("rope_backward", True)] * (f is train and layout != "misaligned")
         if layout == "misaligned":
             assert a[0] is ValueError and a == b
         else:
             assert all(torch.equal(x, y) and x.is_contiguous() and y.is_contiguous() for x, y in zip(a, b)), f.__name__
-    plain = layout in ("bhnd", "bnhd", "qkv", "narrow") or (layout == "transposed" and N == 1)
-    assert both_ways.seen[0] == ("rope_forward", plain)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

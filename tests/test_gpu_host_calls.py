@@ -18,7 +18,8 @@ class _Refuses:
 
 @pytest.fixture
 def both_ways(pkg, monkeypatch):
-    """run(f) -> [f() through the native host side, f() through the Python binding]; an exception counts as its type and text."""
+    """run(f) -> [f() through the native host side, f() through the Python binding]; an exception counts as its type and text.  run.seen: (name, whether
+    it took the call) for the calls that the native side was asked for."""
     lib = pkg._lib.load()
     native, seen = lib.host, []
 
@@ -113,7 +114,11 @@ def test_corope_same_bits_both_ways(pkg, both_ways, layout, dtype):
         return [out.detach(), *torch.autograd.grad(out, x, g)]
 
     a, b = both_ways(train)
-    assert a[0] is ValueError and a == b or all(torch.equal(x, y) for x, y in zip(a, b))
+    if layout == "misaligned":
+        assert a[0] is ValueError and a == b and both_ways.seen == [("gqa_forward", False)]
+    else:
+        assert both_ways.seen == [("gqa_forward", True), ("gqa_backward", True)]
+        assert len(a) == len(b) == 4 and all(torch.equal(x, y) for x, y in zip(a, b))
 
 
 def test_tables_of_other_forms_both_ways(pkg, both_ways):

@@ -29,11 +29,11 @@ def _force_path(monkeypatch, pkg, rotated):
     monkeypatch.setattr(pkg.rope_attn, "TRAIN_ROTATED_MIN_ND", 1 if rotated else 1 << 60)
 
 
-def _gpu_fwd_bwd(pkg, q, k, v, g, causal, scale, c, s):
+def _gpu_fwd_bwd(pkg, q, k, v, g, causal, scale, c, s, dtype=torch.bfloat16):
     dev = torch.device("cuda:0")
-    qd, kd, vd = (t.to(dev, torch.bfloat16).requires_grad_(True) for t in (q, k, v))
+    qd, kd, vd = (t.to(dev, dtype).requires_grad_(True) for t in (q, k, v))
     o = pkg.attention(qd, kd, vd, causal, scale, c.to(dev), s.to(dev))
-    o.backward(g.to(dev, torch.bfloat16))
+    o.backward(g.to(dev, dtype))
     torch.cuda.synchronize()
     return tuple(t.detach().float().cpu() for t in (o, qd.grad, kd.grad, vd.grad))
 
@@ -602,22 +602,27 @@ def test_entry_points_on_rotated_copies_agree(pkg, B, Hq, Hkv, N, D, causal):
                   int(dtype == torch.float16), None, 0, st)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("B,Hq,Hkv,N,D", [(1, 2, 1, 1, 128), (2, 8, 2, 63, 64), (1, 8, 1, 65, 128), (3, 4, 4, 129, 64), (1, 6, 3, 129, 256), (2, 16, 4, 511, 128),
-                                          (1, 8, 2, 767, 64), (1, 4, 4, 768, 64)])
-def test_short_sequences_by_the_operators_own_rule(pkg, B, Hq, Hkv, N, D, causal):
+                                          (1, 8, 2, 767, 64), (1, 4, 4, 768, 64),
+                                          (1, 4, 2, 769, 64), (1, 8, 1, 1023, 64)])
+def test_short_sequences_by_the_operators_own_rule(pkg, B, Hq, Hkv, N, D, causal, dtype):
     """Training runs on rotated copies at every length, the forward alone from the lengths of use_rotated_path on (edges on both sides):
-    each against the oracle, and the two forwards within one bf16 step of each other."""
+    each against the oracle, and the two forwards against each other.  They round the same things: a weight by half a step of the type in either (of the
+    largest |v|, since the weights of a row add up to one; fp16 ones below its smallest normal number by 2^-25 of the row's largest), and O by half a step."""
     G, scale = Hq // Hkv, 1 / math.sqrt(D)
-    q, g = (bf16_round(seeded((B, Hq, N, D), 120 + i)) for i in range(2))
-    k, v = (bf16_round(seeded((B, Hkv, N, D), 130 + i)) for i in range(2))
+    q, g = (seeded((B, Hq, N, D), 120 + i).to(dtype).float() for i in range(2))
+    k, v = (seeded((B, Hkv, N, D), 130 + i).to(dtype).float() for i in range(2))
     c, s = O.precompute_freqs_cis(D, N)
-    got = _gpu_fwd_bwd(pkg, q, k, v, g, causal, scale, c, s)
-    alone = pkg.attention(*(t.cuda().bfloat16() for t in (q, k, v)), causal, scale, c.cuda(), s.cuda()).float().cpu()
+    got = _gpu_fwd_bwd(pkg, q, k, v, g, causal, scale, c, s, dtype)
+    alone = pkg.attention(*(t.cuda().to(dtype) for t in (q, k, v)), causal, scale, c.cuda(), s.cuda()).float().cpu()
     ro, _, rdq, rdk, rdv, _ = O.rope_attn_fwd_bwd_blocked(q, k.repeat_interleave(G, 1), v.repeat_interleave(G, 1), g, causal, scale, c, s)
     rdk, rdv = (t.reshape(B, Hkv, G, N, D).sum(2) for t in (rdk, rdv))
     for name, a, b in (("O", got[0], ro), ("O alone", alone, ro), ("dQ", got[1], rdq), ("dK", got[2], rdk), ("dV", got[3], rdv)):
         assert within_bar(a, b, TOL * (math.sqrt(G) if name in ("dK", "dV") else 1))[0], name
+    step, v_max = 2.0 ** (-8 if dtype == torch.bfloat16 else -11), v.abs().max()
+    assert ((got[0] - alone).abs() <= step * (v_max + ro.abs()) + 2 * N * 2.0 ** -25 * v_max).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -19,10 +19,10 @@ import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
 try:
-    from .check_isa import ASM_MFMA_IN_SOURCE, check_asm_mfma
+    from .check_isa import ASM_MFMA_IN_SOURCE, check_asm_mfma, check_tile_loops
 except ImportError:   # run as a script
     sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
-    from check_isa import ASM_MFMA_IN_SOURCE, check_asm_mfma
+    from check_isa import ASM_MFMA_IN_SOURCE, check_asm_mfma, check_tile_loops
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -76,12 +76,13 @@ def _compile(src, extra, suffix=""):
                     raise RuntimeError(f"no device assembly of {src}{suffix} to check")
                 for path in asm:
                     with open(path) as f:
-                        problems += check_asm_mfma(f.read(), src + suffix)
+                        text = f.read()
+                    problems += check_asm_mfma(text, src + suffix) + check_tile_loops(text, src + suffix)
     err = "\n".join(l for l in r.stderr.splitlines() if noise not in l)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed on {src}:\n{err}")
     if problems:
-        raise RuntimeError("asm-issued matrix-core results touched too early:\n" + "\n".join(problems))
+        raise RuntimeError("the generated assembly is not what the kernels rely on:\n" + "\n".join(problems))
     return obj, err
 
 

@@ -15,7 +15,10 @@ such statement of every kernel:
   straight-line code in front of the statement; a label ends the search).
 
 The build fails if a register copy, a spill or anything else has come between (a different compiler version, more
-register pressure, accumulators moved to the other half of the register file)."""
+register pressure, accumulators moved to the other half of the register file).
+
+``check_tile_loops`` looks for scratch memory in the tile loops (the innermost loops with matrix-core instructions) of the kernels that were laid
+out to keep all of a tile in registers: what they spill belongs to a change of items, which a tile does not pay for."""
 from __future__ import annotations
 
 import re
@@ -172,4 +175,43 @@ def check_asm_mfma(asm_text, name="<asm>"):
             verdict = _operand_written_just_before(lines, i + 1, _regs(m.group(2)) | _regs(m.group(3)) | addend)
             if verdict:
                 problems.append(f"{where}: {verdict}")
+    return problems
+
+
+#: kernels whose tile loops keep to registers: the pipelined forwards (but for the four-wave form with bf16 probabilities, which keeps one value
+#: there at D = 128) and, at head dim 256, the backward on rotated operands
+REGISTERS_ONLY = re.compile(r"rope_attn_fwd_pipe_kernelILi\d+ELb[01]E(Li8ELb[01]ELb[01]|Li4ELb0ELb1)E|rope_attn_fwd_pipe32_kernel|"
+                            r"rope_attn_bwd_dq_kernelILi256E\w*?ELb[01]ELb1ELb|rope_attn_bwd_dkdv_kernelILi256E\w*?ELb[01]ELb1ELb1ELb1E")
+
+
+def check_tile_loops(asm_text, name="<asm>", kernels=REGISTERS_ONLY):
+    """Returns a list of problems: scratch instructions in a tile loop of a kernel that matches.  (The compiler notes at each block which loop it
+    belongs to: "Loop Header: Depth=2", "in Loop: Header=BB3_40 Depth=2".)"""
+    problems, kernel, label, block = [], None, None, None
+    loops = {}   # header -> [depth, matrix-core instructions, scratch instructions]
+
+    def settle():
+        with_products = [l for l in loops.values() if l[1]]
+        for depth, _, scratch in with_products:
+            if scratch and depth == max(l[0] for l in with_products):
+                problems.append(f"{name}: {kernel}: {scratch} scratch instructions in a tile loop")
+
+    for line in asm_text.split("\n"):
+        if line.startswith("_Z") and line.split(";")[0].strip().endswith(":"):
+            kernel, block, loops = line.split(":")[0], None, {}
+        elif kernel is None or kernels.search(kernel) is None:
+            continue
+        if m := re.match(r"(?:\.L|; %)(\w+|bb\.\d+):", line):
+            label, block = m.group(1), None
+        if h := re.search(r"=>\s*This (?:Inner )?Loop Header: Depth=(\d+)", line):   # (on the label's line or the next)
+            block = loops.setdefault(label, [int(h.group(1)), 0, 0])
+        elif h := re.search(r"in Loop: Header=(\w+) Depth=(\d+)", line):
+            block = loops.setdefault(h.group(1), [int(h.group(2)), 0, 0])
+        elif block is not None and line.strip().startswith("v_mfma"):
+            block[1] += 1
+        elif block is not None and line.strip().startswith("scratch_"):
+            block[2] += 1
+        if line.startswith(".Lfunc_end"):
+            settle()
+            kernel, loops = None, {}
     return problems

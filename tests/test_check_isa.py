@@ -6,6 +6,7 @@ import re
 import pytest
 
 check = importlib.import_module("co-rope_amd.check_isa").check_asm_mfma
+check_tile_loops = importlib.import_module("co-rope_amd.check_isa").check_tile_loops
 
 ASM = "\t;;#ASMSTART\n\tv_mfma_f32_32x32x16_bf16 v[16:31], v[32:35], v[48:51], v[0:15]\n\t;;#ASMEND\n"
 ACCUMULATE = "\tv_mfma_f32_32x32x16_bf16 v[16:31], v[36:39], v[52:55], v[16:31]\n"
@@ -69,6 +70,39 @@ def test_sources_with_asm_matrix_instructions_are_found():
     assert "rope_rotate.hip" not in checked and "abi.hip" not in checked
 
 
+ITEMS = """_ZN6corope23rope_attn_bwd_dq_kernelILi256ELi4ELi32ELb1ELb1ELb0EEEvNS_9BwdParamsE: ; @kernel
+; %bb.0:
+	s_load_dword s0, s[4:5], 0x0
+.LBB0_1:                                ; =>This Loop Header: Depth=1
+                                        ;     Child Loop BB0_2 Depth 2
+	scratch_load_dword v1, off, off
+.LBB0_2:                                ;   Parent Loop BB0_1 Depth=1
+                                        ; =>  This Inner Loop Header: Depth=2
+	{header}
+	v_mfma_f32_32x32x16_bf16 a[16:31], v[36:39], v[52:55], a[16:31]
+; %bb.3:                                ;   in Loop: Header=BB0_2 Depth=2
+	{inner}
+	s_cbranch_scc1 .LBB0_2
+; %bb.4:                                ;   in Loop: Header=BB0_1 Depth=1
+	scratch_store_dword off, v1, off
+	s_cbranch_scc1 .LBB0_1
+; %bb.5:
+	s_endpgm
+.Lfunc_end0:
+"""
+
+
+def test_scratch_in_a_tile_loop_is_reported():
+    """What a kernel spills at a change of items passes; in its tile loop, in the loop's first block or another, it does not."""
+    nop, spill = "s_nop 0", "scratch_store_dword off, v2, off offset:4"
+    assert check_tile_loops(ITEMS.format(header=nop, inner=nop)) == []
+    for where in (dict(header=spill, inner=nop), dict(header=nop, inner=spill)):
+        problems = check_tile_loops(ITEMS.format(**where))
+        assert len(problems) == 1 and "1 scratch" in problems[0] and "dq_kernel" in problems[0]
+    # kernels that do not claim it are not held to it
+    assert check_tile_loops(ITEMS.format(header=spill, inner=spill).replace("ELb1ELb1ELb0E", "ELb1ELb0ELb0E")) == []
+
+
 def _kernels_of_the_library(path):
     """What the compiler noted of every kernel in a built library: the AMDGPU note (type 32) of each code object, a msgpack map."""
     msgpack = pytest.importorskip("msgpack")
@@ -90,3 +124,18 @@ def test_corope_forward_kernels_keep_their_registers():
     assert any("corope_f16" in n for n in kernels) and any("corope_f16" not in n for n in kernels)
     spilled = {n: k[".vgpr_spill_count"] for n, k in kernels.items() if k[".vgpr_spill_count"] > 4}
     assert not spilled, spilled
+
+
+@pytest.mark.parametrize("kernels,most", [
+    (r"corope_f16\d+rope_attn_fwd_pipe_kernelILi64ELb[01]ELi[48]ELb[01]ELb1E", 0),       # fp16 probabilities, D = 64
+    (r"corope_f16\d+rope_attn_fwd_pipe_kernelILi128ELb[01]ELi8ELb[01]ELb1E", 16),        # D = 128, eight waves, whole and cut
+    (r"corope_f16\d+rope_attn_fwd_pipe_kernelILi128ELb[01]ELi4ELb0ELb1E", 32),           # four waves
+    (r"rope_attn_bwd_dq_kernelILi256ELi4ELi32ELb[01]ELb1ELb0E", 40),                     # D = 256 on rotated operands: dQ, whole blocks
+    (r"rope_attn_bwd_dkdv_kernelILi256ELi4ELi32ELb[01]ELb1ELb1ELb1ELb[01]E", 8),         # dK+dV, whole and cut
+])
+def test_streamed_kernels_keep_their_registers(kernels, most):
+    """What these kernels spill lies at their changes of items (the build looks at the tile loops); more of it than when they were measured would
+    show there, where nothing overlaps it."""
+    notes = _kernels_of_the_library(importlib.import_module("co-rope_amd._lib").LIB_PATH)
+    found = {n: k[".vgpr_spill_count"] for n, k in notes.items() if re.search(kernels, n)}
+    assert len(found) >= 2 and max(found.values()) <= most, found

@@ -16,9 +16,9 @@ import torch
 
 from . import _lib
 
+# 256 (the largest head dim of the reference, fused_rope_attn.py:661) runs one wave per SIMD, on rotated copies a pipelined forward (bf16; fp16
+# takes the single-launch kernel there) and, like the others, dQ and fused dK+dV.
 _SUPPORTED_D = (64, 128, 256)
-# 256 (the largest head dim of the reference, fused_rope_attn.py:661) runs one wave per SIMD: the single-launch forward
-# kernel (on a rotated key copy from the rotated path's lengths on) and separate dQ, dV and dK kernels.
 _ROTATED_PATH_MAX_D = 256
 # Head dims of the reference (fused_rope_attn.py:661) below the kernels' own: run at D = 64 with each half of a row padded
 # with zeros (the rotation pairs column j with column j + D/2, so the halves must stay the starts of the new halves).
@@ -167,6 +167,15 @@ def _view_strides(t):
     return (ctypes.c_int64 * 3)(sb, sh, sn)
 
 
+def _readable(t):
+    """t, or a copy where the kernels cannot read it where it lies, with its (batch, head, row) strides."""
+    strides = None if t.is_contiguous() else _view_strides(t)
+    if strides is not None:
+        return t, strides
+    _, h, n, d = t.shape
+    return t.contiguous(), (ctypes.c_int64 * 3)(h * n * d, n * d, d)   # (an axis of length 1 may say otherwise)
+
+
 def _route(q, k, causal, keep_rotated, two_launch=None):
     """(rotate K ahead?, keep P and V in fp16 there?) for a forward."""
     B, H, N, D = q.shape
@@ -218,88 +227,24 @@ def _forward(q, k, v, causal, sm_scale, freqs_cos, freqs_sin, two_launch=None, k
     if fc.stride(0) != fs.stride(0):
         fc, fs = fc.contiguous(), fs.contiguous()
     B, H, N, D = q.shape
-    strides = None
-    if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
-        strides = tuple(_view_strides(t) for t in (q, k, v))
-        if any(st is None for st in strides) or D > _ROTATED_PATH_MAX_D:
-            q, k, v, strides = q.contiguous(), k.contiguous(), v.contiguous(), None
-    o = torch.empty(q.shape, device=q.device, dtype=q.dtype)
-    M = torch.empty((B, H, N), device=q.device, dtype=torch.float32)
-    two_launch, exact = _route(q, k, causal, keep_rotated, two_launch)
-    fp16 = q.dtype == torch.float16
-    rotated = None
     Hkv = k.shape[1]
+    (q, q_st), (k, k_st), (v, v_st) = (_readable(t) for t in (q, k, v))
+    two_launch, exact = _route(q, k, causal, keep_rotated, two_launch)
+    empty = lambda shape, dtype=torch.float32: torch.empty(shape, device=q.device, dtype=dtype)
+    ptr = lambda t: None if t is None else t.data_ptr()
     with _on_device(q):
         parts, nbytes = _fwd_parts(lib, q, causal) if two_launch else (None, 0)
-        if strides is None and (parts is not None or (exact and D <= 128)):
-            strides = tuple((ctypes.c_int64 * 3)(h * N * D, N * D, D) for h in (H, Hkv, Hkv))   # (contiguous; an axis of length 1 may say otherwise)
-        if strides is not None:
-            q_rot = torch.empty(q.shape, device=q.device, dtype=q.dtype) if (two_launch and keep_rotated) else None
-            k_rot = torch.empty(k.shape, device=q.device, dtype=q.dtype) if two_launch else None
-            kmax = torch.empty((B, Hkv, (N + 63) // 64), device=q.device, dtype=torch.float32) if (two_launch and not exact) else None
-            rc = lib.corope_rope_attn_fwd_keep(q.data_ptr(), strides[0], k.data_ptr(), strides[1], v.data_ptr(), strides[2],
-                                              fc.data_ptr(), fs.data_ptr(), fc.stride(0), o.data_ptr(), M.data_ptr(),
-                                              q_rot.data_ptr() if q_rot is not None else None,
-                                              k_rot.data_ptr() if k_rot is not None else None,
-                                              kmax.data_ptr() if kmax is not None else None, B, H, Hkv, N, D,
-                                              float(sm_scale), int(bool(causal)), int(fp16),
-                                              parts.data_ptr() if parts is not None else None, nbytes, None, _stream_ptr(q))
-            _lib.check(rc, "corope_rope_attn_fwd_keep")
-            if q_rot is not None:
-                rotated = (q_rot, k_rot)
-        elif q.dtype == torch.float16:
-            # the reference's dtype: one entry point covers the forms, grouped-query K/V included.  With key-norm maxima: the
-            # pipelined kernel (bf16 probabilities against a V converted to bf16 on its way into LDS); without (here D = 256):
-            # the single-launch kernel on the rotated copy, P and V in fp16
-            q_rot = torch.empty_like(q) if (two_launch and keep_rotated) else None
-            k_rot = torch.empty_like(k) if two_launch else None
-            kmax = torch.empty((B, Hkv, (N + 63) // 64), device=q.device, dtype=torch.float32) if (two_launch and not exact) else None
-            rc = lib.corope_rope_attn_fwd_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), fc.data_ptr(), fs.data_ptr(),
-                                              fc.stride(0), o.data_ptr(), M.data_ptr(),
-                                              q_rot.data_ptr() if q_rot is not None else None,
-                                              k_rot.data_ptr() if k_rot is not None else None,
-                                              kmax.data_ptr() if kmax is not None else None, B, H, Hkv, N, D,
-                                              float(sm_scale), int(bool(causal)), _stream_ptr(q))
-            _lib.check(rc, "corope_rope_attn_fwd_f16")
-            if q_rot is not None:
-                rotated = (q_rot, k_rot)
-        elif Hkv != H:   # grouped-query attention: one entry point covers the three forms
-            q_rot = torch.empty_like(q) if (two_launch and keep_rotated) else None
-            k_rot = torch.empty_like(k) if two_launch else None
-            kmax = torch.empty((B, Hkv, (N + 63) // 64), device=q.device, dtype=torch.float32) if two_launch else None
-            rc = lib.corope_rope_attn_fwd_gqa(q.data_ptr(), k.data_ptr(), v.data_ptr(), fc.data_ptr(), fs.data_ptr(),
-                                              fc.stride(0), o.data_ptr(), M.data_ptr(),
-                                              q_rot.data_ptr() if q_rot is not None else None,
-                                              k_rot.data_ptr() if k_rot is not None else None,
-                                              kmax.data_ptr() if kmax is not None else None, B, H, Hkv, N, D,
-                                              float(sm_scale), int(bool(causal)), _stream_ptr(q))
-            _lib.check(rc, "corope_rope_attn_fwd_gqa")
-            if q_rot is not None:
-                rotated = (q_rot, k_rot)
-        elif two_launch and keep_rotated:
-            q_rot, k_rot = torch.empty_like(q), torch.empty_like(k)
-            kmax = torch.empty((B, H, (N + 63) // 64), device=q.device, dtype=torch.float32)
-            rc = lib.corope_rope_attn_fwd_train(q.data_ptr(), k.data_ptr(), v.data_ptr(), fc.data_ptr(), fs.data_ptr(),
-                                                fc.stride(0), o.data_ptr(), M.data_ptr(), q_rot.data_ptr(), k_rot.data_ptr(),
-                                                kmax.data_ptr(), B, H, N, D, float(sm_scale), int(bool(causal)),
-                                                _stream_ptr(q))
-            _lib.check(rc, "corope_rope_attn_fwd_train")
-            rotated = (q_rot, k_rot)
-        elif two_launch:
-            nbytes = lib.corope_rope_attn_fwd_workspace_bytes(B, H, N, D)
-            if nbytes < 0:
-                _lib.check(lib.corope_rope_attn_check(B, H, N, D, fc.stride(0), float(sm_scale), 0), "corope_rope_attn_check")
-            ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-            rc = lib.corope_rope_attn_fwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), fc.data_ptr(), fs.data_ptr(),
-                                             fc.stride(0), o.data_ptr(), M.data_ptr(), B, H, N, D, float(sm_scale),
-                                             int(bool(causal)), ws.data_ptr(), nbytes, _stream_ptr(q))
-            _lib.check(rc, "corope_rope_attn_fwd_ws")
-        else:
-            rc = lib.corope_rope_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), fc.data_ptr(), fs.data_ptr(),
-                                          fc.stride(0), o.data_ptr(), M.data_ptr(), B, H, N, D, float(sm_scale),
-                                          int(bool(causal)), _stream_ptr(q))
-            _lib.check(rc, "corope_rope_attn_fwd")
-    return o, M, fc, fs, rotated
+        o, M = empty(q.shape, q.dtype), empty((B, H, N))
+        q_rot = empty(q.shape, q.dtype) if two_launch and keep_rotated else None
+        k_rot = empty(k.shape, q.dtype) if two_launch else None
+        # with key-norm maxima: the pipelined kernel, for fp16 with bf16 probabilities against a V converted to bf16 on its way into LDS; without:
+        # P and V in fp16, pipelined as well up to D = 128, in the single-launch kernel on the rotated copy at 256
+        kmax = empty((B, Hkv, (N + 63) // 64)) if two_launch and not exact else None
+        rc = lib.corope_rope_attn_fwd_keep(q.data_ptr(), q_st, k.data_ptr(), k_st, v.data_ptr(), v_st, fc.data_ptr(), fs.data_ptr(), fc.stride(0),
+                                           o.data_ptr(), M.data_ptr(), ptr(q_rot), ptr(k_rot), ptr(kmax), B, H, Hkv, N, D, float(sm_scale),
+                                           int(bool(causal)), int(q.dtype == torch.float16), ptr(parts), nbytes, None, _stream_ptr(q))
+    _lib.check(rc, "corope_rope_attn_fwd_keep")
+    return o, M, fc, fs, (None if q_rot is None else (q_rot, k_rot))
 
 
 def _backward_rotated(lib, q_rot, k_rot, v, o, do, M, fc, fs, sm_scale, causal):
@@ -372,6 +317,8 @@ class _FusedRopeAttn(torch.autograd.Function):
         B, H, N, D = q.shape
         if ctx.rotated:   # q, k are the rotated copies the forward kept; dO is read where it lies if its layout allows it
             return _backward_rotated(lib, q, k, v, o, do, M, fc, fs, ctx.sm_scale, ctx.causal)
+        # A forward of which only the tables ask for a gradient kept nothing rotated: the copies are made here.  (Without them, the kernels on unrotated
+        # operands, whose entry points callers of the C ABI have: here only where TRAIN_ROTATED_MIN_ND and TWO_LAUNCH_MIN_N are raised.)
         do = do.contiguous()
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         delta = torch.empty_like(M)

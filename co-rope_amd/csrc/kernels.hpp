@@ -116,6 +116,25 @@ inline int64_t most_tiles_dealt(int64_t n_items, int grid, F&& tiles_of) {
   return most;
 }
 
+// Most items that one of `shares` equal pieces of a list of tiles meets (list: QueryTiles or DkdvTiles, `per` tiles a head).
+template <class Tiles>
+inline int most_items_met(const Tiles& list, int per, int shares) {
+  int most = 1, block = 0;
+  int64_t head = 0, item_end = list.first(1);
+  const auto next_item = [&] {
+    if (++block == list.nb) block = 0, head += per;
+    item_end = head + list.first(block + 1);
+  };
+  for (int w = 1; w <= shares; ++w) {
+    const int64_t end = (int64_t)w * list.total_tiles / shares;
+    int met = 1;
+    for (; item_end < end; next_item()) ++met;
+    if (item_end == end) next_item();
+    most = met > most ? met : most;
+  }
+  return most;
+}
+
 struct FwdParams {
   COROPE_TRACE_FIELD
   const uint16_t* q;

@@ -1049,6 +1049,11 @@ static bool dkdv_small_tiles(int N, int slabs) {
 // shorter), 6 TB/s for the partial sums, 10 us for the launch and the longer change of items.  Backward, whole / cut, B Hq Hkv N at
 // D = 128: 1 32 8 3001 676 / 285 us, 4 8 1 1500 633 / 129, 1 8 8 4096 337 / 244, 1 16 16 2048 181 / 150, and on the other side
 // 2 16 16 2048 182 / 188, 2 40 40 1500 196 / 254.
+// At D = 256 (one wave per SIMD) what is not tiles weighs more: the constants there are those of a fit to both forms' launches at 660 shapes, 1 to 96
+// heads of 200 to 8000 rows, grouped ones among them, with the most items that a piece meets; 3 to 5 % of a launch off at the root mean square.  The form chosen
+// is more than 3 % slower than the other at 9 of them (with the constants of D = 128: 39, by up to 26 %).  dK+dV launch, whole / cut with its sums, B1 H N:
+// causal 1 2048 115 / 32, 4 4096 219 / 126, 10 2048 119 / 103, 10 500 40 / 29, not 24 1500 182 / 150, and on the other side causal 16 2048 123 / 135, 20 1024
+// 68 / 76, 10 4096 236 / 257, not 40 1500 194 / 222.
 template <int D>
 static int dkdv_shares(int N, int slabs, int group, bool causal) {
   constexpr int BM = kDkdvBlockM<D>, CW = kDkdvCutWaves<D>, kMost = 16;
@@ -1063,10 +1068,16 @@ static int dkdv_shares(int N, int slabs, int group, bool causal) {
   const int64_t longest = most_tiles_dealt(n_items, grid, [&](int64_t i) -> int64_t { return group * (m_tiles - (causal ? (int)(i / slabs) * (block / BM) : 0)); });
   const DkdvTiles t((N + CW * 32 - 1) / (CW * 32), slabs, group, m_tiles, causal ? CW * 32 / BM : 0);
   const int shares = std::max(1, std::min(cus, t.total_tiles / 4));
+  const float moved = (float)(shares + std::min<int64_t>(t.nb * (int64_t)slabs, shares)) * kDkdvSlotFloats<D, CW> * 8;
+  if constexpr (D > 128) {
+    const float busy = std::min(1.f, (float)t.total_tiles / ((float)longest * cus));
+    const float whole = 1.9f * longest * (0.75f + 0.25f * busy) + 4.f * ((n_items + grid - 1) / grid) + 11.f;
+    const int tiles = (t.total_tiles + shares - 1) / shares;
+    return (causal ? 2.3f : 1.92f) * tiles + 4.5f * most_items_met(t, t.per_slab, shares) + 11.5f + moved / 9e6f < whole ? shares : 0;
+  }
   const float tile_us = D == 64 ? 1.7f : 3.3f;
   const float busy = std::min(1.f, (float)t.total_tiles * (block == CW * 32 ? 1.f : 2.f) / ((float)longest * cus));
   const float whole = (small ? 0.85f : 1.f) * longest * tile_us * (0.75f + 0.25f * busy);
-  const float moved = (float)(shares + std::min<int64_t>(t.nb * (int64_t)slabs, shares)) * kDkdvSlotFloats<D, CW> * 8;
   const float cut = t.total_tiles * tile_us / shares + 10.f + moved / 6e6f;
   return cut < 0.95f * whole ? shares : 0;
 }
@@ -1137,12 +1148,13 @@ static hipError_t launch_dq_waves(BwdParams p, hipStream_t stream) {
 
 // How many pieces the key tiles of the dQ launch on rotated operands are cut into; 0: whole items.  As dkdv_shares: with few heads the longest
 // whole item (a sequence's last queries, which see all of its keys) sets the time however many compute units are idle.  Measured
-// constants, in microseconds: a tile of a full chip, a change of items (at head dim 256 nothing hides it with one wave per SIMD, and the cut kernel sends
-// 130 registers through scratch there, none in the tile loop), the launch; a causal piece of T tiles crosses up to sqrt(2 T / step) of a head's lightest items
-// (items_crossed), one that is not T / k_tiles (at head dims up to 128, where a change is short, the constants hold with one for less than one).  dQ launch, whole / cut
+// constants, in microseconds: a tile of a full chip, a change of items (items_crossed: at most so many a piece, and one), the launch.  dQ launch, whole / cut
 // with its sums, B1 H N: D = 128: 8 4096 159 / 87, 4 8192 296 / 132, 1 10000 330 / 66, 8 3000 not causal 119 / 80, and on the other side 16 4096 153 / 152, 40 1100 53 / 64; D = 64: 8 4096 63 / 50, 4 16384 276 / 239, 2 3000
-// not causal 46 / 27, 16 1500 27.5 / 28.2; D = 256: 2 2048 112 / 58, 4 4096 212 / 185, 8 2048 115 / 129, 16 2048 124 / 199,
-// not causal 12 4096 435 / 377, 8 1024 66 / 47, and on the other side 40 2304 397 / 451, 32 4096 888 / 973.
+// not causal 46 / 27, 16 1500 27.5 / 28.2.
+// At D = 256 nothing hides a change of items with one wave per SIMD, and the cut kernels send 130 to 147 registers through scratch there (none in the tile
+// loop): the constants are those of a fit as in dkdv_shares, with the most items that a piece meets.  The form chosen is more than 3 % slower than the
+// other at 4 of the 660 shapes (with the constants of the kernels before: 56, by up to 50 %).  Causal 2 2048 92 / 58, 4 1500 73 / 58, 1 1024 54 / 48, and on the other side 3 8000 308 / 367, 4 4096
+// 168 / 187, 8 2048 95 / 131; not causal 4 1024 57 / 43, 12 4096 373 / 341, 24 1500 162 / 148, and on the other side 6 700 45 / 66, 10 2048 103 / 120, 40 1500 171 / 235.
 template <int D>
 static int dq_shares(int N, int BH, bool causal) {
   constexpr int BN = kDqBlockN<D>, CW = kDqCutWaves<D>, kMost = 16;
@@ -1157,13 +1169,20 @@ static int dq_shares(int N, int BH, bool causal) {
   const int64_t longest = most_tiles_dealt(n_items, grid, [&](int64_t i) -> int64_t { return causal ? std::min((nb - (int)(i / BH)) * (block / BN), k_tiles) : k_tiles; });
   const QueryTiles t((N + CW * 32 - 1) / (CW * 32), BH, k_tiles, causal ? CW * 32 / BN : 0);
   const int shares = std::max(1, std::min(cus, t.total_tiles / 4));
-  constexpr float kWholeTile = D == 64 ? 1.25f : D == 128 ? 2.8f : 1.75f, kTile = D == 64 ? 1.5f : D == 128 ? 2.9f : 1.6f;
-  constexpr float kChange = D == 64 ? 3.5f : D == 128 ? 5.f : 21.f;
-  const float busy = std::min(1.f, (float)t.total_tiles * (block == CW * 32 ? 1.f : 2.f) / ((float)longest * cus));
-  const float whole = (small ? 0.85f : 1.f) * longest * kWholeTile * (0.75f + 0.25f * busy) + kChange * ((n_items + grid - 1) / grid);
-  const float tiles = (float)t.total_tiles / shares, crossed = D > 128 && !causal ? tiles / k_tiles : items_crossed(t, tiles);
   const float moved = (float)(shares + std::min<int64_t>(t.nb * (int64_t)BH, shares)) * kDqSlotFloats<D, CW> * 8;
-  const float cut = tiles * kTile + kChange * (1.f + crossed) + 9.f + moved / 12e6f;
+  const int rounds = (int)((n_items + grid - 1) / grid);
+  if constexpr (D > 128) {
+    const float busy = std::min(1.f, (float)t.total_tiles / ((float)longest * cus));
+    const float whole = 1.5f * longest * (0.75f + 0.25f * busy) + 6.4f * rounds + 11.6f;
+    const int tiles = (t.total_tiles + shares - 1) / shares, met = most_items_met(t, t.per_head, shares);
+    const float cut = causal ? 3.5f * tiles + 3.3f * met + 22.f + moved / 3.4e6f : 1.45f * tiles + 21.f * met + 3.f + moved / 5.4e6f;
+    return cut < whole ? shares : 0;
+  }
+  constexpr float kWholeTile = D == 64 ? 1.25f : 2.8f, kTile = D == 64 ? 1.5f : 2.9f, kChange = D == 64 ? 3.5f : 5.f;
+  const float busy = std::min(1.f, (float)t.total_tiles * (block == CW * 32 ? 1.f : 2.f) / ((float)longest * cus));
+  const float whole = (small ? 0.85f : 1.f) * longest * kWholeTile * (0.75f + 0.25f * busy) + kChange * rounds;
+  const float tiles = (float)t.total_tiles / shares;
+  const float cut = tiles * kTile + kChange * (1.f + items_crossed(t, tiles)) + 9.f + moved / 12e6f;
   return cut < 0.9f * whole ? shares : 0;
 }
 

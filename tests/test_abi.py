@@ -357,6 +357,19 @@ def test_rotated_path_rule_answers_for_every_head_dim(pkg):
     assert not rule(300, 96, False, 4) and rule(1024, 96, False, 4) and not rule(5000, 512, False, 4)
 
 
+def test_where_launches_are_cut_at_head_dim_256(pkg):
+    """The rules at D = 256 on either side of their lines, where the two forms were measured apart (256 compute units).  The scratch is the larger of both
+    launches': 256 pieces of dQ take 64 MiB, of dK+dV 128."""
+    lib = pkg._lib.load()
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rules depend on the number of compute units")
+    need = lambda H, N, causal, Hkv=None: lib.corope_rope_attn_bwd_rotated_parts_bytes(1, H, Hkv or H, N, 256, causal) >> 20
+    for H, N, causal in ((1, 2048, 1), (4, 4096, 1), (10, 2048, 1), (16, 500, 1), (10, 500, 0), (8, 2048, 0), (24, 1500, 0), (12, 4096, 0)):
+        assert need(H, N, causal) > 64, (H, N, causal)                          # dK+dV cut
+    for H, N, causal in ((16, 2048, 1), (20, 1024, 1), (20, 1280, 1), (10, 4096, 1), (6, 8000, 1), (12, 3000, 1), (40, 1500, 0), (40, 1500, 1), (16, 3000, 1)):
+        assert need(H, N, causal) == 0, (H, N, causal)                          # nothing cut
+
+
 def test_where_a_forward_alone_takes_rotated_keys(pkg):
     """Both sides of the rule for forwards alone below 1024 rows, at shapes where one path was measured to be the faster (256 compute units)."""
     rule = lambda N, D, slabs, causal=True, kv=None: pkg.rope_attn.use_rotated_path(N, D, False, slabs, kv, causal)

@@ -680,7 +680,7 @@ struct QueryTiles {
 // were cut that should not be.  Whole / cut with its join or sums, us, D = 64: BH 4096 N 64 causal, forward 91 / 133, dQ + dK+dV 145 / 184, N 200 not causal 198 /
 // 230, 396 / 411; D = 128: BH 3072 N 128 not causal 162 / 210, 351 / 379.
 inline float items_crossed(const QueryTiles& t, float tiles) {
-  if (t.step == 0) return std::max(1.f, tiles / t.k_tiles);
+  if (t.step == 0) return std::max(1.f, 0.75f * tiles / t.k_tiles);   // (as launches of 16 to 6000 heads have it; 0.5 cuts too much, 1 leaves one that pays)
   const float heads = std::floor(tiles / t.per_head);
   return heads * t.nb + std::min((float)t.nb, std::sqrt(2.f * (tiles - heads * t.per_head) / t.step));
 }

@@ -345,6 +345,7 @@ def test_short_items_are_not_cut(pkg):
         for causal in (0, 1):
             assert not any(f(B, 32, N, D, causal) for f in (fwd, bwd) for B in (48, 64, 96, 128) for N in (16, 64, 100, 128, 200, 300)), (D, causal)
     assert not fwd(16, 128, 512, 64, 0) and not bwd(16, 96, 300, 128, 0)
+    assert fwd(1, 40, 1660, 128, 0)     # a little more than an item to a piece: 100.5 us whole, 95.4 cut
 
 
 def test_rotated_path_rule_answers_for_every_head_dim(pkg):

@@ -101,11 +101,12 @@ inline unsigned persistent_grid(int64_t n_items, int waves, int lds_bytes) {
 }
 
 // Tiles of the workgroup that a persistent launch deals the most: items come in rounds, heaviest first, every other round from the other end
-// (ItemList).  tiles_of(i): tiles of item i.  Every eighth workgroup is looked at, one per round of the XCDs.
+// (ItemList).  tiles_of(i): tiles of item i.  Every eighth workgroup is looked at, one per round of the XCDs, and the last one, to which a round that runs
+// from the other end deals its first item (the only one to be dealt any, where the last round has one).
 template <class F>
 inline int64_t most_tiles_dealt(int64_t n_items, int grid, F&& tiles_of) {
   int64_t most = 0;
-  for (int w = 0; w < grid; w += 8) {
+  for (int w = 0; w < grid; w = w < grid - 1 && w + 8 >= grid ? grid - 1 : w + 8) {
     int64_t sum = 0;
     for (int r = 0; (int64_t)r * grid < n_items; ++r) {
       const int64_t i = (int64_t)r * grid + ((r & 1) ? grid - 1 - w : w);

@@ -371,6 +371,18 @@ def test_where_launches_are_cut_at_head_dim_256(pkg):
         assert need(H, N, causal) == 0, (H, N, causal)                          # nothing cut
 
 
+def test_a_second_round_of_a_few_items_counts(pkg):
+    """257 to 263 items of equal length on 256 compute units take two rounds, as 264 do: cut into equal pieces they take little more than one (B1 H20 N1600 D256
+    not causal: dQ 169 us whole, 147 cut; dK+dV 187, 153)."""
+    lib = pkg._lib.load()
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rules depend on the number of compute units")
+    need = lambda H, N, D: lib.corope_rope_attn_bwd_rotated_parts_bytes(1, H, H, N, D, 0)
+    assert need(20, 1600, 256) > 0 and need(37, 850, 256) > 0       # 260 and 259 blocks of 128 rows
+    for H, N in ((13, 5120), (26, 2560), (37, 1792), (43, 1536)):   # 260, 260, 259 and 258 of 256 rows
+        assert need(H, N, 128) > 0 and lib.corope_rope_attn_fwd_parts_bytes(1, H, N, 128, 0) > 0, (H, N)
+
+
 def test_where_a_forward_alone_takes_rotated_keys(pkg):
     """Both sides of the rule for forwards alone below 1024 rows, at shapes where one path was measured to be the faster (256 compute units)."""
     rule = lambda N, D, slabs, causal=True, kv=None: pkg.rope_attn.use_rotated_path(N, D, False, slabs, kv, causal)

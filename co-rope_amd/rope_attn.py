@@ -179,12 +179,12 @@ def _readable(t):
 def _route(q, k, causal, keep_rotated, two_launch=None):
     """(rotate K ahead?, keep P and V in fp16 there?) for a forward."""
     B, H, N, D = q.shape
-    asked = two_launch is not None
+    asked, fp16 = two_launch is not None, q.dtype == torch.float16
     if not asked:
-        two_launch = use_rotated_path(N, D, keep_rotated, B * H if q.dtype == torch.bfloat16 or D <= 128 else None, B * k.shape[1], causal,
-                                      _compute_units(q.device.index))
+        two_launch = use_rotated_path(N, D, True) if keep_rotated else use_rotated_path(
+            N, D, False, None if fp16 and D > 128 else B * H, B * k.shape[1], causal, _compute_units(q.device.index))
     # fp16 with gradients, or so short that the fast form's kernel never served it: P and V stay fp16 (no key-norm maxima)
-    return two_launch, (q.dtype == torch.float16 and two_launch and
+    return two_launch, (fp16 and two_launch and
                         (FP16_TRAINING_FORWARD != "fast" if keep_rotated else not asked and not use_rotated_path(N, D, False)))
 
 

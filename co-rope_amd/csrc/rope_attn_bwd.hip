@@ -40,8 +40,8 @@ constexpr int kDkdvBothWaysPad = kStaggerPad;
 //   dK_r^T += Q_r^T dS        (A = Q_r tile read transposed, B = dS)
 // DO_PAD: row padding of the dO tile.  The dV-only kernel reads dO through the transposing load alone and takes the
 // padding that is conflict-free for it (32); the dK kernel reads dO row-wise (8).
-// V_LDS: the waves' V rows live in LDS instead of registers -- the fused dK+dV kernel, whose two sets of accumulators
-// leave no room for them.
+// V_LDS: the waves' V rows live in LDS instead of registers -- the fused dK+dV kernel up to D = 128, whose two sets of accumulators
+// leave no room for them (at D = 256, with one wave per SIMD, they do).
 //
 // Persistent, like the other attention kernels: one workgroup per compute unit walks a balanced list of (key/value slab,
 // key block) items and the stream of query tiles runs on from item to item.  Behind the two tile stages every wave has an

@@ -34,7 +34,8 @@
 // again against its true maximum.  The comparison is issued one MFMA ahead of the branch that waits for it.
 // Two branches a tile cost 1 to 3 % beside the form without; the single-launch kernel on rotated keys, whose comparisons the branches wait
 // for and which starts a workgroup per query block, took, with the rotation pass, B2 H32 N4096 D128 causal 387 us, this 330; B1 H13 N29504 D64
-// 1953 / 1610; few heads, whose blocks this one cuts, B1 H8 N4096 D128 143 / 78.
+// 1953 / 1610; few heads, whose blocks this one cuts, B1 H8 N4096 D128 143 / 78.  Hot logits, where halves outgrow fp16 and are done again, cost either
+// kernel about the same: B2 H32 N4096 D128 at sm_scale 1/sqrt(D) / 0.5 / 1, 357 / 366 / 364 and 320 / 320 / 333 us; B1 H8 N4096 138 / 139 / 140 and 74 / 76 / 81.
 #include "common.hpp"
 #include "kernels.hpp"
 

@@ -104,6 +104,8 @@ def _freq_table(f):
 # 64.3 -> 39.2, B3 Hq64 Hkv32 N64 D64 30.9 -> 26.7, B2 Hq32 Hkv4 N700 D64 299 -> 71, B2 Hq16 Hkv4 N400 D128 243 -> 77, B2 H8 N200
 # D256 133 -> 84, B128 H32 N64 D64 265 -> 249, B512 H32 N16 D64 920 -> 869, B128 H32 N16 D256 1013 -> 571 (from N * D = 65536 on it was before).
 # The forward alone pays the rotation pass's launch (3 to 4 us) and its way through memory (_forward_pays_rotation).
+# What it costs: the rotated q and k beside the caller's own between forward and backward (537 MB at B256 H32 N256 D64, where the step on unrotated
+# operands kept references), and a short forward with gradients whose backward never runs (B4 H8 N300 D64 fp16 9.8 -> 11.6).
 TWO_LAUNCH_MIN_N = 1024
 TRAIN_ROTATED_MIN_ND = 0
 _FWD_ROTATED_MIN_ND = 65536
@@ -120,7 +122,9 @@ def _forward_pays_rotation(N, D, slabs, kv_slabs, causal, cus):
     D = 128, fewer 256-row items than compute units (from there on the unrotated kernel's 256-row form holds out: H128 N300 25.2 -> 26.6): H8 N129
     15.4 -> 14.4, H96 N257 27.4 -> 26.1, H255 N129 not causal 33.0 -> 31.4; causal, up to three blocks of 128 rows, only while those are about one
     round: H128 N160 18.1 -> 18.2; beyond, H160 N160 23.0 -> 26.6, H192 N256 28.4 -> 31.2, H112 N320 28.4 -> 29.9.
-    D = 256: H32 N128 26.1 -> 26.7, N160 35.5 -> 27.1, H255 N129 75.9 -> 48.9."""
+    D = 256: H32 N128 26.1 -> 26.7, N160 35.5 -> 27.1, H255 N129 75.9 -> 48.9.
+    fp16 (D = 64 and 128; the pipelined kernel with P and V in fp16) goes the same way: D = 64 H32 N1000 22.1 -> 21.2, H192 N800 not causal 74.8 -> 67.5; D = 128
+    H32 N160 16.2 -> 14.7, N300 22.5 -> 17.6, and beyond H192 N160 23.4 -> 29.2."""
     items = (N + 255) // 256 * slabs
     if D == 256:
         return N > 128

@@ -237,7 +237,7 @@ int corope_rope_attn_bwd_ws(const void *q, const void *k, const void *v, const v
  * the rotation in its loop and with its own bookkeeping -- P and V stay fp16, as in the reference -- and q_rot as above.
  * Backward: prerotated = 1: q, k are those rotated copies (corope_rope_attn_bwd_rotated without parts); else preprocess + dV + dK + dQ as in corope_rope_attn_bwd, or -- given a workspace of
  * corope_rope_attn_bwd_workspace_bytes (may be NULL) -- the rotation of q and k into it followed by the dQ and the fused
- * dK+dV kernel as in corope_rope_attn_bwd_ws, the faster form from N * D = 65536 on.  `delta` is (B,H,N) fp32 scratch.
+ * dK+dV kernel as in corope_rope_attn_bwd_ws, the faster form at every length.  `delta` is (B,H,N) fp32 scratch.
  * k, v, dk, dv have Hkv heads (H a multiple of Hkv; Hkv = H: the reference's form), as in the grouped-query entry points below.
  * Replaces _attention.forward / .backward (fused-rope/fused_rope_attn.py:655-777) for callers that keep the reference's dtype. */
 int corope_rope_attn_fwd_f16(const void *q, const void *k, const void *v,

@@ -296,9 +296,9 @@ def test_head_dims_below_the_kernels_own(pkg, B, H, N, D, causal):
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("B,Hq,Hkv,N", [(1, 2, 2, 300), (2, 2, 2, 128), (1, 1, 1, 1), (1, 3, 3, 1100), (1, 4, 2, 260), (1, 40, 40, 200)])
 def test_head_dim_256(pkg, monkeypatch, B, Hq, Hkv, N, causal, two_launch):
-    """The largest head dim the reference admits (fused-rope/fused_rope_attn.py:661), one wave per SIMD: the single-launch
-    forward kernel and separate dQ, dV and dK kernels, on the original operands and (two_launch) on copies rotated
-    beforehand; ragged lengths, grouped-query K/V, more items than compute units' worth of one round and fewer."""
+    """The largest head dim the reference admits (fused-rope/fused_rope_attn.py:661), one wave per SIMD: on the original operands
+    the single-launch forward kernel and separate dQ, dV and dK kernels, and (two_launch) on copies rotated beforehand the pipelined forward, dQ and
+    fused dK+dV; ragged lengths, grouped-query K/V, more items than compute units' worth of one round and fewer."""
     D = 256
     print(f"case D=256 B={B} Hq={Hq} Hkv={Hkv} N={N} causal={causal} two_launch={two_launch}", flush=True)
     _force_path(monkeypatch, pkg, two_launch)
